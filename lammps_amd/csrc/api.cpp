@@ -233,17 +233,17 @@ int mdx_create(int device, mdx_ctx **out) {
     delete c;
     return hip_fail(e, "stream");
   }
-  if (hipMalloc(&c->dflags_base, 128) != hipSuccess || hipMalloc(&c->red_out, sizeof(double) * MDX_RED_SLOTS) != hipSuccess ||
+  if (hipMalloc(&c->dflags_base, sizeof(int) * 2 * kFlagWords) != hipSuccess || hipMalloc(&c->red_out, sizeof(double) * MDX_RED_SLOTS) != hipSuccess ||
       hipHostMalloc(&c->red_host, sizeof(double) * MDX_RED_SLOTS, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&c->trig_host, 64, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
-      hipHostMalloc(&c->bflags_host, 64, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc(&c->bflags_host, sizeof(int) * kFlagInts, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
       hipMalloc(&c->trig_dev, 64) != hipSuccess || hipMalloc(&c->lj_dev, sizeof(LJTab)) != hipSuccess) {
     set_error("Insufficient memory on accelerator");
     return MDX_ERR_NOMEM;
   }
   memset(c->trig_host, 0, 64);
   c->dflags = c->dflags_base;
-  if (hipMemset(c->dflags_base, 0, 128) != hipSuccess || hipMemset(c->trig_dev, 0, 64) != hipSuccess ||
+  if (hipMemset(c->dflags_base, 0, sizeof(int) * 2 * kFlagWords) != hipSuccess || hipMemset(c->trig_dev, 0, 64) != hipSuccess ||
       hipEventCreateWithFlags(&c->step_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->build_ev, hipEventDisableTiming) != hipSuccess) {
     set_error("device flags initialisation failed");

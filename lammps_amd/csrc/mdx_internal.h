@@ -41,6 +41,17 @@
 
 namespace mdx {
 
+// Build flags of one list build: kFlagInts words ([0] largest row, [4] lost
+// atom, [5] bin overflow, [8..9] 64-bit entry total), then kListSlots
+// counters of the list pass, each on a cache line of its own.
+struct ListSlot {
+  int most, pad;            // largest row the slot's workgroups saw
+  unsigned long long sum;   // entries they listed
+  int line[12];
+};
+constexpr int kFlagInts = 16, kListSlots = 256;
+constexpr int kFlagWords = kFlagInts + kListSlots * (int)(sizeof(ListSlot) / sizeof(int));
+
 // Bin geometry of the reference's Neighbor::setup_bins (neighbor.cpp:1538-1702),
 // used only to decide which side of a periodic pair the reference would
 // have evaluated the distance from (matters only at exact cutoff ties).
@@ -358,7 +369,7 @@ struct mdx_ctx {
   double skin = 0.3;
   int every = 1, delay = 10, check = 1, one = 2000;
   double triggersq = 0.0225, cutneighmax = 0.0;
-  // dflags: [0] max count, [4] lost atom, [8..9] 64-bit neighbour total
+  // dflags: kFlagWords words of the current build (see kFlagInts)
   int *nbr = nullptr, *numneigh = nullptr, *dflags = nullptr;
   // ghost-shell exchange (halo.hip): per swap, the device indices of the
   // atoms to send (valid until the next list build) and their image shift
@@ -406,7 +417,7 @@ struct mdx_ctx {
   int *trig_host = nullptr;
   int *trig_dev = nullptr;       // device copy of the trigger word
   int *bflags_host = nullptr;    // pinned copy of the last build's flags
-  int *dflags_base = nullptr;    // two halves of 16 build flags (null: dflags alone, cleared per build)
+  int *dflags_base = nullptr;    // two sets of kFlagWords build flags (null: dflags alone, cleared per build)
   bool flags_dirty = false;      // a build started and did not pass its flags check
   bool bins_dirty = true;        // bin counters not known to be clear
   hipEvent_t build_ev = nullptr; // recorded after that copy

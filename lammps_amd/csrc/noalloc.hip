@@ -46,7 +46,7 @@ constexpr size_t kPerAtomBytes = align_up(sizeof(double4) * kAtoms) * 6 +  // x,
                                  align_up(sizeof(int4) * kAtoms) * 2;       // xq, xqb
 constexpr size_t kScratchBytes = kPerAtomBytes + align_up(sizeof(int) * kListEntries) +
                                  align_up(sizeof(int) * kBins) * 2 + align_up(sizeof(double) * kPartials) +
-                                 kScanBytes + align_up(64) + align_up(sizeof(double) * MDX_RED_SLOTS);
+                                 kScanBytes + align_up(sizeof(int) * kFlagWords) + align_up(sizeof(double) * MDX_RED_SLOTS);
 static_assert(kScratchBytes <= (size_t)MDX_NOALLOC_SCRATCH_BYTES, "scratch layout exceeds its stated size");
 
 }  // namespace
@@ -235,7 +235,7 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
   s.cap_partials = (long)kPartials;
   s.scan_tmp = cv.take<unsigned char>(kScanBytes);
   s.scan_tmp_bytes = kScanBytes;
-  s.dflags = cv.take<int>(16);
+  s.dflags = cv.take<int>(kFlagWords);
   s.red_out = cv.take<double>(MDX_RED_SLOTS);
   if ((size_t)(cv.p - base) > (size_t)MDX_NOALLOC_SCRATCH_BYTES) {
     set_error("mdx_compute_noalloc: scratch layout overrun");
