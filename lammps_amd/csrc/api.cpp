@@ -237,7 +237,7 @@ int mdx_create(int device, mdx_ctx **out) {
       hipHostMalloc(&c->red_host, sizeof(double) * MDX_RED_SLOTS, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&c->trig_host, 64, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
       hipHostMalloc(&c->bflags_host, sizeof(int) * kFlagInts, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
-      hipMalloc(&c->trig_dev, 64) != hipSuccess || hipMalloc(&c->lj_dev, sizeof(LJTab)) != hipSuccess) {
+      hipMalloc(&c->trig_dev, 64) != hipSuccess || hipMalloc(&c->na_dev, sizeof(NeighArgs)) != hipSuccess || hipMalloc(&c->lj_dev, sizeof(LJTab)) != hipSuccess) {
     set_error("Insufficient memory on accelerator");
     return MDX_ERR_NOMEM;
   }
@@ -263,7 +263,7 @@ int mdx_destroy(mdx_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_atoms(c);
-  void *ptrs[] = {c->dflags_base, c->trig_dev, c->red_out, c->lj_dev, c->eam_tab, c->eam_tab_f, c->eam_pk, c->eam_pk_f, c->bin_count, c->bin_start,
+  void *ptrs[] = {c->dflags_base, c->trig_dev, c->na_dev, c->red_out, c->lj_dev, c->eam_tab, c->eam_tab_f, c->eam_pk, c->eam_pk_f, c->bin_count, c->bin_start,
                   c->scan_tmp};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);

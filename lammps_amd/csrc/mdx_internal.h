@@ -361,6 +361,7 @@ struct mdx_ctx {
   // bins / sort
   int nbins = 0, cap_bins = 0;
   mdx::NeighArgs na{};
+  mdx::NeighArgs *na_dev = nullptr;  // device copy of the current build's (its first kernel writes it)
   unsigned *bkey = nullptr, *bkey_s = nullptr;
   int *bidx = nullptr, *bidx_s = nullptr, *bin_count = nullptr, *bin_start = nullptr;
   void *scan_tmp = nullptr;

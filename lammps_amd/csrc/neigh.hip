@@ -8,8 +8,8 @@
 // box (Domain::pbc, src/domain.cpp:478), binned on the reference's own bin
 // grid (binsize = cutneigh/2, src/neighbor.cpp:1580-1620), and stably
 // sorted by bin (counting sort: arrival slots, then ranks by atom index)
-// so that every x-row of bins is one contiguous atom range.  One lane per
-// atom then scans the 5x5 rows of its stencil (each row at most 3
+// so that every x-row of bins is one contiguous atom range.  One lane
+// per atom (32 lanes in systems too small to fill the chip that way) then scans the 5x5 rows of its stencil (each row at most 3
 // contiguous segments: wrapped-low, main, wrapped-high; k_build_flat takes
 // them a plane at a time as one candidate stream) and keeps j iff
 // rsq <= cutneighsq, with the rsq the reference computes for a ghost atom:
@@ -156,9 +156,9 @@ __device__ __forceinline__ void stage_band(const NeighArgs &a, float *lo, float 
 
 // The list pass's largest row and entry total: each workgroup adds into one
 // of kListSlots counters, k_build_flags combines them.  Atomics on one
-// address complete one after the other, ~12 ns each on the eight XCDs, so a
-// single pair of words (two atomics per wavefront) is 0.1 ms at 256,000
-// atoms and 0.77 ms at 2.048 M: builds 224 -> 163 us and 1061 -> 934 us.
+// address complete one after the other, ~12 ns each on the eight XCDs: a
+// single pair of words took 0.77 ms of the 0.95 ms list pass at 2.048 M
+// atoms (64,000 of them), and 50 us at 32,000 atoms with one per workgroup.
 __device__ __forceinline__ void count_rows(ListSlot *slots, int most, unsigned long long sum) {
   ListSlot &s = slots[blockIdx.x % kListSlots];
   atomicMax(&s.most, most);
@@ -197,16 +197,31 @@ __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ df
   host[threadIdx.x] = v;
 }
 
+// The fixed-point position of a list entry's atom: a 32-bit byte offset from
+// the array's base (index < 2^27, 16 B each), so the address stays in one
+// register and the base in scalar registers.
+__device__ __forceinline__ int4 gather_q(const int4 *__restrict__ xq, unsigned entry) {
+  return *reinterpret_cast<const int4 *>(reinterpret_cast<const char *>(xq) + ((entry << 5) >> 1));
+}
+
 // Domain::pbc + bin index + histogram; one thread per atom.  slot[i] is the
 // atom's arrival order in its bin (not deterministic; k_bin_rank orders
 // each bin by atom index).  Atoms arrive nearly bin-sorted (the previous
 // build's order), so the lanes of a wavefront with equal bins form runs: one
 // returning atomic per run reserves the run's slots, and no two lanes of a
 // wavefront hit one counter.
+// The build's arguments also go to device memory (args): the list pass reads
+// the few that only its rare exact test needs from there, where they cost no
+// registers (as kernel arguments the compiler held them in spilled scalar
+// registers through the candidate loop).  With gather_q: builds 2-8% faster.
 __global__ void k_wrap_bin(NeighArgs a, double4 *__restrict__ x, int *__restrict__ image,
                            unsigned *__restrict__ key, int *__restrict__ slot, int *__restrict__ count,
-                           int *__restrict__ dflags) {
+                           int *__restrict__ dflags, NeighArgs *__restrict__ args) {
+  static_assert(sizeof(NeighArgs) % sizeof(int) == 0, "copied by words");
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < (int)(sizeof(NeighArgs) / sizeof(int)); k += blockDim.x)
+      reinterpret_cast<int *>(args)[k] = reinterpret_cast<const int *>(&a)[k];
   const int lane = threadIdx.x & 63;
   unsigned b = 0xffffffffu;  // past the end: its own run, no atomic
   if (i < a.n) {
@@ -564,7 +579,8 @@ __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(Neigh
                                                    const int4 *__restrict__ xq, QStep qs,
                                                    const unsigned *__restrict__ bkey,
                                                    const int *__restrict__ bin_start, int *__restrict__ nbr,
-                                                   int *__restrict__ numneigh, ListSlot *__restrict__ slots, FlatConst fc) {
+                                                   int *__restrict__ numneigh, ListSlot *__restrict__ slots, FlatConst fc,
+                                                   const NeighArgs *__restrict__ ax) {
   __shared__ double s_cut[MDX_NT1 * MDX_NT1];
   __shared__ float s_lo[Q ? MDX_NT1 * MDX_NT1 : 1], s_hi[Q ? MDX_NT1 * MDX_NT1 : 1];
   __shared__ double s_cmax[MDX_NT1];
@@ -714,9 +730,8 @@ __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(Neigh
         int4 qj[Q ? kLaneU : 1];
 #pragma unroll
         for (int u = 0; u < kLaneU; u++) {
-          const int j = eu[u] & MDX_IDX_MASK;
-          if constexpr (Q) qj[u] = xq[j];
-          else xj[u] = x[j];
+          if constexpr (Q) qj[u] = gather_q(xq, eu[u]);
+          else xj[u] = x[eu[u] & MDX_IDX_MASK];
         }
 #pragma unroll
         for (int u = 0; u < kLaneU; u++) {
@@ -733,8 +748,8 @@ __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(Neigh
             keep = valid && rq <= lo;
             if (valid && !keep && rq <= hi) {
               double shx, shy, shz;
-              code_shift(a, code, shx, shy, shz);
-              keep = keep_exact(a, xi, x[eu[u] & MDX_IDX_MASK], shx, shy, shz, code, ONE ? c_cut : s_cut[t]);
+              code_shift(*ax, code, shx, shy, shz);
+              keep = keep_exact(*ax, x[i], x[eu[u] & MDX_IDX_MASK], shx, shy, shz, code, ONE ? c_cut : s_cut[t]);
             }
           } else {
             double shx, shy, shz;
@@ -765,6 +780,237 @@ __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(Neigh
   count_rows(slots, cnt, (unsigned long long)cnt);
 }
 
+// The list build with a group of 32 lanes per atom, for systems too small to
+// fill the chip with one lane each.  k_build_flat's time is one lane's serial
+// walk of its candidates, 95-150 us (the denser, the longer) whatever the
+// atom count, until every SIMD holds a few of its wavefronts.  Here a group
+// shares one atom: each lane forms the bin ranges of one row of the 5x5
+// stencil rows, in scan order, and reads their bin_start entries, all rows in
+// one memory latency; a scan over the lanes gives each row's place in the
+// atom's candidate sequence, and the lanes write the sequence (list entries
+// j | code << MDX_IDX_BITS) to LDS; then the group tests candidates 32 at a
+// time, kGroupU gathers in flight, and a ballot gives each accepted entry its
+// place in the row.  Candidate order, keep test and tie rule are
+// k_build_flat's: the rows are entry for entry the same.  A group lies in one
+// wavefront, so its LDS exchange needs no barrier.  Sequences longer than
+// kGroupCand (about 200 candidates on the lj/cut melt, 290 on the denser
+// Kob-Andersen mixture) are taken in windows of that length.
+// It is bound by latency below ~30,000 atoms and by VALU issue above (about
+// 350 instructions per atom, k_build_flat 250).  Whole build, this against
+// k_build_flat: lj/cut 500 atoms 32 against 132 us, 32,000 atoms 55 against
+// 119, 107,880 (eam) 105 against 129, 157,216 135 against 144, 186,624 151
+// against 142; Kob-Andersen 8,000 atoms 40 against 184, 195,112 210 against
+// 215.  16 lanes per atom (two rows each) gain 3% from 100,000 atoms and lose
+// 20% at 8,000; 64 lose at every size; six wavefronts per SIMD (spills) lose
+// 7%.  The grid is capped (persistent tiles): one row count per workgroup
+// goes to the slots at its end, not one per tile.
+constexpr int kGroupMaxAtoms = 163840;  // 2.5 wavefronts of k_build_flat per SIMD
+constexpr int kGroupLanes = 32;
+constexpr int kGroupU = 4;
+constexpr int kGroupBlock = 256;
+constexpr int kGroupGrid = 2048;   // 8 workgroups per CU
+constexpr int kGroupCand = 384;    // candidates of a group's LDS window
+template <bool Q, bool ONE>
+__global__ __launch_bounds__(kGroupBlock, 5) void k_build_group(NeighArgs a, const double4 *__restrict__ x,
+                                                   const int4 *__restrict__ xq, QStep qs,
+                                                   const int *__restrict__ bin_start, int *__restrict__ nbr,
+                                                   int *__restrict__ numneigh, ListSlot *__restrict__ slots, FlatConst fc,
+                                                   const NeighArgs *__restrict__ ax) {
+  constexpr int GL = kGroupLanes, NG = kGroupBlock / GL;  // lanes per atom, atoms per block
+  constexpr int RPL = (kFlatRows * kFlatRows + GL - 1) / GL;  // stencil rows per lane
+  __shared__ double s_cut[ONE ? 1 : MDX_NT1 * MDX_NT1];
+  __shared__ float s_lo[Q && !ONE ? MDX_NT1 * MDX_NT1 : 1], s_hi[Q && !ONE ? MDX_NT1 * MDX_NT1 : 1];
+  __shared__ double s_cmax[ONE ? 1 : MDX_NT1];
+  __shared__ int s_cand[NG * kGroupCand];
+  __shared__ int s_max[NG], s_sum[NG];
+  if constexpr (!ONE) {
+    if constexpr (Q) stage_band(a, s_lo, s_hi);
+    stage_cmax(a, s_cmax);
+    stage_cutneighsq(a, s_cut);
+  }
+  const int lane = threadIdx.x % GL, grp = threadIdx.x / GL;
+  const int sub = (threadIdx.x & 63) / GL * GL;  // first lane of the group in its wavefront
+  const unsigned long long gmask = ((GL == 64 ? 0ull : (1ull << (GL & 63))) - 1ull) << sub;
+  int *const cand = s_cand + grp * kGroupCand;
+  const int nbx = a.nbin[0], nby = a.nbin[1], nbz = a.nbin[2];
+  // tiles of NG atoms, each XCD taking a contiguous range of them, its
+  // workgroups side by side
+  const int tiles = (a.n + NG - 1) / NG, per_xcd = (tiles + kXCD - 1) / kXCD;
+  const int xcd = blockIdx.x % kXCD, step = gridDim.x / kXCD;
+  int most = 0, sum = 0;
+  for (int tt = blockIdx.x / kXCD; tt < per_xcd; tt += step) {
+    const int i = (xcd * per_xcd + tt) * NG + grp;
+    const bool live = i < a.n;
+    const double4 xi = x[live ? i : 0];
+    const int ti = static_cast<int>(xi.w);
+    int4 qi = make_int4(0, 0, 0, 0);
+    if constexpr (Q) qi = xq[live ? i : 0];
+    // the bin of the atom as k_wrap_bin formed it, and its place in bins
+    const double bx = (xi.x - a.lo[0]) * a.bininv[0], by = (xi.y - a.lo[1]) * a.bininv[1],
+                 bz = (xi.z - a.lo[2]) * a.bininv[2];
+    const int ix = min(max(static_cast<int>(bx), 0), nbx - 1), iy = min(max(static_cast<int>(by), 0), nby - 1),
+              iz = min(max(static_cast<int>(bz), 0), nbz - 1);
+    const float tx = static_cast<float>(bx), ty = static_cast<float>(by), tz = static_cast<float>(bz);
+    const float reach = ONE ? fc.reach : static_cast<float>(s_cmax[ONE ? 0 : ti] * (1.0 + 1e-4));
+    const int prune = fc.prune;
+    const int self = i | (MDX_NOSHIFT << MDX_IDX_BITS);
+    unsigned blo[RPL][2], bhi[RPL][2], tag[RPL][2];
+#pragma unroll
+    for (int q = 0; q < RPL; q++) {
+      const int r = lane * RPL + q;
+      const int dz = r / kFlatRows - kFlatRows / 2, dy = r % kFlatRows - kFlatRows / 2;
+      blo[q][0] = bhi[q][0] = blo[q][1] = bhi[q][1] = 0u;  // empty
+      tag[q][0] = tag[q][1] = 0u;
+      if (!live || r >= kFlatRows * kFlatRows || dz < -a.S[2] || dz > a.S[2] || dy < -a.S[1] || dy > a.S[1]) continue;
+      const float gz = (dz > 0 ? (iz + dz) - tz : dz < 0 ? tz - (iz + dz + 1) : 0.0f) - 1e-3f;
+      const float gy = (dy > 0 ? (iy + dy) - ty : dy < 0 ? ty - (iy + dy + 1) : 0.0f) - 1e-3f;
+      const float dz2 = gz > 0.0f ? gz * gz * fc.bsz * fc.bsz : 0.0f;
+      const float dyz2 = dz2 + (gy > 0.0f ? gy * gy * fc.bsy * fc.bsy : 0.0f);
+      if (prune && dyz2 > reach) continue;
+      int jz = iz + dz, sz = 0, jy = iy + dy, sy = 0;
+      if (jz < 0) {
+        if (!a.periodic[2]) continue;
+        jz += nbz;
+        sz = -1;
+      } else if (jz >= nbz) {
+        if (!a.periodic[2]) continue;
+        jz -= nbz;
+        sz = 1;
+      }
+      if (jy < 0) {
+        if (!a.periodic[1]) continue;
+        jy += nby;
+        sy = -1;
+      } else if (jy >= nby) {
+        if (!a.periodic[1]) continue;
+        jy -= nby;
+        sy = 1;
+      }
+      const unsigned rowbase = static_cast<unsigned>(bin_row(a, jy, jz) * nbx);
+      int x0 = ix - a.S[0], x1 = ix + a.S[0];
+      if (prune == 1) {
+        const float wb = sqrtf(reach - dyz2) * fc.binx + 1e-3f;
+        x0 = max(x0, static_cast<int>(ceilf(tx - 1.0f - wb)));
+        x1 = min(x1, static_cast<int>(floorf(tx + wb)));
+      }
+      const int cyz = 3 * (sy + 1) + 9 * (sz + 1);
+      const int mlo = max(x0, 0), mhi = min(x1, nbx - 1);
+      const bool wlo = x0 < 0 && a.periodic[0], whi = x1 >= nbx && a.periodic[0];
+      // the main piece (tag 1 + cyz), and before it a piece wrapped below
+      // bin 0 or after it one wrapped above nbx - 1 (2S <= nbx: not both)
+      const unsigned m0 = mlo <= mhi ? rowbase + mlo : rowbase, m1 = mlo <= mhi ? rowbase + mhi + 1 : rowbase;
+      const int p = wlo ? 1 : 0;
+      blo[q][0] = p ? rowbase + (x0 + nbx) : m0;
+      bhi[q][0] = p ? rowbase + nbx : m1;
+      tag[q][0] = static_cast<unsigned>(p ? cyz : 1 + cyz) << MDX_IDX_BITS;
+      blo[q][1] = p ? m0 : whi ? rowbase : 0u;
+      bhi[q][1] = p ? m1 : whi ? rowbase + (x1 - nbx) + 1 : 0u;
+      tag[q][1] = static_cast<unsigned>(p ? 1 + cyz : 2 + cyz) << MDX_IDX_BITS;
+    }
+    int jlo[RPL][2], len[RPL][2], mine = 0;
+#pragma unroll
+    for (int q = 0; q < RPL; q++)
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        jlo[q][p] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(bin_start) + blo[q][p] * 4u);
+        len[q][p] = *reinterpret_cast<const int *>(reinterpret_cast<const char *>(bin_start) + bhi[q][p] * 4u) - jlo[q][p];
+        mine += len[q][p];
+      }
+    int incl = mine;
+#pragma unroll
+    for (int off = 1; off < GL; off <<= 1) {
+      const int up = __shfl_up(incl, off, GL);
+      if (lane >= off) incl += up;
+    }
+    const int total = __shfl(incl, GL - 1, GL);
+    const int first = incl - mine;
+    int cnt = 0;
+    for (int w = 0; w < total; w += kGroupCand) {
+      const int wn = min(total - w, kGroupCand);
+      int at = first - w;
+#pragma unroll
+      for (int q = 0; q < RPL; q++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+          const int t0 = max(0, -at), t1 = min(len[q][p], kGroupCand - at);
+          const unsigned e0 = static_cast<unsigned>(jlo[q][p]) | tag[q][p];
+          for (int t = t0; t < t1; t++) cand[at + t] = static_cast<int>(e0 + t);
+          at += len[q][p];
+        }
+      // the entries that other lanes of the wavefront read next are written
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int c0 = lane; c0 - lane < wn; c0 += GL * kGroupU) {
+        int e[kGroupU];
+        double4 xj[Q ? 1 : kGroupU];
+        int4 qj[Q ? kGroupU : 1];
+#pragma unroll
+        for (int u = 0; u < kGroupU; u++) {
+          const int c = c0 + u * GL;
+          e[u] = c < wn ? cand[c] : self;  // past the end: the atom itself, rejected below
+        }
+#pragma unroll
+        for (int u = 0; u < kGroupU; u++) {
+          if constexpr (Q) qj[u] = gather_q(xq, e[u]);
+          else xj[u] = x[e[u] & MDX_IDX_MASK];
+        }
+#pragma unroll
+        for (int u = 0; u < kGroupU; u++) {
+          const bool valid = e[u] != self;
+          const int code = static_cast<int>(static_cast<unsigned>(e[u]) >> MDX_IDX_BITS);
+          bool keep;
+          if constexpr (Q) {
+            const float dx = static_cast<float>(static_cast<int>((unsigned)qi.x - (unsigned)qj[u].x)) * qs.s[0];
+            const float dy = static_cast<float>(static_cast<int>((unsigned)qi.y - (unsigned)qj[u].y)) * qs.s[1];
+            const float dz = static_cast<float>(static_cast<int>((unsigned)qi.z - (unsigned)qj[u].z)) * qs.s[2];
+            const float rq = dx * dx + dy * dy + dz * dz;
+            const int t = ONE ? 0 : ti * a.ntypes1 + qj[u].w;
+            const float lo = ONE ? fc.c_lo : s_lo[ONE ? 0 : t], hi = ONE ? fc.c_hi : s_hi[ONE ? 0 : t];
+            keep = valid && rq <= lo;
+            if (valid && !keep && rq <= hi) {
+              double shx, shy, shz;
+              code_shift(*ax, code, shx, shy, shz);
+              keep = keep_exact(*ax, x[i], x[e[u] & MDX_IDX_MASK], shx, shy, shz, code, ONE ? fc.c_cut : s_cut[ONE ? 0 : t]);
+            }
+          } else {
+            double shx, shy, shz;
+            code_shift(a, code, shx, shy, shz);
+            const double c = ONE ? fc.c_cut : s_cut[ONE ? 0 : ti * a.ntypes1 + static_cast<int>(xj[u].w)];
+            keep = valid && keep_exact(a, xi, xj[u], shx, shy, shz, code, c);
+          }
+          const unsigned long long m = __ballot(keep) & gmask;
+          if (keep) {
+            // accepted lanes of the group before this one
+            const int k = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+            if (k < a.maxneigh) nbr[list_index(i, k, a.npad)] = e[u];
+          }
+          cnt += __popcll(m);
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the window is read before it is written again
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if (live && lane == 0) numneigh[i] = cnt;
+    most = max(most, cnt);
+    sum += cnt;
+  }
+  if (lane == 0) {
+    s_max[grp] = most;
+    s_sum[grp] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long all = 0;
+    for (int g = 0; g < NG; g++) {
+      most = max(most, s_max[g]);
+      all += (unsigned long long)s_sum[g];
+    }
+    count_rows(slots, most, all);
+  }
+}
+
 // The fixed-point build needs the mirror (written by k_permute just before
 // the build, in either precision, where its resolution fits the band; mixed
 // precision also keeps it current between builds for its gathers) and a
@@ -786,7 +1032,7 @@ void launch_build(mdx_ctx *c) {
     hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bkey_s, c->bin_start, c->nbr,
                        c->numneigh, slots);
   };
-  // the flat build takes stencils of at most 5x5 rows with at most two
+  // the group and flat builds take stencils of at most 5x5 rows with at most two
   // pieces per row (no row wraps around the box at both ends: a row spans
   // 2S+1 bins).  Larger stencils come from bins thinner than half the
   // cutoff, in a box dimension below it (one bin): the per-row build.
@@ -810,8 +1056,21 @@ void launch_build(mdx_ctx *c) {
     }
     auto goflat = [&](auto kernel, const int4 *xq) {
       hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bkey_s, c->bin_start,
-                         c->nbr, c->numneigh, slots, fc);
+                         c->nbr, c->numneigh, slots, fc, c->na_dev);
     };
+    if (c->n <= kGroupMaxAtoms) {
+      constexpr int per = kGroupBlock / kGroupLanes;
+      const int Gg = std::min(xcd_grid((c->n + per - 1) / per), kGroupGrid);
+      auto gogroup = [&](auto kernel, const int4 *xq) {
+        hipLaunchKernelGGL(kernel, dim3(Gg), dim3(kGroupBlock), 0, c->stream, c->na, c->x, xq, qs, c->bin_start,
+                           c->nbr, c->numneigh, slots, fc, c->na_dev);
+      };
+      if (q && one) gogroup(k_build_group<true, true>, c->xq);
+      else if (q) gogroup(k_build_group<true, false>, c->xq);
+      else if (one) gogroup(k_build_group<false, true>, nullptr);
+      else gogroup(k_build_group<false, false>, nullptr);
+      return;
+    }
     if (q && one) goflat(k_build_flat<true, true>, c->xq);
     else if (q) goflat(k_build_flat<true, false>, c->xq);
     else if (one) goflat(k_build_flat<false, true>, nullptr);
@@ -946,7 +1205,7 @@ int neigh_build_launch(mdx_ctx *c) {
   if (c->bins_dirty && (e = hipMemsetAsync(c->bin_count, 0, sizeof(int) * (c->nbins + 1), c->stream)) != hipSuccess)
     return hip_fail(e, "memset bins");
   hipLaunchKernelGGL(k_wrap_bin, dim3(G), dim3(B), 0, c->stream, a, c->x, c->image, c->bkey, c->bidx,
-                     c->bin_count, c->dflags);
+                     c->bin_count, c->dflags, c->na_dev);
   c->bins_dirty = true;  // until the scatter pass clears them
   // stable sort of (bin, current index): bin_start from the counts, then
   // scatter by arrival slot and rank within each bin (deterministic order)

@@ -285,6 +285,45 @@ def test_crowded_bin_gives_the_oracle_pair_set(prec):
     ctx.close()
 
 
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("n", [163839, 163840, 163841])
+def test_list_on_both_sides_of_the_build_size_line_matches_the_oracle(n, fmt):
+    """Around 163,840 atoms the build changes from 32 lanes per atom to one:
+    two types, a closed y dimension, an odd last atom, FP64 and fixed-point
+    candidates; the pair set equals the oracle's."""
+    from lammps_amd import mdx
+    cells = (35, 34, 35)
+    rng = np.random.default_rng(5)
+    lo, hi, x = mdx.lattice("fcc", 0.8442, "lj", (0, 0, 0), cells)
+    x = x[rng.permutation(len(x))[:n]] + rng.uniform(-0.1, 0.1, (n, 3))
+    lo, hi = np.asarray(lo).copy(), np.asarray(hi).copy()
+    x[:, 0::2] = np.mod(x[:, 0::2], hi[0::2])
+    lo[1], hi[1] = -0.5, hi[1] + 0.5
+    t = np.where(rng.random(n) < 0.2, 2, 1).astype(np.int32)
+    coeffs = {(1, 1): (1.0, 1.0, 2.5), (1, 2): (1.5, 0.8, 2.0), (2, 2): (0.5, 0.88, 2.2)}
+    ref = M.Ref(M.LJ)
+    ref.box(lo, hi, (1, 0, 1), ntypes=2)
+    ref.add_atoms(x, t)
+    ref.mass(1, 1.0)
+    ref.mass(2, 1.0)
+    ref.pair_lj(2.5)
+    for (i, j), (e, s, c) in coeffs.items():
+        ref.pair_coeff(i, j, e, s, c)
+    ref.neighbor(0.3)
+    ref.setup()
+    ctx = mdx.Context(0)
+    ctx.set_box(lo, hi, (1, 0, 1))
+    ctx.set_atoms(x, t, np.array([0.0, 1.0, 1.0]), tags=np.arange(1, n + 1))
+    ctx.pair_lj_from_coeffs(2, coeffs)
+    ctx.position_format(fmt)
+    ctx.neigh_modify(0.3)
+    ctx.neigh_build()
+    got, want = (np.sort(np.asarray(p, dtype=np.int64), axis=1) for p in (ctx.neigh_pairs(), ref.list_pairs()))
+    assert ctx.stats()["total_neighbors"] == 2 * len(want)
+    assert np.array_equal(np.sort(got[:, 0] << 32 | got[:, 1]), np.sort(want[:, 0] << 32 | want[:, 1]))
+    ctx.close()
+
+
 def test_collapsed_bin_is_reported_as_overflow():
     """2500 atoms in one bin with one = 2000: every one of them has more than
     `one` neighbours, the reference's "Neighbor list overflow"
