@@ -881,16 +881,17 @@ int mdx_set_launch(mdx_ctx *c, int block, int tpa) {
     set_error("threads per atom must be one of 1, 2, 4, 8, 16, 32");
     return MDX_ERR_ARG;
   }
-  c->launch.block = block ? block : 256;
-  c->launch.tpa = tpa ? tpa : 8;
+  c->launch.block = block;
+  c->launch.tpa = tpa;
   return MDX_OK;
 }
 
 int mdx_get_launch(mdx_ctx *c, int *block, int *tpa) {
   int rc = check_ctx(c);
   if (rc) return rc;
-  if (block) *block = c->launch.block;
-  if (tpa) *tpa = c->launch.tpa;
+  const mdx::Launch l = pair_launch(c);
+  if (block) *block = l.block;
+  if (tpa) *tpa = l.tpa;
   return MDX_OK;
 }
 

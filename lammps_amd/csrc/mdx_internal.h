@@ -247,6 +247,19 @@ __device__ __forceinline__ int4 quantize(const QScale &q, const double4 &p) {
   return make_int4(qcoord(p.x, q.lo[0], q.scale[0]), qcoord(p.y, q.lo[1], q.scale[1]),
                    qcoord(p.z, q.lo[2], q.scale[2]), static_cast<int>(p.w));
 }
+// The position of a list entry's atom, fixed point or FP64: a 32-bit byte
+// offset from the array's base (index < 2^27, 16 or 32 B each; the image code
+// in bits 27-31 is shifted out), so the address takes one register and the
+// base stays in scalar registers.
+__device__ __forceinline__ int4 gather_q(const int4 *__restrict__ xq, unsigned entry) {
+  return *reinterpret_cast<const int4 *>(reinterpret_cast<const char *>(xq) + ((entry << 5) >> 1));
+}
+__device__ __forceinline__ double4 gather_x(const double4 *__restrict__ x, unsigned entry) {
+  return *reinterpret_cast<const double4 *>(reinterpret_cast<const char *>(x) + (entry << 5));
+}
+__device__ __forceinline__ double gather_d(const double *__restrict__ a, unsigned entry) {
+  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a) + ((entry << 5) >> 2));
+}
 // separation q_i - q_j of one dimension in length units (FP64, exact product)
 __device__ __forceinline__ double qdelta(int qi, int qj, double step) {
   return (double)(int)((unsigned)qi - (unsigned)qj) * step;
@@ -326,8 +339,8 @@ struct IntegArgs {
 };
 
 struct Launch {
-  int block = 256;     // threads per workgroup of the pair kernels
-  int tpa = 8;         // threads per atom in the pair kernels
+  int block = 0;  // threads per workgroup of the pair kernels (0: by pair_launch)
+  int tpa = 0;    // threads per atom in the pair kernels (0: by pair_launch)
 };
 
 }  // namespace mdx
@@ -499,6 +512,7 @@ int neigh_check_displacement(mdx_ctx *c, int *flag);
 // sorted order), per-atom energy in f.w, per-atom virial in vatom, and the
 // global energy/virial into c->red_host (after a sync) when ev is set.
 int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig = nullptr);
+Launch pair_launch(const mdx_ctx *c);  // the context's launch shape, defaults filled in for its size
 
 // integrator (integrate.hip)
 int nve_initial(mdx_ctx *c, double dtv, double dtf, int check);

@@ -197,13 +197,6 @@ __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ df
   host[threadIdx.x] = v;
 }
 
-// The fixed-point position of a list entry's atom: a 32-bit byte offset from
-// the array's base (index < 2^27, 16 B each), so the address stays in one
-// register and the base in scalar registers.
-__device__ __forceinline__ int4 gather_q(const int4 *__restrict__ xq, unsigned entry) {
-  return *reinterpret_cast<const int4 *>(reinterpret_cast<const char *>(xq) + ((entry << 5) >> 1));
-}
-
 // Domain::pbc + bin index + histogram; one thread per atom.  slot[i] is the
 // atom's arrival order in its bin (not deterministic; k_bin_rank orders
 // each bin by atom index).  Atoms arrive nearly bin-sorted (the previous

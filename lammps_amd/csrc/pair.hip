@@ -119,6 +119,19 @@ __device__ __forceinline__ double group_sum(double v) {
   return v;
 }
 
+// Mixed precision with four lanes per atom keeps two sets of sums per lane,
+// set h holding the lane's trips (eam: entries) of parity h, and adds the
+// sets before the lanes: the order of the additions, and so every bit of the
+// result, is that of eight lanes per atom.  A mixed trajectory then does not
+// depend on which of the two the default launch takes for its size; the
+// fixed-point mirror otherwise turns a last-bit difference of a sum into a
+// rounding step of a position (about 1e-8 of the box).
+__host__ __device__ constexpr bool split_sums(bool mixed, int tpa) { return mixed && tpa == 4; }
+template <int NS>
+__device__ __forceinline__ double set_sum(const double (&v)[NS]) {
+  return NS == 2 ? v[0] + v[NS - 1] : v[0];
+}
+
 __device__ __forceinline__ void image_shift(int code, double px, double py, double pz, double &sx, double &sy,
                                             double &sz) {
   sx = ((code % 3) - 1) * px;
@@ -315,7 +328,8 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
   (void)t11;
   const double o_clo = one.clo, o_chi = one.chi, o_cut = one.cut, o_lj1 = one.lj1, o_lj2 = one.lj2;
   const float o_f1 = one.f1, o_f2 = one.f2;
-  double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
+  constexpr int NS = split_sums(MIXED, TPA) ? 2 : 1;
+  double fx[NS] = {}, fy[NS] = {}, fz[NS] = {}, e = 0.0;
   double w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
   double4 vpre = make_double4(0.0, 0.0, 0.0, 0.0), hpre = vpre;
@@ -324,9 +338,9 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     if (ig.check) hpre = ig.xhold[i];
   }
   if (i < n) {
-    xi = x[i];
+    if (!Q) xi = x[i];  // Q reads it where it is used: the re-test, the end
     const int4 qi = Q ? xq[i] : make_int4(0, 0, 0, 0);
-    const int row = static_cast<int>(xi.w) * nt1;
+    const int row = (Q ? qi.w : static_cast<int>(xi.w)) * nt1;
     const int jn = numneigh[i];
     const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
     // UNROLL entries per lane per trip: all index loads, then all gathers,
@@ -344,7 +358,11 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     // kernel 0.395 ms against 0.452; the 16-B fixed-point gathers gain
     // nothing (0.310 against 0.304), so Q keeps the lane's own chunk.
     constexpr bool TRANS = CHUNK && TPA == 4 && kTransLJ && !Q;
-    for (int k0 = TRANS ? 0 : CHUNK ? 4 * lane : lane; k0 < jn; k0 += U * TPA) {
+    for (int kt = TRANS ? 0 : CHUNK ? 4 * lane : lane; kt < jn; kt += NS * U * TPA) {
+#pragma unroll
+    for (int h = 0; h < NS; h++) {  // trip h of NS adds into set h
+      const int k0 = kt + h * U * TPA;
+      if (h > 0 && k0 >= jn) break;
       int jc[U];
       double4 xj[Q ? 1 : U];
       int4 qj[Q ? U : 1];
@@ -372,8 +390,8 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        if (Q) qj[u] = xq[jc[u] & MDX_IDX_MASK];
-        else xj[Q ? 0 : u] = x[jc[u] & MDX_IDX_MASK];
+        if (Q) qj[u] = gather_q(xq, jc[u]);
+        else xj[Q ? 0 : u] = gather_x(x, jc[u]);
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
@@ -391,7 +409,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
           inside = rsq < (HOIST ? o_clo : s_clo[t]);
           if (!inside && rsq < (HOIST ? o_chi : s_chi[t])) {
             double ex, ey, ez;
-            pair_delta(xi, x[jc[u] & MDX_IDX_MASK], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
+            pair_delta(x[i], x[jc[u] & MDX_IDX_MASK], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
             inside = ex * ex + ey * ey + ez * ez < (HOIST ? o_cut : s_cutsq[t]);
           }
         } else {
@@ -416,9 +434,9 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
             fpair = forcelj * r2inv;
             if (EV) evdwl = HOIST ? r6inv * (one.lj3 * r6inv - one.lj4) - one.off : r6inv * (s_lj3[t] * r6inv - s_lj4[t]) - s_off[t];
           }
-          fx += delx * fpair;
-          fy += dely * fpair;
-          fz += delz * fpair;
+          fx[h] += delx * fpair;
+          fy[h] += dely * fpair;
+          fz[h] += delz * fpair;
           if (EV) {
             e += 0.5 * evdwl;
             virial_entry(w, ig.pervir, (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz, fpair);
@@ -426,8 +444,10 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
         }
       }
     }
+    }
   }
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, fx, fy, fz, e, w, ig, vpre, hpre, f, vatom,
+  if (Q && i < n && lane == 0) xi = x[i];
+  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f, vatom,
                               partials);
 }
 
@@ -435,7 +455,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
 // a pair inside the cutoff, for the FP64/mixed gathers (Q false) or the
 // fixed-point gathers with the FP64 re-test near the cutoff (Q true)
 template <bool Q>
-__device__ __forceinline__ bool pair_inside(const double4 &xi, const int4 &qi, const double4 *__restrict__ x,
+__device__ __forceinline__ bool pair_inside(const double4 &xi, int i, const int4 &qi, const double4 *__restrict__ x,
                                             int entry, const double4 &xj, const int4 &qj, const QScale &qs,
                                             double px, double py, double pz, double cutsq, double clo, double chi,
                                             double &delx, double &dely, double &delz, double &rsq) {
@@ -447,7 +467,7 @@ __device__ __forceinline__ bool pair_inside(const double4 &xi, const int4 &qi, c
     if (rsq < clo) return true;
     if (!(rsq < chi)) return false;
     double ex, ey, ez;
-    pair_delta(xi, x[entry & MDX_IDX_MASK], (unsigned)entry >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
+    pair_delta(x[i], x[entry & MDX_IDX_MASK], (unsigned)entry >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
     return ex * ex + ey * ey + ez * ez < cutsq;
   }
   pair_delta(xi, xj, (unsigned)entry >> MDX_IDX_BITS, px, py, pz, delx, dely, delz);
@@ -477,13 +497,14 @@ __global__ MDX_PAIR_BOUNDS void k_eam_rho(int n, int npad, int cap, double px, d
   __syncthreads();
   const int i = (xcd_block() * blockDim.x + threadIdx.x) / TPA;
   const int lane = threadIdx.x % TPA;
-  double rho = 0.0;
+  constexpr int NS = split_sums(MIXED, TPA) ? 2 : 1;
+  double rhos[NS] = {};
   int ti = 0;
   const double clo = a.clo, chi = a.chi;  // kernel arguments: scalar registers
   if (i < n) {
-    const double4 xi = x[i];
+    const double4 xi = Q ? make_double4(0.0, 0.0, 0.0, 0.0) : x[i];
     const int4 qi = Q ? xq[i] : make_int4(0, 0, 0, 0);
-    ti = static_cast<int>(xi.w);
+    ti = Q ? qi.w : static_cast<int>(xi.w);
     const int jn = numneigh[i];
     const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
     constexpr bool CHUNK = kChunkEAM;
@@ -506,29 +527,29 @@ __global__ MDX_PAIR_BOUNDS void k_eam_rho(int n, int npad, int cap, double px, d
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        if (Q) qj[u] = xq[jc[u] & MDX_IDX_MASK];
-        else xj[Q ? 0 : u] = x[jc[u] & MDX_IDX_MASK];
+        if (Q) qj[u] = gather_q(xq, jc[u]);
+        else xj[Q ? 0 : u] = gather_x(x, jc[u]);
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
         if (k0 + u * KS >= jn) continue;  // entries carry image bits: test the index, not the sign
         double delx, dely, delz, rsq;
-        if (pair_inside<Q>(xi, qi, x, jc[u], xj[Q ? 0 : u], qj[Q ? u : 0], qs, px, py, pz, a.cutforcesq, clo, chi,
+        if (pair_inside<Q>(xi, i, qi, x, jc[u], xj[Q ? 0 : u], qj[Q ? u : 0], qs, px, py, pz, a.cutforcesq, clo, chi,
                            delx, dely, delz, rsq)) {
           const int tj = Q ? qj[Q ? u : 0].w : static_cast<int>(xj[Q ? 0 : u].w);
           if constexpr (TL) {
             int m;
             float p;
             (void)eam_index_mixed(rsq, a.rdr, a.nr, m, p);
-            rho += (double)eam_rho_eval(s_eam_tab[m], p);
+            rhos[u % NS] += (double)eam_rho_eval(s_eam_tab[m], p);
           } else {
-            rho += eam_rho_term<MIXED>(a, s_t2r[ONE ? a.ntypes1 + 1 : tj * a.ntypes1 + ti], rsq);
+            rhos[u % NS] += eam_rho_term<MIXED>(a, s_t2r[ONE ? a.ntypes1 + 1 : tj * a.ntypes1 + ti], rsq);
           }
         }
       }
     }
   }
-  rho = group_sum<TPA>(rho);
+  const double rho = group_sum<TPA>(set_sum<NS>(rhos));
   if (i < n && lane == 0) {
     // fp pass (pair_eam.cpp:213-228), FP64 in both modes: one per atom
     double p = rho * a.rdrho + 1.0;
@@ -580,7 +601,8 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
   __syncthreads();
   const int i = (xcd_block() * blockDim.x + threadIdx.x) / TPA;
   const int lane = threadIdx.x % TPA;
-  double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
+  constexpr int NS = split_sums(MIXED, TPA) ? 2 : 1;
+  double fx[NS] = {}, fy[NS] = {}, fz[NS] = {}, e = 0.0;
   double w[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
   double4 vpre = make_double4(0.0, 0.0, 0.0, 0.0), hpre = vpre;
@@ -590,9 +612,9 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
   }
   const double clo = a.clo, chi = a.chi;  // kernel arguments: scalar registers
   if (i < n) {
-    xi = x[i];
+    if (!Q) xi = x[i];  // Q reads it where it is used: the re-test, the end
     const int4 qi = Q ? xq[i] : make_int4(0, 0, 0, 0);
-    const int ti = static_cast<int>(xi.w);
+    const int ti = Q ? qi.w : static_cast<int>(xi.w);
     const double fpi = fp[i];
     const int jn = numneigh[i];
     const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
@@ -617,16 +639,15 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const int jj = jc[u] & MDX_IDX_MASK;
-        if (Q) qjv[u] = xq[jj];
-        else xjv[Q ? 0 : u] = x[jj];
-        fpjv[u] = fp[jj];
+        if (Q) qjv[u] = gather_q(xq, jc[u]);
+        else xjv[Q ? 0 : u] = gather_x(x, jc[u]);
+        fpjv[u] = gather_d(fp, jc[u]);
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
       if (k0 + u * KS >= jn) continue;  // entries carry image bits: test the index, not the sign
       double delx, dely, delz, rsq;
-      if (pair_inside<Q>(xi, qi, x, jc[u], xjv[Q ? 0 : u], qjv[Q ? u : 0], qs, px, py, pz, a.cutforcesq, clo, chi,
+      if (pair_inside<Q>(xi, i, qi, x, jc[u], xjv[Q ? 0 : u], qjv[Q ? u : 0], qs, px, py, pz, a.cutforcesq, clo, chi,
                          delx, dely, delz, rsq)) {
         const int tj = Q ? qjv[Q ? u : 0].w : static_cast<int>(xjv[Q ? 0 : u].w);
         const int tij = ONE ? a.ntypes1 + 1 : ti * a.ntypes1 + tj, tji = ONE ? tij : tj * a.ntypes1 + ti;
@@ -640,9 +661,9 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
         } else {
           eam_pair_term<MIXED>(a, s_t2r[tij], s_t2r[tji], s_t2z[tij], rsq, fpi, fpjv[u], fpair, phi);
         }
-        fx += delx * fpair;
-        fy += dely * fpair;
-        fz += delz * fpair;
+        fx[u % NS] += delx * fpair;
+        fy[u % NS] += dely * fpair;
+        fz[u % NS] += delz * fpair;
         if (EV) {
           e += 0.5 * phi;
           virial_entry(w, ig.pervir, (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz, fpair);
@@ -652,7 +673,8 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
     }
     if (EV && lane == 0) e += eemb[i];
   }
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, fx, fy, fz, e, w, ig, vpre, hpre, f, vatom,
+  if (Q && i < n && lane == 0) xi = x[i];
+  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f, vatom,
                               partials);
 }
 
@@ -772,9 +794,10 @@ void launch_eam(mdx_ctx *c, int B, const IntegArgs &ig) {
 }
 
 template <bool MIXED, bool EV, bool INTEG, bool Q>
-int dispatch_tpa(mdx_ctx *c, int B, const IntegArgs &ig) {
+int dispatch_tpa(mdx_ctx *c, const Launch &l, const IntegArgs &ig) {
+  const int B = l.block;
   const bool lj = c->pair_style == MDX_PAIR_LJ;
-  switch (c->launch.tpa) {
+  switch (l.tpa) {
     case 1: lj ? launch_lj<MIXED, EV, 1, INTEG, Q>(c, B, ig) : launch_eam<MIXED, EV, 1, INTEG, Q>(c, B, ig); break;
     case 2: lj ? launch_lj<MIXED, EV, 2, INTEG, Q>(c, B, ig) : launch_eam<MIXED, EV, 2, INTEG, Q>(c, B, ig); break;
     case 4: lj ? launch_lj<MIXED, EV, 4, INTEG, Q>(c, B, ig) : launch_eam<MIXED, EV, 4, INTEG, Q>(c, B, ig); break;
@@ -790,19 +813,50 @@ int dispatch_tpa(mdx_ctx *c, int B, const IntegArgs &ig) {
 
 template <bool INTEG>
 int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
-  const int B = c->launch.block;
+  const Launch l = pair_launch(c);
   if (c->precision == MDX_MIXED) {
     if (c->qpos) {
       int rc = refresh_xq(c);
       if (rc) return rc;
-      return ev ? dispatch_tpa<true, true, INTEG, true>(c, B, ig) : dispatch_tpa<true, false, INTEG, true>(c, B, ig);
+      return ev ? dispatch_tpa<true, true, INTEG, true>(c, l, ig) : dispatch_tpa<true, false, INTEG, true>(c, l, ig);
     }
-    return ev ? dispatch_tpa<true, true, INTEG, false>(c, B, ig) : dispatch_tpa<true, false, INTEG, false>(c, B, ig);
+    return ev ? dispatch_tpa<true, true, INTEG, false>(c, l, ig) : dispatch_tpa<true, false, INTEG, false>(c, l, ig);
   }
-  return ev ? dispatch_tpa<false, true, INTEG, false>(c, B, ig) : dispatch_tpa<false, false, INTEG, false>(c, B, ig);
+  return ev ? dispatch_tpa<false, true, INTEG, false>(c, l, ig) : dispatch_tpa<false, false, INTEG, false>(c, l, ig);
 }
 
 }  // namespace
+
+// Launch shape where the caller set none.  Few lanes per atom do the least
+// work (fewer partial sums, longer index chunks) and win once they fill the
+// chip; below that more lanes per atom shorten the one chain of dependent
+// loads that a small launch consists of.  Measured per step kernel (us, lanes
+// 4 / 8 / 16 / 32 per atom, FP64):
+//   lj/cut            500 atoms  8.3 /  6.9 /  5.0 /  4.9
+//                   4,000        8.1 /  7.3 /  4.9 /  5.3
+//                  32,000       10.4 / 10.8 / 13.0 / 16.7  (mixed 8.0 / 7.7 / 10.1)
+//                 108,000       24.6 / 30.5 / 36.5 / 51
+//               2,048,000        381 /  508 /  685 / 1096  (mixed  286 /  329)
+//   Kob-Andersen    2,744       11.1 /  7.9 /  5.8 /  5.3
+//                   8,000       11.0 /  7.7 /  6.5 /  6.6
+//   eam (rho+force) 4,000       26.3 / 17.3 / 13.1 / 12.6
+//                  13,500       26.2 / 22.2 / 23.2 / 24.3
+//                 108,000        100 /  106 /  118 /  142
+// Mixed precision takes only 8 and 4, which give the same bits (split_sums):
+// a mixed trajectory amplifies any other difference to its own error.
+// Workgroups of one wavefront spread a small launch evenly over the CUs
+// (13,500 lj/cut atoms at 8 lanes: 6.8 against 7.9 us); with 1024 or more
+// workgroups of 256 there is nothing to gain.  The mixed single-type eam
+// kernels copy their spline tables to LDS once per workgroup, so they keep
+// 256 (13,500 atoms: 15.9 against 22.1 us).
+Launch pair_launch(const mdx_ctx *c) {
+  Launch l = c->launch;
+  const bool eam = c->pair_style == MDX_PAIR_EAM;
+  const bool mixed = c->precision == MDX_MIXED;
+  if (!l.tpa) l.tpa = c->n > 48000 ? 4 : c->n > 10000 || mixed ? 8 : c->n > (eam ? 6000 : 3000) ? 16 : 32;
+  if (!l.block) l.block = (long)c->n * l.tpa < 1024L * 256 && !(eam && mixed) ? 64 : 256;
+  return l;
+}
 
 // Pair::compute on the device.  With `ig` the force
 // kernel also runs fix nve's final integrate of this step and, if ig->next,

@@ -513,3 +513,35 @@ def test_shifted_two_type_lj_energies_match_the_oracle(prec):
     np.testing.assert_allclose(out["eatom"], ea_ref, rtol=0, atol=100 * etol * np.abs(ea_ref).max())
     np.testing.assert_allclose(out["vatom"], va_ref, rtol=0, atol=100 * etol * np.abs(va_ref).max())
     ctx.close()
+
+
+@pytest.mark.parametrize("style,n", [("lj", 3000), ("lj", 3001), ("lj", 10000), ("lj", 10001), ("lj", 48000),
+                                     ("lj", 48001), ("eam", 6000), ("eam", 6001), ("eam", 10001), ("eam", 48001)])
+def test_default_launch_shapes_agree_with_a_fixed_one(style, n):
+    """On both sides of the sizes where the default launch shape changes:
+    forces equal those of 8 lanes per atom in workgroups of 256 to the order
+    of the sums (FP64: 1e-12 of the rms force)."""
+    from gpu_helpers import CU_U3
+    from lammps_amd import mdx
+    rng = np.random.default_rng(n)
+    cells = int(np.ceil((n / 4.0) ** (1.0 / 3.0)))
+    a = (4.0 / 0.8442) ** (1.0 / 3.0) if style == "lj" else 3.615
+    lo, hi, x = mdx.lattice("fcc", 0.8442 if style == "lj" else 3.615, "lj" if style == "lj" else "metal", (0, 0, 0),
+                            (cells,) * 3)
+    x = np.mod(x[rng.permutation(len(x))[:n]] + rng.uniform(-0.04 * a, 0.04 * a, (n, 3)), hi)
+    ctx = mdx.Context(0)
+    ctx.set_box(lo, hi, (1, 1, 1))
+    ctx.set_atoms(x, np.ones(n, dtype=np.int32), np.array([0.0, 1.0 if style == "lj" else 63.55]))
+    if style == "lj":
+        ctx.pair_lj_from_coeffs(1, {(1, 1): (1.0, 1.0, 2.5)})
+    else:
+        mdx.eam_context_tables(ctx, CU_U3)
+    ctx.neigh_modify(0.3 if style == "lj" else 1.0)
+    ctx.precision(mdx.FP64)
+    got = ctx.compute(1, 1)
+    ctx.set_launch(256, 8)
+    want = ctx.compute(1, 1)
+    assert ctx.get_launch() == dict(block=256, tpa=8)
+    assert force_errors(got["f"], want["f"])[0] <= 1e-12
+    assert abs(got["eng"] - want["eng"]) <= 1e-12 * abs(want["eng"])
+    ctx.close()
