@@ -279,6 +279,17 @@ __device__ __forceinline__ void mark_trigger(bool moved, int *trig, int *trig_de
   }
 }
 
+// The list pass's largest row and entry total: each workgroup adds into one
+// of kListSlots counters, k_build_flags combines them.  Atomics on one
+// address complete one after the other, ~12 ns each on the eight XCDs: a
+// single pair of words took 0.77 ms of the 0.95 ms list pass at 2.048 M
+// atoms (64,000 of them), and 50 us at 32,000 atoms with one per workgroup.
+__device__ __forceinline__ void count_rows(ListSlot *slots, int most, unsigned long long sum) {
+  ListSlot &s = slots[blockIdx.x % kListSlots];
+  atomicMax(&s.most, most);
+  atomicAdd(&s.sum, sum);
+}
+
 // Gate of a step's kernels queued before the host has checked what they
 // depend on (mdx_run's look-ahead): they do nothing when
 //   * the displacement trigger they were queued behind fired (the device
@@ -491,6 +502,9 @@ int prof_resolve(mdx_ctx *c);
 
 // Pair::init + Neighbor::init cutoffs, bin grid, first list and partials (api.cpp)
 int prepare_ctx(mdx_ctx *c);
+// combines a list pass's slots into its build flags and writes those to the
+// mapped host words `host` as well (neigh.hip)
+void launch_build_flags(hipStream_t stream, int *dflags, int *host);
 // no-allocation compute (noalloc.hip)
 int noalloc_init(int device);
 int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int eflag, int vflag, double *f,

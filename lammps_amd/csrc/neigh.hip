@@ -154,17 +154,6 @@ __device__ __forceinline__ void stage_band(const NeighArgs &a, float *lo, float 
   }
 }
 
-// The list pass's largest row and entry total: each workgroup adds into one
-// of kListSlots counters, k_build_flags combines them.  Atomics on one
-// address complete one after the other, ~12 ns each on the eight XCDs: a
-// single pair of words took 0.77 ms of the 0.95 ms list pass at 2.048 M
-// atoms (64,000 of them), and 50 us at 32,000 atoms with one per workgroup.
-__device__ __forceinline__ void count_rows(ListSlot *slots, int most, unsigned long long sum) {
-  ListSlot &s = slots[blockIdx.x % kListSlots];
-  atomicMax(&s.most, most);
-  atomicAdd(&s.sum, sum);
-}
-
 // The list pass's counters into the build flags, and the flags into pinned
 // host memory (in place of a copy): one workgroup, one slot per thread.
 __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ dflags, int *__restrict__ host) {
@@ -1078,6 +1067,10 @@ void launch_build(mdx_ctx *c) {
 
 }  // namespace
 
+void launch_build_flags(hipStream_t stream, int *dflags, int *host) {
+  hipLaunchKernelGGL(k_build_flags, dim3(1), dim3(kListSlots), 0, stream, dflags, host);
+}
+
 int neigh_setup_grid(mdx_ctx *c) {
   NeighArgs &a = c->na;
   const double cut = c->cutneighmax;
@@ -1251,7 +1244,7 @@ int launch_list(mdx_ctx *c, bool again) {
       return hip_fail(e, "memset flags");
   }
   launch_build(c);
-  hipLaunchKernelGGL(k_build_flags, dim3(1), dim3(kListSlots), 0, c->stream, c->dflags, c->bflags_host);
+  launch_build_flags(c->stream, c->dflags, c->bflags_host);
   prof_end(c);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "list build launch");
   if ((e = hipEventRecord(c->build_ev, c->stream)) != hipSuccess) return hip_fail(e, "build event");

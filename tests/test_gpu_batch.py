@@ -264,3 +264,30 @@ def test_neighbour_counts_match_brute_force_small_boxes():
         cnt += int(np.sum(r2 < 2.5 ** 2)) - 1
     assert total == cnt
     b.close()
+
+
+@pytest.mark.parametrize("density", [0.9, 7.0])
+@pytest.mark.parametrize("side", [(2.1, 2.3, 2.2), (2.6, 5.3, 3.1), (9.7, 2.6, 2.6)])
+def test_neighbour_counts_match_brute_force(side, density):
+    """Boxes of four bins a side (FP64 candidates) and of more (fixed-point
+    candidates), a free cluster beside each, rows of more candidates than one
+    window of the build holds (density 7: about 460 neighbours per atom)."""
+    rng = np.random.default_rng(8)
+    L = 2.5 * np.array(side)
+    n1 = int(density * np.prod(L))
+    x1 = rng.uniform(0, 1, size=(n1, 3)) * L
+    x2 = rng.uniform(0, 1, size=(n1 // 2 + 1, 3)) * L
+    b = B.Batch([n1, len(x2)], [[0, 0, 0]] * 2, [L, L], [[1, 1, 1], [0, 0, 0]], 1, np.ones(n1 + len(x2), np.int32))
+    b.set_positions(np.concatenate([x1, x2]))
+    one = np.ones((2, 2))
+    b.lj_init(one, one * 0.5, one * 2.5)
+    total, most = b.neigh_stats()
+    counts = []
+    for x, periodic in ((x1, True), (x2, False)):
+        for i in range(len(x)):
+            d = x - x[i]
+            if periodic:
+                d -= L * np.round(d / L)
+            counts.append(int(np.sum(np.sum(d * d, 1) < 2.5 ** 2)) - 1)
+    assert total == sum(counts) and most == max(counts)
+    b.close()
