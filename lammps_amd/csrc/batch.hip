@@ -34,6 +34,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <cmath>
+#include <type_traits>
 
 #include "../../include/mdx_batch.h"
 #include "mdx_internal.h"
@@ -52,6 +53,7 @@ struct RepGeom {
   // difference is the minimum-image separation), qstep = prd * 2^-32
   // (periodic) or prd * 2^-30, exact
   double qscale[3], qstep[3];
+  double iprd[3];  // 1 / prd in periodic dimensions, 0 in the others
   int nbin[3], periodic[3];
   int bin_off;
 };
@@ -107,38 +109,6 @@ __device__ __forceinline__ void shift_of(int code, double &sx, double &sy, doubl
   sx = (double)(code / 9 - 1);
   sy = (double)((code / 3) % 3 - 1);
   sz = (double)(code % 3 - 1);
-}
-
-// Separation of the pair (i, list entry) and whether it lies inside cutsq:
-// from the FP64 positions with the entry's image shift, or (MIXED) from the
-// fixed-point mirror with the FP64 re-test within kQBand of the cutoff.
-template <bool MIXED>
-__device__ __forceinline__ bool b_pair(const double4 &xi, const int4 &qi, const double4 *__restrict__ x,
-                                       const int4 *__restrict__ xq, const RepGeom &g, int ent, double cutsq,
-                                       double &dx, double &dy, double &dz, double &rsq) {
-  const int j = ent & MDX_IDX_MASK;
-  if (MIXED) {
-    const int4 qj = xq[j];
-    dx = qsep(qi.x, qj.x, g.qstep[0]);
-    dy = qsep(qi.y, qj.y, g.qstep[1]);
-    dz = qsep(qi.z, qj.z, g.qstep[2]);
-    rsq = dx * dx + dy * dy + dz * dz;
-    if (rsq < cutsq * (1.0 - kQBand)) return true;
-    if (!(rsq < cutsq * (1.0 + kQBand))) return false;
-  }
-  double sx, sy, sz;
-  shift_of((int)((unsigned)ent >> MDX_IDX_BITS), sx, sy, sz);
-  const double4 xj = x[j];
-  const double ex = xi.x - (xj.x + sx * g.prd[0]), ey = xi.y - (xj.y + sy * g.prd[1]),
-               ez = xi.z - (xj.z + sz * g.prd[2]);
-  const double esq = ex * ex + ey * ey + ez * ez;
-  if (!MIXED) {
-    dx = ex;
-    dy = ey;
-    dz = ez;
-    rsq = esq;
-  }
-  return esq < cutsq;
 }
 
 __device__ __forceinline__ int local_bin(const RepGeom &g, double x, int d) {
@@ -388,6 +358,37 @@ __global__ __launch_bounds__(kBuildBlock, 5) void k_b_build(int n, const double4
   }
 }
 
+// ---------------------------------------------------------------- pair helpers
+
+// sqrt(x) and 1/sqrt(x) in FP64 to about an ulp: the hardware reciprocal
+// square root refined in coupled steps, half the instructions of sqrt and a
+// divide
+__device__ __forceinline__ void sqrt_and_inverse(double x, double &r, double &ri) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, x), h, g);
+  ri = h + h;
+  ri = fma(ri, fma(-ri, g, 1.0), ri);
+  r = g;
+}
+
+// One lane's four consecutive entries k0 .. k0+3 of a row (rows start 16-B
+// aligned; entries past jn are not written and become the atom itself)
+__device__ __forceinline__ void row_chunk(const int *__restrict__ row, int k0, int jn, int self, int (&ent)[4]) {
+  const int4 e4 = *reinterpret_cast<const int4 *>(row + k0);
+  ent[0] = e4.x;
+  ent[1] = k0 + 1 < jn ? e4.y : self;
+  ent[2] = k0 + 2 < jn ? e4.z : self;
+  ent[3] = k0 + 3 < jn ? e4.w : self;
+}
+
+// separation of a pair within half the box, in FP64: the nearest image
+// (periodic boxes are at least two cutoffs wide, so it is the list's)
+__device__ __forceinline__ double nearest(double d, double prd, double iprd) { return fma(-prd, rint(d * iprd), d); }
+
 // ---------------------------------------------------------------- lj/cut
 
 // MIXED: neighbours are read from the fixed-point mirror (16 B instead of
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           ent[u] = k0 + u < jn ? ev[u] : i;  // the row's tail past jn is not written
-          qj[u] = xq[ent[u] & MDX_IDX_MASK];
+          qj[u] = gather_q(xq, ent[u]);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -478,15 +479,13 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           ent[u] = k0 + u < jn ? ev[u] : i;
-          xj[u] = x[ent[u] & MDX_IDX_MASK];
+          xj[u] = gather_x(x, ent[u]);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           if (k0 + u >= jn) continue;
-          double sx, sy, sz;
-          shift_of((unsigned)ent[u] >> MDX_IDX_BITS, sx, sy, sz);
-          const double dx = xi.x - (xj[u].x + sx * px), dy = xi.y - (xj[u].y + sy * py),
-                       dz = xi.z - (xj[u].z + sz * pz);
+          const double dx = nearest(xi.x - xj[u].x, px, g.iprd[0]), dy = nearest(xi.y - xj[u].y, py, g.iprd[1]),
+                       dz = nearest(xi.z - xj[u].z, pz, g.iprd[2]);
           const double rsq = dx * dx + dy * dy + dz * dz;
           const int t = ti * nt1 + (int)xj[u].w;
           if (rsq < s_tab[T_CUTSQ * kNT + t]) {
@@ -510,22 +509,38 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
   }
 }
 
-// per-block partial rows: [eps grad (nt1^2) | sigma grad (nt1^2)]
-template <bool MIXED, int TPA>
+// Parameter gradients, FP64.  A pair's gradient factor is the same in both of
+// its atoms' rows, so each pair is taken once (entry j > i) with G_i - G_j;
+// its sums go to the type pair (lower, higher type).  Per-block partial rows:
+// [eps grad | sigma grad], nt1^2 each.
+// One or two atom types: the NT(NT+1)/2 type pairs' sums stay in registers
+// for the whole launch and are added up once, at its end.
+template <int NT, int TPA>
 __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4 *__restrict__ x,
                                                    const int *__restrict__ rep, const RepGeom *__restrict__ geom,
                                                    const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                                    int cap, const double *__restrict__ tab,
                                                    const double4 *__restrict__ gin, double *__restrict__ partials) {
-  __shared__ double s_tab[T_N * kNT];
-  __shared__ double s_acc[2 * kNT];
-  for (int k = threadIdx.x; k < T_N * kNT; k += blockDim.x) s_tab[k] = tab[k];
-  for (int k = threadIdx.x; k < 2 * kNT; k += blockDim.x) s_acc[k] = 0.0;
+  constexpr bool FEW = NT <= 2;
+  constexpr int NP = NT * (NT + 1) / 2;
+  constexpr int NA = FEW ? NP : NT;  // sums per lane: type pairs, or the partner's types
+  __shared__ double s_cut[kNT];
+  __shared__ double2 s_a[kNT], s_b[kNT];
+  __shared__ double s_acc[FEW ? 2 * NP * 16 : 2 * kNT];
+  const int cols = nt1 * nt1;
+  for (int k = threadIdx.x; k < cols; k += blockDim.x) {
+    s_cut[k] = tab[T_CUTSQ * kNT + k];
+    s_a[k] = make_double2(tab[T_A1 * kNT + k], tab[T_A2 * kNT + k]);
+    s_b[k] = make_double2(tab[T_B1 * kNT + k], tab[T_B2 * kNT + k]);
+  }
+  if (!FEW)
+    for (int k = threadIdx.x; k < 2 * kNT; k += blockDim.x) s_acc[k] = 0.0;
   __syncthreads();
   const int apb = blockDim.x / TPA;
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  double ae[NA] = {}, as[NA] = {};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -533,70 +548,117 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
     const double4 gi = gin[i];
     const int ti = (int)xi.w;
     const RepGeom &g = geom[rep[i]];
-    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2];
+    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
-    double ae[MDX_NT1], as[MDX_NT1];
+    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+      int ent[4];
+      double4 xj[4], gj[4];
+      row_chunk(row, k0, jn, i, ent);
+      bool any = false;
 #pragma unroll
-    for (int t = 0; t < MDX_NT1; t++) ae[t] = as[t] = 0.0;
-    for (int k = lane; k < jn; k += TPA) {
-      const int ent = row[k];
-      const int j = ent & MDX_IDX_MASK;
-      double sx, sy, sz;
-      shift_of((unsigned)ent >> MDX_IDX_BITS, sx, sy, sz);
-      const double4 xj = x[j];
-      const double dx = xi.x - (xj.x + sx * px), dy = xi.y - (xj.y + sy * py), dz = xi.z - (xj.z + sz * pz);
-      const double rsq = dx * dx + dy * dy + dz * dz;
-      const int tj = (int)xj.w;
-      const int t = ti * nt1 + tj;
-      if (rsq < s_tab[T_CUTSQ * kNT + t]) {
-        const double a = gi.x * dx + gi.y * dy + gi.z * dz;
-        double de, ds;
-        if (MIXED) {
-          const float r2inv = 1.0f / (float)rsq;
-          const float r6inv = r2inv * r2inv * r2inv;
-          const float r8 = r2inv * r6inv;
-          de = (double)(r8 * ((float)s_tab[T_A1 * kNT + t] * r6inv - (float)s_tab[T_A2 * kNT + t]));
-          ds = (double)(r8 * ((float)s_tab[T_B1 * kNT + t] * r6inv - (float)s_tab[T_B2 * kNT + t]));
-        } else {
+      for (int q = 0; q < 4; q++) any |= (ent[q] & MDX_IDX_MASK) > i;
+      if (!any) continue;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        xj[q] = gather_x(x, ent[q]);
+        gj[q] = gather_x(gin, ent[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        if ((ent[q] & MDX_IDX_MASK) <= i) continue;  // the pair's other row, or past the end
+        const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
+                     dz = nearest(xi.z - xj[q].z, pz, iz);
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        const int tj = (int)xj[q].w;
+        const int t = ti * nt1 + tj;
+        if (rsq < s_cut[t]) {
+          const double a = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
           const double r2inv = 1.0 / rsq;
           const double r6inv = r2inv * r2inv * r2inv;
-          const double r8 = r2inv * r6inv;
-          de = r8 * (s_tab[T_A1 * kNT + t] * r6inv - s_tab[T_A2 * kNT + t]);
-          ds = r8 * (s_tab[T_B1 * kNT + t] * r6inv - s_tab[T_B2 * kNT + t]);
-        }
+          const double ar8 = a * (r2inv * r6inv);
+          const double2 ca = s_a[t], cb = s_b[t];
+          const double de = ca.x * r6inv - ca.y, ds = cb.x * r6inv - cb.y;
+          const int slot = FEW ? ti + tj - 2 : tj - 1;  // (1,1), (1,2), (2,2), or the partner's type
 #pragma unroll
-        for (int tt = 1; tt < MDX_NT1; tt++)
-          if (tt == tj) {
-            ae[tt] += a * de;
-            as[tt] += a * ds;
-          }
+          for (int c = 0; c < NA; c++)
+            if (NA == 1 || slot == c) {
+              ae[c] += ar8 * de;
+              as[c] += ar8 * ds;
+            }
+        }
       }
     }
+    if constexpr (!FEW) {
 #pragma unroll
-    for (int tt = 1; tt < MDX_NT1; tt++) {
-      if (tt < nt1) {
-        const double se = gsum<TPA>(ae[tt]), ss = gsum<TPA>(as[tt]);
-        if (lane == 0) {
-          atomicAdd(&s_acc[ti * nt1 + tt], se);
-          atomicAdd(&s_acc[kNT + ti * nt1 + tt], ss);
+      for (int c = 0; c < NA; c++)
+        if (c + 1 < nt1) {
+          const double se = gsum<TPA>(ae[c]), ss = gsum<TPA>(as[c]);
+          if (lane == 0) {
+            const int t = min(ti, c + 1) * nt1 + max(ti, c + 1);
+            atomicAdd(&s_acc[t], se);
+            atomicAdd(&s_acc[kNT + t], ss);
+          }
+          ae[c] = as[c] = 0.0;
         }
-      }
     }
   }
-  __syncthreads();
-  double *out = partials + (size_t)blockIdx.x * 2 * kNT;
-  for (int k = threadIdx.x; k < 2 * kNT; k += blockDim.x) out[k] = s_acc[k];
+  double *out = partials + (size_t)blockIdx.x * 2 * cols;
+  if constexpr (FEW) {
+#pragma unroll
+    for (int c = 0; c < NP; c++) {
+      const double se = gsum<64>(ae[c]), ss = gsum<64>(as[c]);
+      if ((threadIdx.x & 63) == 0) {
+        s_acc[(2 * c) * 16 + (threadIdx.x >> 6)] = se;
+        s_acc[(2 * c + 1) * 16 + (threadIdx.x >> 6)] = ss;
+      }
+    }
+    __syncthreads();
+    const int nw = blockDim.x >> 6;
+    for (int k = threadIdx.x; k < 2 * cols; k += blockDim.x) {
+      const int t = k % cols, lo = t / nt1, hi = t % nt1;
+      double v = 0.0;
+      if (lo >= 1 && hi >= lo) {
+        const double *w = s_acc + (2 * (lo + hi - 2) + (k >= cols ? 1 : 0)) * 16;
+        for (int q = 0; q < nw; q++) v += w[q];
+      }
+      out[k] = v;
+    }
+  } else {
+    __syncthreads();
+    for (int k = threadIdx.x; k < 2 * cols; k += blockDim.x) out[k] = s_acc[k < cols ? k : kNT + k - cols];
+  }
 }
 
 // ---------------------------------------------------------------- eam
 
-// spline tables (n+1)*7 in LDS when they fit, else read from global memory
-template <typename T>
-__device__ __forceinline__ const T *stage(T *lds, const T *g, int count, bool use_lds) {
-  if (!use_lds) return g;
-  for (int k = threadIdx.x; k < count; k += blockDim.x) lds[k] = g[k];
-  return lds;
+// The spline tables of the pair passes: per knot two 4-vectors, {c0,c1,c2,0}
+// (derivative) and {c3,c4,c5,c6} (value), so a lookup is one or two vector
+// reads.  They are copied to LDS when they fit (kTabLDS), one vector kind
+// after the other; persistent grids make that once per workgroup.
+template <bool MIXED>
+struct Real {
+  using T = double;
+  using V = double4;
+};
+template <>
+struct Real<true> {
+  using T = float;
+  using V = float4;
+};
+struct EamKnots {
+  const double4 *rhor_d, *z2r_d;
+  const float4 *rhor_f, *z2r_f;
+};
+template <bool MIXED>
+__device__ __forceinline__ const typename Real<MIXED>::V *rhor_knots(const EamKnots &t) {
+  if constexpr (MIXED) return t.rhor_f;
+  else return t.rhor_d;
+}
+template <bool MIXED>
+__device__ __forceinline__ const typename Real<MIXED>::V *z2r_knots(const EamKnots &t) {
+  if constexpr (MIXED) return t.z2r_f;
+  else return t.z2r_d;
 }
 
 template <typename T>
@@ -608,20 +670,51 @@ __device__ __forceinline__ void r_spline(const EamTab &et, T r, int &m, T &p) {
   p = pp < (T)1 ? pp : (T)1;
 }
 
-template <bool MIXED, int TPA>
+// Whether the pair (i, entry) lies inside cutsq, and its separation: from the
+// fixed-point mirror with the FP64 re-test within kQBand of the cutoff
+// (MIXED), or from the FP64 positions.
+template <bool MIXED>
+__device__ __forceinline__ bool eam_inside(const double4 &xi, const int4 &qi, int i, const double4 *__restrict__ x,
+                                           const double4 &xj, const int4 &qj, const RepGeom &g, int ent, double cutsq,
+                                           const double (&step)[3], const double (&ip)[3], double &dx, double &dy,
+                                           double &dz, double &rsq) {
+  if constexpr (MIXED) {
+    dx = qsep(qi.x, qj.x, step[0]);
+    dy = qsep(qi.y, qj.y, step[1]);
+    dz = qsep(qi.z, qj.z, step[2]);
+    rsq = dx * dx + dy * dy + dz * dz;
+    if (rsq < cutsq * (1.0 - kQBand)) return true;
+    if (!(rsq < cutsq * (1.0 + kQBand))) return false;
+    double sx, sy, sz;
+    shift_of((int)((unsigned)ent >> MDX_IDX_BITS), sx, sy, sz);
+    const double4 pi = x[i], pj = x[ent & MDX_IDX_MASK];
+    const double ex = pi.x - (pj.x + sx * g.prd[0]), ey = pi.y - (pj.y + sy * g.prd[1]),
+                 ez = pi.z - (pj.z + sz * g.prd[2]);
+    return ex * ex + ey * ey + ez * ez < cutsq;
+  } else {
+    dx = nearest(xi.x - xj.x, step[0], ip[0]);
+    dy = nearest(xi.y - xj.y, step[1], ip[1]);
+    dz = nearest(xi.z - xj.z, step[2], ip[2]);
+    rsq = dx * dx + dy * dy + dz * dz;
+    return rsq < cutsq;
+  }
+}
+
+template <bool MIXED, int TPA, bool TL>
 __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__restrict__ x,
                                                     const int4 *__restrict__ xq, const int *__restrict__ rep,
                                                     const RepGeom *__restrict__ geom, const int *__restrict__ nbr,
                                                     const int *__restrict__ numneigh, int cap, EamTab et,
-                                                    const double *__restrict__ rhor_d, const float *__restrict__ rhor_f,
-                                                    const double *__restrict__ frho_d, int use_lds,
+                                                    EamKnots knots, const double *__restrict__ frho_d,
                                                     double *__restrict__ rho, double *__restrict__ fp,
                                                     double *__restrict__ eemb) {
-  extern __shared__ double s_dyn[];
-  using T = typename std::conditional<MIXED, float, double>::type;
-  const T *rhor;
-  if (MIXED) rhor = (const T *)stage((float *)s_dyn, rhor_f, (et.nr + 1) * 7, use_lds);
-  else rhor = (const T *)stage((double *)s_dyn, rhor_d, (et.nr + 1) * 7, use_lds);
+  extern __shared__ double4 s_knots[];
+  using T = typename Real<MIXED>::T;
+  using V = typename Real<MIXED>::V;
+  const V *const tab = rhor_knots<MIXED>(knots);
+  V *const s_val = reinterpret_cast<V *>(s_knots);
+  if constexpr (TL)
+    for (int m = threadIdx.x; m <= et.nr; m += blockDim.x) s_val[m] = tab[2 * m + 1];
   __syncthreads();
   const int apb = blockDim.x / TPA;
   int end;
@@ -630,21 +723,46 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
-    const double4 xi = x[i];
-    const int4 qi = MIXED ? xq[i] : make_int4(0, 0, 0, 0);
+    double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
+    int4 qi = make_int4(0, 0, 0, 0);
+    if constexpr (MIXED) qi = xq[i];
+    else xi = x[i];
     const RepGeom &g = geom[rep[i]];
+    double step[3], ip[3];
+    for (int d = 0; d < 3; d++) {
+      step[d] = MIXED ? g.qstep[d] : g.prd[d];
+      ip[d] = g.iprd[d];
+    }
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double acc = 0.0;
-    for (int k = lane; k < jn; k += TPA) {
-      double dx, dy, dz, rsq;
-      if (b_pair<MIXED>(xi, qi, x, xq, g, row[k], et.cutsq, dx, dy, dz, rsq)) {
-        int m;
-        T p;
-        if constexpr (MIXED) (void)eam_index_mixed(rsq, et.rdr, et.nr, m, p);
-        else r_spline<T>(et, (T)sqrt(rsq), m, p);
-        const T *c = rhor + m * 7;
-        acc += (double)(((c[3] * p + c[4]) * p + c[5]) * p + c[6]);
+    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+      int ent[4];
+      double4 xj[MIXED ? 1 : 4];
+      int4 qj[MIXED ? 4 : 1];
+      row_chunk(row, k0, jn, i, ent);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
+        else xj[u] = gather_x(x, ent[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        double dx, dy, dz, rsq;
+        if (k0 + u < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
+                                             step, ip, dx, dy, dz, rsq)) {
+          int m;
+          T p;
+          if constexpr (MIXED) {
+            (void)eam_index_mixed(rsq, et.rdr, et.nr, m, p);
+          } else {
+            double r, ri;
+            sqrt_and_inverse(rsq, r, ri);
+            r_spline<T>(et, r, m, p);
+          }
+          const V c = TL ? s_val[m] : tab[2 * m + 1];
+          acc += (double)(((c.x * p + c.y) * p + c.z) * p + c.w);
+        }
       }
     }
     acc = gsum<TPA>(acc);
@@ -666,26 +784,25 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
   }
 }
 
-template <bool MIXED, int TPA>
+template <bool MIXED, int TPA, bool TL>
 __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__restrict__ x,
-                                                      const int4 *__restrict__ xq, const int *__restrict__ rep, const RepGeom *__restrict__ geom,
-                                                      const int *__restrict__ nbr, const int *__restrict__ numneigh,
-                                                      int cap, EamTab et, const double *__restrict__ rhor_d,
-                                                      const double *__restrict__ z2r_d, const float *__restrict__ rhor_f,
-                                                      const float *__restrict__ z2r_f, int use_lds,
-                                                      const double *__restrict__ fp, const double *__restrict__ eemb,
-                                                      double4 *__restrict__ f) {
-  extern __shared__ double s_dyn[];
-  using T = typename std::conditional<MIXED, float, double>::type;
-  const int tn = (et.nr + 1) * 7;
-  const T *rhor, *z2r;
-  if (MIXED) {
-    rhor = (const T *)stage((float *)s_dyn, rhor_f, tn, use_lds);
-    z2r = (const T *)stage((float *)s_dyn + tn, z2r_f, tn, use_lds);
-  } else {
-    rhor = (const T *)stage((double *)s_dyn, rhor_d, tn, use_lds);
-    z2r = (const T *)stage((double *)s_dyn + tn, z2r_d, tn, use_lds);
-  }
+                                                      const int4 *__restrict__ xq, const int *__restrict__ rep,
+                                                      const RepGeom *__restrict__ geom, const int *__restrict__ nbr,
+                                                      const int *__restrict__ numneigh, int cap, EamTab et,
+                                                      EamKnots knots, const double *__restrict__ fp,
+                                                      const double *__restrict__ eemb, double4 *__restrict__ f) {
+  extern __shared__ double4 s_knots[];
+  using T = typename Real<MIXED>::T;
+  using V = typename Real<MIXED>::V;
+  const V *const rtab = rhor_knots<MIXED>(knots), *const ztab = z2r_knots<MIXED>(knots);
+  const int kn = et.nr + 1;
+  V *const s_tab = reinterpret_cast<V *>(s_knots);  // rho' | z2' | z2
+  if constexpr (TL)
+    for (int m = threadIdx.x; m < kn; m += blockDim.x) {
+      s_tab[m] = rtab[2 * m];
+      s_tab[kn + m] = ztab[2 * m];
+      s_tab[2 * kn + m] = ztab[2 * m + 1];
+    }
   __syncthreads();
   const int apb = blockDim.x / TPA;
   int end;
@@ -694,39 +811,61 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
-    const double4 xi = x[i];
-    const int4 qi = MIXED ? xq[i] : make_int4(0, 0, 0, 0);
+    double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
+    int4 qi = make_int4(0, 0, 0, 0);
+    if constexpr (MIXED) qi = xq[i];
+    else xi = x[i];
     const double fpi = fp[i];
     const RepGeom &g = geom[rep[i]];
+    double step[3], ip[3];
+    for (int d = 0; d < 3; d++) {
+      step[d] = MIXED ? g.qstep[d] : g.prd[d];
+      ip[d] = g.iprd[d];
+    }
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
-    for (int k = lane; k < jn; k += TPA) {
-      const int ent = row[k];
-      double dx, dy, dz, rsq;
-      if (b_pair<MIXED>(xi, qi, x, xq, g, ent, et.cutsq, dx, dy, dz, rsq)) {
-        const double fpj = fp[ent & MDX_IDX_MASK];
-        int m;
-        T p, r;
-        if constexpr (MIXED) r = eam_index_mixed(rsq, et.rdr, et.nr, m, p);
-        else {
-          r = (T)sqrt(rsq);
-          r_spline<T>(et, r, m, p);
+    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+      int ent[4];
+      double4 xj[MIXED ? 1 : 4];
+      int4 qj[MIXED ? 4 : 1];
+      double fpj[4];
+      row_chunk(row, k0, jn, i, ent);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
+        else xj[u] = gather_x(x, ent[u]);
+        fpj[u] = gather_d(fp, ent[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        double dx, dy, dz, rsq;
+        if (k0 + u < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
+                                             step, ip, dx, dy, dz, rsq)) {
+          int m;
+          T p, r, recip;
+          if constexpr (MIXED) {
+            r = eam_index_mixed(rsq, et.rdr, et.nr, m, p);
+            recip = __builtin_amdgcn_rcpf(r);  // hardware reciprocal, 1 ulp
+          } else {
+            sqrt_and_inverse(rsq, r, recip);
+            r_spline<T>(et, r, m, p);
+          }
+          const V rd = TL ? s_tab[m] : rtab[2 * m];
+          const V zd = TL ? s_tab[kn + m] : ztab[2 * m];
+          const V zv = TL ? s_tab[2 * kn + m] : ztab[2 * m + 1];
+          const T rhop = (rd.x * p + rd.y) * p + rd.z;
+          const T z2p = (zd.x * p + zd.y) * p + zd.z;
+          const T z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
+          const T phi = z2 * recip;
+          const T phip = z2p * recip - phi * recip;
+          const T psip = (T)fpi * rhop + (T)fpj[u] * rhop + phip;
+          const double fpair = (double)(-psip * recip);
+          fx += dx * fpair;
+          fy += dy * fpair;
+          fz += dz * fpair;
+          e += 0.5 * (double)phi;
         }
-        const T *c = rhor + m * 7;
-        const T rhop = (c[0] * p + c[1]) * p + c[2];
-        c = z2r + m * 7;
-        const T z2p = (c[0] * p + c[1]) * p + c[2];
-        const T z2 = ((c[3] * p + c[4]) * p + c[5]) * p + c[6];
-        const T recip = MIXED ? (T)__builtin_amdgcn_rcpf((float)r) : (T)1 / r;
-        const T phi = z2 * recip;
-        const T phip = z2p * recip - phi * recip;
-        const T psip = (T)fpi * rhop + (T)fpj * rhop + phip;
-        const double fpair = (double)(-psip * recip);
-        fx += dx * fpair;
-        fy += dy * fpair;
-        fz += dz * fpair;
-        e += 0.5 * (double)phi;
       }
     }
     fx = gsum<TPA>(fx);
@@ -737,26 +876,36 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
   }
 }
 
-// partial row layout: [frho c3..c6 (nrho+1)*4 | rhor (nr+1)*4 | z2r (nr+1)*4]
-template <bool MIXED, int TPA>
+// Adjoint passes, FP64.  A pair appears in both of its atoms' rows at one
+// distance, so the spline terms are taken once per pair (entry j > i) with
+// both rows' factors added: half the LDS atomics, which bound these passes,
+// together with their conflicts (a thermalised crystal's distances fall on a
+// few knots).  Each workgroup therefore keeps `copies` accumulator sets, one
+// per thread modulo copies, coefficient-major (neighbouring knots in
+// neighbouring banks).  Row of partials: [frho c3..c6 (nrho+1)*4 | rhor
+// (nr+1)*4 | z2r (nr+1)*4] from pass A, rhor alone from pass B.
+// stride of one accumulator set of `terms` coefficients: offset by 8 doubles
+// modulo 32 from copy to copy
+__host__ __device__ inline int adj_stride(int terms, int kn) { return (terms * kn + 31) / 32 * 32 + 8; }
+
+template <int TPA, bool TL>
 __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__restrict__ x,
                                                       const int *__restrict__ rep, const RepGeom *__restrict__ geom,
                                                       const int *__restrict__ nbr, const int *__restrict__ numneigh,
-                                                      int cap, EamTab et, const double *__restrict__ rhor_d,
-                                                      const float *__restrict__ rhor_f,
+                                                      int cap, EamTab et, const double4 *__restrict__ rhor,
                                                       const double *__restrict__ frho_d, const double *__restrict__ rho,
                                                       const double *__restrict__ fp, const double4 *__restrict__ gin,
-                                                      double *__restrict__ vout, double *__restrict__ partials) {
-  extern __shared__ double s_dyn[];
-  using T = typename std::conditional<MIXED, float, double>::type;
-  const int P = 4 * (et.nrho + 1) + 8 * (et.nr + 1);
-  double *s_gf = s_dyn, *s_gr = s_dyn + 4 * (et.nrho + 1), *s_gz = s_gr + 4 * (et.nr + 1);
-  for (int k = threadIdx.x; k < P; k += blockDim.x) s_dyn[k] = 0.0;
-  const int tn = (et.nr + 1) * 7;
-  const T *rhor;
-  if (MIXED) rhor = (const T *)stage((float *)(s_dyn + P), rhor_f, tn, false);
-  else rhor = (const T *)stage((double *)(s_dyn + P), rhor_d, tn, false);
+                                                      int copies, double *__restrict__ vout,
+                                                      double *__restrict__ partials) {
+  extern __shared__ double4 s_knots[];
+  const int kn = et.nr + 1, kf = et.nrho + 1, stride = adj_stride(7, kn);
+  double4 *const s_rd = s_knots;  // TL: rho' {c0,c1,c2,0}
+  double *const s_gf = reinterpret_cast<double *>(s_knots + (TL ? kn : 0)), *const s_g = s_gf + 3 * kf;
+  for (int k = threadIdx.x; k < 3 * kf + copies * stride; k += blockDim.x) s_gf[k] = 0.0;
+  if constexpr (TL)
+    for (int m = threadIdx.x; m < kn; m += blockDim.x) s_rd[m] = rhor[2 * m];
   __syncthreads();
+  double *const mine = s_g + (threadIdx.x % copies) * stride;  // z2r terms t*kn, then rhor terms (4+t)*kn
   const int apb = blockDim.x / TPA;
   int end;
   const int b0 = chunk_begin(n, apb, &end);
@@ -769,43 +918,46 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
     const double4 gi = gin[i];
     const double fpi = fp[i];
     const RepGeom &g = geom[rep[i]];
-    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2];
+    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double u = 0.0;
-    for (int k = lane; k < jn; k += TPA) {
-      const int ent = row[k];
-      const int j = ent & MDX_IDX_MASK;
-      double sx, sy, sz;
-      shift_of((unsigned)ent >> MDX_IDX_BITS, sx, sy, sz);
-      const double4 xj = x[j];
-      const double dx = xi.x - (xj.x + sx * px), dy = xi.y - (xj.y + sy * py), dz = xi.z - (xj.z + sz * pz);
-      const double rsq = dx * dx + dy * dy + dz * dz;
-      if (rsq < et.cutsq) {
-        const double4 gj = gin[j];
-        const double fpj = fp[j];
-        int m;
-        T p;
-        const T r = MIXED ? (T)sqrtf((float)rsq) : (T)sqrt(rsq);
-        r_spline<T>(et, r, m, p);
-        const T *c = rhor + m * 7;
-        const double rhop = (double)((c[0] * p + c[1]) * p + c[2]);
-        const double rr = (double)r;
-        const double b = -(gi.x * dx + gi.y * dy + gi.z * dz) / rr;
-        const double bs = -((gi.x - gj.x) * dx + (gi.y - gj.y) * dy + (gi.z - gj.z) * dz) / rr;
-        const double pd = (double)p;
-        const double dw0 = 3.0 * pd * pd * rdr, dw1 = 2.0 * pd * rdr, dw2 = rdr;
-        const double vw0 = pd * pd * pd, vw1 = pd * pd, vw2 = pd;
-        const double gz2p = b / rr, gz2 = -b / (rr * rr), grp = b * (fpi + fpj);
-        double *gz = s_gz + 4 * m, *gr = s_gr + 4 * m;
-        atomicAdd(gz + 0, gz2p * dw0 + gz2 * vw0);
-        atomicAdd(gz + 1, gz2p * dw1 + gz2 * vw1);
-        atomicAdd(gz + 2, gz2p * dw2 + gz2 * vw2);
-        atomicAdd(gz + 3, gz2);
-        atomicAdd(gr + 0, grp * dw0);
-        atomicAdd(gr + 1, grp * dw1);
-        atomicAdd(gr + 2, grp * dw2);
-        u += bs * rhop;
+    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+      int ent[4];
+      double4 xj[4], gj[4];
+      row_chunk(row, k0, jn, i, ent);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        xj[q] = gather_x(x, ent[q]);
+        gj[q] = gather_x(gin, ent[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        if (k0 + q >= jn) continue;
+        const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
+                     dz = nearest(xi.z - xj[q].z, pz, iz);
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        if (rsq < et.cutsq) {
+          double r, ri, p;
+          int m;
+          sqrt_and_inverse(rsq, r, ri);
+          r_spline<double>(et, r, m, p);
+          const double4 c = TL ? s_rd[m] : rhor[2 * m];
+          const double b = -((gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz) * ri;
+          u += b * ((c.x * p + c.y) * p + c.z);
+          const int j = ent[q] & MDX_IDX_MASK;
+          if (j > i) {
+            const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * (fpi + fp[j]) * rdr, gzr = gz1 * rdr, pp = p * p;
+            double *a = mine + m;
+            atomicAdd(a, 3.0 * pp * gzr + gz0 * pp * p);
+            atomicAdd(a + kn, 2.0 * p * gzr + gz0 * pp);
+            atomicAdd(a + 2 * kn, gzr + gz0 * p);
+            atomicAdd(a + 3 * kn, gz0);
+            atomicAdd(a + 4 * kn, 3.0 * pp * grp);
+            atomicAdd(a + 5 * kn, 2.0 * p * grp);
+            atomicAdd(a + 6 * kn, grp);
+          }
+        }
       }
     }
     u = gsum<TPA>(u);
@@ -819,32 +971,42 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
       const bool clamped = p > 1.0;
       p = fmin(p, 1.0);
       const double rdrho = et.rdrho;
-      double *gf = s_gf + 4 * m;
-      atomicAdd(gf + 0, u * 3.0 * p * p * rdrho);
-      atomicAdd(gf + 1, u * 2.0 * p * rdrho);
-      atomicAdd(gf + 2, u * rdrho);
+      atomicAdd(s_gf + m, u * 3.0 * p * p * rdrho);
+      atomicAdd(s_gf + kf + m, u * 2.0 * p * rdrho);
+      atomicAdd(s_gf + 2 * kf + m, u * rdrho);
       const double *c = frho_d + m * 7;
       const double fpp = clamped ? 0.0 : (2.0 * c[0] * p + c[1]) * rdrho;
       vout[i] = u * fpp;
     }
   }
   __syncthreads();
+  const int P = 4 * kf + 8 * kn;
   double *out = partials + (size_t)blockIdx.x * P;
-  for (int k = threadIdx.x; k < P; k += blockDim.x) out[k] = s_dyn[k];
+  for (int k = threadIdx.x; k < P; k += blockDim.x) {
+    double v = 0.0;
+    if (k < 4 * kf) {
+      if ((k & 3) < 3) v = s_gf[(k & 3) * kf + (k >> 2)];
+    } else {
+      const int q = k - 4 * kf, z = q >= 4 * kn, m = (z ? q - 4 * kn : q) >> 2, t = q & 3;
+      if (z || t < 3)
+        for (int c = 0; c < copies; c++) v += s_g[c * stride + (z ? t : 4 + t) * kn + m];
+    }
+    out[k] = v;
+  }
 }
 
-template <bool MIXED, int TPA>
+template <int TPA>
 __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__restrict__ x,
                                                       const int *__restrict__ rep, const RepGeom *__restrict__ geom,
                                                       const int *__restrict__ nbr, const int *__restrict__ numneigh,
-                                                      int cap, EamTab et, const double *__restrict__ vin,
+                                                      int cap, EamTab et, const double *__restrict__ vin, int copies,
                                                       double *__restrict__ partials) {
-  extern __shared__ double s_dyn[];
-  using T = typename std::conditional<MIXED, float, double>::type;
-  const int P = 4 * (et.nrho + 1) + 8 * (et.nr + 1);
-  double *s_gr = s_dyn + 4 * (et.nrho + 1);
-  for (int k = threadIdx.x; k < P; k += blockDim.x) s_dyn[k] = 0.0;
+  extern __shared__ double4 s_knots[];
+  const int kn = et.nr + 1, stride = adj_stride(4, kn);
+  double *const s_g = reinterpret_cast<double *>(s_knots);
+  for (int k = threadIdx.x; k < copies * stride; k += blockDim.x) s_g[k] = 0.0;
   __syncthreads();
+  double *const mine = s_g + (threadIdx.x % copies) * stride;
   const int apb = blockDim.x / TPA;
   int end;
   const int b0 = chunk_begin(n, apb, &end);
@@ -853,36 +1015,53 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
     const double vi = vin[i];
-    if (vi == 0.0) continue;
     const double4 xi = x[i];
     const RepGeom &g = geom[rep[i]];
-    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2];
+    const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
-    for (int k = lane; k < jn; k += TPA) {
-      const int ent = row[k];
-      const int j = ent & MDX_IDX_MASK;
-      double sx, sy, sz;
-      shift_of((unsigned)ent >> MDX_IDX_BITS, sx, sy, sz);
-      const double4 xj = x[j];
-      const double dx = xi.x - (xj.x + sx * px), dy = xi.y - (xj.y + sy * py), dz = xi.z - (xj.z + sz * pz);
-      const double rsq = dx * dx + dy * dy + dz * dz;
-      if (rsq < et.cutsq) {
-        int m;
-        T p;
-        r_spline<T>(et, MIXED ? (T)sqrtf((float)rsq) : (T)sqrt(rsq), m, p);
-        const double pd = (double)p;
-        double *gr = s_gr + 4 * m;
-        atomicAdd(gr + 0, vi * pd * pd * pd);
-        atomicAdd(gr + 1, vi * pd * pd);
-        atomicAdd(gr + 2, vi * pd);
-        atomicAdd(gr + 3, vi);
+    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+      int ent[4];
+      double4 xj[4];
+      double vj[4];
+      row_chunk(row, k0, jn, i, ent);
+      bool any = false;
+#pragma unroll
+      for (int q = 0; q < 4; q++) any |= (ent[q] & MDX_IDX_MASK) > i;
+      if (!any) continue;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        xj[q] = gather_x(x, ent[q]);
+        vj[q] = gather_d(vin, ent[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        if ((ent[q] & MDX_IDX_MASK) <= i) continue;  // the pair's other row, or past the end
+        const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
+                     dz = nearest(xi.z - xj[q].z, pz, iz);
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        const double v = vi + vj[q];
+        if (rsq < et.cutsq && v != 0.0) {
+          double r, ri, p;
+          int m;
+          sqrt_and_inverse(rsq, r, ri);
+          r_spline<double>(et, r, m, p);
+          double *a = mine + m;
+          atomicAdd(a, v * p * p * p);
+          atomicAdd(a + kn, v * p * p);
+          atomicAdd(a + 2 * kn, v * p);
+          atomicAdd(a + 3 * kn, v);
+        }
       }
     }
   }
   __syncthreads();
-  double *out = partials + (size_t)blockIdx.x * P;
-  for (int k = threadIdx.x; k < P; k += blockDim.x) out[k] = s_dyn[k];
+  double *out = partials + (size_t)blockIdx.x * 4 * kn;
+  for (int k = threadIdx.x; k < 4 * kn; k += blockDim.x) {
+    double v = 0.0;
+    for (int c = 0; c < copies; c++) v += s_g[c * stride + (k & 3) * kn + (k >> 2)];
+    out[k] = v;
+  }
 }
 
 // ---------------------------------------------------------------- utilities
@@ -891,33 +1070,42 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
 // (deterministic): k_b_colsum_chunks sums chunk ry of the rows (rows
 // [rows*ry/nchunk, rows*(ry+1)/nchunk)) for 64 columns per block, four row
 // lanes per column combined in LDS; k_b_colsum then sums the nchunk chunk
-// rows.  One thread per column over every row leaves the device mostly idle
-// (a few hundred columns, thousands of rows).
+// rows the same way, into mapped host memory.  A second set of rows (partB)
+// covers colsB columns from c0B on.
 constexpr int kColChunks = 64;
+__device__ __forceinline__ void colsum_store(double (&s)[4][64], double acc, int c, int cols, double *out) {
+  const int l = threadIdx.x & 63, sub = threadIdx.x >> 6;
+  s[sub][l] = acc;
+  __syncthreads();
+  if (sub == 0 && c < cols) out[c] = ((s[0][l] + s[1][l]) + s[2][l]) + s[3][l];
+}
 __global__ __launch_bounds__(256) void k_b_colsum_chunks(const double *__restrict__ part, int rows, int cols,
-                                                         double *__restrict__ mid) {
+                                                         const double *__restrict__ partB, int rowsB, int c0B,
+                                                         int colsB, double *__restrict__ mid) {
   __shared__ double s[4][64];
   const int c = blockIdx.x * 64 + (threadIdx.x & 63), sub = threadIdx.x >> 6;
   const int ry = blockIdx.y, nchunk = gridDim.y;
-  const int r0 = (int)((long)rows * ry / nchunk), r1 = (int)((long)rows * (ry + 1) / nchunk);
+  double acc = 0.0;
+  if (c < cols) {
+    const int r0 = (int)((long)rows * ry / nchunk), r1 = (int)((long)rows * (ry + 1) / nchunk);
+    for (int r = r0 + sub; r < r1; r += 4) acc += part[(size_t)r * cols + c];
+  }
+  const int cb = c - c0B;
+  if (cb >= 0 && cb < colsB) {
+    const int r0 = (int)((long)rowsB * ry / nchunk), r1 = (int)((long)rowsB * (ry + 1) / nchunk);
+    for (int r = r0 + sub; r < r1; r += 4) acc += partB[(size_t)r * colsB + cb];
+  }
+  colsum_store(s, acc, c, cols, mid + (size_t)ry * cols);
+}
+__global__ __launch_bounds__(256) void k_b_colsum(const double *__restrict__ mid, int rows, int cols,
+                                                  double *__restrict__ out) {
+  __shared__ double s[4][64];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63);
   double acc = 0.0;
   if (c < cols)
-    for (int r = r0 + sub; r < r1; r += 4) acc += part[(size_t)r * cols + c];
-  s[sub][threadIdx.x & 63] = acc;
-  __syncthreads();
-  if (sub == 0 && c < cols) {
-    const int l = threadIdx.x & 63;
-    mid[(size_t)ry * cols + c] = ((s[0][l] + s[1][l]) + s[2][l]) + s[3][l];
-  }
-}
-
-// column sums over rows in a fixed order (deterministic)
-__global__ void k_b_colsum(const double *__restrict__ part, int rows, int cols, double *__restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  double s = 0.0;
-  for (int r = 0; r < rows; r++) s += part[(size_t)r * cols + c];
-  out[c] = s;
+#pragma unroll 4
+    for (int r = threadIdx.x >> 6; r < rows; r += 4) acc += mid[(size_t)r * cols + c];
+  colsum_store(s, acc, c, cols, out);
 }
 
 // per-replica energy: one block per replica, fixed-order tree
@@ -999,14 +1187,18 @@ struct mdx_batch {
   size_t partials_cap = 0;  // doubles
   double *colsum = nullptr;
   size_t colsum_cap = 0;
+  double *sums_host = nullptr;  // mapped: the column sums
+  size_t sums_cap = 0;
   // pair
   int pair = MDX_PAIR_NONE;
   double *ljtab = nullptr;  // T_N * kNT
   double lj_cutmax = 0.0;
   std::vector<double> lj_tab;  // the table last uploaded (a repeated init uploads nothing)
   EamTab et{};
-  double *frho_d = nullptr, *rhor_d = nullptr, *z2r_d = nullptr;
-  float *rhor_f = nullptr, *z2r_f = nullptr;
+  double *frho_d = nullptr;
+  EamKnots knots{};             // packed rhor and z2r (into knots_d, knots_f)
+  double4 *knots_d = nullptr;
+  float4 *knots_f = nullptr;
   std::vector<double> eam_knots[3];
   double eam_drho = 0.0, eam_dr = 0.0, eam_cut = 0.0;
   int eam_rho_prec = -1;  // precision of the rho/fp on the device for the current positions and tables (-1: stale)
@@ -1074,6 +1266,7 @@ int timed(mdx_batch *b, int kind, const Tune &t, F &&launch, float *ms_out = nul
 
 // kernels that flush per-block partial rows cap the grid at kPartialBlocksPerCU per CU
 constexpr int kPartialBlocksPerCU = 8;
+constexpr size_t kAdjLDS = 20480;  // LDS per workgroup of the eam adjoint with small tables
 int persistent_grid(mdx_batch *b, const Tune &t, bool partial_rows = false) {
   const int apb = t.block / t.tpa;
   const long tiles = (b->n + apb - 1) / apb;
@@ -1140,20 +1333,29 @@ int ensure_partials(mdx_batch *b, size_t doubles) {
   return dalloc(&b->partials, doubles);
 }
 
-int colsum(mdx_batch *b, int rows, int cols, std::vector<double> &out) {
-  const size_t need = (size_t)(kColChunks + 1) * cols;  // chunk sums, then the result
+// column sums of `rows` partial rows (and rowsB rows of colsB columns at partB,
+// into the columns from c0B on), left in b->sums_host when this returns
+int colsum(mdx_batch *b, int rows, int cols, const double *partB = nullptr, int rowsB = 0, int c0B = 0, int colsB = 0) {
+  const size_t need = (size_t)kColChunks * cols;
   if (need > b->colsum_cap) {
     int rc = dalloc(&b->colsum, need);
     if (rc) return rc;
     b->colsum_cap = need;
   }
-  const int nchunk = std::max(1, std::min(kColChunks, rows));
-  double *mid = b->colsum + cols;
+  if ((size_t)cols > b->sums_cap) {
+    if (b->sums_host) (void)hipHostFree(b->sums_host);
+    b->sums_host = nullptr;
+    b->sums_cap = 0;
+    hipError_t e = hipHostMalloc(&b->sums_host, sizeof(double) * cols, hipHostMallocCoherent | hipHostMallocMapped);
+    if (e != hipSuccess) return bfail(e, "gradient buffer");
+    b->sums_cap = cols;
+  }
+  const int nchunk = std::max(1, std::min(kColChunks, std::max(rows, rowsB)));
   hipLaunchKernelGGL(k_b_colsum_chunks, dim3((cols + 63) / 64, nchunk), dim3(256), 0, b->stream, b->partials, rows,
-                     cols, mid);
-  hipLaunchKernelGGL(k_b_colsum, dim3((cols + 255) / 256), dim3(256), 0, b->stream, mid, nchunk, cols, b->colsum);
-  out.assign(cols, 0.0);
-  hipError_t e = hipMemcpyAsync(out.data(), b->colsum, sizeof(double) * cols, hipMemcpyDeviceToHost, b->stream);
+                     cols, partB, rowsB, c0B, colsB, b->colsum);
+  hipLaunchKernelGGL(k_b_colsum, dim3((cols + 63) / 64), dim3(256), 0, b->stream, b->colsum, nchunk, cols,
+                     b->sums_host);
+  hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
   return e == hipSuccess ? MDX_OK : bfail(e, "gradient reduction");
 }
@@ -1338,16 +1540,36 @@ void spline_coeffs(int n, const double *f /* [n] */, double *c /* (n+1)*4: c3..c
   }
 }
 
+// dL/d(knots) from dL/d(c3..c6): the transpose of spline_coeffs, one sweep
 void knot_gradient(int n, const double *gc, double *g) {
-  std::vector<double> e(n, 0.0), c(4 * (n + 1));
-  for (int k = 0; k < n; k++) {
-    e[k] = 1.0;
-    spline_coeffs(n, e.data(), c.data());
-    double acc = 0.0;
-    for (int t = 4; t < 4 * (n + 1); t++) acc += gc[t] * c[t];
-    g[k] = acc;
-    e[k] = 0.0;
+  std::vector<double> gk(n + 1, 0.0), g5(n + 1, 0.0);  // by knot 1..n: F and c5
+  for (int m = 1; m <= n; m++) {
+    g5[m] += gc[4 * m + 2];
+    gk[m] += gc[4 * m + 3];
   }
+  for (int m = 1; m <= n - 1; m++) {
+    const double a = gc[4 * m], b = gc[4 * m + 1];
+    gk[m + 1] += 3.0 * b - 2.0 * a;
+    gk[m] -= 3.0 * b - 2.0 * a;
+    g5[m] += a - 2.0 * b;
+    g5[m + 1] += a - b;
+  }
+  gk[2] += g5[1];
+  gk[1] -= g5[1];
+  gk[3] += 0.5 * g5[2];
+  gk[1] -= 0.5 * g5[2];
+  gk[n] += 0.5 * g5[n - 1];
+  gk[n - 2] -= 0.5 * g5[n - 1];
+  gk[n] += g5[n];
+  gk[n - 1] -= g5[n];
+  for (int m = 3; m <= n - 2; m++) {
+    const double q = g5[m] / 12.0;
+    gk[m - 2] += q;
+    gk[m + 2] -= q;
+    gk[m + 1] += 8.0 * q;
+    gk[m - 1] -= 8.0 * q;
+  }
+  for (int k = 0; k < n; k++) g[k] = gk[k + 1];
 }
 
 // full 7-coefficient table from knots (host copy uploaded to the device)
@@ -1429,6 +1651,7 @@ int mdx_batch_create(int device, int nrep, const int *natoms, const double *lo, 
       const double span = periodic[3 * r + d] ? 4294967296.0 : 1073741824.0;
       b->geom_h[r].qscale[d] = span / b->geom_h[r].prd[d];
       b->geom_h[r].qstep[d] = b->geom_h[r].prd[d] / span;
+      b->geom_h[r].iprd[d] = periodic[3 * r + d] ? 1.0 / b->geom_h[r].prd[d] : 0.0;
     }
   hipError_t e;
   int rc;
@@ -1476,10 +1699,11 @@ int mdx_batch_destroy(mdx_batch *b) {
                   b->f,       b->g,        b->rep,      b->orig,     b->inv,     b->key,     b->slot,    b->order,
                   b->bin_count, b->bin_start, b->scan_tmp, b->nbr,    b->numneigh, b->dflags,
                   b->rho,     b->fp,       b->eemb,     b->vadj,     b->partials, b->colsum,  b->ljtab,   b->frho_d,
-                  b->rhor_d,  b->z2r_d,    b->rhor_f,   b->z2r_f};
+                  b->knots_d, b->knots_f};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->flags_host) (void)hipHostFree(b->flags_host);
+  if (b->sums_host) (void)hipHostFree(b->sums_host);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->own_stream) {
@@ -1635,23 +1859,25 @@ int mdx_batch_lj_vjp(mdx_batch *b, const double *gf, double *geps, double *gsigm
   auto launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);
     grid_used = G;
-    TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_lj_vjp<false, TP>), dim3(G), dim3(t.block), 0, b->stream, b->n, nt1,
-                                           b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->ljtab, b->g,
-                                           b->partials))
+    auto go = [&](auto nt) {
+      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_lj_vjp<decltype(nt)::value, TP>), dim3(G), dim3(t.block), 0,
+                                             b->stream, b->n, nt1, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
+                                             b->ljtab, b->g, b->partials))
+    };
+    if (b->ntypes == 1) go(std::integral_constant<int, 1>{});
+    else if (b->ntypes == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, MDX_MAXT>{});
   };
   // partial rows for the largest grid any candidate can use
   const long maxgrid = (long)kPartialBlocksPerCU * b->num_cu;
-  if ((rc = ensure_partials(b, (size_t)maxgrid * 2 * kNT))) return rc;
+  if ((rc = ensure_partials(b, (size_t)maxgrid * 2 * nt1 * nt1))) return rc;
   if ((rc = run_kind(b, MDX_BK_LJ_VJP, launch))) return rc;
-  std::vector<double> sums;
-  if ((rc = colsum(b, grid_used, 2 * kNT, sums))) return rc;
-  for (int k = 0; k < nt1 * nt1; k++) geps[k] = gsigma[k] = 0.0;
-  for (int a = 1; a < nt1; a++)
-    for (int c = 1; c < nt1; c++) {
-      const int lo = std::min(a, c), hi = std::max(a, c);
-      geps[lo * nt1 + hi] += sums[a * nt1 + c];
-      gsigma[lo * nt1 + hi] += sums[kNT + a * nt1 + c];
-    }
+  const int cols = nt1 * nt1;
+  if ((rc = colsum(b, grid_used, 2 * cols))) return rc;
+  for (int k = 0; k < cols; k++) {
+    geps[k] = b->sums_host[k];
+    gsigma[k] = b->sums_host[cols + k];
+  }
   return MDX_OK;
 }
 
@@ -1671,21 +1897,28 @@ int mdx_batch_eam_init(mdx_batch *b, int nrho, double drho, int nr, double dr, d
   spline7(nrho, drho, frho, sf);
   spline7(nr, dr, rhor, sr);
   spline7(nr, dr, z2r, sz);
-  std::vector<float> fr(sr.begin(), sr.end()), fz(sz.begin(), sz.end());
+  // rhor and z2r as two 4-vectors per knot, in both precisions
+  const size_t kn = (size_t)nr + 1;
+  std::vector<double4> kd(4 * kn);
+  std::vector<float4> kf(4 * kn);
+  for (size_t q = 0; q < 2 * kn; q++) {
+    const double *c = (q < kn ? sr.data() + 7 * q : sz.data() + 7 * (q - kn));
+    kd[2 * q] = make_double4(c[0], c[1], c[2], 0.0);
+    kd[2 * q + 1] = make_double4(c[3], c[4], c[5], c[6]);
+    kf[2 * q] = make_float4((float)c[0], (float)c[1], (float)c[2], 0.0f);
+    kf[2 * q + 1] = make_float4((float)c[3], (float)c[4], (float)c[5], (float)c[6]);
+  }
   if (b->et.nrho != nrho || !b->frho_d) {
     if ((rc = dalloc(&b->frho_d, sf.size()))) return rc;
   }
-  if (b->et.nr != nr || !b->rhor_d) {
-    if ((rc = dalloc(&b->rhor_d, sr.size())) || (rc = dalloc(&b->z2r_d, sz.size())) ||
-        (rc = dalloc(&b->rhor_f, fr.size())) || (rc = dalloc(&b->z2r_f, fz.size())))
-      return rc;
+  if (b->et.nr != nr || !b->knots_d) {
+    if ((rc = dalloc(&b->knots_d, kd.size())) || (rc = dalloc(&b->knots_f, kf.size()))) return rc;
   }
   if ((rc = upload(b->frho_d, sf.data(), sizeof(double) * sf.size())) ||
-      (rc = upload(b->rhor_d, sr.data(), sizeof(double) * sr.size())) ||
-      (rc = upload(b->z2r_d, sz.data(), sizeof(double) * sz.size())) ||
-      (rc = upload(b->rhor_f, fr.data(), sizeof(float) * fr.size())) ||
-      (rc = upload(b->z2r_f, fz.data(), sizeof(float) * fz.size())))
+      (rc = upload(b->knots_d, kd.data(), sizeof(double4) * kd.size())) ||
+      (rc = upload(b->knots_f, kf.data(), sizeof(float4) * kf.size())))
     return rc;
+  b->knots = {b->knots_d, b->knots_d + 2 * kn, b->knots_f, b->knots_f + 2 * kn};
   b->et.nrho = nrho;
   b->et.nr = nr;
   b->et.rdrho = 1.0 / drho;
@@ -1709,36 +1942,35 @@ int eam_forward(mdx_batch *b, bool with_force, int precision) {
   int rc;
   if ((rc = ensure_built(b))) return rc;
   const bool mixed = precision == MDX_MIXED;
-  const int tn = (b->et.nr + 1) * 7;
-  const size_t esz = mixed ? sizeof(float) : sizeof(double);
-  const bool lds1 = (size_t)tn * esz <= (size_t)kTabLDS * 8;
-  const bool lds2 = (size_t)2 * tn * esz <= (size_t)kTabLDS * 8;
-  const size_t sh1 = lds1 ? tn * esz : 0, sh2 = lds2 ? 2 * tn * esz : 0;
+  const size_t vec = (size_t)(b->et.nr + 1) * (mixed ? sizeof(float4) : sizeof(double4));
+  const bool lds1 = vec <= (size_t)kTabLDS * 8, lds2 = 3 * vec <= (size_t)kTabLDS * 8;
+  // precision and table place as types, threads per atom from the tune
+  auto choose = [&](bool lds, auto &&go) {
+    if (mixed && lds) go(std::true_type{}, std::true_type{});
+    else if (mixed) go(std::true_type{}, std::false_type{});
+    else if (lds) go(std::false_type{}, std::true_type{});
+    else go(std::false_type{}, std::false_type{});
+  };
   auto rho_launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t);
-    if (mixed)
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_rho<true, TP>), dim3(G), dim3(t.block), sh1, b->stream, b->n,
-                                             b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->rhor_d,
-                                             b->rhor_f, b->frho_d, lds1 ? 1 : 0, b->rho, b->fp, b->eemb))
-    else
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_rho<false, TP>), dim3(G), dim3(t.block), sh1, b->stream, b->n,
-                                             b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->rhor_d,
-                                             b->rhor_f, b->frho_d, lds1 ? 1 : 0, b->rho, b->fp, b->eemb))
+    choose(lds1, [&](auto mx, auto tl) {
+      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_rho<decltype(mx)::value, TP, decltype(tl)::value>), dim3(G),
+                                             dim3(t.block), lds1 ? vec : 0, b->stream, b->n, b->x, b->xq, b->rep,
+                                             b->geom, b->nbr, b->numneigh, b->cap, b->et, b->knots, b->frho_d, b->rho,
+                                             b->fp, b->eemb))
+    });
   };
   if ((rc = run_kind(b, MDX_BK_EAM_RHO, rho_launch))) return rc;
   b->eam_rho_prec = precision;
   if (!with_force) return MDX_OK;
   auto force_launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t);
-    if (mixed)
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_force<true, TP>), dim3(G), dim3(t.block), sh2, b->stream, b->n,
-                                             b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->rhor_d,
-                                             b->z2r_d, b->rhor_f, b->z2r_f, lds2 ? 1 : 0, b->fp, b->eemb, b->f))
-    else
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_force<false, TP>), dim3(G), dim3(t.block), sh2, b->stream,
-                                             b->n, b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et,
-                                             b->rhor_d, b->z2r_d, b->rhor_f, b->z2r_f, lds2 ? 1 : 0, b->fp, b->eemb,
+    choose(lds2, [&](auto mx, auto tl) {
+      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_force<decltype(mx)::value, TP, decltype(tl)::value>), dim3(G),
+                                             dim3(t.block), lds2 ? 3 * vec : 0, b->stream, b->n, b->x, b->xq, b->rep,
+                                             b->geom, b->nbr, b->numneigh, b->cap, b->et, b->knots, b->fp, b->eemb,
                                              b->f))
+    });
   };
   return run_kind(b, MDX_BK_EAM_FORCE, force_launch);
 }
@@ -1790,36 +2022,48 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
   if ((rc = read_g(b, gf))) return rc;
   // FP64 adjoint arithmetic in both precision modes, as for lj/cut
   const int P = 4 * (b->et.nrho + 1) + 8 * (b->et.nr + 1);
-  const size_t shA = sizeof(double) * P, shB = sizeof(double) * P;
-  if ((long)shA > b->lds_max) {
+  if ((long)sizeof(double) * P > b->lds_max) {
     set_error("eam tables too large for the adjoint's LDS accumulators");
     return MDX_ERR_ARG;
   }
+  const int kn = b->et.nr + 1, kf = b->et.nrho + 1;
+  // accumulator sets per workgroup: as many of 4, 2, 1 as keep it within an
+  // eighth of a CU's LDS (small tables), and rho' beside them if it fits
+  const size_t tabA = sizeof(double4) * kn, gfA = sizeof(double) * 3 * kf, setA = sizeof(double) * adj_stride(7, kn),
+               setB = sizeof(double) * adj_stride(4, kn);
+  int cA = 4, cB = 4;
+  while (cA > 1 && gfA + tabA + cA * setA > kAdjLDS) cA /= 2;
+  while (cB > 1 && cB * setB > kAdjLDS) cB /= 2;
+  const bool tlA = tabA + gfA + cA * setA <= (size_t)b->lds_max;
+  const size_t shA = (tlA ? tabA : 0) + gfA + cA * setA, shB = cB * setB;
   const long maxgrid = (long)kPartialBlocksPerCU * b->num_cu;
-  if ((rc = ensure_partials(b, (size_t)2 * maxgrid * P))) return rc;
+  if ((rc = ensure_partials(b, (size_t)maxgrid * (P + 4 * kn)))) return rc;
   int gA = 0, gB = 0;
   auto launchA = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);
     gA = G;
-    TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_a<false, TP>), dim3(G), dim3(t.block), shA, b->stream, b->n,
-                                           b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->rhor_d,
-                                           b->rhor_f, b->frho_d, b->rho, b->fp, b->g, b->vadj, b->partials))
+    auto go = [&](auto tl) {
+      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_a<TP, decltype(tl)::value>), dim3(G), dim3(t.block), shA,
+                                             b->stream, b->n, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
+                                             b->et, b->knots.rhor_d, b->frho_d, b->rho, b->fp, b->g, cA, b->vadj,
+                                             b->partials))
+    };
+    if (tlA) go(std::true_type{});
+    else go(std::false_type{});
   };
   if ((rc = run_kind(b, MDX_BK_EAM_ADJ_A, launchA))) return rc;
   double *partB = b->partials + (size_t)gA * P;
   auto launchB = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);
     gB = G;
-    TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_b<false, TP>), dim3(G), dim3(t.block), shB, b->stream, b->n,
-                                           b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->vadj, partB))
+    TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_b<TP>), dim3(G), dim3(t.block), shB, b->stream, b->n, b->x,
+                                           b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->vadj, cB, partB))
   };
   if ((rc = run_kind(b, MDX_BK_EAM_ADJ_B, launchB))) return rc;
-  std::vector<double> gc;
-  if ((rc = colsum(b, gA + gB, P, gc))) return rc;
-  const int nrho = b->et.nrho, nr = b->et.nr;
-  knot_gradient(nrho, gc.data(), g_frho);
-  knot_gradient(nr, gc.data() + 4 * (nrho + 1), g_rhor);
-  knot_gradient(nr, gc.data() + 4 * (nrho + 1) + 4 * (nr + 1), g_z2r);
+  if ((rc = colsum(b, gA, P, partB, gB, 4 * kf, 4 * kn))) return rc;
+  knot_gradient(b->et.nrho, b->sums_host, g_frho);
+  knot_gradient(b->et.nr, b->sums_host + 4 * kf, g_rhor);
+  knot_gradient(b->et.nr, b->sums_host + 4 * kf + 4 * kn, g_z2r);
   return MDX_OK;
 }
 
