@@ -89,7 +89,9 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
 
 /* Launch shape per kernel kind: block (64..1024, multiple of 64), threads
    per atom (1..64, power of two), grid (blocks; 0 = one block per
-   atom tile).  Kernels loop over their share of atoms, so any grid is valid. */
+   atom tile).  Kernels loop over their share of atoms, so any grid is valid.
+   A kind that was neither set nor tuned takes a shape for the batch's size;
+   the list build always takes its own. */
 int mdx_batch_set_launch(mdx_batch *b, int kind, int block, int tpa, int grid);
 int mdx_batch_get_launch(mdx_batch *b, int kind, int *block, int *tpa, int *grid);
 /* Autotuner: when on, the next call of each kernel kind times a set of

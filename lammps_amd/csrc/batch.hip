@@ -85,7 +85,7 @@ struct EamTab {
 };
 
 struct Tune {
-  int block = 256, tpa = 8, grid = 0;
+  int block = 0, tpa = 0, grid = 0;  // tpa 0: by default_tune
 };
 
 __device__ __forceinline__ int chunk_begin(int n, int apb, int *end) {
@@ -1244,6 +1244,30 @@ int check_b(mdx_batch *b) {
   return e == hipSuccess ? MDX_OK : bfail(e, "hipSetDevice");
 }
 
+// The launch shape of a kernel kind that was neither set nor tuned.  A grid
+// of as many workgroups as the chip holds at once (512 threads, two per CU)
+// lets each copy its tables to LDS once and loop; four lanes per atom read a
+// row in whole 64-B pieces and waste the least.  Small batches take more
+// lanes per atom, as one launch is then one chain of loads.  Measured (us):
+//   eam 1.37 M atoms, one workgroup of 256 at 8 lanes per tile (the former
+//   default) against this: rho 347 / 156, force 538 / 198, FP64 rho 435 / 196,
+//   adjoint 525 / 414 and 256 / 188; lj 512,000 atoms: forces 111 / 85 mixed,
+//   134 / 118 FP64, gradient 192 / 158
+//   at 4 / 16 lanes: eam 3,164 atoms rho 12.7 / 7.9, adjoint 29 / 15.5, 22,401
+//   atoms 9.5 / 12.3 and 22.7 / 25.3; lj 21,952 atoms 21.5 / 17.6, 101,250
+//   atoms 35 / 46; 16 / 32 lanes: lj 4,000 atoms 10.4 / 9.5
+Tune default_tune(const mdx_batch *b, int kind) {
+  Tune t;
+  const bool lj = kind == MDX_BK_LJ || kind == MDX_BK_LJ_VJP;
+  const bool large = b->n > (lj ? 50000 : 10000);
+  t.tpa = large ? 4 : lj && b->n <= 10000 ? 32 : 16;
+  t.block = large ? 512 : 256;
+  t.grid = (large ? 2 : 4) * b->num_cu;
+  return t;
+}
+
+Tune tune_of(const mdx_batch *b, int kind) { return b->tune[kind].tpa ? b->tune[kind] : default_tune(b, kind); }
+
 // run one launch of kind `kind` under timing; `launch(tune)` enqueues it
 template <typename F>
 int timed(mdx_batch *b, int kind, const Tune &t, F &&launch, float *ms_out = nullptr, bool count = true) {
@@ -1298,7 +1322,7 @@ template <typename F>
 int run_kind(mdx_batch *b, int kind, F &&launch) {
   if (b->autotune && !b->tuned[kind]) {
     float best = 1e30f;
-    Tune bt = b->tune[kind];
+    Tune bt = tune_of(b, kind);
     for (const Tune &t : candidates(b)) {
       float ms = 0.0f;
       for (int rep = 0; rep < 2; rep++) {  // second timing counts (warm caches)
@@ -1313,7 +1337,7 @@ int run_kind(mdx_batch *b, int kind, F &&launch) {
     b->tune[kind] = bt;
     b->tuned[kind] = true;
   }
-  return timed(b, kind, b->tune[kind], launch);
+  return timed(b, kind, tune_of(b, kind), launch);
 }
 
 #define TPA_DISPATCH(tpa, CALL)                      \
@@ -2089,9 +2113,10 @@ int mdx_batch_get_launch(mdx_batch *b, int kind, int *block, int *tpa, int *grid
     set_error("invalid kernel kind");
     return MDX_ERR_ARG;
   }
-  if (block) *block = b->tune[kind].block;
-  if (tpa) *tpa = b->tune[kind].tpa;
-  if (grid) *grid = b->tune[kind].grid;
+  const Tune t = tune_of(b, kind);
+  if (block) *block = t.block;
+  if (tpa) *tpa = t.tpa;
+  if (grid) *grid = t.grid;
   return MDX_OK;
 }
 
