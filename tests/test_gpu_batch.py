@@ -291,3 +291,78 @@ def test_neighbour_counts_match_brute_force(side, density):
             counts.append(int(np.sum(np.sum(d * d, 1) < 2.5 ** 2)) - 1)
     assert total == sum(counts) and most == max(counts)
     b.close()
+
+
+@pytest.mark.parametrize("ntypes", [1, 3, 8])
+def test_lj_gradient_for_other_type_counts(ntypes):
+    """One type, and the general kernel of three or more (two: the
+    Kob-Andersen tests): forces and gradients equal the oracle's, a periodic
+    box and a free one, a different cutoff for every type pair."""
+    rng = np.random.default_rng(ntypes)
+    L, n = 9.3, (701, 307)
+    grid = np.stack(np.meshgrid(*(np.arange(9),) * 3, indexing="ij"), -1).reshape(-1, 3) * (L / 9) + 0.2
+    x = np.concatenate([grid[rng.permutation(len(grid))[:m]] + rng.uniform(-0.15, 0.15, (m, 3)) for m in n])
+    t = rng.integers(1, ntypes + 1, len(x)).astype(np.int32)
+    e, s, c = (np.zeros((ntypes + 1, ntypes + 1)) for _ in range(3))
+    for i in range(1, ntypes + 1):
+        for j in range(i, ntypes + 1):
+            e[i, j] = e[j, i] = rng.uniform(0.5, 1.5)
+            s[i, j] = s[j, i] = rng.uniform(0.8, 1.0)
+            c[i, j] = c[j, i] = rng.uniform(2.0, 2.5)
+    geo = (list(n), [[0, 0, 0], [0, 0, 0]], [[L, L, L]] * 2, [[1, 1, 1], [0, 0, 0]], ntypes, t)
+    x = np.clip(x, 0.0, L - 1e-9)
+    ref = FR.Batch(*geo, x)
+    G = rng.normal(size=x.shape)
+    ge_ref, gs_ref = ref.lj_vjp(e, s, c, G)
+    b = B.Batch(*geo)
+    b.set_positions(x)
+    b.lj_init(e, s, c)
+    assert force_errors(b.lj_forces()[0], ref.lj_forces(e, s, c)[0])[0] <= 1e-11
+    ge, gs = b.lj_vjp(G)
+    assert rel(ge, ge_ref) <= 1e-9 and rel(gs, gs_ref) <= 1e-9
+    b.close()
+
+
+@pytest.mark.parametrize("nknots", [16, 300, 511, 512, 660])
+def test_eam_table_sizes(nknots):
+    """Tables in LDS and beyond it (the FP64 force pass to 511 knots, several
+    adjoint accumulator sets only below ~90): forces and knot gradients equal
+    the oracle's."""
+    pot = W.synthetic_knots(nknots)
+    rng = np.random.default_rng(nknots)
+    xs = [q + rng.normal(scale=0.1, size=q.shape) for q in (W.fcc_cluster(331), W.fcc_cluster(120))]
+    x = np.concatenate(xs)
+    geo = ([len(q) for q in xs], [q.min(0) - 2.0 for q in xs], [q.max(0) + 2.0 for q in xs], [[0, 0, 0]] * 2, 1,
+           np.ones(len(x), np.int32))
+    ref = FR.Batch(*geo, x)
+    ref.eam_set(pot["drho"], pot["dr"], pot["cut"], pot["frho"], pot["rhor"], pot["z2r"])
+    G = rng.normal(size=x.shape)
+    g_ref = ref.eam_vjp(G)
+    f_ref = ref.eam_forces()[0]
+    for prec, tol in ((B.FP64, 1e-11), (B.MIXED, 1e-5)):
+        b = B.Batch(*geo)
+        b.set_positions(x)
+        b.precision(prec)
+        b.eam_init(pot["drho"], pot["dr"], pot["cut"], pot["frho"], pot["rhor"], pot["z2r"])
+        assert force_errors(b.eam_forces()[0], f_ref)[0] <= tol
+        for gd, gr in zip(b.eam_vjp(G), g_ref):
+            assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
+        b.close()
+
+
+@pytest.mark.parametrize("nrep,nside", [(2, 17), (3, 15), (10, 17), (11, 17)])
+def test_default_batch_launch_shapes_agree_with_a_fixed_one(nrep, nside):
+    """Batches on both sides of the sizes (10,000 and 50,000 atoms) where the
+    default launch shape changes, against workgroups of 256 at 8 lanes."""
+    natoms, lo, hi, per, t, x = ka_batch_inputs(nrep, nside)
+    b = B.Batch(natoms, lo, hi, per, 2, t)
+    b.set_positions(x)
+    b.lj_init(*ka_tables())
+    G = np.random.default_rng(2).normal(size=x.shape)
+    f0, (ge0, gs0) = b.lj_forces()[0], b.lj_vjp(G)
+    for kind in (B.BK_LJ, B.BK_LJ_VJP):
+        b.set_launch(kind, 256, 8, 0)
+    f1, (ge1, gs1) = b.lj_forces()[0], b.lj_vjp(G)
+    assert force_errors(f0, f1)[0] <= 1e-12
+    assert rel(ge0, ge1) <= 1e-12 and rel(gs0, gs1) <= 1e-12
+    b.close()
