@@ -360,21 +360,6 @@ __global__ __launch_bounds__(kBuildBlock, 5) void k_b_build(int n, const double4
 
 // ---------------------------------------------------------------- pair helpers
 
-// sqrt(x) and 1/sqrt(x) in FP64 to about an ulp: the hardware reciprocal
-// square root refined in coupled steps, half the instructions of sqrt and a
-// divide
-__device__ __forceinline__ void sqrt_and_inverse(double x, double &r, double &ri) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double e = fma(-h, g, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  g = fma(fma(-g, g, x), h, g);
-  ri = h + h;
-  ri = fma(ri, fma(-ri, g, 1.0), ri);
-  r = g;
-}
-
 // One lane's four consecutive entries k0 .. k0+3 of a row (rows start 16-B
 // aligned; entries past jn are not written and become the atom itself)
 __device__ __forceinline__ void row_chunk(const int *__restrict__ row, int k0, int jn, int self, int (&ent)[4]) {

@@ -90,6 +90,21 @@ struct EAMArgs {
   const float4 *rhor_pf, *z2r_pf;
 };
 
+// sqrt(x) and 1/sqrt(x) in FP64 to about an ulp: the hardware reciprocal
+// square root refined in coupled steps, half the instructions of sqrt and a
+// divide
+__device__ __forceinline__ void sqrt_and_inverse(double x, double &r, double &ri) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, x), h, g);
+  ri = h + h;
+  ri = fma(ri, fma(-ri, g, 1.0), ri);
+  r = g;
+}
+
 // ---- eam spline evaluation of the pair kernels (every variant of the
 // density and force passes uses these, so a pair gives the same bits in
 // each).  The spline
@@ -137,8 +152,9 @@ __device__ __forceinline__ double eam_rho_term(const EAMArgs &a, int tab, double
     (void)eam_index_mixed(rsq, a.rdr, a.nr, m, p);
     return (double)eam_rho_eval(a.rhor_pf[2 * ((size_t)tab * (a.nr + 1) + m) + 1], p);  // c3..c6
   }
-  double p;
-  eam_spline_index<double>(sqrt(rsq), a.rdr, a.nr, m, p);
+  double p, r, ri;
+  sqrt_and_inverse(rsq, r, ri);
+  eam_spline_index<double>(r, a.rdr, a.nr, m, p);
   const double4 c = a.rhor_p[2 * ((size_t)tab * (a.nr + 1) + m) + 1];
   return ((c.x * p + c.y) * p + c.z) * p + c.w;
 }
@@ -161,6 +177,20 @@ __device__ __forceinline__ void eam_pair_eval(const float4 &ci, const float4 &cj
   phi = (double)phif;
 }
 
+// the same in FP64, with 1/r given
+__device__ __forceinline__ void eam_pair_eval64(const double4 &ci, const double4 &cj, const double4 &zd,
+                                                const double4 &zv, double recip, double p, double fpi, double fpj,
+                                                double &fpair, double &phi) {
+  const double rhoip = (ci.x * p + ci.y) * p + ci.z;
+  const double rhojp = (cj.x * p + cj.y) * p + cj.z;
+  const double z2p = (zd.x * p + zd.y) * p + zd.z;
+  const double z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
+  phi = z2 * recip;
+  const double phip = z2p * recip - phi * recip;
+  const double psip = fpi * rhojp + fpj * rhoip + phip;
+  fpair = -psip * recip;
+}
+
 // pair force factor fpair (f_i += del * fpair) and phi of the force pass
 // (pair_eam.cpp:245-282); ri = type2rhor[ti][tj], rj = type2rhor[tj][ti],
 // zi = type2z2r[ti][tj]
@@ -178,23 +208,15 @@ __device__ __forceinline__ void eam_pair_term(const EAMArgs &a, int ri, int rj, 
     eam_pair_eval(ci, cj, a.z2r_pf[2 * (zi * kn + m)], a.z2r_pf[2 * (zi * kn + m) + 1], r, p, fpi, fpj, fpair, phi);
     return;
   }
-  const double r = sqrt(rsq);
+  double r, recip, p;
   int m;
-  double p;
+  sqrt_and_inverse(rsq, r, recip);
   eam_spline_index<double>(r, a.rdr, a.nr, m, p);
   const double4 ci = a.rhor_p[2 * (ri * kn + m)];
   double4 cj = ci;
   if (ri != rj) cj = a.rhor_p[2 * (rj * kn + m)];
   const double4 zd = a.z2r_p[2 * (zi * kn + m)], zv = a.z2r_p[2 * (zi * kn + m) + 1];
-  const double rhoip = (ci.x * p + ci.y) * p + ci.z;
-  const double rhojp = (cj.x * p + cj.y) * p + cj.z;
-  const double z2p = (zd.x * p + zd.y) * p + zd.z;
-  const double z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
-  const double recip = 1.0 / r;
-  phi = z2 * recip;
-  const double phip = z2p * recip - phi * recip;
-  const double psip = fpi * rhojp + fpj * rhoip + phip;
-  fpair = -psip * recip;
+  eam_pair_eval64(ci, cj, zd, zv, recip, p, fpi, fpj, fpair, phi);
 }
 
 __host__ __device__ inline int imax2(int a, int b) { return a > b ? a : b; }

@@ -51,6 +51,8 @@ constexpr int kUnrollQ = MDX_GATHER_UNROLL_Q;
 #define MDX_PAIR_MIN_WAVES 1
 #endif
 #define MDX_PAIR_BOUNDS __launch_bounds__(256, MDX_PAIR_MIN_WAVES)
+// the FP64 eam kernels with LDS tables run in workgroups of up to 512 threads
+#define MDX_EAM_BOUNDS(WIDE) __launch_bounds__((WIDE) ? 512 : 256, MDX_PAIR_MIN_WAVES)
 
 // A lane's share of a row is either strided, entries lane, lane+TPA, ...,
 // or chunked, four consecutive entries 4*lane .. 4*lane+3, then
@@ -475,24 +477,30 @@ __device__ __forceinline__ bool pair_inside(const double4 &xi, int i, const int4
   return rsq < cutsq;
 }
 
-// TL (mixed, one type): the spline knots the kernel reads are copied into
-// LDS first (dynamic shared memory, (nr+1) float4 per vector kind), so a
-// lookup is an LDS read instead of a cached global gather; same arithmetic.
+// TL (one type): the spline knots the kernel reads are copied into LDS first
+// (dynamic shared memory), so a lookup is an LDS read instead of a cached
+// global gather; same arithmetic.
 template <bool MIXED, bool EV, int TPA, bool Q, bool ONE, bool TL>
-__global__ MDX_PAIR_BOUNDS void k_eam_rho(int n, int npad, int cap, double px, double py, double pz, EAMArgs a,
+__global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_rho(int n, int npad, int cap, double px, double py, double pz, EAMArgs a,
                                                 const double4 *__restrict__ x, const int4 *__restrict__ xq, QScale qs,
                                                 const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                                 double *__restrict__ rho_out, double *__restrict__ fp_out,
                                                 double *__restrict__ eemb, StepGate gate) {
-  static_assert(!TL || (MIXED && ONE), "LDS tables hold the one FP32 table of a single-type system");
+  static_assert(!TL || ONE, "LDS tables hold the one table of a single-type system");
   if (gate_closed(gate)) return;
   // type map in LDS: a kernel-argument array indexed per lane is a memory read
   __shared__ int s_t2r[kNT2];
-  extern __shared__ float4 s_eam_tab[];  // TL: c3..c6 of knots 0..nr
+  extern __shared__ float4 s_eam_tab[];  // TL: c3..c6 of knots 0..nr (FP64: two double2 each)
+  [[maybe_unused]] double2 *const s_eam_tab64 = reinterpret_cast<double2 *>(s_eam_tab);
   for (int q = threadIdx.x; q < a.ntypes1 * a.ntypes1; q += blockDim.x) s_t2r[q] = a.type2rhor[q];
   if constexpr (TL) {
     const size_t kn = (size_t)(a.nr + 1), t = a.type2rhor[a.ntypes1 + 1];
-    for (int m = threadIdx.x; m < (int)kn; m += blockDim.x) s_eam_tab[m] = a.rhor_pf[2 * (t * kn + m) + 1];
+    if constexpr (MIXED) {
+      for (int m = threadIdx.x; m < (int)kn; m += blockDim.x) s_eam_tab[m] = a.rhor_pf[2 * (t * kn + m) + 1];
+    } else {
+      const double2 *src = reinterpret_cast<const double2 *>(a.rhor_p + 2 * t * kn);
+      for (int q = threadIdx.x; q < 2 * (int)kn; q += blockDim.x) s_eam_tab64[q] = src[4 * (q >> 1) + 2 + (q & 1)];
+    }
   }
   __syncthreads();
   const int i = (xcd_block() * blockDim.x + threadIdx.x) / TPA;
@@ -539,9 +547,17 @@ __global__ MDX_PAIR_BOUNDS void k_eam_rho(int n, int npad, int cap, double px, d
           const int tj = Q ? qj[Q ? u : 0].w : static_cast<int>(xj[Q ? 0 : u].w);
           if constexpr (TL) {
             int m;
-            float p;
-            (void)eam_index_mixed(rsq, a.rdr, a.nr, m, p);
-            rhos[u % NS] += (double)eam_rho_eval(s_eam_tab[m], p);
+            if constexpr (MIXED) {
+              float p;
+              (void)eam_index_mixed(rsq, a.rdr, a.nr, m, p);
+              rhos[u % NS] += (double)eam_rho_eval(s_eam_tab[m], p);
+            } else {
+              double p, r, ri;
+              sqrt_and_inverse(rsq, r, ri);
+              eam_spline_index<double>(r, a.rdr, a.nr, m, p);
+              const double2 c0 = s_eam_tab64[2 * m], c1 = s_eam_tab64[2 * m + 1];
+              rhos[u % NS] += ((c0.x * p + c0.y) * p + c1.x) * p + c1.y;
+            }
           } else {
             rhos[u % NS] += eam_rho_term<MIXED>(a, s_t2r[ONE ? a.ntypes1 + 1 : tj * a.ntypes1 + ti], rsq);
           }
@@ -570,21 +586,23 @@ __global__ MDX_PAIR_BOUNDS void k_eam_rho(int n, int npad, int cap, double px, d
 }
 
 template <bool MIXED, bool EV, int TPA, bool INTEG, bool Q, bool ONE, bool TL>
-__global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px, double py, double pz,
+__global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int cap, double px, double py, double pz,
                                                   EAMArgs a, const double4 *__restrict__ x,
                                                   const int4 *__restrict__ xq, QScale qs,
                                                   const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                                   const double *__restrict__ fp, const double *__restrict__ eemb,
                                                   double4 *__restrict__ f, double *__restrict__ vatom,
                                                   double *__restrict__ partials, IntegArgs ig) {
-  static_assert(!TL || (MIXED && ONE), "LDS tables hold the one FP32 table of a single-type system");
+  static_assert(!TL || ONE, "LDS tables hold the one table of a single-type system");
   if constexpr (INTEG) {
     if (gate_closed(ig.gate)) return;
   }
   // type maps in LDS: kernel-argument arrays indexed per lane are memory reads
   __shared__ int s_t2r[kNT2], s_t2z[kNT2];
-  // TL: rho' c0..c2, z2' c0..c2 and z2 c3..c6 of knots 0..nr, one after the other
+  // TL: rho' c0..c2, z2' c0..c2 and z2 c3..c6 of knots 0..nr, one after the
+  // other (mixed), or as five double2 per knot (FP64)
   extern __shared__ float4 s_eam_tab[];
+  [[maybe_unused]] double2 *const s_eam_tab64 = reinterpret_cast<double2 *>(s_eam_tab);
   for (int q = threadIdx.x; q < a.ntypes1 * a.ntypes1; q += blockDim.x) {
     s_t2r[q] = a.type2rhor[q];
     s_t2z[q] = a.type2z2r[q];
@@ -593,9 +611,20 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
   if constexpr (TL) {
     const size_t t = a.type2rhor[a.ntypes1 + 1], z = a.type2z2r[a.ntypes1 + 1];
     for (int m = threadIdx.x; m < kn; m += blockDim.x) {
-      s_eam_tab[m] = a.rhor_pf[2 * (t * kn + m)];
-      s_eam_tab[kn + m] = a.z2r_pf[2 * (z * kn + m)];
-      s_eam_tab[2 * kn + m] = a.z2r_pf[2 * (z * kn + m) + 1];
+      if constexpr (MIXED) {
+        s_eam_tab[m] = a.rhor_pf[2 * (t * kn + m)];
+        s_eam_tab[kn + m] = a.z2r_pf[2 * (z * kn + m)];
+        s_eam_tab[2 * kn + m] = a.z2r_pf[2 * (z * kn + m) + 1];
+      } else {
+        const double4 rd = a.rhor_p[2 * (t * kn + m)], zd = a.z2r_p[2 * (z * kn + m)],
+                      zv = a.z2r_p[2 * (z * kn + m) + 1];
+        double2 *const d = s_eam_tab64 + 5 * m;
+        d[0] = make_double2(rd.x, rd.y);
+        d[1] = make_double2(rd.z, zd.x);
+        d[2] = make_double2(zd.y, zd.z);
+        d[3] = make_double2(zv.x, zv.y);
+        d[4] = make_double2(zv.z, zv.w);
+      }
     }
   }
   __syncthreads();
@@ -654,10 +683,21 @@ __global__ MDX_PAIR_BOUNDS void k_eam_force(int n, int npad, int cap, double px,
         double fpair, phi;
         if constexpr (TL) {
           int m;
-          float p;
-          const float r = eam_index_mixed(rsq, a.rdr, a.nr, m, p);
-          const float4 ci = s_eam_tab[m];
-          eam_pair_eval(ci, ci, s_eam_tab[kn + m], s_eam_tab[2 * kn + m], r, p, fpi, fpjv[u], fpair, phi);
+          if constexpr (MIXED) {
+            float p;
+            const float r = eam_index_mixed(rsq, a.rdr, a.nr, m, p);
+            const float4 ci = s_eam_tab[m];
+            eam_pair_eval(ci, ci, s_eam_tab[kn + m], s_eam_tab[2 * kn + m], r, p, fpi, fpjv[u], fpair, phi);
+          } else {
+            double r, recip, p;
+            sqrt_and_inverse(rsq, r, recip);
+            eam_spline_index<double>(r, a.rdr, a.nr, m, p);
+            const double2 *const d = s_eam_tab64 + 5 * m;
+            const double2 d0 = d[0], d1 = d[1], d2 = d[2], d3 = d[3], d4 = d[4];
+            const double4 ci = make_double4(d0.x, d0.y, d1.x, 0.0);
+            eam_pair_eval64(ci, ci, make_double4(d1.y, d2.x, d2.y, 0.0), make_double4(d3.x, d3.y, d4.x, d4.y), recip,
+                            p, fpi, fpjv[u], fpair, phi);
+          }
         } else {
           eam_pair_term<MIXED>(a, s_t2r[tij], s_t2r[tji], s_t2z[tij], rsq, fpi, fpjv[u], fpair, phi);
         }
@@ -746,9 +786,11 @@ void launch_lj_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   c->last_grid = G;
 }
 
-// knots (nr+1) up to which the single-type FP32 tables go to LDS: the force
-// pass holds three float4 per knot (48 KiB at this limit)
-constexpr int kEamLdsKnots = 1024;
+// knots (nr+1) up to which the single-type tables go to LDS: the force pass
+// holds three float4 per knot (48 KiB at this limit), or in FP64 five double2
+// (62.5 KiB).  FP64 from LDS against gathers through L1: rho + force 23.1
+// against 35.6 us at 32,000 atoms, 106 against 212 at 256,000.
+constexpr int kEamLdsKnots = 1024, kEamLdsKnots64 = 800;
 
 template <bool MIXED, bool EV, int TPA, bool INTEG, bool Q, bool ONE, bool TL>
 void launch_eam_t(mdx_ctx *c, int B, const IntegArgs &ig) {
@@ -759,17 +801,23 @@ void launch_eam_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   ea.chi = ea.cutforcesq * (1.0 + kBand);
   prof_begin(c, MDX_K_EAM_RHO);
   hipLaunchKernelGGL((k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>), dim3(G), dim3(B),
-                     occupancy_lds(static_lds<k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>>(), B, TL ? kn * sizeof(float4) : 0, 0), c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs,
+                     occupancy_lds(static_lds<k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>>(), B, TL ? kn * (MIXED ? sizeof(float4) : sizeof(double4)) : 0, 0), c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs,
                      c->nbr, c->numneigh, c->rho, c->fp, c->eemb, INTEG ? ig.gate : StepGate{});
   prof_end(c);
   prof_begin(c, INTEG ? MDX_K_FUSED : MDX_K_EAM_FORCE);
-  const size_t tl_bytes = TL ? 3 * kn * sizeof(float4) : 0;
+  const size_t tl_bytes = TL ? kn * (MIXED ? 3 * sizeof(float4) : 5 * sizeof(double2)) : 0;
   hipLaunchKernelGGL((k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>), dim3(G), dim3(B),
                      INTEG ? occupancy_lds(static_lds<k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>>(), B, tl_bytes, 0) : tl_bytes, c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1],
                      c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp, c->eemb, c->f, c->vatom,
                      c->partials, ig);
   prof_end(c);
   c->last_grid = G;
+}
+
+// whether the eam kernels take the LDS tables of a single-type system
+bool eam_lds_tables(const mdx_ctx *c, int tpa) {
+  return c->ntypes == 1 && (tpa == 4 || tpa == 8 || tpa == 16) &&
+         c->eam.nr + 1 <= (c->precision == MDX_MIXED ? kEamLdsKnots : kEamLdsKnots64);
 }
 
 template <bool MIXED, bool EV, int TPA, bool INTEG, bool Q>
@@ -784,9 +832,7 @@ template <bool MIXED, bool EV, int TPA, bool INTEG, bool Q>
 void launch_eam(mdx_ctx *c, int B, const IntegArgs &ig) {
   if constexpr (TPA == 4 || TPA == 8 || TPA == 16) {
     if (c->ntypes == 1) {
-      if constexpr (MIXED) {
-        if (c->eam.nr + 1 <= kEamLdsKnots) return launch_eam_t<MIXED, EV, TPA, INTEG, Q, true, true>(c, B, ig);
-      }
+      if (eam_lds_tables(c, TPA)) return launch_eam_t<MIXED, EV, TPA, INTEG, Q, true, true>(c, B, ig);
       return launch_eam_t<MIXED, EV, TPA, INTEG, Q, true, false>(c, B, ig);
     }
   }
@@ -839,22 +885,27 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 //               2,048,000        381 /  508 /  685 / 1096  (mixed  286 /  329)
 //   Kob-Andersen    2,744       11.1 /  7.9 /  5.8 /  5.3
 //                   8,000       11.0 /  7.7 /  6.5 /  6.6
-//   eam (rho+force) 4,000       26.3 / 17.3 / 13.1 / 12.6
-//                  13,500       26.2 / 22.2 / 23.2 / 24.3
-//                 108,000        100 /  106 /  118 /  142
+//   eam (rho+force)   500       19.3 / 14.6 / 12.2 / 10.5
+//                   4,000       19.6 / 14.7 / 12.4 / 12.6
+//                  13,500       22.6 / 16.5 / 17.4 / 24.2
+//                 108,000         57 /   65 /   89 /  136
 // Mixed precision takes only 8 and 4, which give the same bits (split_sums):
 // a mixed trajectory amplifies any other difference to its own error.
 // Workgroups of one wavefront spread a small launch evenly over the CUs
 // (13,500 lj/cut atoms at 8 lanes: 6.8 against 7.9 us); with 1024 or more
-// workgroups of 256 there is nothing to gain.  The mixed single-type eam
-// kernels copy their spline tables to LDS once per workgroup, so they keep
-// 256 (13,500 atoms: 15.9 against 22.1 us).
+// workgroups of 256 there is nothing to gain.  The single-type eam kernels
+// copy their spline tables to LDS once per workgroup, so they keep 256 (mixed,
+// 13,500 atoms: 15.9 against 22.1 us), and 512 for the larger FP64 tables
+// above 10,000 atoms (32,000: 23.1 against 24.7 us, 665,500: 269 against 283;
+// 1024: 283).
 Launch pair_launch(const mdx_ctx *c) {
   Launch l = c->launch;
-  const bool eam = c->pair_style == MDX_PAIR_EAM;
   const bool mixed = c->precision == MDX_MIXED;
-  if (!l.tpa) l.tpa = c->n > 48000 ? 4 : c->n > 10000 || mixed ? 8 : c->n > (eam ? 6000 : 3000) ? 16 : 32;
-  if (!l.block) l.block = (long)c->n * l.tpa < 1024L * 256 && !(eam && mixed) ? 64 : 256;
+  if (!l.tpa) l.tpa = c->n > 48000 ? 4 : c->n > 10000 || mixed ? 8 : c->n > 3000 ? 16 : 32;
+  if (!l.block) {
+    const bool tables = c->pair_style == MDX_PAIR_EAM && eam_lds_tables(c, l.tpa);
+    l.block = tables ? (mixed || c->n <= 10000 ? 256 : 512) : (long)c->n * l.tpa < 1024L * 256 ? 64 : 256;
+  }
   return l;
 }
 
