@@ -17,7 +17,9 @@
  *  - Per-type tables are (ntypes+1)^2 row-major doubles, indexed [i][j] with
  *    1-based types, exactly as Pair::init_one fills them.
  *  - A context owns all device memory; one context per host thread.
- *    Calls are synchronous at return.
+ *    Calls are synchronous at return; mdx_set_atoms and mdx_set_positions
+ *    return when the caller's arrays have been read, and every later call of
+ *    the context runs after their device work.
  *  - Plain pointers and sizes only; no HIP or torch types cross the ABI.
  */
 #ifndef MDX_H

@@ -9,6 +9,7 @@
 // |x - xhold|^2 > (skin/2)^2 and raises a device flag, so the trigger costs
 // no extra pass over x.
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <thread>
 #include <vector>
@@ -117,7 +118,8 @@ __global__ __launch_bounds__(256) void k_reduce_records(const double *__restrict
   if ((int)threadIdx.x < nslots) out[(size_t)blockIdx.x * nslots + threadIdx.x] = s[threadIdx.x][0];
 }
 
-// caller-order host positions -> device (sorted) order, type kept in w
+// caller-order positions (device or mapped host memory) -> device (sorted)
+// order, type kept in w
 __global__ void k_scatter_x(int n, const double *__restrict__ hx, const int *__restrict__ orig,
                             double4 *__restrict__ x, int4 *__restrict__ xq, QScale qs) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -131,6 +133,51 @@ __global__ void k_scatter_x(int n, const double *__restrict__ hx, const int *__r
   if (xq) xq[i] = quantize(qs, p);
 }
 
+// the caller's arrays as uploaded -> a context's atoms in caller order (v, tag
+// may be null: zero velocities, tags 1..n); forces are cleared up to npad
+__global__ void k_load_atoms(int n, int npad, const double *__restrict__ hx, const double *__restrict__ hv,
+                             const int *__restrict__ type, const int *__restrict__ htag, int img0,
+                             double4 *__restrict__ x, double4 *__restrict__ v, double4 *__restrict__ f,
+                             int *__restrict__ tag, int *__restrict__ orig, int *__restrict__ inv,
+                             int *__restrict__ image) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npad) return;
+  f[i] = make_double4(0.0, 0.0, 0.0, 0.0);
+  if (i >= n) return;
+  const size_t k = 3 * (size_t)i;
+  x[i] = make_double4(hx[k], hx[k + 1], hx[k + 2], (double)type[i]);
+  v[i] = hv ? make_double4(hv[k], hv[k + 1], hv[k + 2], 0.0) : make_double4(0.0, 0.0, 0.0, 0.0);
+  tag[i] = htag ? htag[i] : i + 1;
+  orig[i] = i;
+  inv[i] = i;
+  image[i] = img0;
+}
+
+// a context's atoms -> caller-order arrays (device or mapped host memory;
+// null: not wanted), the image counts unpacked to three ints
+__global__ void k_store_atoms(int n, const int *__restrict__ orig, const double4 *__restrict__ x,
+                              const double4 *__restrict__ v, const double4 *__restrict__ f,
+                              const int *__restrict__ image, double *__restrict__ ox, double *__restrict__ ov,
+                              double *__restrict__ of, int *__restrict__ oi) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const size_t k = 3 * (size_t)orig[i];
+  auto put = [k](double *o, const double4 &p) {
+    o[k] = p.x;
+    o[k + 1] = p.y;
+    o[k + 2] = p.z;
+  };
+  if (ox) put(ox, x[i]);
+  if (ov) put(ov, v[i]);
+  if (of) put(of, f[i]);
+  if (oi) {
+    const int im = image[i];
+    oi[k] = (im & MDX_IMGMASK) - MDX_IMGMAX;
+    oi[k + 1] = ((im >> 10) & MDX_IMGMASK) - MDX_IMGMAX;
+    oi[k + 2] = (im >> 20) - MDX_IMGMAX;
+  }
+}
+
 // fixed-point mirror of all positions (after a change of precision or
 // position format)
 __global__ void k_quantize(int n, const double4 *__restrict__ x, int4 *__restrict__ xq, QScale qs) {
@@ -138,33 +185,11 @@ __global__ void k_quantize(int n, const double4 *__restrict__ x, int4 *__restric
   if (i < n) xq[i] = quantize(qs, x[i]);
 }
 
-// device order -> caller order [n][3]
-__global__ void k_gather3(int n, const int *__restrict__ orig, const double4 *__restrict__ src,
+// device order -> caller order, one value per atom
+__global__ void k_gather1(int n, const int *__restrict__ orig, const double *__restrict__ src,
                           double *__restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int o = orig[i];
-  const double4 p = src[i];
-  out[3 * o] = p.x;
-  out[3 * o + 1] = p.y;
-  out[3 * o + 2] = p.z;
-}
-
-// device order -> caller order for the w component (per-atom energy)
-__global__ void k_gather_w(int n, const int *__restrict__ orig, const double4 *__restrict__ src,
-                           double *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  out[orig[i]] = src[i].w;
-}
-
-// device order SoA [ncols][npad] -> caller order [n][ncols]
-__global__ void k_gather_soa(int n, int npad, int ncols, const int *__restrict__ orig, const double *__restrict__ src,
-                             double *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int o = orig[i];
-  for (int c = 0; c < ncols; c++) out[(size_t)o * ncols + c] = src[(size_t)c * npad + i];
+  if (i < n) out[orig[i]] = src[i];
 }
 
 // streaming copy of known size (HBM calibration: bytes moved = 2 * bytes)
@@ -211,26 +236,25 @@ int neigh_check_displacement(mdx_ctx *c, int *flag) {
   return MDX_OK;
 }
 
-// Sum of the per-block records into red_host.  Many records (64,000 for the
+// Sum of the per-block records into red_host (mapped).  Many records (64,000 for the
 // fused lj/cut kernel at 2.048 M atoms) are first reduced by up to 1024
 // blocks of at least 256 contiguous records each, into the space after the
-// records, then by one block: the partition depends only on nblocks, so the
+// records (partials_for holds it), then by one block: the partition depends only on nblocks, so the
 // sums are reproducible.
-int finish_reduction(mdx_ctx *c, int nblocks, int nslots) {
+int finish_reduction(mdx_ctx *c, int nblocks, int nslots, bool wait) {
   const int per = std::max(256, (nblocks + 1023) / 1024);
   const int nlev = (nblocks + per - 1) / per;
-  if (nblocks > 2 * per && (long)(nblocks + nlev) * nslots <= c->cap_partials) {
+  if (nblocks > 2 * per) {
     double *lev = c->partials + (size_t)nblocks * nslots;
     hipLaunchKernelGGL(k_reduce_records, dim3(nlev), dim3(256), 0, c->stream, c->partials, nblocks, nslots, per, lev);
-    hipLaunchKernelGGL(k_reduce_records, dim3(1), dim3(256), 0, c->stream, lev, nlev, nslots, nlev, c->red_out);
+    hipLaunchKernelGGL(k_reduce_records, dim3(1), dim3(256), 0, c->stream, lev, nlev, nslots, nlev, c->red_host);
   } else {
     hipLaunchKernelGGL(k_reduce_records, dim3(1), dim3(256), 0, c->stream, c->partials, nblocks, nslots, nblocks,
-                       c->red_out);
+                       c->red_host);
   }
-  hipError_t e = hipMemcpyAsync(c->red_host, c->red_out, sizeof(double) * nslots, hipMemcpyDeviceToHost, c->stream);
-  if (e != hipSuccess) return hip_fail(e, "reduction copy");
-  if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return hip_fail(e, "reduction sync");
-  return MDX_OK;
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && wait) e = hipStreamSynchronize(c->stream);
+  return e == hipSuccess ? MDX_OK : hip_fail(e, "reduction");
 }
 
 int reduce_ke(mdx_ctx *c) {
@@ -243,117 +267,223 @@ int reduce_ke(mdx_ctx *c) {
   return finish_reduction(c, G, 1);
 }
 
-// Host copy between the caller's arrays and the pinned staging buffer.  One
-// thread copies about 10 GB/s, well under the link's rate, so copies above
-// 8 MiB are split over up to eight threads.
-void host_copy(void *dst, const void *src, size_t bytes) {
-  constexpr size_t kSplit = size_t(8) << 20;
-  if (bytes < kSplit) {
-    memcpy(dst, src, bytes);
-    return;
-  }
-  const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<size_t>(std::min(8u, hw), bytes / (size_t(2) << 20));
-  const size_t chunk = ((bytes + nt - 1) / nt + 63) / 64 * 64;
-  std::vector<std::thread> pool;
-  for (int t = 1; t < nt; t++) {
-    const size_t off = chunk * t;
-    if (off >= bytes) break;
-    pool.emplace_back([=] { memcpy((char *)dst + off, (const char *)src + off, std::min(chunk, bytes - off)); });
-  }
-  memcpy(dst, src, std::min(chunk, bytes));
-  for (auto &th : pool) th.join();
-}
+// ---- transfers between the caller's arrays and the device
+//
+// Everything goes through the pinned stage in pieces: a piece's DMA overlaps
+// the host's copies of its neighbours.  One thread copies about 10 GB/s, well
+// under the link's rate, so transfers of 2 MiB and more are split over up to
+// eight threads, each taking its slice of every piece.
+constexpr size_t kPiece = size_t(2) << 20;
+constexpr int kPiecesInFlight = 64;
 
-// Large transfers through the pinned stage go in chunks so that the host
-// copy of one chunk overlaps the DMA of the previous (host -> device) or the
-// next (device -> host).
-constexpr size_t kStageChunk = size_t(8) << 20;
+struct Piece {
+  char *host, *dev, *stage;
+  size_t len;
+  bool add;
+};
 
-static int stage_events(mdx_ctx *c) {
-  for (hipEvent_t &ev : c->stage_ev)
-    if (!ev) {
-      hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-      if (e != hipSuccess) {
-        ev = nullptr;
-        return hip_fail(e, "staging events");
-      }
+static std::vector<Piece> pieces_of(const Seg *segs, int nseg, size_t &total) {
+  std::vector<Piece> v;
+  total = 0;
+  for (int s = 0; s < nseg; s++)
+    for (size_t off = 0; off < segs[s].bytes; off += kPiece) {
+      const size_t len = std::min(kPiece, segs[s].bytes - off);
+      v.push_back({(char *)segs[s].host + off, (char *)segs[s].dev + off, nullptr, len, segs[s].add});
+      total += len;
     }
-  return MDX_OK;
+  return v;
 }
 
-// host -> stage -> device, chunked; returns after the copies are queued
-static int upload_staged(mdx_ctx *c, void *dev, const void *host, size_t bytes) {
-  size_t chunk = std::max(kStageChunk, ((bytes + 7) / 8 + 63) / 64 * 64);  // whole doubles per chunk
-  for (size_t off = 0; off < bytes; off += chunk) {
-    const size_t len = std::min(chunk, bytes - off);
-    host_copy((char *)c->host_stage + off, (const char *)host + off, len);
-    hipError_t e = hipMemcpyAsync((char *)dev + off, (char *)c->host_stage + off, len, hipMemcpyHostToDevice,
-                                  c->stream);
-    if (e != hipSuccess) return hip_fail(e, "staged upload");
-  }
-  return MDX_OK;
+// slice t of nt of `len` bytes, on whole 64-byte lines
+static void slice(size_t len, int t, int nt, size_t &a, size_t &b) {
+  const size_t per = ((len + nt - 1) / nt + 63) / 64 * 64;
+  a = std::min(len, per * t);
+  b = std::min(len, a + per);
 }
 
-// host[k] += stage[k] over `count` doubles, split as host_copy splits
 void host_add(double *dst, const double *src, size_t count) {
-  constexpr size_t kSplit = size_t(1) << 20;
-  auto add = [](double *d, const double *s, size_t n) {
-    for (size_t k = 0; k < n; k++) d[k] += s[k];
-  };
-  if (count < kSplit) {
-    add(dst, src, count);
-    return;
-  }
+  for (size_t k = 0; k < count; k++) dst[k] += src[k];
+}
+
+// Runs work(t, nt) on nt threads, the caller's among them as t = 0; fewer
+// threads than asked for if the system gives no more.
+template <typename W>
+static void on_threads(size_t bytes, W &&work) {
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<size_t>(std::min(8u, hw), count / (size_t(1) << 18));
-  const size_t chunk = ((count + nt - 1) / nt + 7) / 8 * 8;
+  const int want = bytes < kPiece ? 1 : (int)std::min<size_t>(std::min(8u, hw), bytes >> 20);
+  std::atomic<int> nt{0};
   std::vector<std::thread> pool;
-  for (int t = 1; t < nt; t++) {
-    const size_t off = chunk * t;
-    if (off >= count) break;
-    pool.emplace_back([=] { add(dst + off, src + off, std::min(chunk, count - off)); });
+  try {
+    pool.reserve(want);
+    for (int t = 1; t < want; t++)
+      pool.emplace_back([&nt, &work, t] {
+        int n;
+        while (!(n = nt.load(std::memory_order_acquire))) std::this_thread::yield();
+        work(t, n);
+      });
+  } catch (...) {
   }
-  add(dst, src, std::min(chunk, count));
+  const int n = (int)pool.size() + 1;
+  nt.store(n, std::memory_order_release);
+  work(0, n);
   for (auto &th : pool) th.join();
 }
 
-// device -> stage -> host, chunked; waits for the last chunk.  With `add`
-// the host array receives host += device (doubles) instead of a copy.
-static int download_staged(mdx_ctx *c, void *host, const void *dev, size_t bytes, bool add = false) {
-  int rc = stage_events(c);
-  if (rc) return rc;
-  size_t chunk = std::max(kStageChunk, ((bytes + 7) / 8 + 63) / 64 * 64);  // whole doubles per chunk
-  const int nchunk = (int)((bytes + chunk - 1) / chunk);  // at most 8
-  hipError_t e;
-  for (int k = 0; k < nchunk; k++) {
-    const size_t off = chunk * k, len = std::min(chunk, bytes - off);
-    if ((e = hipMemcpyAsync((char *)c->host_stage + off, (const char *)dev + off, len, hipMemcpyDeviceToHost,
-                            c->stream)) != hipSuccess ||
-        (e = hipEventRecord(c->stage_ev[k], c->stream)) != hipSuccess)
-      return hip_fail(e, "staged download");
+int stage_ready(mdx_ctx *c) {
+  if (!c->stage_busy) return MDX_OK;
+  hipError_t e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) return hip_fail(e, "staging memory");
+  c->stage_busy = false;
+  return MDX_OK;
+}
+
+// the next pieces that fit the stage, from piece `first` on
+static size_t place(mdx_ctx *c, std::vector<Piece> &v, size_t first) {
+  const size_t cap = (size_t)(sizeof(double) * kStageDoubles * c->cap_atoms);
+  size_t off = 0, k = first;
+  for (; k < v.size() && k - first < (size_t)kPiecesInFlight && off + v[k].len <= cap; k++) {
+    v[k].stage = (char *)c->host_stage + off;
+    off += (v[k].len + 63) / 64 * 64;
   }
-  for (int k = 0; k < nchunk; k++) {
-    const size_t off = chunk * k, len = std::min(chunk, bytes - off);
-    if ((e = hipEventSynchronize(c->stage_ev[k])) != hipSuccess) return hip_fail(e, "staged download");
-    if (add)
-      host_add(reinterpret_cast<double *>((char *)host + off), reinterpret_cast<const double *>((char *)c->host_stage + off),
-               len / sizeof(double));
-    else
-      host_copy((char *)host + off, (char *)c->host_stage + off, len);
+  return k;
+}
+
+int upload(mdx_ctx *c, const Seg *segs, int nseg) {
+  size_t total;
+  std::vector<Piece> v = pieces_of(segs, nseg, total);
+  hipError_t e = hipSuccess;
+  for (size_t first = 0, last; first < v.size(); first = last) {
+    int rc = stage_ready(c);
+    if (rc) return rc;
+    if ((last = place(c, v, first)) == first) {
+      set_error("staging memory too small");
+      return MDX_ERR_ARG;
+    }
+    std::vector<std::atomic<int>> done(last - first);
+    c->stage_busy = true;
+    on_threads(total, [&](int t, int nt) {
+      for (size_t k = first; k < last; k++) {
+        size_t a, b;
+        slice(v[k].len, t, nt, a, b);
+        memcpy(v[k].stage + a, v[k].host + a, b - a);
+        if (t) {
+          done[k - first].fetch_add(1, std::memory_order_release);
+        } else {
+          while (done[k - first].load(std::memory_order_acquire) < nt - 1) std::this_thread::yield();
+          if (e == hipSuccess) e = hipMemcpyAsync(v[k].dev, v[k].stage, v[k].len, hipMemcpyHostToDevice, c->stream);
+        }
+      }
+    });
+    if (e != hipSuccess) return hip_fail(e, "upload");
+  }
+  return MDX_OK;
+}
+
+int download(mdx_ctx *c, const Seg *segs, int nseg) {
+  size_t total;
+  std::vector<Piece> v = pieces_of(segs, nseg, total);
+  hipError_t e = hipSuccess;
+  for (size_t first = 0, last; first < v.size(); first = last) {
+    if ((last = place(c, v, first)) == first) {
+      set_error("staging memory too small");
+      return MDX_ERR_ARG;
+    }
+    while (c->stage_ev.size() < last - first) {
+      hipEvent_t ev;
+      if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return hip_fail(e, "staging events");
+      c->stage_ev.push_back(ev);
+    }
+    for (size_t k = first; k < last; k++)
+      if ((e = hipMemcpyAsync(v[k].stage, v[k].dev, v[k].len, hipMemcpyDeviceToHost, c->stream)) != hipSuccess ||
+          (e = hipEventRecord(c->stage_ev[k - first], c->stream)) != hipSuccess) {
+        (void)hipStreamSynchronize(c->stream);
+        return hip_fail(e, "download");
+      }
+    std::vector<std::atomic<int>> state(last - first);  // 1: in the stage, 2: failed
+    on_threads(total, [&](int t, int nt) {
+      for (size_t k = first; k < last; k++) {
+        if (t == 0) {
+          if (e == hipSuccess) e = hipEventSynchronize(c->stage_ev[k - first]);
+          state[k - first].store(e == hipSuccess ? 1 : 2, std::memory_order_release);
+        }
+        int st;
+        while (!(st = state[k - first].load(std::memory_order_acquire))) std::this_thread::yield();
+        if (st == 2) return;
+        size_t a, b;
+        slice(v[k].len, t, nt, a, b);
+        if (v[k].add)
+          host_add(reinterpret_cast<double *>(v[k].host + a), reinterpret_cast<const double *>(v[k].stage + a),
+                   (b - a) / sizeof(double));
+        else
+          memcpy(v[k].host + a, v[k].stage + a, b - a);
+      }
+    });
+    if (e != hipSuccess) return hip_fail(e, "download");
+    c->stage_busy = false;  // the stream has passed everything queued before
   }
   return MDX_OK;
 }
 
 int scatter_positions(mdx_ctx *c, const double *host_x) {
   const int B = 256, G = (c->n + B - 1) / B;
-  double *dtmp = c->dscratch;
-  int rc = upload_staged(c, dtmp, host_x, sizeof(double) * 3 * c->n);
+  const size_t bytes = sizeof(double) * 3 * c->n;
+  const double *src = c->dscratch;
+  int rc;
+  if (c->n <= kIoAtoms) {
+    if ((rc = stage_ready(c))) return rc;
+    memcpy(c->host_in, host_x, bytes);
+    src = c->host_in;
+    c->stage_busy = true;
+  } else {
+    const Seg seg{const_cast<double *>(host_x), c->dscratch, bytes, false};
+    if ((rc = upload(c, &seg, 1))) return rc;
+  }
+  hipLaunchKernelGGL(k_scatter_x, dim3(G), dim3(B), 0, c->stream, c->n, src, c->orig, c->x, c->qpos ? c->xq : nullptr,
+                     c->qs);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? MDX_OK : hip_fail(e, "positions scatter");
+}
+
+int load_atoms(mdx_ctx *c, const double *x, const double *v, const int *type, const int *tag) {
+  const size_t n = (size_t)c->n, n3 = 3 * n;
+  Seg segs[4];
+  int ns = 0;
+  segs[ns++] = {const_cast<double *>(x), c->dscratch, sizeof(double) * n3, false};
+  if (v) segs[ns++] = {const_cast<double *>(v), c->dscratch + n3, sizeof(double) * n3, false};
+  segs[ns++] = {const_cast<int *>(type), c->bidx, sizeof(int) * n, false};
+  if (tag) segs[ns++] = {const_cast<int *>(tag), c->bidx_s, sizeof(int) * n, false};
+  int rc = upload(c, segs, ns);
   if (rc) return rc;
-  hipError_t e;
-  hipLaunchKernelGGL(k_scatter_x, dim3(G), dim3(B), 0, c->stream, c->n, dtmp, c->orig, c->x,
-                     c->qpos ? c->xq : nullptr, c->qs);
-  if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return hip_fail(e, "positions scatter");
+  const int img0 = (MDX_IMGMAX << 20) | (MDX_IMGMAX << 10) | MDX_IMGMAX;
+  const int B = 256, G = (c->npad + B - 1) / B;
+  hipLaunchKernelGGL(k_load_atoms, dim3(G), dim3(B), 0, c->stream, c->n, c->npad, c->dscratch,
+                     v ? c->dscratch + n3 : nullptr, c->bidx, tag ? c->bidx_s : nullptr, img0, c->x, c->v, c->f, c->tag,
+                     c->orig, c->inv, c->image);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? MDX_OK : hip_fail(e, "atom upload");
+}
+
+int store_atoms(mdx_ctx *c, double *x, double *v, double *f, int *image) {
+  const size_t n3 = 3 * (size_t)c->n;
+  const bool small = c->n <= kIoAtoms;
+  // x | v | f | image, in mapped host memory or in two device scratch arrays
+  double *dx = small ? c->host_out : c->dscratch, *dv = dx + n3, *df = small ? dv + n3 : c->vatom;
+  int *di = reinterpret_cast<int *>(df + n3);
+  const int B = 256, G = (c->n + B - 1) / B;
+  hipLaunchKernelGGL(k_store_atoms, dim3(G), dim3(B), 0, c->stream, c->n, c->orig, c->x, c->v, c->f, c->image,
+                     x ? dx : nullptr, v ? dv : nullptr, f ? df : nullptr, image ? di : nullptr);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "atom download");
+  Seg segs[4];
+  int ns = 0;
+  if (x) segs[ns++] = {x, dx, sizeof(double) * n3, false};
+  if (v) segs[ns++] = {v, dv, sizeof(double) * n3, false};
+  if (f) segs[ns++] = {f, df, sizeof(double) * n3, false};
+  if (image) segs[ns++] = {image, di, sizeof(int) * n3, false};
+  if (!small) return download(c, segs, ns);
+  if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return hip_fail(e, "atom download");
+  c->stage_busy = false;
+  for (int k = 0; k < ns; k++) memcpy(segs[k].host, segs[k].dev, segs[k].bytes);
   return MDX_OK;
 }
 
@@ -365,12 +495,6 @@ int refresh_xq(mdx_ctx *c) {
   if (e != hipSuccess) return hip_fail(e, "fixed-point positions");
   c->xq_stale = false;
   return MDX_OK;
-}
-
-int gather_vec3(mdx_ctx *c, const double4 *dev, double *host_out, bool add) {
-  const int B = 256, G = (c->n + B - 1) / B;
-  hipLaunchKernelGGL(k_gather3, dim3(G), dim3(B), 0, c->stream, c->n, c->orig, dev, c->dscratch);
-  return download_staged(c, host_out, c->dscratch, sizeof(double) * 3 * c->n, add);
 }
 
 int copy_probe(mdx_ctx *c, long nbytes, int iters, double *gbs) {
@@ -410,21 +534,11 @@ int copy_probe(mdx_ctx *c, long nbytes, int iters, double *gbs) {
   return MDX_OK;
 }
 
-static int copy_back(mdx_ctx *c, size_t count, double *host_out) {
-  return download_staged(c, host_out, c->dscratch, sizeof(double) * count);
-}
-
-int gather_w(mdx_ctx *c, const double4 *dev, double *host_out) {
+int gather_value(mdx_ctx *c, const double *dev, double *host_out) {
   const int B = 256, G = (c->n + B - 1) / B;
-  hipLaunchKernelGGL(k_gather_w, dim3(G), dim3(B), 0, c->stream, c->n, c->orig, dev, c->dscratch);
-  return copy_back(c, (size_t)c->n, host_out);
-}
-
-int gather_soa(mdx_ctx *c, const double *dev, int ncols, double *host_out) {
-  const int B = 256, G = (c->n + B - 1) / B;
-  hipLaunchKernelGGL(k_gather_soa, dim3(G), dim3(B), 0, c->stream, c->n, c->npad, ncols, c->orig, dev,
-                     c->dscratch);
-  return copy_back(c, (size_t)c->n * ncols, host_out);
+  hipLaunchKernelGGL(k_gather1, dim3(G), dim3(B), 0, c->stream, c->n, c->orig, dev, c->dscratch);
+  const Seg seg{host_out, c->dscratch, sizeof(double) * c->n, false};
+  return download(c, &seg, 1);
 }
 
 }  // namespace mdx

@@ -16,7 +16,7 @@
 //                                bits 0-26 of an entry hold the neighbour
 //                                index, bits 27-31 a periodic image code
 //                                (sx+1) + 3(sy+1) + 9(sz+1)
-//   vatom  double[6][npad] per-atom virial (SoA)
+//   vatom  double[npad][6] per-atom virial, caller order
 #pragma once
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -49,6 +49,8 @@ struct ListSlot {
   unsigned long long sum;   // entries they listed
   int line[12];
 };
+constexpr int kIoAtoms = 1024;      // systems whose positions and results travel through mapped host memory
+constexpr double kStageDoubles = 7.5;  // pinned staging per atom
 constexpr int kFlagInts = 16, kListSlots = 256;
 constexpr int kFlagWords = kFlagInts + kListSlots * (int)(sizeof(ListSlot) / sizeof(int));
 
@@ -349,6 +351,14 @@ __host__ __device__ __forceinline__ size_t list_index(int i, int k, int npad) {
   return (((size_t)(k >> 2) * npad + i) << 2) + (k & 3);
 }
 
+// Results that a force kernel without fused integration also writes in the
+// caller's atom order (null: not wanted): f [n][3], per-atom energy [n] and
+// virial [n][6] (energy/virial launches).  Device or mapped host memory.
+struct PairOut {
+  double *f, *e, *v;
+  const int *orig;  // caller index of each atom
+};
+
 struct IntegArgs {
   double mass[MDX_NT1];
   double dtf, dtv, triggersq;
@@ -369,6 +379,7 @@ struct IntegArgs {
   // plus the image-shift term of the pairs that cross a periodic boundary
   // (virial_fdotr_compute), about 6 FMAs per pair cheaper
   int pervir;
+  PairOut out;
 };
 
 struct Launch {
@@ -386,7 +397,7 @@ struct mdx_ctx {
   int periodic[3] = {1, 1, 1};
   bool box_set = false;
   // atoms
-  int n = 0, npad = 0, ntypes = 0, cap_atoms = 0;
+  int n = 0, npad = 0, ntypes = 0, cap_atoms = 0;  // arrays hold cap_atoms >= npad atoms
   double mass[MDX_NT1] = {0};
   double4 *x = nullptr, *xb = nullptr, *v = nullptr, *vb = nullptr, *f = nullptr, *xhold = nullptr;
   // fixed-point positions for the mixed-precision gathers (xqb: the fused
@@ -401,9 +412,12 @@ struct mdx_ctx {
   int *inv = nullptr;  // caller index -> device index
   double *vatom = nullptr;
   double *dscratch = nullptr;    // device, 6*npad doubles (host<->device reordering)
-  double *host_stage = nullptr;  // pinned, 6*npad doubles
-  hipEvent_t stage_ev[8] = {};   // chunked staging copies: one event per chunk in flight
-  int *host_istage = nullptr;    // pinned, 3*npad ints
+  double *host_stage = nullptr;  // pinned, kStageDoubles * cap_atoms doubles
+  bool stage_busy = false;       // queued work may still read host_stage or host_in
+  std::vector<hipEvent_t> stage_ev;  // one per piece in flight to the host
+  // mapped host memory of small systems (kIoAtoms): positions in, results out
+  double *host_in = nullptr, *host_out = nullptr;
+  char *dev_block = nullptr, *host_block = nullptr;  // one allocation each for the context's small arrays
   // bins / sort
   int nbins = 0, cap_bins = 0;
   mdx::NeighArgs na{};
@@ -456,14 +470,13 @@ struct mdx_ctx {
   double *partials = nullptr;
   long cap_partials = 0;
   int last_grid = 0;  // blocks of the last pair launch (partials to reduce)
-  double *red_out = nullptr;    // device, MDX_RED_SLOTS
-  double *red_host = nullptr;   // pinned, MDX_RED_SLOTS
+  double *red_host = nullptr;   // mapped, MDX_RED_SLOTS
   // Rebuild trigger of the displacement check, written by the kernels
   // straight into pinned host memory: a check stores its own stamp, so the
   // word needs no clearing and no device-to-host copy before it is read.
   int *trig_host = nullptr;
   int *trig_dev = nullptr;       // device copy of the trigger word
-  int *bflags_host = nullptr;    // pinned copy of the last build's flags
+  int *bflags_host = nullptr;    // mapped copy of the last build's flags
   int *dflags_base = nullptr;    // two sets of kFlagWords build flags (null: dflags alone, cleared per build)
   bool flags_dirty = false;      // a build started and did not pass its flags check
   bool bins_dirty = true;        // bin counters not known to be clear
@@ -545,20 +558,45 @@ int alloc_list(mdx_ctx *c, int cap);
 int neigh_check_displacement(mdx_ctx *c, int *flag);
 
 // pair kernels (pair.hip); eflag/vflag as Pair::compute.  Writes f (device,
-// sorted order), per-atom energy in f.w, per-atom virial in vatom, and the
+// sorted order), per-atom energy in f.w, and the
 // global energy/virial into c->red_host (after a sync) when ev is set.
-int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig = nullptr);
+// out: results also in caller order; wait: return only when red_host holds the
+// sums (else the caller synchronises).
+int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig = nullptr, const PairOut *out = nullptr, bool wait = true);
 Launch pair_launch(const mdx_ctx *c);  // the context's launch shape, defaults filled in for its size
 
 // integrator (integrate.hip)
 int nve_initial(mdx_ctx *c, double dtv, double dtf, int check);
 int nve_final(mdx_ctx *c, double dtf);
 int reduce_ke(mdx_ctx *c);
-int finish_reduction(mdx_ctx *c, int nblocks, int nslots);
+// doubles of the reduction records for n atoms: a record per workgroup of the
+// smallest launch shape (64 threads, up to 32 threads per atom), and the
+// first level's sums after them
+constexpr size_t partials_for(size_t n) {
+  const size_t G = (n * 32 + 63) / 64 + 1 + kXCD;
+  return (G + G / 256 + 2) * MDX_RED_SLOTS;
+}
+int finish_reduction(mdx_ctx *c, int nblocks, int nslots, bool wait = true);
 int scatter_positions(mdx_ctx *c, const double *host_x);
 int refresh_xq(mdx_ctx *c);  // rebuild the fixed-point positions if stale
 int copy_probe(mdx_ctx *c, long nbytes, int iters, double *gbs);
-// device order -> caller order [n][3] on the host; add: host += device
-int gather_vec3(mdx_ctx *c, const double4 *dev, double *host_out, bool add = false);
+// Transfers between device memory and the caller's arrays through the pinned
+// stage (integrate.hip): all segments in pieces, the host's share of one piece
+// overlapping the next piece's DMA.  upload returns when the host arrays have
+// been read, download when they are written; add: host += device (doubles).
+struct Seg {
+  void *host;
+  void *dev;
+  size_t bytes;
+  bool add;
+};
+int upload(mdx_ctx *c, const Seg *segs, int nseg);
+int download(mdx_ctx *c, const Seg *segs, int nseg);
+// caller's arrays -> the context's atoms, and the other way (null: not wanted)
+int load_atoms(mdx_ctx *c, const double *x, const double *v, const int *type, const int *tag);
+int store_atoms(mdx_ctx *c, double *x, double *v, double *f, int *image);
+// waits until queued work has read the staging memory
+int stage_ready(mdx_ctx *c);
+void host_add(double *dst, const double *src, size_t count);
 
 }  // namespace mdx

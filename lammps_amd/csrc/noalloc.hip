@@ -35,7 +35,7 @@ constexpr size_t align_up(size_t b) { return (b + kAlign - 1) / kAlign * kAlign;
 constexpr size_t kAtoms = MDX_NOALLOC_MAX_ATOMS;
 constexpr size_t kListEntries = (size_t)MDX_NOALLOC_MAX_ATOMS * MDX_NOALLOC_NEIGH_PER_ATOM;
 constexpr size_t kBins = MDX_NOALLOC_MAX_BINS;  // bin counters, including the scan's end slot
-constexpr size_t kPartials = (((size_t)MDX_NOALLOC_MAX_ATOMS * 32 + 63) / 64 + 1 + kXCD) * 8;
+constexpr size_t kPartials = partials_for(MDX_NOALLOC_MAX_ATOMS);
 constexpr size_t kScanBytes = size_t(1) << 20;  // hipcub scan temporary storage over kBins counters
 
 constexpr size_t kPerAtomBytes = align_up(sizeof(double4) * kAtoms) * 6 +  // x, xb, v, vb, f, xhold
@@ -46,7 +46,7 @@ constexpr size_t kPerAtomBytes = align_up(sizeof(double4) * kAtoms) * 6 +  // x,
                                  align_up(sizeof(int4) * kAtoms) * 2;       // xq, xqb
 constexpr size_t kScratchBytes = kPerAtomBytes + align_up(sizeof(int) * kListEntries) +
                                  align_up(sizeof(int) * kBins) * 2 + align_up(sizeof(double) * kPartials) +
-                                 kScanBytes + align_up(sizeof(int) * kFlagWords) + align_up(sizeof(double) * MDX_RED_SLOTS);
+                                 kScanBytes + align_up(sizeof(int) * kFlagWords);
 static_assert(kScratchBytes <= (size_t)MDX_NOALLOC_SCRATCH_BYTES, "scratch layout exceeds its stated size");
 
 }  // namespace
@@ -237,7 +237,6 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
   s.scan_tmp = cv.take<unsigned char>(kScanBytes);
   s.scan_tmp_bytes = kScanBytes;
   s.dflags = cv.take<int>(kFlagWords);
-  s.red_out = cv.take<double>(MDX_RED_SLOTS);
   if ((size_t)(cv.p - base) > (size_t)MDX_NOALLOC_SCRATCH_BYTES) {
     set_error("mdx_compute_noalloc: scratch layout overrun");
     return MDX_ERR_ARG;

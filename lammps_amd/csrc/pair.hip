@@ -227,10 +227,13 @@ __device__ __forceinline__ double integrate_atom(int i, const double4 &xi, doubl
 // per-atom results of one group: lane 0 stores (and integrates when fused),
 // all lanes join the block sum of {e, virial[6], m v^2}
 template <int TPA, bool EV, bool INTEG, bool LATE = false>
-__device__ __forceinline__ void finish_atom(int i, bool owner, int npad, const double4 &xi, double fx, double fy,
+__device__ __forceinline__ void finish_atom(int i, bool owner, const double4 &xi, double fx, double fy,
                                             double fz, double e, double (&w)[6], const IntegArgs &ig,
                                             double4 vpre, double4 hpre, double4 *__restrict__ f,
-                                            double *__restrict__ vatom, double *__restrict__ partials) {
+                                            double *__restrict__ partials) {
+  int o = 0;  // caller index: its load overlaps the lane sums
+  const bool caller = !INTEG && owner && (ig.out.f || (EV && (ig.out.e || ig.out.v)));
+  if (caller) o = ig.out.orig[i];
   fx = group_sum<TPA>(fx);
   fy = group_sum<TPA>(fy);
   fz = group_sum<TPA>(fz);
@@ -242,10 +245,21 @@ __device__ __forceinline__ void finish_atom(int i, bool owner, int npad, const d
   double mv2 = 0.0;
   if (owner) {
     if (!INTEG || EV || ig.write_f) f[i] = make_double4(fx, fy, fz, e);
-    if (EV && ig.pervir) {
+    if (caller) {
+      if (ig.out.f) {
+        double *const d = ig.out.f + 3 * (size_t)o;
+        d[0] = fx;
+        d[1] = fy;
+        d[2] = fz;
+      }
+      if (EV && ig.out.e) ig.out.e[o] = e;
+      if (EV && ig.pervir && ig.out.v) {
+        double *const d = ig.out.v + 6 * (size_t)o;
 #pragma unroll
-      for (int q = 0; q < 6; q++) vatom[(size_t)q * npad + i] = w[q];
-    } else if (EV) {  // the x_i f_i share of the global virial
+        for (int q = 0; q < 6; q++) d[q] = w[q];
+      }
+    }
+    if (EV && !ig.pervir) {  // the x_i f_i share of the global virial
       w[0] += xi.x * fx;
       w[1] += xi.y * fy;
       w[2] += xi.z * fz;
@@ -293,7 +307,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
                                            const double4 *__restrict__ x, const int4 *__restrict__ xq, QScale qs,
                                            const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                            const LJTab *__restrict__ tab, double4 *__restrict__ f,
-                                           double *__restrict__ vatom, double *__restrict__ partials, IntegArgs ig,
+                                           double *__restrict__ partials, IntegArgs ig,
                                            LJOne one) {
   if constexpr (INTEG) {
     if (gate_closed(ig.gate)) return;
@@ -449,7 +463,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     }
   }
   if (Q && i < n && lane == 0) xi = x[i];
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f, vatom,
+  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
                               partials);
 }
 
@@ -591,8 +605,8 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int ca
                                                   const int4 *__restrict__ xq, QScale qs,
                                                   const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                                   const double *__restrict__ fp, const double *__restrict__ eemb,
-                                                  double4 *__restrict__ f, double *__restrict__ vatom,
-                                                  double *__restrict__ partials, IntegArgs ig) {
+                                                  double4 *__restrict__ f, double *__restrict__ partials,
+                                                  IntegArgs ig) {
   static_assert(!TL || ONE, "LDS tables hold the one table of a single-type system");
   if constexpr (INTEG) {
     if (gate_closed(ig.gate)) return;
@@ -714,7 +728,7 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int ca
     if (EV && lane == 0) e += eemb[i];
   }
   if (Q && i < n && lane == 0) xi = x[i];
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, npad, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f, vatom,
+  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
                               partials);
 }
 
@@ -781,7 +795,7 @@ void launch_lj_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   }
   hipLaunchKernelGGL((k_lj<MIXED, EV, TPA, INTEG, Q, ONE>), dim3(G), dim3(B), lds, c->stream, c->n, c->npad, c->maxneigh,
                      c->ntypes + 1, c->prd[0], c->prd[1], c->prd[2], c->x, c->xq, c->qs, c->nbr, c->numneigh,
-                     c->lj_dev, c->f, c->vatom, c->partials, ig, one);
+                     c->lj_dev, c->f, c->partials, ig, one);
   prof_end(c);
   c->last_grid = G;
 }
@@ -808,7 +822,7 @@ void launch_eam_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   const size_t tl_bytes = TL ? kn * (MIXED ? 3 * sizeof(float4) : 5 * sizeof(double2)) : 0;
   hipLaunchKernelGGL((k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>), dim3(G), dim3(B),
                      INTEG ? occupancy_lds(static_lds<k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>>(), B, tl_bytes, 0) : tl_bytes, c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1],
-                     c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp, c->eemb, c->f, c->vatom,
+                     c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp, c->eemb, c->f,
                      c->partials, ig);
   prof_end(c);
   c->last_grid = G;
@@ -915,7 +929,7 @@ Launch pair_launch(const mdx_ctx *c) {
 // forces only, 1 also energy and global virial, 2 also the per-atom virial;
 // with ev the reduction's slots are {eng_vdwl, virial[6], sum m v^2 (fused
 // only)}.
-int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig) {
+int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig, const PairOut *out, bool wait) {
   if (c->n == 0) {  // no atoms: zero energy, virial and kinetic sums
     for (int k = 0; k < MDX_RED_SLOTS; k++) c->red_host[k] = 0.0;
     return MDX_OK;
@@ -928,13 +942,14 @@ int pair_compute(mdx_ctx *c, int ev, const IntegArgs *ig) {
   const int nslots = 8;
   IntegArgs args = ig ? *ig : IntegArgs{};
   args.pervir = ev >= 2 ? 1 : 0;
+  if (out) args.out = *out;
   if (ig) rc = dispatch_prec<true>(c, ev, args);
   else rc = dispatch_prec<false>(c, ev, args);
   if (rc) return rc;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "pair kernel launch");
   // the per-atom energy in f.w already includes the EAM embedding term
-  if (ev) return finish_reduction(c, c->last_grid, nslots);
+  if (ev) return finish_reduction(c, c->last_grid, nslots, wait);
   return MDX_OK;
 }
 

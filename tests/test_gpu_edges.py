@@ -545,3 +545,67 @@ def test_default_launch_shapes_agree_with_a_fixed_one(style, n):
     assert force_errors(got["f"], want["f"])[0] <= 1e-12
     assert abs(got["eng"] - want["eng"]) <= 1e-12 * abs(want["eng"])
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [255, 1023, 1024, 1025])
+def test_transfers_on_both_sides_of_the_mapped_memory_line(n):
+    """Systems up to 1,024 atoms exchange positions and results through mapped
+    host memory, larger ones through copies: what set_atoms took comes back
+    unchanged, and forces, per-atom energies and virials match the oracle's."""
+    from lammps_amd import mdx
+    L = (n / 0.85) ** (1.0 / 3.0)
+    x = random_gas(n, L, 0.8, seed=n)
+    v = np.random.default_rng(n).normal(size=(n, 3))
+    ref = M.Ref(M.LJ)
+    ref.box((0, 0, 0), (L, L, L))
+    ref.add_atoms(x, np.ones(n, dtype=np.int32))
+    ref.mass(1, 1.0)
+    ref.pair_lj(2.5)
+    ref.pair_coeff(1, 1, 1.0, 1.0, 2.5)
+    ref.neighbor(0.3)
+    ref.setup()
+    ref.compute(3, 5)
+    ea, va = ref.peratom()
+    ctx = mdx.Context(0)
+    ctx.set_box((0, 0, 0), (L, L, L), (1, 1, 1))
+    ctx.set_atoms(x, np.ones(n, dtype=np.int32), MASS, v=v)
+    ctx.pair_lj_from_coeffs(1, {(1, 1): (1.0, 1.0, 2.5)})
+    ctx.neigh_modify(0.3)
+    gx, gv, gf, gi = ctx.get_atoms()
+    assert np.array_equal(gx, x) and np.array_equal(gv, v) and not gf.any() and not gi.any()
+    for _ in range(2):  # the second call after a position update
+        out = ctx.compute(3, 5, peratom=True)
+        assert force_errors(out["f"], ref.state()[2])[0] <= 1e-11
+        np.testing.assert_allclose(out["eatom"], ea, rtol=0, atol=1e-10 * np.abs(ea).max())
+        np.testing.assert_allclose(out["vatom"], va, rtol=0, atol=1e-10 * np.abs(va).max())
+        ctx.set_positions(x)
+        ctx.set_positions(x)
+    ctx.close()
+
+
+def test_atoms_handed_over_again_give_what_a_fresh_context_gives():
+    """set_atoms keeps storage that fits: growing, shrinking and regrown atom
+    counts, changed density, types and velocities in one context, each against
+    a context of its own."""
+    from lammps_amd import mdx
+
+    def forces(ctx, k, n, L, ntypes):
+        rng = np.random.default_rng(k)
+        x = random_gas(n, L, 0.8, seed=k)
+        t = rng.integers(1, ntypes + 1, n).astype(np.int32)
+        ctx.set_box((0, 0, 0), (L, L, L), (1, 1, 1))
+        ctx.set_atoms(x, t, np.ones(ntypes + 1), v=None if k % 2 else x)
+        ctx.pair_lj_from_coeffs(ntypes, {(i, i): (1.0, 1.0, 2.5) for i in range(1, ntypes + 1)})
+        ctx.neigh_modify(0.3)
+        ctx.precision(mdx.MIXED if k % 3 == 0 else mdx.FP64)
+        out = ctx.compute(3, 5, peratom=True)
+        return [out["f"], out["eatom"], out["vatom"], np.array([out["eng"]])] + list(ctx.get_atoms())
+
+    kept = mdx.Context(0)
+    for k, (n, L, nt) in enumerate([(3000, 16.0, 1), (2900, 15.5, 1), (3072, 40.0, 1), (1600, 13.0, 1), (1400, 12.5, 1),
+                                    (2999, 15.5, 1), (700, 9.5, 1), (1200, 12.0, 1)]):
+        fresh = mdx.Context(0)
+        for a, b in zip(forces(kept, k, n, L, nt), forces(fresh, k, n, L, nt)):
+            assert np.array_equal(a, b), (k, n)
+        fresh.close()
+    kept.close()
