@@ -245,7 +245,7 @@ int mdx_create(int device, mdx_ctx **out) {
     p += (bytes + 255) / 256 * 256;
     return q;
   };
-  constexpr size_t kHostBlock = 4 * 256 + sizeof(double) * (3 + 11) * kIoAtoms + 512;
+  constexpr size_t kHostBlock = 5 * 256 + sizeof(double) * (3 + 11) * kIoAtoms + 512;
   constexpr size_t kDevBlock = sizeof(int) * 2 * kFlagWords + sizeof(NeighArgs) + sizeof(LJTab) + 5 * 256;
   static_assert(sizeof(double) * MDX_RED_SLOTS <= 256 && sizeof(int) * kFlagInts <= 256, "one slot each");
   if (hipMalloc(&c->dev_block, kDevBlock) != hipSuccess ||
@@ -257,6 +257,7 @@ int mdx_create(int device, mdx_ctx **out) {
   char *hp = c->host_block, *dp = c->dev_block;
   c->red_host = reinterpret_cast<double *>(carve(hp, sizeof(double) * MDX_RED_SLOTS));
   c->trig_host = reinterpret_cast<int *>(carve(hp, 64));
+  c->decided_host = reinterpret_cast<int *>(carve(hp, 64));
   c->bflags_host = reinterpret_cast<int *>(carve(hp, sizeof(int) * kFlagInts));
   c->host_in = reinterpret_cast<double *>(carve(hp, sizeof(double) * 3 * kIoAtoms));
   c->host_out = reinterpret_cast<double *>(carve(hp, sizeof(double) * 11 * kIoAtoms));
@@ -264,12 +265,10 @@ int mdx_create(int device, mdx_ctx **out) {
   c->trig_dev = reinterpret_cast<int *>(carve(dp, 64));
   c->na_dev = reinterpret_cast<NeighArgs *>(carve(dp, sizeof(NeighArgs)));
   c->lj_dev = reinterpret_cast<LJTab *>(carve(dp, sizeof(LJTab)));
-  memset(c->trig_host, 0, 64);
+  memset(c->host_block, 0, kHostBlock);
   c->dflags = c->dflags_base;
   // flags and trigger word, side by side
-  if (hipMemsetAsync(c->dflags_base, 0, (char *)c->trig_dev + 64 - (char *)c->dflags_base, c->stream) != hipSuccess ||
-      hipEventCreateWithFlags(&c->step_ev, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->build_ev, hipEventDisableTiming) != hipSuccess) {
+  if (hipMemsetAsync(c->dflags_base, 0, (char *)c->trig_dev + 64 - (char *)c->dflags_base, c->stream) != hipSuccess) {
     set_error("device flags initialisation failed");
     (void)mdx_destroy(c);
     return MDX_ERR_HIP;
@@ -294,8 +293,6 @@ int mdx_destroy(mdx_ctx *c) {
     if (p) (void)hipFree(p);
   halo_free(c);
   for (hipEvent_t ev : c->stage_ev) (void)hipEventDestroy(ev);
-  if (c->step_ev) (void)hipEventDestroy(c->step_ev);
-  if (c->build_ev) (void)hipEventDestroy(c->build_ev);
   if (c->host_block) (void)hipHostFree(c->host_block);
   for (auto &r : c->evpool) {
     (void)hipEventDestroy(r.a);
@@ -783,18 +780,20 @@ int mdx_run(mdx_ctx *c, int nsteps, double dt, double ftm2v, int thermo_every, m
         if (fused && !pending_initial && !out) {
           // Look-ahead decide: the trigger was computed by the previous
           // step's fused kernel.  This step's kernels are queued before the
-          // host reads it, predicated on its device copy, so the device
-          // never idles while the host decides; when it fired they do
+          // host knows it, predicated on its device word, so the device
+          // never idles while the host decides; the first of them tells the
+          // host the outcome as it starts.  When the trigger fired they do
           // nothing and the step is queued again after the rebuild.
           const int prev = c->trig_stamp;
           IntegArgs ig = step_args(is_last);
           ig.gate.trig = c->trig_dev;
           ig.gate.stamp = prev;
+          ig.gate.decided = c->decided_host;
           if ((rc = pair_compute(c, 0, &ig))) return rc;
           queued = true;
-          hipError_t e = hipEventSynchronize(c->step_ev);
-          if (e != hipSuccess) return hip_fail(e, "trigger wait");
-          flag = __atomic_load_n(c->trig_host, __ATOMIC_ACQUIRE) == prev ? 1 : 0;
+          int word = prev;  // no atoms: no kernel, nothing moved
+          if (c->n > 0 && (rc = wait_word(c->stream, c->decided_host, prev, -prev, &word))) return rc;
+          flag = word < 0 ? 1 : 0;
         } else if ((rc = neigh_check_displacement(c, &flag))) {
           return rc;
         }
@@ -830,13 +829,6 @@ int mdx_run(mdx_ctx *c, int nsteps, double dt, double ftm2v, int thermo_every, m
       if (!queued) {
         IntegArgs ig = step_args(is_last);
         if ((rc = pair_compute(c, out ? 1 : 0, &ig))) return rc;
-      }
-      // the next step's look-ahead decide waits for this step's kernels
-      // (which compute its trigger); an event costs the queue a few us, so
-      // it is recorded only then
-      if (!is_last && c->check && is_decide(c->ago + 1)) {
-        hipError_t e = hipEventRecord(c->step_ev, c->stream);
-        if (e != hipSuccess) return hip_fail(e, "step event");
       }
       if (out) {
         c->eng_vdwl = c->red_host[0];

@@ -1471,7 +1471,7 @@ int build(mdx_batch *b) {
       };
       if (b->mirror_ok) go(k_b_build<true>);
       else go(k_b_build<false>);
-      launch_build_flags(b->stream, b->dflags, b->flags_host);
+      launch_build_flags(b->stream, b->dflags, b->flags_host, 1);  // the event below is waited for
     };
     if ((rc = timed(b, MDX_BK_BUILD, b->tune[MDX_BK_BUILD], launch))) return rc;
     int fl[kFlagInts];

@@ -51,6 +51,7 @@ struct ListSlot {
 };
 constexpr int kIoAtoms = 1024;      // systems whose positions and results travel through mapped host memory
 constexpr double kStageDoubles = 7.5;  // pinned staging per atom
+constexpr int kFlagSerial = 15;  // mapped flags only: the build they belong to, written last
 constexpr int kFlagInts = 16, kListSlots = 256;
 constexpr int kFlagWords = kFlagInts + kListSlots * (int)(sizeof(ListSlot) / sizeof(int));
 
@@ -331,10 +332,21 @@ struct StepGate {
   int stamp;
   const int *bflags;  // build flags, or null
   int cap;            // list capacity the build ran with
+  // Mapped host word, or null: the launch's first thread stores `stamp` when
+  // the trigger had not fired, -stamp when it had.  The launch starts after
+  // the kernels that test the displacements, so the word tells the host their
+  // outcome while the step itself runs; an event recorded between the two
+  // launches idles the queue for about 6 us.
+  int *decided;
 };
 
 __device__ __forceinline__ bool gate_closed(const StepGate &g) {
-  if (g.trig && __hip_atomic_load(g.trig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.stamp) return true;
+  if (g.trig) {
+    const bool fired = __hip_atomic_load(g.trig, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.stamp;
+    if (g.decided && blockIdx.x == 0 && threadIdx.x == 0)
+      __hip_atomic_store(g.decided, fired ? -g.stamp : g.stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (fired) return true;
+  }
   if (g.bflags) {
     const int mx = __hip_atomic_load(g.bflags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int lost = __hip_atomic_load(g.bflags + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -480,9 +492,9 @@ struct mdx_ctx {
   int *dflags_base = nullptr;    // two sets of kFlagWords build flags (null: dflags alone, cleared per build)
   bool flags_dirty = false;      // a build started and did not pass its flags check
   bool bins_dirty = true;        // bin counters not known to be clear
-  hipEvent_t build_ev = nullptr; // recorded after that copy
+  int flag_serial = 0;           // list passes whose flags were asked for (kFlagSerial)
   int trig_stamp = 0;
-  hipEvent_t step_ev = nullptr;  // recorded after each fused step's kernels (look-ahead decide)
+  int *decided_host = nullptr;   // mapped: outcome of the look-ahead decide (StepGate::decided)
   // results of the last compute
   double eng_vdwl = 0.0, virial[6] = {0, 0, 0, 0, 0, 0};
   // launch shape and timing (event pairs recorded on `stream`, resolved
@@ -538,8 +550,12 @@ int prof_resolve(mdx_ctx *c);
 // Pair::init + Neighbor::init cutoffs, bin grid, first list and partials (api.cpp)
 int prepare_ctx(mdx_ctx *c);
 // combines a list pass's slots into its build flags and writes those to the
-// mapped host words `host` as well (neigh.hip)
-void launch_build_flags(hipStream_t stream, int *dflags, int *host);
+// mapped host words `host` as well, `serial` (never 0) into host[kFlagSerial]
+// after all the others (neigh.hip)
+void launch_build_flags(hipStream_t stream, int *dflags, int *host, int serial);
+// Waits until a queued kernel has stored `a` or `b` into a mapped host word;
+// *got is the value.  Fails if the stream fails or ends without it.
+int wait_word(hipStream_t stream, const int *word, int a, int b, int *got);
 // no-allocation compute (noalloc.hip)
 int noalloc_init(int device);
 int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int eflag, int vflag, double *f,

@@ -156,7 +156,8 @@ __device__ __forceinline__ void stage_band(const NeighArgs &a, float *lo, float 
 
 // The list pass's counters into the build flags, and the flags into pinned
 // host memory (in place of a copy): one workgroup, one slot per thread.
-__global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ dflags, int *__restrict__ host) {
+__global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ dflags, int *__restrict__ host,
+                                                             int serial) {
   __shared__ int s_most[kListSlots / 64];
   __shared__ unsigned long long s_sum[kListSlots / 64];
   const ListSlot &slot = reinterpret_cast<const ListSlot *>(dflags + kFlagInts)[threadIdx.x];
@@ -183,7 +184,11 @@ __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ df
   if (threadIdx.x == 8) v = static_cast<int>(sum);
   if (threadIdx.x == 9) v = static_cast<int>(sum >> 32);
   dflags[threadIdx.x] = v;
-  host[threadIdx.x] = v;
+  if (threadIdx.x != kFlagSerial) host[threadIdx.x] = v;
+  // the host waits for this word alone: the flags above are there before it
+  // (the threads are lanes of one wavefront)
+  __threadfence_system();
+  if (threadIdx.x == kFlagSerial) __hip_atomic_store(host + kFlagSerial, serial, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Domain::pbc + bin index + histogram; one thread per atom.  slot[i] is the
@@ -1067,8 +1072,31 @@ void launch_build(mdx_ctx *c) {
 
 }  // namespace
 
-void launch_build_flags(hipStream_t stream, int *dflags, int *host) {
-  hipLaunchKernelGGL(k_build_flags, dim3(1), dim3(kListSlots), 0, stream, dflags, host);
+void launch_build_flags(hipStream_t stream, int *dflags, int *host, int serial) {
+  hipLaunchKernelGGL(k_build_flags, dim3(1), dim3(kListSlots), 0, stream, dflags, host, serial);
+}
+
+int wait_word(hipStream_t stream, const int *word, int a, int b, int *got) {
+  for (long spin = 1;; spin++) {
+    const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if (v == a || v == b) {
+      *got = v;
+      return MDX_OK;
+    }
+    if (spin % 4096) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    // a stream that failed, or ran dry without the store, will not store it
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return hip_fail(e, "queued work");
+    const int last = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if (last != a && last != b) {
+      set_error("queued work ended without its result");
+      return MDX_ERR_HIP;
+    }
+  }
 }
 
 int neigh_setup_grid(mdx_ctx *c) {
@@ -1244,10 +1272,10 @@ int launch_list(mdx_ctx *c, bool again) {
       return hip_fail(e, "memset flags");
   }
   launch_build(c);
-  launch_build_flags(c->stream, c->dflags, c->bflags_host);
+  c->flag_serial = c->flag_serial == 0x7fffffff ? 1 : c->flag_serial + 1;
+  launch_build_flags(c->stream, c->dflags, c->bflags_host, c->flag_serial);
   prof_end(c);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "list build launch");
-  if ((e = hipEventRecord(c->build_ev, c->stream)) != hipSuccess) return hip_fail(e, "build event");
   return MDX_OK;
 }
 
@@ -1257,8 +1285,9 @@ int launch_list(mdx_ctx *c, bool again) {
 int neigh_build_finish(mdx_ctx *c, bool *regrow) {
   *regrow = false;
   if (c->n == 0) return MDX_OK;
-  hipError_t e = hipEventSynchronize(c->build_ev);
-  if (e != hipSuccess) return hip_fail(e, "neighbour build");
+  int serial;
+  int rc = wait_word(c->stream, c->bflags_host + kFlagSerial, c->flag_serial, c->flag_serial, &serial);
+  if (rc) return rc;
   int flags[16];
   memcpy(flags, c->bflags_host, sizeof(flags));
   if (flags[4]) {
@@ -1278,8 +1307,7 @@ int neigh_build_finish(mdx_ctx *c, bool *regrow) {
     // regrow: the accelerator library's max_nbors resize (lal_neighbor.cpp:582-595)
     int cap = ((mx + mx / 4 + 15) / 16) * 16;
     cap = std::min(cap, c->one);
-    int rc = alloc_list(c, cap);
-    if (rc) return rc;
+    if ((rc = alloc_list(c, cap))) return rc;
     *regrow = true;
     return MDX_OK;
   }

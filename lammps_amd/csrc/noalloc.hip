@@ -190,7 +190,7 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
   s.red_host = c->red_host;  // pinned host slots of the caller's context
   s.bflags_host = c->bflags_host;
   s.na_dev = c->na_dev;
-  s.build_ev = c->build_ev;
+  s.flag_serial = c->flag_serial;  // the mapped flags' serial goes on from the caller's context
   s.profile = false;
   s.fixed_storage = true;
   s.n = n;
@@ -251,7 +251,9 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "pack launch");
   int rc = prepare_ctx(&s);
   if (rc) return rc;
-  if ((rc = neigh_build(&s))) return rc;  // synchronises; reads the build flags
+  rc = neigh_build(&s);  // waits for the build flags
+  c->flag_serial = s.flag_serial;
+  if (rc) return rc;
   int bad = 0;
   if ((e = hipMemcpy(&bad, s.dflags + 6, sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess)
     return hip_fail(e, "read flags");

@@ -818,12 +818,14 @@ void launch_eam_t(mdx_ctx *c, int B, const IntegArgs &ig) {
                      occupancy_lds(static_lds<k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>>(), B, TL ? kn * (MIXED ? sizeof(float4) : sizeof(double4)) : 0, 0), c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs,
                      c->nbr, c->numneigh, c->rho, c->fp, c->eemb, INTEG ? ig.gate : StepGate{});
   prof_end(c);
+  IntegArgs fi = ig;
+  fi.gate.decided = nullptr;  // the density pass has told the host
   prof_begin(c, INTEG ? MDX_K_FUSED : MDX_K_EAM_FORCE);
   const size_t tl_bytes = TL ? kn * (MIXED ? 3 * sizeof(float4) : 5 * sizeof(double2)) : 0;
   hipLaunchKernelGGL((k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>), dim3(G), dim3(B),
                      INTEG ? occupancy_lds(static_lds<k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>>(), B, tl_bytes, 0) : tl_bytes, c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1],
                      c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp, c->eemb, c->f,
-                     c->partials, ig);
+                     c->partials, fi);
   prof_end(c);
   c->last_grid = G;
 }
