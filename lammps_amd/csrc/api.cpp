@@ -94,14 +94,14 @@ int check_ctx(mdx_ctx *c) {
 void free_atoms(mdx_ctx *c) {
   if (c->stage_busy) (void)hipStreamSynchronize(c->stream);  // queued copies still read the stage
   void *ptrs[] = {c->x, c->xb, c->v, c->vb, c->f, c->xhold, c->tag, c->tagb, c->orig, c->origb, c->image,
-                  c->imageb, c->inv, c->vatom, c->dscratch, c->bkey, c->bkey_s, c->bidx, c->bidx_s,
+                  c->imageb, c->inv, c->vatom, c->dscratch, c->bkey, c->bidx, c->bidx_s,
                   c->numneigh, c->nbr, c->rho, c->fp, c->eemb, c->partials, c->xq, c->xqb};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   c->x = c->xb = c->v = c->vb = c->f = c->xhold = nullptr;
   c->tag = c->tagb = c->orig = c->origb = c->image = c->imageb = c->inv = nullptr;
   c->vatom = c->dscratch = nullptr;
-  c->bkey = c->bkey_s = nullptr;
+  c->bkey = nullptr;
   c->bidx = c->bidx_s = c->numneigh = c->nbr = nullptr;
   c->rho = c->fp = c->eemb = c->partials = nullptr;
   c->xq = c->xqb = nullptr;
@@ -366,7 +366,7 @@ int mdx_set_atoms(mdx_ctx *c, int n, int ntypes, const double *x, const double *
         (rc = dev_alloc(&c->origb, npad)) || (rc = dev_alloc(&c->image, npad)) ||
         (rc = dev_alloc(&c->imageb, npad)) || (rc = dev_alloc(&c->inv, npad)) ||
         (rc = dev_alloc(&c->vatom, (size_t)6 * npad)) || (rc = dev_alloc(&c->dscratch, (size_t)6 * npad)) ||
-        (rc = dev_alloc(&c->bkey, npad)) || (rc = dev_alloc(&c->bkey_s, npad)) || (rc = dev_alloc(&c->bidx, npad)) ||
+        (rc = dev_alloc(&c->bkey, npad)) || (rc = dev_alloc(&c->bidx, npad)) ||
         (rc = dev_alloc(&c->bidx_s, npad)) || (rc = dev_alloc(&c->numneigh, npad)) ||
         (rc = dev_alloc(&c->rho, npad)) || (rc = dev_alloc(&c->fp, npad)) || (rc = dev_alloc(&c->eemb, npad)) ||
         (rc = dev_alloc(&c->xq, npad)) || (rc = dev_alloc(&c->xqb, npad)))

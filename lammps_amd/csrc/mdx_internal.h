@@ -245,15 +245,6 @@ __host__ __device__ inline int bin_row(const NeighArgs &a, int y, int z) {
 __host__ __device__ inline int bin_index(const NeighArgs &a, int x, int y, int z) {
   return bin_row(a, y, z) * a.nbin[0] + x;
 }
-__host__ __device__ inline void bin_coords(const NeighArgs &a, int b, int &x, int &y, int &z) {
-  x = b % a.nbin[0];
-  const int r = b / a.nbin[0];
-  const int y0 = (r / (kBinTileY * a.nbin[2])) * kBinTileY;
-  const int th = imin2(kBinTileY, a.nbin[1] - y0);
-  const int rem = r - y0 * a.nbin[2];
-  z = rem / th;
-  y = y0 + rem % th;
-}
 
 // 32-bit fixed-point positions read by the mixed-precision gathers (16 B
 // per neighbour instead of 32).  Per dimension q = round((x - lo) * scale)
@@ -434,7 +425,7 @@ struct mdx_ctx {
   int nbins = 0, cap_bins = 0;
   mdx::NeighArgs na{};
   mdx::NeighArgs *na_dev = nullptr;  // device copy of the current build's (its first kernel writes it)
-  unsigned *bkey = nullptr, *bkey_s = nullptr;
+  unsigned *bkey = nullptr;
   int *bidx = nullptr, *bidx_s = nullptr, *bin_count = nullptr, *bin_start = nullptr;
   void *scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ df
 }
 
 // Domain::pbc + bin index + histogram; one thread per atom.  slot[i] is the
-// atom's arrival order in its bin (not deterministic; k_bin_rank orders
+// atom's arrival order in its bin (not deterministic; k_rank_permute orders
 // each bin by atom index).  Atoms arrive nearly bin-sorted (the previous
 // build's order), so the lanes of a wavefront with equal bins form runs: one
 // returning atomic per run reserves the run's slots, and no two lanes of a
@@ -293,13 +293,22 @@ __global__ void k_bin_scatter(int n, const unsigned *__restrict__ key, const int
 // order (still a permutation, so the passes after it stay in bounds) and
 // raises the overflow flag, which the build reports; the scan is thus
 // bounded by `one` + 1 entries per atom.
-__global__ void k_bin_rank(int n, const unsigned *__restrict__ key, const int *__restrict__ bin_start,
-                           const int *__restrict__ tmp, int *__restrict__ src, unsigned *__restrict__ key_s,
-                           int max_occupancy, int *__restrict__ dflags) {
+// The same thread then moves its atom to its place (p stays near it: a bin's
+// entries are a few): one launch and two passes over the order less than
+// ranking into an index array and permuting by it.
+__global__ void k_rank_permute(int n, const unsigned *__restrict__ key, const int *__restrict__ bin_start,
+                               const int *__restrict__ tmp, int max_occupancy, int *__restrict__ dflags,
+                               const double4 *__restrict__ x, const double4 *__restrict__ v,
+                               const int *__restrict__ tag, const int *__restrict__ orig,
+                               const int *__restrict__ image, double4 *__restrict__ xo, double4 *__restrict__ vo,
+                               int *__restrict__ tago, int *__restrict__ origo, int *__restrict__ imageo,
+                               int *__restrict__ inv, double4 *__restrict__ xhold, int4 *__restrict__ xq, QScale qs) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int i = tmp[p];
   const unsigned b = key[i];
+  const double4 q = x[i], w = v[i];
+  const int t = tag[i], o = orig[i], im = image[i];
   const int s = bin_start[b], e = bin_start[b + 1];
   int r = p - s;
   if (e - s <= max_occupancy) {
@@ -308,29 +317,63 @@ __global__ void k_bin_rank(int n, const unsigned *__restrict__ key, const int *_
   } else if (p == s) {
     atomicOr(&dflags[5], 1);
   }
-  src[s + r] = i;
-  key_s[s + r] = b;
+  const int k = s + r;
+  xo[k] = q;
+  xhold[k] = q;
+  if (xq) xq[k] = quantize(qs, q);
+  vo[k] = w;
+  tago[k] = t;
+  origo[k] = o;
+  imageo[k] = im;
+  inv[o] = k;
 }
 
-__global__ void k_permute(int n, const int *__restrict__ src, const double4 *__restrict__ x,
-                          const double4 *__restrict__ v, const int *__restrict__ tag,
-                          const int *__restrict__ orig, const int *__restrict__ image, double4 *__restrict__ xo,
-                          double4 *__restrict__ vo, int *__restrict__ tago, int *__restrict__ origo,
-                          int *__restrict__ imageo, int *__restrict__ inv, double4 *__restrict__ xhold,
-                          int4 *__restrict__ xq, QScale qs) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  int o = src[k];
-  double4 p = x[o];
-  xo[k] = p;
-  xhold[k] = p;
-  if (xq) xq[k] = quantize(qs, p);
-  vo[k] = v[o];
-  tago[k] = tag[o];
-  int oi = orig[o];
-  origo[k] = oi;
-  imageo[k] = image[o];
-  inv[oi] = k;
+// Exclusive scan of the bin counters in one workgroup, for grids of up to
+// kScanBins bins (each thread a run of consecutive counters in 16-B loads):
+// one launch of about 4 us where the library's scan takes two and about 9.
+constexpr int kScanThreads = 1024, kScanPer = 32, kScanBins = kScanThreads * kScanPer;
+__global__ __launch_bounds__(kScanThreads) void k_scan_bins(int m, const int *__restrict__ count,
+                                                           int *__restrict__ start) {
+  __shared__ int s_wave[kScanThreads / 64];
+  const int per = ((m + kScanThreads - 1) / kScanThreads + 3) / 4 * 4;  // <= kScanPer
+  const int b0 = min(m, (int)threadIdx.x * per), b1 = min(m, b0 + per);
+  int4 c[kScanPer / 4];
+  int sum = 0;
+#pragma unroll
+  for (int q = 0; q < kScanPer / 4; q++) {
+    const int k = b0 + 4 * q;
+    c[q] = make_int4(0, 0, 0, 0);
+    if (k + 3 < b1) {
+      c[q] = *reinterpret_cast<const int4 *>(count + k);
+    } else if (k < b1) {  // the last counters
+      c[q].x = count[k];
+      if (k + 1 < b1) c[q].y = count[k + 1];
+      if (k + 2 < b1) c[q].z = count[k + 2];
+    }
+    sum += c[q].x + c[q].y + c[q].z + c[q].w;
+  }
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int incl = sum;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int up = __shfl_up(incl, off);
+    if (lane >= off) incl += up;
+  }
+  if (lane == 63) s_wave[w] = incl;
+  __syncthreads();
+  int at = incl - sum;
+  for (int q = 0; q < w; q++) at += s_wave[q];
+#pragma unroll
+  for (int q = 0; q < kScanPer / 4; q++) {
+    const int k = b0 + 4 * q;
+    if (k < b1) start[k] = at;
+    at += c[q].x;
+    if (k + 1 < b1) start[k + 1] = at;
+    at += c[q].y;
+    if (k + 2 < b1) start[k + 2] = at;
+    at += c[q].z;
+    if (k + 3 < b1) start[k + 3] = at;
+    at += c[q].w;
+  }
 }
 
 // One lane per atom.  A lane walks ~300 candidates, so
@@ -359,7 +402,6 @@ __global__ void k_permute(int n, const int *__restrict__ src, const double4 *__r
 template <bool Q, bool ONE>
 __global__ __launch_bounds__(256, Q ? MDX_BUILD_Q_WAVES : MDX_BUILD_MIN_WAVES) void k_build_lane(NeighArgs a, const double4 *__restrict__ x,
                                                    const int4 *__restrict__ xq, QStep qs,
-                                                   const unsigned *__restrict__ bkey,
                                                    const int *__restrict__ bin_start, int *__restrict__ nbr,
                                                    int *__restrict__ numneigh, ListSlot *__restrict__ slots) {
   __shared__ double s_cut[MDX_NT1 * MDX_NT1];
@@ -374,10 +416,12 @@ __global__ __launch_bounds__(256, Q ? MDX_BUILD_Q_WAVES : MDX_BUILD_MIN_WAVES) v
   const int ti = static_cast<int>(xi.w);
   int4 qi = make_int4(0, 0, 0, 0);
   if constexpr (Q) qi = xq[i];
-  const unsigned b = bkey[i];
   const int nbx = a.nbin[0], nby = a.nbin[1], nbz = a.nbin[2];
-  int ix, iy, iz;
-  bin_coords(a, (int)b, ix, iy, iz);
+  // the bin as k_wrap_bin formed it, and the place in bins
+  const double bx = (xi.x - a.lo[0]) * a.bininv[0], by = (xi.y - a.lo[1]) * a.bininv[1],
+               bz = (xi.z - a.lo[2]) * a.bininv[2];
+  const int ix = min(max(static_cast<int>(bx), 0), nbx - 1), iy = min(max(static_cast<int>(by), 0), nby - 1),
+            iz = min(max(static_cast<int>(bz), 0), nbz - 1);
   // this atom's column of the chunk-major list: chunk c at col[c * npad]
   int4 *col = reinterpret_cast<int4 *>(nbr) + i;
   int cnt = 0;
@@ -385,9 +429,7 @@ __global__ __launch_bounds__(256, Q ? MDX_BUILD_Q_WAVES : MDX_BUILD_MIN_WAVES) v
   const int t11 = a.ntypes1 + 1;       // (1, 1) in the type tables
   const float c_lo = (ONE && Q) ? s_lo[Q ? t11 : 0] : 0.0f, c_hi = (ONE && Q) ? s_hi[Q ? t11 : 0] : 0.0f;
   const double c_cut = ONE ? s_cut[t11] : 0.0;
-  const float tx = static_cast<float>((xi.x - a.lo[0]) * a.bininv[0]),
-              ty = static_cast<float>((xi.y - a.lo[1]) * a.bininv[1]),
-              tz = static_cast<float>((xi.z - a.lo[2]) * a.bininv[2]);
+  const float tx = static_cast<float>(bx), ty = static_cast<float>(by), tz = static_cast<float>(bz);
   const float bsy = static_cast<float>(1.0 / a.bininv[1]), bsz = static_cast<float>(1.0 / a.bininv[2]);
   const float reach = static_cast<float>(s_cmax[ti] * (1.0 + 1e-4));
   // FP32 bin coordinates stay within the margins up to 8192 bins a side
@@ -564,7 +606,6 @@ struct FlatConst {
 template <bool Q, bool ONE>
 __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(NeighArgs a, const double4 *__restrict__ x,
                                                    const int4 *__restrict__ xq, QStep qs,
-                                                   const unsigned *__restrict__ bkey,
                                                    const int *__restrict__ bin_start, int *__restrict__ nbr,
                                                    int *__restrict__ numneigh, ListSlot *__restrict__ slots, FlatConst fc,
                                                    const NeighArgs *__restrict__ ax) {
@@ -582,19 +623,19 @@ __global__ __launch_bounds__(kFlatBlock, MDX_FLAT_WAVES) void k_build_flat(Neigh
   const int ti = static_cast<int>(xi.w);
   int4 qi = make_int4(0, 0, 0, 0);
   if constexpr (Q) qi = xq[i];
-  const unsigned b = bkey[i];
   const int nbx = a.nbin[0], nby = a.nbin[1], nbz = a.nbin[2];
-  int ix, iy, iz;
-  bin_coords(a, (int)b, ix, iy, iz);
+  // the bin as k_wrap_bin formed it, and the place in bins
+  const double bx = (xi.x - a.lo[0]) * a.bininv[0], by = (xi.y - a.lo[1]) * a.bininv[1],
+               bz = (xi.z - a.lo[2]) * a.bininv[2];
+  const int ix = min(max(static_cast<int>(bx), 0), nbx - 1), iy = min(max(static_cast<int>(by), 0), nby - 1),
+            iz = min(max(static_cast<int>(bz), 0), nbz - 1);
   int4 *col = reinterpret_cast<int4 *>(nbr) + i;
   int cnt = 0;
   int q0 = 0, q1 = 0, q2 = 0, q3 = 0;
   const int t11 = a.ntypes1 + 1;
   const float c_lo = fc.c_lo, c_hi = fc.c_hi;
   const double c_cut = fc.c_cut;
-  const float tx = static_cast<float>((xi.x - a.lo[0]) * a.bininv[0]),
-              ty = static_cast<float>((xi.y - a.lo[1]) * a.bininv[1]),
-              tz = static_cast<float>((xi.z - a.lo[2]) * a.bininv[2]);
+  const float tx = static_cast<float>(bx), ty = static_cast<float>(by), tz = static_cast<float>(bz);
   const float bsy = fc.bsy, bsz = fc.bsz;
   const float reach = ONE ? fc.reach : static_cast<float>(s_cmax[ti] * (1.0 + 1e-4));
   const int prune = fc.prune;
@@ -1016,7 +1057,7 @@ void launch_build(mdx_ctx *c) {
   ListSlot *slots = reinterpret_cast<ListSlot *>(c->dflags + kFlagInts);
   const bool q = q_build_ok(c), one = c->ntypes == 1;
   auto go = [&](auto kernel, const int4 *xq) {
-    hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bkey_s, c->bin_start, c->nbr,
+    hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bin_start, c->nbr,
                        c->numneigh, slots);
   };
   // the group and flat builds take stencils of at most 5x5 rows with at most two
@@ -1042,7 +1083,7 @@ void launch_build(mdx_ctx *c) {
       fc.reach = static_cast<float>(m * (1.0 + 1e-4));
     }
     auto goflat = [&](auto kernel, const int4 *xq) {
-      hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bkey_s, c->bin_start,
+      hipLaunchKernelGGL(kernel, dim3(G), dim3(B), 0, c->stream, c->na, c->x, xq, qs, c->bin_start,
                          c->nbr, c->numneigh, slots, fc, c->na_dev);
     };
     if (c->n <= kGroupMaxAtoms) {
@@ -1223,30 +1264,32 @@ int neigh_build_launch(mdx_ctx *c) {
   c->bins_dirty = true;  // until the scatter pass clears them
   // stable sort of (bin, current index): bin_start from the counts, then
   // scatter by arrival slot and rank within each bin (deterministic order)
-  size_t need = 0;
-  (void)hipcub::DeviceScan::ExclusiveSum(nullptr, need, c->bin_count, c->bin_start, c->nbins + 1, c->stream);
-  if (need > c->scan_tmp_bytes) {
-    if (c->fixed_storage) {
-      set_error("bin scan storage exceeds the fixed storage");
-      return MDX_ERR_ARG;
+  if (c->nbins + 1 <= kScanBins) {
+    hipLaunchKernelGGL(k_scan_bins, dim3(1), dim3(kScanThreads), 0, c->stream, c->nbins + 1, c->bin_count, c->bin_start);
+  } else {
+    size_t need = 0;
+    (void)hipcub::DeviceScan::ExclusiveSum(nullptr, need, c->bin_count, c->bin_start, c->nbins + 1, c->stream);
+    if (need > c->scan_tmp_bytes) {
+      if (c->fixed_storage) {
+        set_error("bin scan storage exceeds the fixed storage");
+        return MDX_ERR_ARG;
+      }
+      (void)hipFree(c->scan_tmp);
+      c->scan_tmp_bytes = need;
+      if (hipMalloc(&c->scan_tmp, need) != hipSuccess) {
+        set_error("Insufficient memory on accelerator (scan)");
+        return MDX_ERR_NOMEM;
+      }
     }
-    (void)hipFree(c->scan_tmp);
-    c->scan_tmp_bytes = need;
-    if (hipMalloc(&c->scan_tmp, need) != hipSuccess) {
-      set_error("Insufficient memory on accelerator (scan)");
-      return MDX_ERR_NOMEM;
-    }
+    e = hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, need, c->bin_count, c->bin_start, c->nbins + 1, c->stream);
+    if (e != hipSuccess) return hip_fail(e, "bin scan");
   }
-  e = hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, need, c->bin_count, c->bin_start, c->nbins + 1, c->stream);
-  if (e != hipSuccess) return hip_fail(e, "bin scan");
   hipLaunchKernelGGL(k_bin_scatter, dim3(G), dim3(B), 0, c->stream, c->n, c->bkey, c->bidx, c->bin_start, c->bidx_s,
                      c->bin_count, c->nbins + 1, next_flags);
   c->bins_dirty = false;
-  hipLaunchKernelGGL(k_bin_rank, dim3(G), dim3(B), 0, c->stream, c->n, c->bkey, c->bin_start, c->bidx_s, c->bidx,
-                     c->bkey_s, c->one + 1, c->dflags);
-  hipLaunchKernelGGL(k_permute, dim3(G), dim3(B), 0, c->stream, c->n, c->bidx, c->x, c->v, c->tag, c->orig,
-                     c->image, c->xb, c->vb, c->tagb, c->origb, c->imageb, c->inv, c->xhold,
-                     (c->qpos || c->qbuild) ? c->xq : nullptr, c->qs);
+  hipLaunchKernelGGL(k_rank_permute, dim3(G), dim3(B), 0, c->stream, c->n, c->bkey, c->bin_start, c->bidx_s,
+                     c->one + 1, c->dflags, c->x, c->v, c->tag, c->orig, c->image, c->xb, c->vb, c->tagb, c->origb,
+                     c->imageb, c->inv, c->xhold, (c->qpos || c->qbuild) ? c->xq : nullptr, c->qs);
   if (c->qpos) c->xq_stale = false;
   std::swap(c->x, c->xb);
   std::swap(c->v, c->vb);
@@ -1295,7 +1338,7 @@ int neigh_build_finish(mdx_ctx *c, bool *regrow) {
     return MDX_ERR_ARG;
   }
   const int mx = flags[0];
-  if (mx > c->one || flags[5]) {  // flags[5]: a bin holds more than one + 1 atoms (k_bin_rank)
+  if (mx > c->one || flags[5]) {  // flags[5]: a bin holds more than one + 1 atoms (k_rank_permute)
     set_error("Neighbor list overflow, boost neigh_modify one");
     return MDX_ERR_OVERFLOW;
   }

@@ -39,7 +39,7 @@ constexpr size_t kPartials = partials_for(MDX_NOALLOC_MAX_ATOMS);
 constexpr size_t kScanBytes = size_t(1) << 20;  // hipcub scan temporary storage over kBins counters
 
 constexpr size_t kPerAtomBytes = align_up(sizeof(double4) * kAtoms) * 6 +  // x, xb, v, vb, f, xhold
-                                 align_up(sizeof(int) * kAtoms) * 12 +      // tag/b, orig/b, image/b, inv, bkey/_s,
+                                 align_up(sizeof(int) * kAtoms) * 11 +      // tag/b, orig/b, image/b, inv, bkey,
                                                                             // bidx/_s, numneigh
                                  align_up(sizeof(double) * 6 * kAtoms) +    // vatom
                                  align_up(sizeof(double) * kAtoms) * 3 +    // rho, fp, eemb
@@ -212,7 +212,6 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
   s.imageb = cv.take<int>(kAtoms);
   s.inv = cv.take<int>(kAtoms);
   s.bkey = cv.take<unsigned>(kAtoms);
-  s.bkey_s = cv.take<unsigned>(kAtoms);
   s.bidx = cv.take<int>(kAtoms);
   s.bidx_s = cv.take<int>(kAtoms);
   s.numneigh = cv.take<int>(kAtoms);
