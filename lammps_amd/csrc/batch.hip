@@ -31,6 +31,7 @@
 // over the knot spacing) in LDS with ds_add_f64, flushed per block and
 // summed over blocks in a fixed order; the host maps coefficient gradients
 // to knot gradients with the transpose of the spline construction.
+#include <hip/hip_ext.h>
 #include <hipcub/hipcub.hpp>
 
 #include <cmath>
@@ -358,6 +359,22 @@ __global__ __launch_bounds__(kBuildBlock, 5) void k_b_build(int n, const double4
   }
 }
 
+// Results of a force pass: the atom's energy in sorted order (for the replica
+// sums), its force straight into the caller's order (f null: not wanted)
+struct ForceOut {
+  double *e;
+  double *f;
+  const int *orig;
+  __device__ __forceinline__ void store(int i, double fx, double fy, double fz, double energy) const {
+    e[i] = energy;
+    if (!f) return;
+    double *const d = f + 3 * (size_t)orig[i];
+    d[0] = fx;
+    d[1] = fy;
+    d[2] = fz;
+  }
+};
+
 // ---------------------------------------------------------------- pair helpers
 
 // One lane's four consecutive entries k0 .. k0+3 of a row (rows start 16-B
@@ -386,7 +403,7 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
                                                const int4 *__restrict__ xq, const int *__restrict__ rep,
                                                const RepGeom *__restrict__ geom, const int *__restrict__ nbr,
                                                const int *__restrict__ numneigh, int cap,
-                                               const double *__restrict__ tab, double4 *__restrict__ f) {
+                                               const double *__restrict__ tab, ForceOut out) {
   __shared__ double s_tab[T_N * kNT];
   __shared__ double s_qlo[MIXED ? kNT : 1], s_qhi[MIXED ? kNT : 1];
   __shared__ float s_f[MIXED ? 4 * kNT : 1];
@@ -490,7 +507,7 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
     fy = gsum<TPA>(fy);
     fz = gsum<TPA>(fz);
     e = gsum<TPA>(e);
-    if (lane == 0) f[i] = make_double4(fx, fy, fz, e);
+    if (lane == 0) out.store(i, fx, fy, fz, e);
   }
 }
 
@@ -775,7 +792,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
                                                       const RepGeom *__restrict__ geom, const int *__restrict__ nbr,
                                                       const int *__restrict__ numneigh, int cap, EamTab et,
                                                       EamKnots knots, const double *__restrict__ fp,
-                                                      const double *__restrict__ eemb, double4 *__restrict__ f) {
+                                                      const double *__restrict__ eemb, ForceOut out) {
   extern __shared__ double4 s_knots[];
   using T = typename Real<MIXED>::T;
   using V = typename Real<MIXED>::V;
@@ -857,7 +874,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
     fy = gsum<TPA>(fy);
     fz = gsum<TPA>(fz);
     e = gsum<TPA>(e);
-    if (lane == 0) f[i] = make_double4(fx, fy, fz, e + eemb[i]);
+    if (lane == 0) out.store(i, fx, fy, fz, e + eemb[i]);
   }
 }
 
@@ -1094,11 +1111,11 @@ __global__ __launch_bounds__(256) void k_b_colsum(const double *__restrict__ mid
 }
 
 // per-replica energy: one block per replica, fixed-order tree
-__global__ void k_b_rep_energy(const double4 *__restrict__ f, const int *__restrict__ off, double *__restrict__ out) {
+__global__ void k_b_rep_energy(const double *__restrict__ e, const int *__restrict__ off, double *__restrict__ out) {
   __shared__ double s[256];
   const int r = blockIdx.x;
   double acc = 0.0;
-  for (int i = off[r] + threadIdx.x; i < off[r + 1]; i += 256) acc += f[i].w;
+  for (int i = off[r] + threadIdx.x; i < off[r + 1]; i += 256) acc += e[i];
   s[threadIdx.x] = acc;
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
@@ -1106,16 +1123,6 @@ __global__ void k_b_rep_energy(const double4 *__restrict__ f, const int *__restr
     __syncthreads();
   }
   if (threadIdx.x == 0) out[r] = s[0];
-}
-
-__global__ void k_b_gather_f(int n, const int *__restrict__ inv, const double4 *__restrict__ f,
-                             double *__restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-  const double4 v = f[inv[c]];
-  out[3 * (size_t)c] = v.x;
-  out[3 * (size_t)c + 1] = v.y;
-  out[3 * (size_t)c + 2] = v.z;
 }
 
 __global__ void k_b_gather_s(int n, const int *__restrict__ inv, const double *__restrict__ a, double *__restrict__ out) {
@@ -1151,7 +1158,9 @@ struct mdx_batch {
   // atoms
   double *xin = nullptr;  // caller order staging [N][3]
   int *type_c = nullptr, *rep_c = nullptr;
-  double4 *xw = nullptr, *x = nullptr, *f = nullptr, *g = nullptr;
+  double4 *xw = nullptr, *x = nullptr, *g = nullptr;
+  double *eat = nullptr;       // per-atom energies of the last force pass
+  double *rep_host = nullptr;  // mapped: replica energies
   int4 *xq = nullptr;  // fixed-point copy of x (mixed-precision force passes)
   int *rep = nullptr, *orig = nullptr, *inv = nullptr;
   unsigned *key = nullptr;
@@ -1163,6 +1172,7 @@ struct mdx_batch {
   int cap = 0;
   int *dflags = nullptr;       // kFlagWords: [0] max count, [4] outside box, [8..9] u64 total
   int *flags_host = nullptr;   // mapped copy of the first kFlagInts
+  int flag_serial = 0;         // list passes whose flags were asked for (kFlagSerial)
   bool mirror_ok = false;      // the fixed-point mirror can decide the list's candidates
   long total_neighbors = 0;
   int max_neighbors = 0;
@@ -1194,7 +1204,15 @@ struct mdx_batch {
   double kms[MDX_BK_NKIND] = {0};
   long klaunch[MDX_BK_NKIND] = {0};
   int num_cu = 256;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // start and stop events of the launches not yet added to kms (read when the
+  // times are asked for, or when the ring is full)
+  struct Launched {
+    hipEvent_t a, b;
+    int kind;
+  };
+  std::vector<Launched> ring;
+  size_t pending = 0;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;  // of the launch being queued
   int lds_max = 65536;
 };
 
@@ -1253,24 +1271,64 @@ Tune default_tune(const mdx_batch *b, int kind) {
 
 Tune tune_of(const mdx_batch *b, int kind) { return b->tune[kind].tpa ? b->tune[kind] : default_tune(b, kind); }
 
-// run one launch of kind `kind` under timing; `launch(tune)` enqueues it
-template <typename F>
-int timed(mdx_batch *b, int kind, const Tune &t, F &&launch, float *ms_out = nullptr, bool count = true) {
-  (void)hipEventRecord(b->ev0, b->stream);
-  launch(t);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return bfail(e, "batch kernel launch");
-  (void)hipEventRecord(b->ev1, b->stream);
-  e = hipEventSynchronize(b->ev1);
+// adds the times of the launches since the last call to kms; waits for them
+int resolve_times(mdx_batch *b) {
+  if (b->pending == 0) return MDX_OK;
+  hipError_t e = hipEventSynchronize(b->ring[b->pending - 1].b);
   if (e != hipSuccess) return bfail(e, "batch kernel");
-  float ms = 0.0f;
-  (void)hipEventElapsedTime(&ms, b->ev0, b->ev1);
-  if (ms_out) *ms_out = ms;
-  if (count) {
-    b->kms[kind] += ms;
-    b->klaunch[kind]++;
+  for (size_t k = 0; k < b->pending; k++) {
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, b->ring[k].a, b->ring[k].b);
+    b->kms[b->ring[k].kind] += ms;
   }
+  b->pending = 0;
   return MDX_OK;
+}
+
+// A launch whose own start and stop times go to the events b->ev0 and ev1:
+// they come with the dispatch, so nothing is queued around it and the host
+// does not wait for it (two recorded events and a wait per kernel cost a
+// 64 x 8,000 atom loss and gradient about 100 us).
+#define BATCH_LAUNCH(KERNEL, G, B, LDS, ...) \
+  hipExtLaunchKernelGGL(KERNEL, dim3(G), dim3(B), LDS, b->stream, b->ev0, b->ev1, 0, __VA_ARGS__)
+
+// run one launch of kind `kind` under timing; `launch(tune)` enqueues it.
+// With ms_out it is waited for and timed on its own, else it is queued.
+constexpr size_t kRing = 64;
+template <typename F>
+int timed(mdx_batch *b, int kind, const Tune &t, F &&launch, float *ms_out = nullptr) {
+  int rc;
+  hipError_t e;
+  if (b->pending == kRing && (rc = resolve_times(b))) return rc;
+  if (b->ring.size() == b->pending) {
+    mdx_batch::Launched l{};
+    if ((e = hipEventCreate(&l.a)) != hipSuccess) return bfail(e, "batch events");
+    if ((e = hipEventCreate(&l.b)) != hipSuccess) {
+      (void)hipEventDestroy(l.a);
+      return bfail(e, "batch events");
+    }
+    b->ring.push_back(l);
+  }
+  mdx_batch::Launched &l = b->ring[b->pending];
+  l.kind = kind;
+  b->ev0 = l.a;
+  b->ev1 = l.b;
+  launch(t);
+  if ((e = hipGetLastError()) != hipSuccess) return bfail(e, "batch kernel launch");
+  if (ms_out) {
+    if ((e = hipEventSynchronize(l.b)) != hipSuccess) return bfail(e, "batch kernel");
+    (void)hipEventElapsedTime(ms_out, l.a, l.b);
+    return MDX_OK;
+  }
+  b->pending++;
+  b->klaunch[kind]++;
+  return MDX_OK;
+}
+
+int finish(mdx_batch *b, const char *what) {
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+  return e == hipSuccess ? MDX_OK : bfail(e, what);
 }
 
 // kernels that flush per-block partial rows cap the grid at kPartialBlocksPerCU per CU
@@ -1311,7 +1369,7 @@ int run_kind(mdx_batch *b, int kind, F &&launch) {
     for (const Tune &t : candidates(b)) {
       float ms = 0.0f;
       for (int rep = 0; rep < 2; rep++) {  // second timing counts (warm caches)
-        int rc = timed(b, kind, t, launch, &ms, false);
+        int rc = timed(b, kind, t, launch, &ms);
         if (rc) return rc;
       }
       if (ms < best) {
@@ -1465,16 +1523,17 @@ int build(mdx_batch *b) {
       constexpr int per = kBuildBlock / kBuildLanes;
       const int G = std::min(xcd_grid((n + per - 1) / per), kBuildGrid);
       auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(G), dim3(kBuildBlock), 0, b->stream, n, b->x, b->xq, b->rep, b->geom,
-                           b->bin_start, cutneighsq, c_lo, c_hi, reach, b->cap, b->nbr, b->numneigh,
-                           reinterpret_cast<ListSlot *>(b->dflags + kFlagInts));
+        BATCH_LAUNCH(kernel, G, kBuildBlock, 0, n, b->x, b->xq, b->rep, b->geom, b->bin_start, cutneighsq, c_lo, c_hi,
+                     reach, b->cap, b->nbr, b->numneigh, reinterpret_cast<ListSlot *>(b->dflags + kFlagInts));
       };
       if (b->mirror_ok) go(k_b_build<true>);
       else go(k_b_build<false>);
-      launch_build_flags(b->stream, b->dflags, b->flags_host, 1);  // the event below is waited for
     };
-    if ((rc = timed(b, MDX_BK_BUILD, b->tune[MDX_BK_BUILD], launch))) return rc;
-    int fl[kFlagInts];
+    if ((rc = timed(b, MDX_BK_BUILD, Tune{}, launch))) return rc;
+    b->flag_serial = b->flag_serial == 0x7fffffff ? 1 : b->flag_serial + 1;
+    launch_build_flags(b->stream, b->dflags, b->flags_host, b->flag_serial);
+    int fl[kFlagInts], got;
+    if ((rc = wait_word(b->stream, b->flags_host + kFlagSerial, b->flag_serial, b->flag_serial, &got))) return rc;
     std::memcpy(fl, b->flags_host, sizeof(fl));
     if (fl[4]) {
       set_error("an atom lies outside its replica's box in a non-periodic dimension");
@@ -1502,16 +1561,23 @@ int ensure_built(mdx_batch *b) {
   return build(b);
 }
 
-// copy [N][3] output from the sorted double4 array to a host or device pointer
-int write_vec3(mdx_batch *b, const double4 *src, double *out) {
-  const int n = b->n;
-  const bool dev = is_device_ptr(out, b->device);
-  double *dst = dev ? out : b->staging;
-  hipLaunchKernelGGL(k_b_gather_f, dim3((n + 255) / 256), dim3(256), 0, b->stream, n, b->inv, src, dst);
-  hipError_t e = hipSuccess;
-  if (!dev) e = hipMemcpyAsync(out, b->staging, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, b->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-  return e == hipSuccess ? MDX_OK : bfail(e, "force output");
+// where a force pass writes: the caller's device array, or staging for a host one
+ForceOut force_out(mdx_batch *b, double *f) {
+  return {b->eat, !f ? nullptr : is_device_ptr(f, b->device) ? f : b->staging, b->orig};
+}
+
+// what follows a force pass: replica energies, the copy to a host force array,
+// and the one wait of the call
+int force_results(mdx_batch *b, const ForceOut &out, double *f, double *energy) {
+  if (energy)
+    hipLaunchKernelGGL(k_b_rep_energy, dim3(b->nrep), dim3(256), 0, b->stream, b->eat, b->off_d, b->rep_host);
+  if (f && out.f != f) {
+    hipError_t e = hipMemcpyAsync(f, out.f, sizeof(double) * 3 * b->n, hipMemcpyDeviceToHost, b->stream);
+    if (e != hipSuccess) return bfail(e, "force output");
+  }
+  int rc = finish(b, "batch forces");
+  if (!rc && energy) std::memcpy(energy, b->rep_host, sizeof(double) * b->nrep);
+  return rc;
 }
 
 int read_g(mdx_batch *b, const double *gf) {
@@ -1665,13 +1731,15 @@ int mdx_batch_create(int device, int nrep, const int *natoms, const double *lo, 
   hipError_t e;
   int rc;
   if ((e = hipSetDevice(device)) != hipSuccess || (e = hipStreamCreate(&b->own_stream)) != hipSuccess ||
-      (e = hipEventCreate(&b->ev0)) != hipSuccess || (e = hipEventCreate(&b->ev1)) != hipSuccess ||
       (e = hipHostMalloc(&b->flags_host, sizeof(int) * kFlagInts, hipHostMallocCoherent | hipHostMallocMapped)) !=
+          hipSuccess ||
+      (e = hipHostMalloc(&b->rep_host, sizeof(double) * nrep, hipHostMallocCoherent | hipHostMallocMapped)) !=
           hipSuccess) {
     rc = bfail(e, "batch stream");
     mdx_batch_destroy(b);
     return rc;
   }
+  std::memset(b->flags_host, 0, sizeof(int) * kFlagInts);  // no serial yet
   b->stream = b->own_stream;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
@@ -1684,7 +1752,7 @@ int mdx_batch_create(int device, int nrep, const int *natoms, const double *lo, 
     for (int i = b->off[r]; i < b->off[r + 1]; i++) rep_c[i] = r;
   if ((rc = dalloc(&b->geom, nrep)) || (rc = dalloc(&b->off_d, nrep + 1)) || (rc = dalloc(&b->xin, 3 * (size_t)n)) ||
       (rc = dalloc(&b->staging, std::max<size_t>(3 * (size_t)n, nrep))) || (rc = dalloc(&b->type_c, n)) || (rc = dalloc(&b->rep_c, n)) ||
-      (rc = dalloc(&b->xw, n)) || (rc = dalloc(&b->x, n)) || (rc = dalloc(&b->xq, n)) || (rc = dalloc(&b->f, n)) ||
+      (rc = dalloc(&b->xw, n)) || (rc = dalloc(&b->x, n)) || (rc = dalloc(&b->xq, n)) || (rc = dalloc(&b->eat, n)) ||
       (rc = dalloc(&b->g, n)) ||
       (rc = dalloc(&b->rep, n)) || (rc = dalloc(&b->orig, n)) || (rc = dalloc(&b->inv, n)) ||
       (rc = dalloc(&b->key, n)) || (rc = dalloc(&b->slot, n)) || (rc = dalloc(&b->order, n)) ||
@@ -1705,16 +1773,19 @@ int mdx_batch_destroy(mdx_batch *b) {
   (void)hipSetDevice(b->device);
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   void *ptrs[] = {b->xq, b->geom,    b->off_d,    b->xin,      b->staging,  b->type_c,  b->rep_c,   b->xw,      b->x,
-                  b->f,       b->g,        b->rep,      b->orig,     b->inv,     b->key,     b->slot,    b->order,
+                  b->eat,     b->g,        b->rep,      b->orig,     b->inv,     b->key,     b->slot,    b->order,
                   b->bin_count, b->bin_start, b->scan_tmp, b->nbr,    b->numneigh, b->dflags,
                   b->rho,     b->fp,       b->eemb,     b->vadj,     b->partials, b->colsum,  b->ljtab,   b->frho_d,
                   b->knots_d, b->knots_f};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->flags_host) (void)hipHostFree(b->flags_host);
+  if (b->rep_host) (void)hipHostFree(b->rep_host);
   if (b->sums_host) (void)hipHostFree(b->sums_host);
-  if (b->ev0) (void)hipEventDestroy(b->ev0);
-  if (b->ev1) (void)hipEventDestroy(b->ev1);
+  for (auto &l : b->ring) {
+    (void)hipEventDestroy(l.a);
+    (void)hipEventDestroy(l.b);
+  }
   if (b->own_stream) {
     (void)hipStreamSynchronize(b->own_stream);
     (void)hipStreamDestroy(b->own_stream);
@@ -1825,27 +1896,18 @@ int mdx_batch_lj_forces(mdx_batch *b, double *f, double *energy) {
   if ((rc = ensure_built(b))) return rc;
   const int nt1 = b->ntypes + 1;
   const bool mixed = b->precision == MDX_MIXED;
+  const ForceOut out = force_out(b, f);
   auto launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t);
     if (mixed)
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_lj<true, TP>), dim3(G), dim3(t.block), 0, b->stream, b->n, nt1,
-                                             b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->ljtab,
-                                             b->f))
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_lj<true, TP>), G, t.block, 0, b->n, nt1, b->x, b->xq, b->rep, b->geom, b->nbr,
+                                       b->numneigh, b->cap, b->ljtab, out))
     else
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_lj<false, TP>), dim3(G), dim3(t.block), 0, b->stream, b->n, nt1,
-                                             b->x, b->xq, b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->ljtab,
-                                             b->f))
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_lj<false, TP>), G, t.block, 0, b->n, nt1, b->x, b->xq, b->rep, b->geom, b->nbr,
+                                       b->numneigh, b->cap, b->ljtab, out))
   };
   if ((rc = run_kind(b, MDX_BK_LJ, launch))) return rc;
-  if (energy) {
-    double *ed = b->staging;
-    hipLaunchKernelGGL(k_b_rep_energy, dim3(b->nrep), dim3(256), 0, b->stream, b->f, b->off_d, ed);
-    hipError_t e = hipMemcpyAsync(energy, ed, sizeof(double) * b->nrep, hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    if (e != hipSuccess) return bfail(e, "energy output");
-  }
-  if (f && (rc = write_vec3(b, b->f, f))) return rc;
-  return MDX_OK;
+  return force_results(b, out, f, energy);
 }
 
 int mdx_batch_lj_vjp(mdx_batch *b, const double *gf, double *geps, double *gsigma) {
@@ -1869,8 +1931,7 @@ int mdx_batch_lj_vjp(mdx_batch *b, const double *gf, double *geps, double *gsigm
     const int G = persistent_grid(b, t, true);
     grid_used = G;
     auto go = [&](auto nt) {
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_lj_vjp<decltype(nt)::value, TP>), dim3(G), dim3(t.block), 0,
-                                             b->stream, b->n, nt1, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_lj_vjp<decltype(nt)::value, TP>), G, t.block, 0, b->n, nt1, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
                                              b->ljtab, b->g, b->partials))
     };
     if (b->ntypes == 1) go(std::integral_constant<int, 1>{});
@@ -1947,7 +2008,7 @@ int mdx_batch_eam_init(mdx_batch *b, int nrho, double drho, int nr, double dr, d
 
 namespace {
 // rho + fp pass in `precision`, then (with_force) the force pass
-int eam_forward(mdx_batch *b, bool with_force, int precision) {
+int eam_forward(mdx_batch *b, bool with_force, int precision, double *f = nullptr) {
   int rc;
   if ((rc = ensure_built(b))) return rc;
   const bool mixed = precision == MDX_MIXED;
@@ -1963,8 +2024,8 @@ int eam_forward(mdx_batch *b, bool with_force, int precision) {
   auto rho_launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t);
     choose(lds1, [&](auto mx, auto tl) {
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_rho<decltype(mx)::value, TP, decltype(tl)::value>), dim3(G),
-                                             dim3(t.block), lds1 ? vec : 0, b->stream, b->n, b->x, b->xq, b->rep,
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_rho<decltype(mx)::value, TP, decltype(tl)::value>), G, t.block,
+                                       lds1 ? vec : 0, b->n, b->x, b->xq, b->rep,
                                              b->geom, b->nbr, b->numneigh, b->cap, b->et, b->knots, b->frho_d, b->rho,
                                              b->fp, b->eemb))
     });
@@ -1972,13 +2033,14 @@ int eam_forward(mdx_batch *b, bool with_force, int precision) {
   if ((rc = run_kind(b, MDX_BK_EAM_RHO, rho_launch))) return rc;
   b->eam_rho_prec = precision;
   if (!with_force) return MDX_OK;
+  const ForceOut out = force_out(b, f);
   auto force_launch = [&](const Tune &t) {
     const int G = persistent_grid(b, t);
     choose(lds2, [&](auto mx, auto tl) {
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_force<decltype(mx)::value, TP, decltype(tl)::value>), dim3(G),
-                                             dim3(t.block), lds2 ? 3 * vec : 0, b->stream, b->n, b->x, b->xq, b->rep,
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_force<decltype(mx)::value, TP, decltype(tl)::value>), G, t.block,
+                                       lds2 ? 3 * vec : 0, b->n, b->x, b->xq, b->rep,
                                              b->geom, b->nbr, b->numneigh, b->cap, b->et, b->knots, b->fp, b->eemb,
-                                             b->f))
+                                             out))
     });
   };
   return run_kind(b, MDX_BK_EAM_FORCE, force_launch);
@@ -1992,24 +2054,17 @@ int mdx_batch_eam_forces(mdx_batch *b, double *f, double *energy, double *rho, d
     set_error("eam not initialised (mdx_batch_eam_init)");
     return MDX_ERR_ARG;
   }
-  if ((rc = eam_forward(b, true, b->precision))) return rc;
-  hipError_t e = hipSuccess;
-  if (energy) {
-    hipLaunchKernelGGL(k_b_rep_energy, dim3(b->nrep), dim3(256), 0, b->stream, b->f, b->off_d, b->staging);
-    e = hipMemcpyAsync(energy, b->staging, sizeof(double) * b->nrep, hipMemcpyDeviceToHost, b->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    if (e != hipSuccess) return bfail(e, "energy output");
-  }
+  if ((rc = eam_forward(b, true, b->precision, f))) return rc;
+  if ((rc = force_results(b, force_out(b, f), f, energy))) return rc;
   for (int k = 0; k < 2; k++) {
     double *out = k == 0 ? rho : fp;
     if (!out) continue;
     hipLaunchKernelGGL(k_b_gather_s, dim3((b->n + 255) / 256), dim3(256), 0, b->stream, b->n, b->inv,
                        k == 0 ? b->rho : b->fp, b->staging);
-    e = hipMemcpyAsync(out, b->staging, sizeof(double) * b->n, hipMemcpyDeviceToHost, b->stream);
+    hipError_t e = hipMemcpyAsync(out, b->staging, sizeof(double) * b->n, hipMemcpyDeviceToHost, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) return bfail(e, "rho/fp output");
   }
-  if (f && (rc = write_vec3(b, b->f, f))) return rc;
   return MDX_OK;
 }
 
@@ -2052,8 +2107,7 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
     const int G = persistent_grid(b, t, true);
     gA = G;
     auto go = [&](auto tl) {
-      TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_a<TP, decltype(tl)::value>), dim3(G), dim3(t.block), shA,
-                                             b->stream, b->n, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
+      TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_adj_a<TP, decltype(tl)::value>), G, t.block, shA, b->n, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
                                              b->et, b->knots.rhor_d, b->frho_d, b->rho, b->fp, b->g, cA, b->vadj,
                                              b->partials))
     };
@@ -2065,7 +2119,7 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
   auto launchB = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);
     gB = G;
-    TPA_DISPATCH(t.tpa, hipLaunchKernelGGL((k_b_eam_adj_b<TP>), dim3(G), dim3(t.block), shB, b->stream, b->n, b->x,
+    TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_adj_b<TP>), G, t.block, shB, b->n, b->x,
                                            b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->vadj, cB, partB))
   };
   if ((rc = run_kind(b, MDX_BK_EAM_ADJ_B, launchB))) return rc;
@@ -2121,6 +2175,7 @@ int mdx_batch_kernel_time(mdx_batch *b, int kind, double *ms, long *launches) {
     set_error("invalid kernel kind");
     return MDX_ERR_ARG;
   }
+  if ((rc = resolve_times(b))) return rc;
   if (ms) *ms = b->kms[kind];
   if (launches) *launches = b->klaunch[kind];
   return MDX_OK;
