@@ -60,7 +60,6 @@ constexpr int kUnrollQ = MDX_GATHER_UNROLL_Q;
 // Chunks take 4x fewer index-load requests; measured on MI355X they speed
 // up lj/cut (threads per atom 4) by 3-7% and slow the eam kernels (8) by
 // 10-15%, so k_lj is chunked and the eam kernels are strided.
-constexpr bool kChunkLJ = true, kChunkEAM = false;
 
 #ifndef MDX_TRANS_LJ
 #define MDX_TRANS_LJ 1
@@ -113,11 +112,42 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], double *__re
   }
 }
 
+// Which atom and which of its TPA lanes a thread is.  By default a group's
+// lanes are neighbours in the wavefront.  ACROSS puts neighbouring atoms in
+// neighbouring lanes instead (lane l of a wavefront: atom l mod 64/TPA, share
+// l / (64/TPA)): the chunked lj/cut kernel then reads one chunk of 64/TPA
+// consecutive atoms as contiguous 16-B pieces, not TPA chunks npad * 16 B
+// apart, and the gathers of neighbouring atoms share more cache lines.  The
+// kernel waits for L1: 1.09 line lookups per CU and cycle at 2.048 M atoms
+// (47 per load instruction), its vector units 57% busy.  Per step kernel,
+// grouped / across: mixed, 4 lanes 2.048 M atoms 287 / 272 us, 256,000 35.1 /
+// 32.3; FP64, 8 lanes 32,000 11.0 / 10.2; 16 lanes 8,000 Kob-Andersen 6.37 /
+// 6.15.  Four lanes in FP64 keep the group (its transposed chunks are faster:
+// 381 against 400 us at 2.048 M).  So do the eam kernels: they read entries,
+// not chunks, so the lanes of a group already gather consecutive entries
+// (17-21 lookups per instruction; across, 256,000 atoms FP64 145 against 109).
+constexpr bool lj_across(bool mixed, int tpa) { return tpa >= (mixed ? 4 : 8); }
+// The lj/cut kernel loads a lane's next chunk before it waits for the gathers
+// of the current one where a lane has few trips and the kernel is a chain of
+// latencies (4,000 atoms, 16 lanes: 4.89 against 5.16 us; 32,000 mixed, 8
+// lanes: 7.74 against 7.88).  At 4 lanes the registers cost more (2.048 M
+// mixed: 306 against 272).
+constexpr bool lj_ahead(int tpa) { return tpa >= 8; }
+
+template <int TPA, bool ACROSS>
+__device__ __forceinline__ void group_place(int &i, int &lane) {
+  const unsigned t = xcd_block() * blockDim.x + threadIdx.x;  // workgroups are whole wavefronts
+  constexpr unsigned A = 64 / TPA;
+  i = ACROSS ? (t >> 6) * A + t % A : t / TPA;
+  lane = ACROSS ? (t & 63) / A : t % TPA;
+}
+
 // sum over the TPA lanes of a group; the result is valid in lane 0
-template <int TPA>
+template <int TPA, bool ACROSS = false>
 __device__ __forceinline__ double group_sum(double v) {
+  constexpr int A = ACROSS ? 64 / TPA : 1;
 #pragma unroll
-  for (int off = TPA / 2; off > 0; off >>= 1) v += __shfl_down(v, off, TPA);
+  for (int off = TPA / 2; off > 0; off >>= 1) v += __shfl_down(v, off * A, A > 1 ? 64 : TPA);
   return v;
 }
 
@@ -226,7 +256,7 @@ __device__ __forceinline__ double integrate_atom(int i, const double4 &xi, doubl
 
 // per-atom results of one group: lane 0 stores (and integrates when fused),
 // all lanes join the block sum of {e, virial[6], m v^2}
-template <int TPA, bool EV, bool INTEG, bool LATE = false>
+template <int TPA, bool EV, bool INTEG, bool LATE = false, bool ACROSS = false>
 __device__ __forceinline__ void finish_atom(int i, bool owner, const double4 &xi, double fx, double fy,
                                             double fz, double e, double (&w)[6], const IntegArgs &ig,
                                             double4 vpre, double4 hpre, double4 *__restrict__ f,
@@ -234,13 +264,13 @@ __device__ __forceinline__ void finish_atom(int i, bool owner, const double4 &xi
   int o = 0;  // caller index: its load overlaps the lane sums
   const bool caller = !INTEG && owner && (ig.out.f || (EV && (ig.out.e || ig.out.v)));
   if (caller) o = ig.out.orig[i];
-  fx = group_sum<TPA>(fx);
-  fy = group_sum<TPA>(fy);
-  fz = group_sum<TPA>(fz);
+  fx = group_sum<TPA, ACROSS>(fx);
+  fy = group_sum<TPA, ACROSS>(fy);
+  fz = group_sum<TPA, ACROSS>(fz);
   if (EV) {
-    e = group_sum<TPA>(e);
+    e = group_sum<TPA, ACROSS>(e);
 #pragma unroll
-    for (int q = 0; q < 6; q++) w[q] = group_sum<TPA>(w[q]);
+    for (int q = 0; q < 6; q++) w[q] = group_sum<TPA, ACROSS>(w[q]);
   }
   double mv2 = 0.0;
   if (owner) {
@@ -334,8 +364,9 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     f_off[q] = (float)tab->offset[q];
   }
   __syncthreads();
-  const int i = (xcd_block() * blockDim.x + threadIdx.x) / TPA;
-  const int lane = threadIdx.x % TPA;
+  int i, lane;
+  constexpr bool ACROSS = lj_across(MIXED, TPA);
+  group_place<TPA, ACROSS>(i, lane);
   // single type: the (1,1) coefficients come as kernel arguments, so they
   // stay in scalar registers for the whole loop (no LDS reads, no vector
   // registers)
@@ -361,9 +392,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
     // UNROLL entries per lane per trip: all index loads, then all gathers,
     // are issued before the first use, so a lane has UNROLL gathers in flight
-    constexpr bool CHUNK = kChunkLJ;
-    constexpr int U = CHUNK ? 4 : (Q ? kUnrollQ : kUnroll);
-    constexpr int KS = CHUNK ? 1 : TPA;  // entry stride within a trip
+    constexpr int U = 4;  // entries of a chunk
     const int self = i | (MDX_NOSHIFT << MDX_IDX_BITS);
     // TRANS (four lanes per atom, 32-B FP64 gathers): the group's four
     // chunks are transposed across its lanes, so gather u of the group
@@ -373,8 +402,11 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     // from k0 is k0 + 4u + lane.  Measured at 2.048 M atoms: FP64 fused
     // kernel 0.395 ms against 0.452; the 16-B fixed-point gathers gain
     // nothing (0.310 against 0.304), so Q keeps the lane's own chunk.
-    constexpr bool TRANS = CHUNK && TPA == 4 && kTransLJ && !Q;
-    for (int kt = TRANS ? 0 : CHUNK ? 4 * lane : lane; kt < jn; kt += NS * U * TPA) {
+    constexpr bool TRANS = TPA == 4 && kTransLJ && !Q && !ACROSS;
+    constexpr bool AHEAD = !TRANS && lj_ahead(TPA);
+    int4 pre = make_int4(0, 0, 0, 0);  // AHEAD: the lane's next chunk
+    if (AHEAD && 4 * lane < jn) pre = nb4[(size_t)lane * npad];
+    for (int kt = TRANS ? 0 : 4 * lane; kt < jn; kt += NS * U * TPA) {
 #pragma unroll
     for (int h = 0; h < NS; h++) {  // trip h of NS adds into set h
       const int k0 = kt + h * U * TPA;
@@ -394,15 +426,12 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
         quad_transpose(ev, lane);
 #pragma unroll
         for (int u = 0; u < U; u++) jc[u] = k0 + 4 * u + lane < jn ? ev[u] : self;
-      } else if constexpr (CHUNK) {
-        const int4 e4 = nb4[(size_t)(k0 >> 2) * npad];
+      } else {
+        const int4 e4 = AHEAD ? pre : nb4[(size_t)(k0 >> 2) * npad];
         const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
         for (int u = 0; u < U; u++) jc[u] = k0 + u < jn ? ev[u] : self;
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          jc[u] = (k0 + u * KS < jn) ? list_entry(nbr + list_index(i, k0 + u * KS, npad)) : self;
+        if (AHEAD && k0 + U * TPA < jn) pre = nb4[(size_t)((k0 + U * TPA) >> 2) * npad];
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
@@ -412,7 +441,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
 #pragma unroll
       for (int u = 0; u < U; u++) {
         // entries carry image bits: test the index, not the sign
-        if ((TRANS ? k0 + 4 * u + lane : k0 + u * KS) >= jn) continue;
+        if ((TRANS ? k0 + 4 * u + lane : k0 + u) >= jn) continue;
         double delx, dely, delz, rsq;
         int t;
         bool inside;
@@ -463,7 +492,7 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     }
   }
   if (Q && i < n && lane == 0) xi = x[i];
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
+  finish_atom<TPA, EV, INTEG, kLateV, ACROSS>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
                               partials);
 }
 
@@ -528,25 +557,16 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_rho(int n, int npad, int cap,
     const int4 qi = Q ? xq[i] : make_int4(0, 0, 0, 0);
     ti = Q ? qi.w : static_cast<int>(xi.w);
     const int jn = numneigh[i];
-    const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
-    constexpr bool CHUNK = kChunkEAM;
-    constexpr int U = CHUNK ? 4 : (Q ? kUnrollQ : kUnroll);
-    constexpr int KS = CHUNK ? 1 : TPA;  // entry stride within a trip
+    constexpr int U = Q ? kUnrollQ : kUnroll;
+    constexpr int KS = TPA;  // entry stride within a trip
     const int self = i | (MDX_NOSHIFT << MDX_IDX_BITS);
-    for (int k0 = CHUNK ? 4 * lane : lane; k0 < jn; k0 += U * TPA) {
+    for (int k0 = lane; k0 < jn; k0 += U * TPA) {
       int jc[U];
       double4 xj[Q ? 1 : U];
       int4 qj[Q ? U : 1];
-      if constexpr (CHUNK) {
-        const int4 e4 = nb4[(size_t)(k0 >> 2) * npad];
-        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-        for (int u = 0; u < U; u++) jc[u] = k0 + u < jn ? ev[u] : self;
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          jc[u] = (k0 + u * KS < jn) ? list_entry(nbr + list_index(i, k0 + u * KS, npad)) : self;
-      }
+      for (int u = 0; u < U; u++)
+        jc[u] = (k0 + u * KS < jn) ? list_entry(nbr + list_index(i, k0 + u * KS, npad)) : self;
 #pragma unroll
       for (int u = 0; u < U; u++) {
         if (Q) qj[u] = gather_q(xq, jc[u]);
@@ -660,26 +680,17 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int ca
     const int ti = Q ? qi.w : static_cast<int>(xi.w);
     const double fpi = fp[i];
     const int jn = numneigh[i];
-    const int4 *nb4 = reinterpret_cast<const int4 *>(nbr) + i;  // chunk c at nb4[c * npad]
-    constexpr bool CHUNK = kChunkEAM;
-    constexpr int U = CHUNK ? 4 : (Q ? kUnrollQ : kUnroll);
-    constexpr int KS = CHUNK ? 1 : TPA;  // entry stride within a trip
+    constexpr int U = Q ? kUnrollQ : kUnroll;
+    constexpr int KS = TPA;  // entry stride within a trip
     const int self = i | (MDX_NOSHIFT << MDX_IDX_BITS);
-    for (int k0 = CHUNK ? 4 * lane : lane; k0 < jn; k0 += U * TPA) {
+    for (int k0 = lane; k0 < jn; k0 += U * TPA) {
       int jc[U];
       double4 xjv[Q ? 1 : U];
       int4 qjv[Q ? U : 1];
       double fpjv[U];
-      if constexpr (CHUNK) {
-        const int4 e4 = nb4[(size_t)(k0 >> 2) * npad];
-        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
-        for (int u = 0; u < U; u++) jc[u] = k0 + u < jn ? ev[u] : self;
-      } else {
-#pragma unroll
-        for (int u = 0; u < U; u++)
-          jc[u] = (k0 + u * KS < jn) ? list_entry(nbr + list_index(i, k0 + u * KS, npad)) : self;
-      }
+      for (int u = 0; u < U; u++)
+        jc[u] = (k0 + u * KS < jn) ? list_entry(nbr + list_index(i, k0 + u * KS, npad)) : self;
 #pragma unroll
       for (int u = 0; u < U; u++) {
         if (Q) qjv[u] = gather_q(xq, jc[u]);
@@ -894,13 +905,14 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 // chip; below that more lanes per atom shorten the one chain of dependent
 // loads that a small launch consists of.  Measured per step kernel (us, lanes
 // 4 / 8 / 16 / 32 per atom, FP64):
-//   lj/cut            500 atoms  8.3 /  6.9 /  5.0 /  4.9
-//                   4,000        8.1 /  7.3 /  4.9 /  5.3
-//                  32,000       10.4 / 10.8 / 13.0 / 16.7  (mixed 8.0 / 7.7 / 10.1)
-//                 108,000       24.6 / 30.5 / 36.5 / 51
-//               2,048,000        381 /  508 /  685 / 1096  (mixed  286 /  329)
-//   Kob-Andersen    2,744       11.1 /  7.9 /  5.8 /  5.3
-//                   8,000       11.0 /  7.7 /  6.5 /  6.6
+//   lj/cut            500 atoms  7.9 /  5.3 /  4.7 /  4.4
+//                   4,000        7.5 /  5.3 /  4.8 /  5.0
+//                  32,000       10.7 / 10.1 / 12.2 / 16.1  (mixed 8.4 / 7.7)
+//                  42,592       12.1 / 13.3 / 15.4 / 19.8  (mixed 9.0 / 9.3)
+//                 108,000       25.0 / 27.0 / 34.0 / 50    (mixed 16.8 / 19.3)
+//               2,048,000        380 /  446 /  638 / 1087  (mixed  272 /  342)
+//   Kob-Andersen    2,744        9.9 /  6.5 /  5.4 /  4.9
+//                   8,000       10.5 /  6.8 /  6.1 /  6.2
 //   eam (rho+force)   500       19.3 / 14.6 / 12.2 / 10.5
 //                   4,000       19.6 / 14.7 / 12.4 / 12.6
 //                  13,500       22.6 / 16.5 / 17.4 / 24.2
@@ -908,7 +920,7 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 // Mixed precision takes only 8 and 4, which give the same bits (split_sums):
 // a mixed trajectory amplifies any other difference to its own error.
 // Workgroups of one wavefront spread a small launch evenly over the CUs
-// (13,500 lj/cut atoms at 8 lanes: 6.8 against 7.9 us); with 1024 or more
+// (13,500 lj/cut atoms at 8 lanes: 64 threads 14% faster than 256); with 1024 or more
 // workgroups of 256 there is nothing to gain.  The single-type eam kernels
 // copy their spline tables to LDS once per workgroup, so they keep 256 (mixed,
 // 13,500 atoms: 15.9 against 22.1 us), and 512 for the larger FP64 tables
@@ -917,7 +929,7 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 Launch pair_launch(const mdx_ctx *c) {
   Launch l = c->launch;
   const bool mixed = c->precision == MDX_MIXED;
-  if (!l.tpa) l.tpa = c->n > 48000 ? 4 : c->n > 10000 || mixed ? 8 : c->n > 3000 ? 16 : 32;
+  if (!l.tpa) l.tpa = c->n > 40000 ? 4 : c->n > 10000 || mixed ? 8 : c->n > 3000 ? 16 : 32;
   if (!l.block) {
     const bool tables = c->pair_style == MDX_PAIR_EAM && eam_lds_tables(c, l.tpa);
     l.block = tables ? (mixed || c->n <= 10000 ? 256 : 512) : (long)c->n * l.tpa < 1024L * 256 ? 64 : 256;

@@ -515,8 +515,8 @@ def test_shifted_two_type_lj_energies_match_the_oracle(prec):
     ctx.close()
 
 
-@pytest.mark.parametrize("style,n", [("lj", 3000), ("lj", 3001), ("lj", 10000), ("lj", 10001), ("lj", 48000),
-                                     ("lj", 48001), ("eam", 6000), ("eam", 6001), ("eam", 10001), ("eam", 48001)])
+@pytest.mark.parametrize("style,n", [("lj", 3000), ("lj", 3001), ("lj", 10000), ("lj", 10001), ("lj", 40000),
+                                     ("lj", 40001), ("lj", 48000), ("lj", 48001), ("eam", 6000), ("eam", 6001), ("eam", 10001), ("eam", 48001)])
 def test_default_launch_shapes_agree_with_a_fixed_one(style, n):
     """On both sides of the sizes where the default launch shape changes:
     forces equal those of 8 lanes per atom in workgroups of 256 to the order
