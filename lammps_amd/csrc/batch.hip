@@ -387,6 +387,40 @@ __device__ __forceinline__ void row_chunk(const int *__restrict__ row, int k0, i
   ent[3] = k0 + 3 < jn ? e4.w : self;
 }
 
+// How a lane walks its share of a row.  By chunk: four consecutive entries,
+// the chunks lane, lane + TPA, ...  QUAD with four lanes per atom: the four
+// chunks of a trip are transposed across the lanes, so gather u of the atom
+// covers entries 4u .. 4u+3 of the trip, which share cache lines, instead of
+// entries u, 4+u, 8+u, 12+u.  That pays for the passes that gather 64 B per
+// pair and wait for L1 (40 line lookups per load instruction, chunk / quad at
+// 1,367,136 atoms: eam pass A 412 / 367 us, pass B 186 / 179, FP64 forces 269 /
+// 261; lj gradient 101,250 atoms 45.3 / 40.8); the 16-B gathers of mixed
+// precision, and more lanes in small batches, lose (101,903: 14.8 / 16.0).
+template <int TPA, bool QUAD>
+struct RowWalk {
+  static constexpr bool kQuad = QUAD && TPA == 4;
+  int lane;
+  __device__ __forceinline__ int first() const { return kQuad ? 0 : 4 * lane; }
+  // the entry that gather u of the trip from k0 covers
+  __device__ __forceinline__ int at(int k0, int u) const { return kQuad ? k0 + 4 * u + lane : k0 + u; }
+  __device__ __forceinline__ void read(const int *__restrict__ row, int k0, int jn, int self, int (&ent)[4]) const {
+    if constexpr (kQuad) {  // trips are group-uniform: the transpose reads all four lanes
+      int4 e4 = make_int4(self, self, self, self);
+      if (k0 + 4 * lane < jn) e4 = *reinterpret_cast<const int4 *>(row + k0 + 4 * lane);
+      ent[0] = e4.x;
+      ent[1] = e4.y;
+      ent[2] = e4.z;
+      ent[3] = e4.w;
+      quad_transpose(ent, lane);
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (at(k0, u) >= jn) ent[u] = self;
+    } else {
+      row_chunk(row, k0, jn, self, ent);
+    }
+  }
+};
+
 // separation of a pair within half the box, in FP64: the nearest image
 // (periodic boxes are at least two cutoffs wide, so it is the list's)
 __device__ __forceinline__ double nearest(double d, double prd, double iprd) { return fma(-prd, rint(d * iprd), d); }
@@ -422,6 +456,7 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, false> walk{lane};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -437,19 +472,17 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
       // rows start 16-B aligned), then four 16-B gathers in flight
       const int4 qi = xq[i];
       const double q0 = g.qstep[0], q1 = g.qstep[1], q2 = g.qstep[2];
-      for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
-        const int4 e4 = *reinterpret_cast<const int4 *>(row + k0);
-        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
         int ent[4];
         int4 qj[4];
+        walk.read(row, k0, jn, i, ent);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          ent[u] = k0 + u < jn ? ev[u] : i;  // the row's tail past jn is not written
           qj[u] = gather_q(xq, ent[u]);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          if (k0 + u >= jn) continue;
+          if (walk.at(k0, u) >= jn) continue;
           const double dx = qsep(qi.x, qj[u].x, q0), dy = qsep(qi.y, qj[u].y, q1), dz = qsep(qi.z, qj[u].z, q2);
           const double rsq = dx * dx + dy * dy + dz * dz;
           const int t = ti * nt1 + qj[u].w;
@@ -473,19 +506,17 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
         }
       }
     } else {
-      for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
-        const int4 e4 = *reinterpret_cast<const int4 *>(row + k0);
-        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
         int ent[4];
         double4 xj[4];
+        walk.read(row, k0, jn, i, ent);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          ent[u] = k0 + u < jn ? ev[u] : i;
           xj[u] = gather_x(x, ent[u]);
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-          if (k0 + u >= jn) continue;
+          if (walk.at(k0, u) >= jn) continue;
           const double dx = nearest(xi.x - xj[u].x, px, g.iprd[0]), dy = nearest(xi.y - xj[u].y, py, g.iprd[1]),
                        dz = nearest(xi.z - xj[u].z, pz, g.iprd[2]);
           const double rsq = dx * dx + dy * dy + dz * dz;
@@ -542,6 +573,7 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, true> walk{lane};
   double ae[NA] = {}, as[NA] = {};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
@@ -553,10 +585,10 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
     const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
-    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4], gj[4];
-      row_chunk(row, k0, jn, i, ent);
+      walk.read(row, k0, jn, i, ent);
       bool any = false;
 #pragma unroll
       for (int q = 0; q < 4; q++) any |= (ent[q] & MDX_IDX_MASK) > i;
@@ -722,6 +754,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, false> walk{lane};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -738,11 +771,11 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double acc = 0.0;
-    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[MIXED ? 1 : 4];
       int4 qj[MIXED ? 4 : 1];
-      row_chunk(row, k0, jn, i, ent);
+      walk.read(row, k0, jn, i, ent);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
@@ -751,7 +784,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         double dx, dy, dz, rsq;
-        if (k0 + u < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
+        if (walk.at(k0, u) < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
                                              step, ip, dx, dy, dz, rsq)) {
           int m;
           T p;
@@ -810,6 +843,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, !MIXED> walk{lane};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -827,12 +861,12 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
-    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[MIXED ? 1 : 4];
       int4 qj[MIXED ? 4 : 1];
       double fpj[4];
-      row_chunk(row, k0, jn, i, ent);
+      walk.read(row, k0, jn, i, ent);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
@@ -842,7 +876,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         double dx, dy, dz, rsq;
-        if (k0 + u < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
+        if (walk.at(k0, u) < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
                                              step, ip, dx, dy, dz, rsq)) {
           int m;
           T p, r, recip;
@@ -886,6 +920,10 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
 // per thread modulo copies, coefficient-major (neighbouring knots in
 // neighbouring banks).  Row of partials: [frho c3..c6 (nrho+1)*4 | rhor
 // (nr+1)*4 | z2r (nr+1)*4] from pass A, rhor alone from pass B.
+// The partner's scalar comes with a vector that is gathered anyway: fp in
+// dL/dF's fourth component (pass A: read inside the j > i branch it cost a
+// memory latency per pair, 367 against 329 us at 1,367,136 atoms), dL/drho
+// in that of the positions pass A writes for pass B (179 against 163).
 // stride of one accumulator set of `terms` coefficients: offset by 8 doubles
 // modulo 32 from copy to copy
 __host__ __device__ inline int adj_stride(int terms, int kn) { return (terms * kn + 31) / 32 * 32 + 8; }
@@ -896,8 +934,8 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
                                                       const int *__restrict__ nbr, const int *__restrict__ numneigh,
                                                       int cap, EamTab et, const double4 *__restrict__ rhor,
                                                       const double *__restrict__ frho_d, const double *__restrict__ rho,
-                                                      const double *__restrict__ fp, const double4 *__restrict__ gin,
-                                                      int copies, double *__restrict__ vout,
+                                                      const double4 *__restrict__ gin, int copies,
+                                                      double4 *__restrict__ vout,
                                                       double *__restrict__ partials) {
   extern __shared__ double4 s_knots[];
   const int kn = et.nr + 1, kf = et.nrho + 1, stride = adj_stride(7, kn);
@@ -912,22 +950,22 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, true> walk{lane};
   const double rdr = et.rdr;
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
     const double4 xi = x[i];
     const double4 gi = gin[i];
-    const double fpi = fp[i];
     const RepGeom &g = geom[rep[i]];
     const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double u = 0.0;
-    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4], gj[4];
-      row_chunk(row, k0, jn, i, ent);
+      walk.read(row, k0, jn, i, ent);
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         xj[q] = gather_x(x, ent[q]);
@@ -935,7 +973,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
       }
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        if (k0 + q >= jn) continue;
+        if (walk.at(k0, q) >= jn) continue;
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
@@ -947,9 +985,8 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
           const double4 c = TL ? s_rd[m] : rhor[2 * m];
           const double b = -((gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz) * ri;
           u += b * ((c.x * p + c.y) * p + c.z);
-          const int j = ent[q] & MDX_IDX_MASK;
-          if (j > i) {
-            const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * (fpi + fp[j]) * rdr, gzr = gz1 * rdr, pp = p * p;
+          if ((ent[q] & MDX_IDX_MASK) > i) {
+            const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * (gi.w + gj[q].w) * rdr, gzr = gz1 * rdr, pp = p * p;
             double *a = mine + m;
             atomicAdd(a, 3.0 * pp * gzr + gz0 * pp * p);
             atomicAdd(a + kn, 2.0 * p * gzr + gz0 * pp);
@@ -978,7 +1015,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
       atomicAdd(s_gf + 2 * kf + m, u * rdrho);
       const double *c = frho_d + m * 7;
       const double fpp = clamped ? 0.0 : (2.0 * c[0] * p + c[1]) * rdrho;
-      vout[i] = u * fpp;
+      vout[i] = make_double4(xi.x, xi.y, xi.z, u * fpp);
     }
   }
   __syncthreads();
@@ -998,10 +1035,10 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
 }
 
 template <int TPA>
-__global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__restrict__ x,
+__global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__restrict__ xv,
                                                       const int *__restrict__ rep, const RepGeom *__restrict__ geom,
                                                       const int *__restrict__ nbr, const int *__restrict__ numneigh,
-                                                      int cap, EamTab et, const double *__restrict__ vin, int copies,
+                                                      int cap, EamTab et, int copies,
                                                       double *__restrict__ partials) {
   extern __shared__ double4 s_knots[];
   const int kn = et.nr + 1, stride = adj_stride(4, kn);
@@ -1013,36 +1050,32 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
   int end;
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
+  const RowWalk<TPA, true> walk{lane};
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
-    const double vi = vin[i];
-    const double4 xi = x[i];
+    const double4 xi = xv[i];
     const RepGeom &g = geom[rep[i]];
     const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
-    for (int k0 = 4 * lane; k0 < jn; k0 += 4 * TPA) {
+    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4];
-      double vj[4];
-      row_chunk(row, k0, jn, i, ent);
+      walk.read(row, k0, jn, i, ent);
       bool any = false;
 #pragma unroll
       for (int q = 0; q < 4; q++) any |= (ent[q] & MDX_IDX_MASK) > i;
       if (!any) continue;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        xj[q] = gather_x(x, ent[q]);
-        vj[q] = gather_d(vin, ent[q]);
-      }
+      for (int q = 0; q < 4; q++) xj[q] = gather_x(xv, ent[q]);
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         if ((ent[q] & MDX_IDX_MASK) <= i) continue;  // the pair's other row, or past the end
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
-        const double v = vi + vj[q];
+        const double v = xi.w + xj[q].w;
         if (rsq < et.cutsq && v != 0.0) {
           double r, ri, p;
           int m;
@@ -1130,11 +1163,13 @@ __global__ void k_b_gather_s(int n, const int *__restrict__ inv, const double *_
   if (c < n) out[c] = a[inv[c]];
 }
 
+// dL/dF in sorted order, with a per-atom value w (null: 0) beside it
 __global__ void k_b_scatter_g(int n, const int *__restrict__ inv, const double *__restrict__ gin,
-                              double4 *__restrict__ g) {
+                              const double *__restrict__ w, double4 *__restrict__ g) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
-  g[inv[c]] = make_double4(gin[3 * (size_t)c], gin[3 * (size_t)c + 1], gin[3 * (size_t)c + 2], 0.0);
+  const int i = inv[c];
+  g[i] = make_double4(gin[3 * (size_t)c], gin[3 * (size_t)c + 1], gin[3 * (size_t)c + 2], w ? w[i] : 0.0);
 }
 
 }  // namespace
@@ -1177,7 +1212,8 @@ struct mdx_batch {
   long total_neighbors = 0;
   int max_neighbors = 0;
   double *staging = nullptr;  // [N][3] output staging
-  double *rho = nullptr, *fp = nullptr, *eemb = nullptr, *vadj = nullptr;
+  double *rho = nullptr, *fp = nullptr, *eemb = nullptr;
+  double4 *vadj = nullptr;  // positions with dL/drho beside them
   double *partials = nullptr;
   size_t partials_cap = 0;  // doubles
   double *colsum = nullptr;
@@ -1580,7 +1616,7 @@ int force_results(mdx_batch *b, const ForceOut &out, double *f, double *energy) 
   return rc;
 }
 
-int read_g(mdx_batch *b, const double *gf) {
+int read_g(mdx_batch *b, const double *gf, const double *w = nullptr) {
   const int n = b->n;
   const double *src = gf;
   hipError_t e;
@@ -1590,7 +1626,7 @@ int read_g(mdx_batch *b, const double *gf) {
       return bfail(e, "dL/dF upload");
     src = b->staging;
   }
-  hipLaunchKernelGGL(k_b_scatter_g, dim3((n + 255) / 256), dim3(256), 0, b->stream, n, b->inv, src, b->g);
+  hipLaunchKernelGGL(k_b_scatter_g, dim3((n + 255) / 256), dim3(256), 0, b->stream, n, b->inv, src, w, b->g);
   return MDX_OK;
 }
 
@@ -2083,7 +2119,7 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
   // the adjoint uses FP64 rho/fp (a mixed forward's rho moves the frho
   // spline weights by ~1e-5 relative): rerun the rho pass in FP64 if needed
   if (b->eam_rho_prec != MDX_FP64 && (rc = eam_forward(b, false, MDX_FP64))) return rc;
-  if ((rc = read_g(b, gf))) return rc;
+  if ((rc = read_g(b, gf, b->fp))) return rc;
   // FP64 adjoint arithmetic in both precision modes, as for lj/cut
   const int P = 4 * (b->et.nrho + 1) + 8 * (b->et.nr + 1);
   if ((long)sizeof(double) * P > b->lds_max) {
@@ -2108,7 +2144,7 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
     gA = G;
     auto go = [&](auto tl) {
       TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_adj_a<TP, decltype(tl)::value>), G, t.block, shA, b->n, b->x, b->rep, b->geom, b->nbr, b->numneigh, b->cap,
-                                             b->et, b->knots.rhor_d, b->frho_d, b->rho, b->fp, b->g, cA, b->vadj,
+                                             b->et, b->knots.rhor_d, b->frho_d, b->rho, b->g, cA, b->vadj,
                                              b->partials))
     };
     if (tlA) go(std::true_type{});
@@ -2119,8 +2155,8 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
   auto launchB = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);
     gB = G;
-    TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_adj_b<TP>), G, t.block, shB, b->n, b->x,
-                                           b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, b->vadj, cB, partB))
+    TPA_DISPATCH(t.tpa, BATCH_LAUNCH((k_b_eam_adj_b<TP>), G, t.block, shB, b->n, b->vadj,
+                                           b->rep, b->geom, b->nbr, b->numneigh, b->cap, b->et, cB, partB))
   };
   if ((rc = run_kind(b, MDX_BK_EAM_ADJ_B, launchB))) return rc;
   if ((rc = colsum(b, gA, P, partB, gB, 4 * kf, 4 * kn))) return rc;

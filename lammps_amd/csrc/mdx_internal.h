@@ -276,6 +276,23 @@ __device__ __forceinline__ double4 gather_x(const double4 *__restrict__ x, unsig
 __device__ __forceinline__ double gather_d(const double *__restrict__ a, unsigned entry) {
   return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a) + ((entry << 5) >> 2));
 }
+// 4x4 transpose across the four lanes of an aligned quad: on return lane l
+// holds in a[r] what lane r held in a[l].  Two butterfly rounds of
+// quad-permute moves (DPP, within the quad); all four lanes must be active.
+__device__ __forceinline__ void quad_transpose(int (&a)[4], int l) {
+  int p[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) p[r] = __builtin_amdgcn_mov_dpp(a[r ^ 1], 0xB1, 0xF, 0xF, false);  // lane ^ 1
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if ((l ^ r) & 1) a[r] = p[r];
+#pragma unroll
+  for (int r = 0; r < 4; r++) p[r] = __builtin_amdgcn_mov_dpp(a[r ^ 2], 0x4E, 0xF, 0xF, false);  // lane ^ 2
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if ((l ^ r) & 2) a[r] = p[r];
+}
+
 // separation q_i - q_j of one dimension in length units (FP64, exact product)
 __device__ __forceinline__ double qdelta(int qi, int qj, double step) {
   return (double)(int)((unsigned)qi - (unsigned)qj) * step;
