@@ -95,7 +95,7 @@ void free_atoms(mdx_ctx *c) {
   if (c->stage_busy) (void)hipStreamSynchronize(c->stream);  // queued copies still read the stage
   void *ptrs[] = {c->x, c->xb, c->v, c->vb, c->f, c->xhold, c->tag, c->tagb, c->orig, c->origb, c->image,
                   c->imageb, c->inv, c->vatom, c->dscratch, c->bkey, c->bidx, c->bidx_s,
-                  c->numneigh, c->nbr, c->rho, c->fp, c->eemb, c->partials, c->xq, c->xqb};
+                  c->numneigh, c->nbr, c->rho, c->fp, c->eemb, c->xf, c->partials, c->xq, c->xqb};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   c->x = c->xb = c->v = c->vb = c->f = c->xhold = nullptr;
@@ -104,6 +104,7 @@ void free_atoms(mdx_ctx *c) {
   c->bkey = nullptr;
   c->bidx = c->bidx_s = c->numneigh = c->nbr = nullptr;
   c->rho = c->fp = c->eemb = c->partials = nullptr;
+  c->xf = nullptr;
   c->xq = c->xqb = nullptr;
   c->xq_stale = true;
   if (c->host_stage) (void)hipHostFree(c->host_stage);
@@ -356,7 +357,7 @@ int mdx_set_atoms(mdx_ctx *c, int n, int ntypes, const double *x, const double *
   // A host program hands its atoms over at every reneighbouring, a few more
   // or fewer each time: storage that holds them (and is at most twice what
   // they need) is kept, list included, instead of freed and allocated again
-  // (27 arrays; 2.9 ms with the list build at 108,000 atoms, 0.4 ms kept).
+  // (28 arrays; 2.9 ms with the list build at 108,000 atoms, 0.4 ms kept).
   if (c->cap_atoms < npad || c->cap_atoms / 2 > npad) {
     free_atoms(c);
     c->cap_atoms = npad;
@@ -369,7 +370,7 @@ int mdx_set_atoms(mdx_ctx *c, int n, int ntypes, const double *x, const double *
         (rc = dev_alloc(&c->bkey, npad)) || (rc = dev_alloc(&c->bidx, npad)) ||
         (rc = dev_alloc(&c->bidx_s, npad)) || (rc = dev_alloc(&c->numneigh, npad)) ||
         (rc = dev_alloc(&c->rho, npad)) || (rc = dev_alloc(&c->fp, npad)) || (rc = dev_alloc(&c->eemb, npad)) ||
-        (rc = dev_alloc(&c->xq, npad)) || (rc = dev_alloc(&c->xqb, npad)))
+        (rc = dev_alloc(&c->xf, npad)) || (rc = dev_alloc(&c->xq, npad)) || (rc = dev_alloc(&c->xqb, npad)))
       return drop_atoms(c, rc);
     if (hipHostMalloc(&c->host_stage, (size_t)(sizeof(double) * kStageDoubles * npad), hipHostMallocDefault) !=
         hipSuccess) {

@@ -486,6 +486,7 @@ struct mdx_ctx {
   double *eam_pk = nullptr;  // packed rhor | z2r (EAMArgs::rhor_p, z2r_p)
   float *eam_pk_f = nullptr;
   double *rho = nullptr, *fp = nullptr, *eemb = nullptr;
+  double4 *xf = nullptr;  // position and fp for the eam force pass (mixed: int4 each)
   // reductions
   double *partials = nullptr;
   long cap_partials = 0;

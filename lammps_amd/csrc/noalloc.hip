@@ -260,6 +260,7 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
     set_error("mdx_compute_noalloc: atom type out of range");
     return MDX_ERR_ARG;
   }
+  s.xf = s.vb;  // the velocity copy's storage is free once the list is built
   if ((rc = pair_compute(&s, ev, nullptr))) return rc;
   hipLaunchKernelGGL(k_noalloc_add_forces, dim3(G), dim3(B), 0, s.stream, n, s.orig, s.f, f);
   if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "force scatter launch");
