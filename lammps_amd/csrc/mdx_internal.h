@@ -377,6 +377,7 @@ __host__ __device__ __forceinline__ size_t list_index(int i, int k, int npad) {
 struct PairOut {
   double *f, *e, *v;
   const int *orig;  // caller index of each atom
+  int add;          // f += the forces (0: f = them)
 };
 
 struct IntegArgs {

@@ -261,9 +261,9 @@ __device__ __forceinline__ void finish_atom(int i, bool owner, const double4 &xi
     if (caller) {
       if (ig.out.f) {
         double *const d = ig.out.f + 3 * (size_t)o;
-        d[0] = fx;
-        d[1] = fy;
-        d[2] = fz;
+        d[0] = ig.out.add ? d[0] + fx : fx;
+        d[1] = ig.out.add ? d[1] + fy : fy;
+        d[2] = ig.out.add ? d[2] + fz : fz;
       }
       if (EV && ig.out.e) ig.out.e[o] = e;
       if (EV && ig.pervir && ig.out.v) {
