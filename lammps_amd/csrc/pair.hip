@@ -740,12 +740,14 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int ca
 
 // Resident wavefronts per SIMD of the fused force kernels, held by giving
 // each workgroup enough LDS that no more workgroups fit on a CU (160 KiB of
-// LDS, four SIMDs).  The mixed fused lj/cut kernel runs fastest at 7: with
-// its single-type coefficients in scalar registers it needs 64 vector
-// registers, which would admit 8 (2.048 M atoms: 0.316 ms per launch at 8,
-// 0.306 held to 7; with 66 registers it was 0.303-0.306 at its own 7).  The
-// FP64 one runs fastest held to 5 (0.394 ms; 0.399 at 6, 0.410 at 7, 0.415
-// at 8).  MDX_PAIR_WAVES sets a cap (0: none) on both and on the EAM passes.
+// LDS, four SIMDs).  The FP64 fused lj/cut kernel runs fastest held to 6
+// (2.048 M atoms: 386 us at 5, 380 at 6, 389 at 7, 397 at its own 8; 256,000:
+// 48.3, 46.5, 46.6, 47.0) once it has two rounds of them; below, the last
+// round decides and all that fit run (108,000: 25.8, 26.9, 24.2, 24.6; 157,216:
+// 32.0, 32.2, 32.0, 31.9).  The mixed one runs at the 7 that its registers
+// allow (272 us; held to 6: 283, to 5: 311).  MDX_PAIR_WAVES sets a cap (0:
+// none) on both and on the EAM passes.
+constexpr long kChipSimds = 256 * 4;
 int pair_wave_cap(int dflt) {
   static const int w = [] {
     const char *s = std::getenv("MDX_PAIR_WAVES");
@@ -780,7 +782,8 @@ template <bool MIXED, bool EV, int TPA, bool INTEG, bool Q, bool ONE>
 void launch_lj_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   const int G = xcd_grid(((long)c->n * TPA + B - 1) / B);
   prof_begin(c, INTEG ? MDX_K_FUSED : MDX_K_LJ);
-  const size_t lds = INTEG ? occupancy_lds(static_lds<k_lj<MIXED, EV, TPA, INTEG, Q, ONE>>(), B, 0, MIXED ? 7 : 5) : 0;
+  const int waves = !MIXED && (long)c->n * TPA > 2 * 6 * 64 * kChipSimds ? 6 : 0;
+  const size_t lds = INTEG ? occupancy_lds(static_lds<k_lj<MIXED, EV, TPA, INTEG, Q, ONE>>(), B, 0, waves) : 0;
   LJOne one{};
   if (ONE) {
     const LJTab &t = c->lj_host;
@@ -902,16 +905,16 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 // 4 / 8 / 16 / 32 per atom, FP64):
 //   lj/cut            500 atoms  7.9 /  5.3 /  4.7 /  4.4
 //                   4,000        7.5 /  5.3 /  4.8 /  5.0
-//                  32,000       10.7 / 10.1 / 12.2 / 16.1  (mixed 8.4 / 7.7)
+//                  32,000       10.8 / 10.3 / 12.2 / 15.2  (mixed 7.8 / 7.6)
 //                  42,592       12.1 / 13.3 / 15.4 / 19.8  (mixed 9.0 / 9.3)
-//                 108,000       25.0 / 27.0 / 34.0 / 50    (mixed 16.8 / 19.3)
-//               2,048,000        380 /  446 /  638 / 1087  (mixed  272 /  342)
+//                 108,000       24.6 / 26.8 / 32.8 / 47    (mixed 17.1 / 19.0)
+//               2,048,000        380 /  447 /  591 /  967  (mixed  272 /  329)
 //   Kob-Andersen    2,744        9.9 /  6.5 /  5.4 /  4.9
-//                   8,000       10.5 /  6.8 /  6.1 /  6.2
+//                   8,000       10.6 /  6.8 /  6.1 /  6.2
 //   eam (rho+force)   500       19.3 / 14.6 / 12.2 / 10.5
 //                   4,000       19.6 / 14.7 / 12.4 / 12.6
-//                  13,500       22.6 / 16.5 / 17.4 / 24.2
-//                 108,000         57 /   65 /   89 /  136
+//                  13,500       22.3 / 16.3 / 17.4 / 24.2
+//                 108,000         55 /   58 /   89 /  136
 // Mixed precision takes only 8 and 4, which give the same bits (split_sums):
 // a mixed trajectory amplifies any other difference to its own error.
 // Workgroups of one wavefront spread a small launch evenly over the CUs
