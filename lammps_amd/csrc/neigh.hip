@@ -1039,7 +1039,7 @@ __global__ __launch_bounds__(kGroupBlock, 5) void k_build_group(NeighArgs a, con
   }
 }
 
-// The fixed-point build needs the mirror (written by k_permute just before
+// The fixed-point build needs the mirror (written by k_rank_permute just before
 // the build, in either precision, where its resolution fits the band; mixed
 // precision also keeps it current between builds for its gathers) and a
 // stencil that never holds one atom under two periodic images.

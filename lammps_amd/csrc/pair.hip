@@ -102,7 +102,7 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], double *__re
 // consecutive atoms as contiguous 16-B pieces, not TPA chunks npad * 16 B
 // apart, and the gathers of neighbouring atoms share more cache lines.  The
 // kernel waits for L1: 1.09 line lookups per CU and cycle at 2.048 M atoms
-// (47 per load instruction), its vector units 57% busy.  Per step kernel,
+// (47 per load instruction; across 0.85 and 34), its vector units 57% busy.  Per step kernel,
 // grouped / across: mixed, 4 lanes 2.048 M atoms 287 / 272 us, 256,000 35.1 /
 // 32.3; FP64, 8 lanes 32,000 11.0 / 10.2; 16 lanes 8,000 Kob-Andersen 6.37 /
 // 6.15.  Four lanes in FP64 keep the group (its transposed chunks are faster:
