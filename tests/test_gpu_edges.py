@@ -175,6 +175,27 @@ def test_small_bin_grids_match_the_oracle(prec, shape):
     assert mx <= (1e-11 if prec == "fp64" else 1e-5)
 
 
+@pytest.mark.parametrize("nb", [(5, 5, 5), (15, 21, 13), (16, 16, 16), (43, 37, 5), (16, 16, 32), (25, 31, 21),
+                                (16, 32, 32), (31, 33, 32), (32, 32, 32)])
+def test_bin_counts_around_the_scan_lines(nb):
+    """Grids whose counters (bins + 1) end just below, at and above the lines
+    where the scan of the bin counters changes (4,096, 8,192, 16,384 and
+    32,768 counters), and in between: the pairs are those of a search over
+    all atoms."""
+    from scipy.spatial import cKDTree
+    from lammps_amd import mdx
+    cut = 2.8  # 2.5 and the skin; two bins to the cutoff
+    L = 0.5 * cut * np.array(nb) + 0.2
+    x = np.random.default_rng(sum(nb)).uniform(0.0, 1.0, (3000, 3)) * L
+    ctx = lj_context((0.0, 0.0, 0.0), tuple(L), (1, 1, 1), x, mdx.FP64)
+    ctx.neigh_build()
+    got = {(min(int(a), int(b)) - 1, max(int(a), int(b)) - 1) for a, b in ctx.neigh_pairs()}  # pairs of tags
+    st = ctx.stats()
+    ctx.close()
+    assert tuple(st["nbins"]) == nb
+    assert got == cKDTree(x, boxsize=L).query_pairs(cut)
+
+
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 def test_long_box_beyond_the_pruning_grid_matches_the_oracle(prec):
     """A periodic box 12,000 sigma long in x: more than 8192 bins in x, where
