@@ -68,7 +68,7 @@ unsigned char *g_scratch[kMaxDevices] = {};
 // read as type 1 so that no table is indexed out of range.  The same launch
 // clears the build's flags and bin counters (three memsets before: with the
 // copy of a flag and the launch that added the forces, 154 us per call of
-// 32,000 lj/cut atoms, now 119).
+// 32,000 lj/cut atoms, now 114-119).
 __global__ void k_noalloc_pack(int n, int ntypes, const double *__restrict__ x, const int *__restrict__ type,
                                double4 *__restrict__ xo, double4 *__restrict__ v, int *__restrict__ tag,
                                int *__restrict__ orig, int *__restrict__ inv, int *__restrict__ image, int img0,
