@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "../../include/mdx_batch.h"
+#include "bin_rows.h"
 #include "mdx_internal.h"
 
 namespace mdx {
@@ -243,12 +244,13 @@ __global__ __launch_bounds__(kBuildBlock, 5) void k_b_build(int n, const double4
       jy -= sy * nby;
       const int rowbase = g.bin_off + (jz * nby + jy) * nbx;
       const float wb = sqrtf(reach - dyz2) * (float)g.bininv[0] + 1e-3f;
-      const int x0 = max(ix - kS, (int)ceilf(tx - 1.0f - wb)), x1 = min(ix + kS, (int)floorf(tx + wb));
+      int x0, x1;
+      row_bins(ix, kS, tx, wb, x0, x1);
       const int cyz = 9 * (0 + 1) + 3 * (sy + 1) + (sz + 1);
       const bool wlo = x0 < 0 && g.periodic[0], whi = x1 >= nbx && g.periodic[0];  // 2 kS <= nbx: not both
       const int p = wlo ? 1 : 0;
-      lo[p] = rowbase + max(x0, 0);
-      hi[p] = max(lo[p], rowbase + min(x1, nbx - 1) + 1);
+      lo[p] = rowbase + max(x0, 0);  // x0 <= ix <= x1: never empty
+      hi[p] = rowbase + min(x1, nbx - 1) + 1;
       code[p] = cyz;
       if (wlo) {
         lo[0] = rowbase + x0 + nbx;

@@ -366,3 +366,25 @@ def test_default_batch_launch_shapes_agree_with_a_fixed_one(nrep, nside):
     assert force_errors(f0, f1)[0] <= 1e-12
     assert rel(ge0, ge1) <= 1e-12 and rel(gs0, gs1) <= 1e-12
     b.close()
+
+
+@pytest.mark.parametrize("far", [5.0, 1e9, 1e30, np.inf, -1e9, -np.inf, np.nan])
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_atom_far_outside_a_closed_box_is_reported(d, far):
+    """An atom outside its replica's box in a non-periodic dimension is an
+    error, however far outside it lies; the batch works on afterwards."""
+    rng = np.random.default_rng(3)
+    x = rng.uniform(0.2, 19.8, size=(600, 3))
+    b = B.Batch([400, 200], [[0, 0, 0]] * 2, [[20.0, 20.0, 20.0]] * 2, [[0, 0, 0]] * 2, 1, np.ones(600, np.int32))
+    one = np.ones((2, 2))
+    b.lj_init(one, one * 0.1, one * 2.5)
+    bad = x.copy()
+    bad[399, d] = 20.0 + far if far > 0 or far != far else far
+    b.set_positions(bad)
+    with pytest.raises(Exception, match="outside its replica's box"):
+        b.neigh_stats()
+    b.set_positions(x)
+    total, _ = b.neigh_stats()
+    want = sum(int(np.sum(np.sum((q[:, None] - q[None]) ** 2, -1) < 6.25)) - len(q) for q in (x[:400], x[400:]))
+    assert total == want
+    b.close()

@@ -99,3 +99,11 @@ def test_runner_parser_under_asan_ubsan(build_dir, tmp_path, extra, want_rc):
     r = subprocess.run([exe, "-in", path], capture_output=True, text=True, timeout=120, env=ENV, cwd=str(tmp_path))
     assert "Sanitizer" not in r.stderr and "runtime error" not in r.stderr, r.stderr[-4000:]
     assert r.returncode == want_rc, (r.stdout[-2000:], r.stderr[-2000:])
+
+
+def test_rows_of_bins_stay_in_range_for_atoms_outside_the_box(build_dir):
+    """The batched list build's row bounds (lammps_amd/csrc/bin_rows.h)."""
+    exe = os.path.join(build_dir, "bin_row_checks")
+    _run(["g++", "-std=c++17"] + SAN + ["-I" + os.path.join(ROOT, "lammps_amd", "csrc"),
+                                        os.path.join(HERE, "sanitize", "bin_row_checks.cpp"), "-o", exe])
+    _run([exe], env=ENV, timeout=60)
