@@ -166,8 +166,8 @@ int mdx_compute(mdx_ctx *ctx, int eflag, int vflag, double *f, double *eng_vdwl,
    of MDX_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends,
    so n <= MDX_NOALLOC_MAX_ATOMS, at most MDX_NOALLOC_MAX_BINS bins, and at
    most MDX_NOALLOC_MAX_ATOMS * MDX_NOALLOC_NEIGH_PER_ATOM / n (and `one`)
-   neighbours per atom; beyond these the call returns MDX_ERR_ARG or
-   MDX_ERR_OVERFLOW without computing.  The call allocates nothing, is
+   neighbours per atom; beyond these, or with a type outside 1..ntypes, the
+   call returns MDX_ERR_ARG or MDX_ERR_OVERFLOW and leaves f as it was.  The call allocates nothing, is
    synchronous at return, and every call on one GPU shares that GPU's
    array: calls that overlap on one GPU (from several threads or contexts)
    race. */

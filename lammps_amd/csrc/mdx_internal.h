@@ -42,8 +42,9 @@
 namespace mdx {
 
 // Build flags of one list build: kFlagInts words ([0] largest row, [4] lost
-// atom, [5] bin overflow, [8..9] 64-bit entry total), then kListSlots
-// counters of the list pass, each on a cache line of its own.
+// atom, [5] bin overflow, [6] atom type out of range, [8..9] 64-bit entry
+// total), then kListSlots counters of the list pass, each on a cache line of
+// its own.
 struct ListSlot {
   int most, pad;            // largest row the slot's workgroups saw
   unsigned long long sum;   // entries they listed

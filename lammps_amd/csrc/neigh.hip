@@ -218,6 +218,11 @@ __global__ void k_wrap_bin(NeighArgs a, double4 *__restrict__ x, int *__restrict
   int im[3] = {img & MDX_IMGMASK, (img >> 10) & MDX_IMGMASK, img >> 20};
   int ib[3];
   bool lost = false, moved = false;
+  if (p.w < 1.0) {  // a type that the caller's device array should not hold (noalloc.hip)
+    atomicOr(&dflags[6], 1);
+    p.w = 1.0;
+    moved = true;
+  }
   for (int d = 0; d < 3; d++) {
     double lo = a.lo[d], hi = a.lo[d] + a.prd[d];
     if (a.periodic[d]) {
@@ -240,7 +245,7 @@ __global__ void k_wrap_bin(NeighArgs a, double4 *__restrict__ x, int *__restrict
     ib[d] = b;
   }
   if (lost) atomicOr(&dflags[4], 1);
-  // most atoms stay inside the box between builds: store only the wrapped ones
+  // most atoms stay inside the box between builds: store only the changed ones
   if (moved) {
     p.x = c[0];
     p.y = c[1];
@@ -1353,6 +1358,10 @@ int neigh_build_finish(mdx_ctx *c, bool *regrow) {
   if (rc) return rc;
   int flags[16];
   memcpy(flags, c->bflags_host, sizeof(flags));
+  if (flags[6]) {
+    set_error("atom type out of range");
+    return MDX_ERR_ARG;
+  }
   if (flags[4]) {
     set_error("Lost atoms: an atom left a non-periodic box");
     return MDX_ERR_ARG;

@@ -64,11 +64,12 @@ std::mutex g_scratch_mu;
 unsigned char *g_scratch[kMaxDevices] = {};
 
 // caller arrays -> the shadow context's atoms, in caller order (device index
-// = caller index until the list build sorts them); types outside 1..ntypes are
-// read as type 1 so that no table is indexed out of range.  The same launch
-// clears the build's flags and bin counters (three memsets before: with the
-// copy of a flag and the launch that added the forces, 154 us per call of
-// 32,000 lj/cut atoms, now 114-119).
+// = caller index until the list build sorts them).  The same launch clears the
+// build's flags and bin counters (three memsets before: with the copy of a
+// flag and the launch that added the forces, 154 us per call of 32,000 lj/cut
+// atoms, now 114-119).  It cannot raise a flag beside that, so a type outside
+// 1..ntypes becomes 0, which the build's first kernel (k_wrap_bin) reports
+// and replaces by 1: no table is indexed out of range.
 __global__ void k_noalloc_pack(int n, int ntypes, const double *__restrict__ x, const int *__restrict__ type,
                                double4 *__restrict__ xo, double4 *__restrict__ v, int *__restrict__ tag,
                                int *__restrict__ orig, int *__restrict__ inv, int *__restrict__ image, int img0,
@@ -78,7 +79,7 @@ __global__ void k_noalloc_pack(int n, int ntypes, const double *__restrict__ x, 
   for (int k = i; k < nbins; k += gridDim.x * blockDim.x) bins[k] = 0;
   if (i >= n) return;
   const int t = type[i];
-  xo[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], t < 1 || t > ntypes ? 1.0 : (double)t);
+  xo[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], t < 1 || t > ntypes ? 0.0 : (double)t);
   v[i] = make_double4(0.0, 0.0, 0.0, 0.0);
   tag[i] = i + 1;
   orig[i] = i;

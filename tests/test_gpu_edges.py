@@ -630,3 +630,33 @@ def test_atoms_handed_over_again_give_what_a_fresh_context_gives():
             assert np.array_equal(a, b), (k, n)
         fresh.close()
     kept.close()
+
+
+@pytest.mark.parametrize("bad", [0, -3, 2, 1 << 20])
+def test_noalloc_refuses_types_out_of_range(bad):
+    """One type outside 1..ntypes in device memory: an error, the force array
+    left as it was; the context computes on afterwards."""
+    import torch
+    from lammps_amd import mdx
+    rng = np.random.default_rng(4)
+    lo, hi, x = mdx.lattice("fcc", 0.8442, "lj", (0, 0, 0), (6, 6, 6))
+    x = np.mod(x + rng.uniform(-0.05, 0.05, x.shape), hi)
+    n = len(x)
+    ctx = lj_context((0, 0, 0), hi, (1, 1, 1), x, mdx.FP64)
+    xd = torch.tensor(x, device="cuda:0")
+    t = np.ones(n, dtype=np.int32)
+    t[n - 5] = bad
+    td = torch.tensor(t, device="cuda:0")
+    fd = torch.full((n, 3), 7.0, dtype=torch.float64, device="cuda:0")
+    torch.cuda.synchronize()
+    with pytest.raises(mdx.MdxError, match="type out of range") as e:
+        ctx.compute_noalloc(n, xd.data_ptr(), td.data_ptr(), fd.data_ptr())
+    assert e.value.code == mdx.ERR_ARG
+    assert bool((fd == 7.0).all())
+    td[n - 5] = 1
+    torch.cuda.synchronize()
+    eng, _ = ctx.compute_noalloc(n, xd.data_ptr(), td.data_ptr(), fd.data_ptr())
+    out = ctx.compute(1, 1)
+    assert force_errors(fd.cpu().numpy() - 7.0, out["f"])[0] <= 1e-12
+    assert abs(eng - out["eng"]) <= 1e-12 * abs(out["eng"])
+    ctx.close()
