@@ -192,7 +192,11 @@ int mdx::prepare_ctx(mdx_ctx *c) {
       set_error("reduction partials exceed the fixed storage");
       return MDX_ERR_ARG;
     }
-    if ((rc = dev_alloc(&c->partials, (size_t)need))) return rc;
+    c->cap_partials = 0;
+    if ((rc = dev_alloc(&c->partials, (size_t)need))) {
+      c->run_setup_done = false;
+      return rc;
+    }
     c->cap_partials = need;
   }
   return MDX_OK;
@@ -479,6 +483,10 @@ int mdx_pair_eam_init(mdx_ctx *c, int ntypes, int nrho, double drho, int nr, dou
   memcpy(all.data() + nf + nrr, z2r_spline, sizeof(double) * nz);
   std::vector<float> allf(all.size());
   for (size_t k = 0; k < all.size(); k++) allf[k] = (float)all[k];
+  // no pair style until the new tables are on the device
+  c->pair_style = MDX_PAIR_NONE;
+  c->built = false;
+  c->run_setup_done = false;
   if ((rc = dev_alloc(&c->eam_tab, all.size())) || (rc = dev_alloc(&c->eam_tab_f, all.size()))) return rc;
   hipError_t e;
   if ((e = hipMemcpy(c->eam_tab, all.data(), sizeof(double) * all.size(), hipMemcpyHostToDevice)) != hipSuccess ||
@@ -733,7 +741,8 @@ int mdx_run(mdx_ctx *c, int nsteps, double dt, double ftm2v, int thermo_every, m
     set_error("mdx_run: nsteps >= 0 and dt > 0 required");
     return MDX_ERR_ARG;
   }
-  if (!c->run_setup_done && (rc = mdx_setup(c, cb, user))) return rc;
+  // set up anew too after a step whose build failed: it left no list
+  if ((!c->run_setup_done || !c->built) && (rc = mdx_setup(c, cb, user))) return rc;
   const double dtv = dt, dtf = 0.5 * dt * ftm2v;
   const long last = c->ntimestep + nsteps;
   // Fused path: the force kernel of step n also runs fix nve's final

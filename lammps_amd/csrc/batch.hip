@@ -1189,7 +1189,7 @@ struct mdx_batch {
   std::vector<RepGeom> geom_h;
   RepGeom *geom = nullptr;
   int *off_d = nullptr;
-  int total_bins = 0, bins_cap = 0;
+  int total_bins = 0, count_cap = 0, start_cap = 0;  // bins; elements of bin_count, bin_start
   double cutneigh = 0.0;  // of the current bins/list
   bool positions = false, built = false;
   // atoms
@@ -1203,7 +1203,7 @@ struct mdx_batch {
   unsigned *key = nullptr;
   int *slot = nullptr, *order = nullptr;  // arrival slots; atoms by bin in arrival order
   int *bin_count = nullptr, *bin_start = nullptr;
-  void *scan_tmp = nullptr;
+  char *scan_tmp = nullptr;
   size_t scan_bytes = 0;
   int *nbr = nullptr, *numneigh = nullptr;
   int cap = 0;
@@ -1265,6 +1265,18 @@ int dalloc(P **p, size_t count) {
   if (count == 0) count = 1;
   hipError_t e = hipMalloc((void **)p, count * sizeof(P));
   return e == hipSuccess ? MDX_OK : bfail(e, "batch allocation");
+}
+
+// *p holds at least `count` elements when this returns MDX_OK.  The capacity
+// is 0 while there is no array: after a failed allocation the next call tries
+// again, whatever it asks for.
+template <typename P, typename C>
+int grow(P **p, C *cap, size_t count) {
+  if (*p && count <= (size_t)*cap) return MDX_OK;
+  *cap = 0;
+  const int rc = dalloc(p, count);
+  if (!rc) *cap = (C)count;
+  return rc;
 }
 
 bool is_device_ptr(const void *p, int device) {
@@ -1432,21 +1444,11 @@ int run_kind(mdx_batch *b, int kind, F &&launch) {
     default: { constexpr int TP = 64; CALL; } break; \
   }
 
-int ensure_partials(mdx_batch *b, size_t doubles) {
-  if (doubles <= b->partials_cap) return MDX_OK;
-  b->partials_cap = doubles;
-  return dalloc(&b->partials, doubles);
-}
-
 // column sums of `rows` partial rows (and rowsB rows of colsB columns at partB,
 // into the columns from c0B on), left in b->sums_host when this returns
 int colsum(mdx_batch *b, int rows, int cols, const double *partB = nullptr, int rowsB = 0, int c0B = 0, int colsB = 0) {
-  const size_t need = (size_t)kColChunks * cols;
-  if (need > b->colsum_cap) {
-    int rc = dalloc(&b->colsum, need);
-    if (rc) return rc;
-    b->colsum_cap = need;
-  }
+  int rc = grow(&b->colsum, &b->colsum_cap, (size_t)kColChunks * cols);
+  if (rc) return rc;
   if ((size_t)cols > b->sums_cap) {
     if (b->sums_host) (void)hipHostFree(b->sums_host);
     b->sums_host = nullptr;
@@ -1484,7 +1486,9 @@ int build(mdx_batch *b) {
   }
   int rc;
   hipError_t e;
-  if (cutneigh != b->cutneigh || !b->bin_start) {
+  b->built = false;  // a failed build leaves no list
+  if (cutneigh != b->cutneigh) {
+    b->cutneigh = 0.0;  // until the bins for it are there
     const double binsize = 0.5 * cutneigh;
     long total = 0;
     for (int r = 0; r < b->nrep; r++) {
@@ -1509,12 +1513,9 @@ int build(mdx_batch *b) {
     b->total_bins = (int)total;
     if ((e = hipMemcpy(b->geom, b->geom_h.data(), sizeof(RepGeom) * b->nrep, hipMemcpyHostToDevice)) != hipSuccess)
       return bfail(e, "replica geometry upload");
-    if (b->total_bins + 1 > b->bins_cap) {
-      if ((rc = dalloc(&b->bin_count, b->total_bins + 1)) || (rc = dalloc(&b->bin_start, b->total_bins + 1)))
-        return rc;
-      b->bins_cap = b->total_bins + 1;
-    }
-    b->cutneigh = cutneigh;
+    if ((rc = grow(&b->bin_count, &b->count_cap, b->total_bins + 1)) ||
+        (rc = grow(&b->bin_start, &b->start_cap, b->total_bins + 1)))
+      return rc;
     // list candidates are decided on the mirror where its rounding stays well
     // inside the re-test band and the wrapping difference is a candidate's own
     // image (no atom in a stencil under two images)
@@ -1526,12 +1527,8 @@ int build(mdx_batch *b) {
     size_t need = 0;
     (void)hipcub::DeviceScan::ExclusiveSum(nullptr, need, b->bin_count, b->bin_start, b->total_bins + 1,
                                            b->stream);
-    if (need > b->scan_bytes) {
-      (void)hipFree(b->scan_tmp);
-      b->scan_tmp = nullptr;
-      if ((e = hipMalloc(&b->scan_tmp, need)) != hipSuccess) return bfail(e, "scan scratch");
-      b->scan_bytes = need;
-    }
+    if ((rc = grow(&b->scan_tmp, &b->scan_bytes, need))) return rc;
+    b->cutneigh = cutneigh;
   }
   const int n = b->n;
   if ((e = hipMemsetAsync(b->bin_count, 0, sizeof(int) * (b->total_bins + 1), b->stream)) != hipSuccess ||
@@ -1547,10 +1544,13 @@ int build(mdx_batch *b) {
                      b->order);
   hipLaunchKernelGGL(k_b_rank_permute, dim3((n + 255) / 256), dim3(256), 0, b->stream, n, b->order, b->key,
                      b->bin_start, b->xw, b->rep_c, b->geom, b->x, b->xq, b->rep, b->orig, b->inv);
-  if (b->cap == 0) {
-    b->cap = 96;
-    if ((rc = dalloc(&b->nbr, (size_t)b->cap * n))) return rc;
-  }
+  auto alloc_rows = [&](int cap) {  // cap stays 0 without a list
+    b->cap = 0;
+    rc = dalloc(&b->nbr, (size_t)cap * n);
+    if (!rc) b->cap = cap;
+    return rc;
+  };
+  if (b->cap == 0 && alloc_rows(96)) return rc;
   const double cutneighsq = cutneigh * cutneigh;
   const float c_lo = (float)(cutneighsq * (1.0 - kBuildBand)), c_hi = (float)(cutneighsq * (1.0 + kBuildBand)),
               reach = (float)(cutneighsq * (1.0 + 1e-4));
@@ -1586,8 +1586,7 @@ int build(mdx_batch *b) {
       b->eam_rho_prec = -1;
       return MDX_OK;
     }
-    b->cap = (fl[0] + 16 + 15) / 16 * 16;
-    if ((rc = dalloc(&b->nbr, (size_t)b->cap * n))) return rc;
+    if (alloc_rows((fl[0] + 16 + 15) / 16 * 16)) return rc;
   }
   set_error("neighbour list capacity did not converge");
   return MDX_ERR_OVERFLOW;
@@ -1978,7 +1977,7 @@ int mdx_batch_lj_vjp(mdx_batch *b, const double *gf, double *geps, double *gsigm
   };
   // partial rows for the largest grid any candidate can use
   const long maxgrid = (long)kPartialBlocksPerCU * b->num_cu;
-  if ((rc = ensure_partials(b, (size_t)maxgrid * 2 * nt1 * nt1))) return rc;
+  if ((rc = grow(&b->partials, &b->partials_cap, (size_t)maxgrid * 2 * nt1 * nt1))) return rc;
   if ((rc = run_kind(b, MDX_BK_LJ_VJP, launch))) return rc;
   const int cols = nt1 * nt1;
   if ((rc = colsum(b, grid_used, 2 * cols))) return rc;
@@ -2016,12 +2015,12 @@ int mdx_batch_eam_init(mdx_batch *b, int nrho, double drho, int nr, double dr, d
     kf[2 * q] = make_float4((float)c[0], (float)c[1], (float)c[2], 0.0f);
     kf[2 * q + 1] = make_float4((float)c[3], (float)c[4], (float)c[5], (float)c[6]);
   }
-  if (b->et.nrho != nrho || !b->frho_d) {
-    if ((rc = dalloc(&b->frho_d, sf.size()))) return rc;
-  }
-  if (b->et.nr != nr || !b->knots_d) {
-    if ((rc = dalloc(&b->knots_d, kd.size())) || (rc = dalloc(&b->knots_f, kf.size()))) return rc;
-  }
+  // no pair style until the new tables are on the device
+  const bool same_nrho = b->et.nrho == nrho, same_nr = b->et.nr == nr;
+  if (b->pair == MDX_PAIR_EAM) b->pair = MDX_PAIR_NONE;
+  b->et.nrho = b->et.nr = 0;
+  if (!same_nrho && (rc = dalloc(&b->frho_d, sf.size()))) return rc;
+  if (!same_nr && ((rc = dalloc(&b->knots_d, kd.size())) || (rc = dalloc(&b->knots_f, kf.size())))) return rc;
   if ((rc = upload(b->frho_d, sf.data(), sizeof(double) * sf.size())) ||
       (rc = upload(b->knots_d, kd.data(), sizeof(double4) * kd.size())) ||
       (rc = upload(b->knots_f, kf.data(), sizeof(float4) * kf.size())))
@@ -2139,7 +2138,7 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
   const bool tlA = tabA + gfA + cA * setA <= (size_t)b->lds_max;
   const size_t shA = (tlA ? tabA : 0) + gfA + cA * setA, shB = cB * setB;
   const long maxgrid = (long)kPartialBlocksPerCU * b->num_cu;
-  if ((rc = ensure_partials(b, (size_t)maxgrid * (P + 4 * kn)))) return rc;
+  if ((rc = grow(&b->partials, &b->partials_cap, (size_t)maxgrid * (P + 4 * kn)))) return rc;
   int gA = 0, gB = 0;
   auto launchA = [&](const Tune &t) {
     const int G = persistent_grid(b, t, true);

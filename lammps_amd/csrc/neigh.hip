@@ -1207,15 +1207,18 @@ int neigh_setup_grid(mdx_ctx *c) {
     }
     (void)hipFree(c->bin_count);
     (void)hipFree(c->bin_start);
-    c->cap_bins = c->nbins + 1;
-    if (hipMalloc(&c->bin_count, sizeof(int) * c->cap_bins) != hipSuccess ||
-        hipMalloc(&c->bin_start, sizeof(int) * c->cap_bins) != hipSuccess) {
+    (void)hipFree(c->scan_tmp);
+    c->bin_count = c->bin_start = nullptr;
+    c->scan_tmp = nullptr;
+    c->scan_tmp_bytes = 0;
+    c->cap_bins = 0;  // until both arrays are there: the next call tries again
+    c->built = c->run_setup_done = false;
+    if (hipMalloc(&c->bin_count, sizeof(int) * (c->nbins + 1)) != hipSuccess ||
+        hipMalloc(&c->bin_start, sizeof(int) * (c->nbins + 1)) != hipSuccess) {
       set_error("Insufficient memory on accelerator (bins)");
       return MDX_ERR_NOMEM;
     }
-    (void)hipFree(c->scan_tmp);
-    c->scan_tmp = nullptr;
-    c->scan_tmp_bytes = 0;
+    c->cap_bins = c->nbins + 1;
   }
   a.ntypes1 = c->ntypes + 1;
   c->bins_dirty = true;  // a new grid starts from cleared counters
@@ -1300,11 +1303,13 @@ int neigh_build_launch(mdx_ctx *c) {
         return MDX_ERR_ARG;
       }
       (void)hipFree(c->scan_tmp);
-      c->scan_tmp_bytes = need;
+      c->scan_tmp = nullptr;
+      c->scan_tmp_bytes = 0;
       if (hipMalloc(&c->scan_tmp, need) != hipSuccess) {
         set_error("Insufficient memory on accelerator (scan)");
         return MDX_ERR_NOMEM;
       }
+      c->scan_tmp_bytes = need;
     }
     e = hipcub::DeviceScan::ExclusiveSum(c->scan_tmp, need, c->bin_count, c->bin_start, c->nbins + 1, c->stream);
     if (e != hipSuccess) return hip_fail(e, "bin scan");
