@@ -95,10 +95,12 @@ struct EAMArgs {
 };
 
 // sqrt(x) and 1/sqrt(x) in FP64 to about an ulp: the hardware reciprocal
-// square root refined in coupled steps, half the instructions of sqrt and a
-// divide
+// square root refined by Goldschmidt's coupled iteration, half the
+// instructions of sqrt and a divide.  The bound on the estimate (above that of
+// every x > 0) makes x = 0 give 0 and, as the last step overflows, infinity;
+// the products of 0 with an infinite estimate would be NaN.
 __device__ __forceinline__ void sqrt_and_inverse(double x, double &r, double &ri) {
-  const double y = __builtin_amdgcn_rsq(x);
+  const double y = fmin(__builtin_amdgcn_rsq(x), 1e308);
   double g = x * y, h = 0.5 * y;
   const double e = fma(-h, g, 0.5);
   g = fma(g, e, g);

@@ -388,3 +388,29 @@ def test_atom_far_outside_a_closed_box_is_reported(d, far):
     want = sum(int(np.sum(np.sum((q[:, None] - q[None]) ** 2, -1) < 6.25)) - len(q) for q in (x[:400], x[400:]))
     assert total == want
     b.close()
+
+
+@pytest.mark.parametrize("tpa,nknots", [(4, 64), (16, 64), (4, 660), (16, 660)])
+def test_coincident_eam_atoms_have_the_density_of_zero_separation(tpa, nknots):
+    """Two atoms of a cluster in one place (FP64, tables in LDS and not):
+    densities and the forces on all other atoms are the oracle's."""
+    pot = W.synthetic_knots(nknots)
+    rng = np.random.default_rng(nknots)
+    x = W.fcc_cluster(331) + rng.normal(scale=0.1, size=(331, 3))
+    x[200] = x[17]
+    geo = ([331], [x.min(0) - 2.0], [x.max(0) + 2.0], [[0, 0, 0]], 1, np.ones(331, np.int32))
+    ref = FR.Batch(*geo, x)
+    ref.eam_set(pot["drho"], pot["dr"], pot["cut"], pot["frho"], pot["rhor"], pot["z2r"])
+    f_ref, _, rho_ref, fp_ref = ref.eam_forces()
+    b = B.Batch(*geo)
+    b.set_positions(x)
+    b.eam_init(pot["drho"], pot["dr"], pot["cut"], pot["frho"], pot["rhor"], pot["z2r"])
+    for kind in (B.BK_EAM_RHO, B.BK_EAM_FORCE):
+        b.set_launch(kind, 256, tpa, 0)
+    f, _, rho, fp = b.eam_forces(rho_fp=True)
+    assert np.isfinite(rho_ref).all()
+    np.testing.assert_allclose(rho, rho_ref, rtol=1e-11)
+    np.testing.assert_allclose(fp, fp_ref, rtol=0, atol=1e-10 * np.abs(fp_ref).max())
+    rest = np.setdiff1d(np.arange(331), [17, 200])
+    assert force_errors(f[rest], f_ref[rest])[0] <= 1e-11
+    b.close()

@@ -660,3 +660,53 @@ def test_noalloc_refuses_types_out_of_range(bad):
     assert force_errors(fd.cpu().numpy() - 7.0, out["f"])[0] <= 1e-12
     assert abs(eng - out["eng"]) <= 1e-12 * abs(out["eng"])
     ctx.close()
+
+
+def copper(cells, seed, amp=0.1):
+    """fcc copper with atoms displaced by up to amp: box and wrapped positions."""
+    from lammps_amd import mdx
+    lo, hi, x = mdx.lattice("fcc", 3.615, "metal", (0, 0, 0), cells)
+    x = x + np.random.default_rng(seed).uniform(-amp, amp, x.shape)
+    return np.asarray(lo), np.asarray(hi), np.mod(x, hi)
+
+
+def eam_pair(path, hi, x, skin=1.0):
+    """One system of one-element eam atoms in the oracle (set up) and in a context (FP64)."""
+    from lammps_amd import mdx
+    ref = M.Ref(M.METAL)
+    ref.box((0, 0, 0), hi)
+    ref.add_atoms(x, np.ones(len(x), dtype=np.int32))
+    ref.pair_eam(path)
+    ref.neighbor(skin)
+    ref.setup()
+    ref.compute(3, 5)
+    ctx = mdx.Context(0)
+    ctx.set_box((0, 0, 0), hi, (1, 1, 1))
+    ctx.set_atoms(x, np.ones(len(x), dtype=np.int32), np.array([0.0, 63.55]))
+    mdx.eam_context_tables(ctx, path)
+    ctx.neigh_modify(skin)
+    return ref, ctx
+
+
+@pytest.mark.parametrize("tpa", [4, 8, 16, 32])
+def test_coincident_eam_atoms_have_the_density_of_zero_separation(tpa):
+    """Two atoms in one place (FP64, spline tables in LDS and not): densities,
+    and the forces and energies of all other atoms, are the oracle's; the
+    pair's energy is infinite there and here."""
+    from gpu_helpers import CU_U3
+    lo, hi, x = copper((5, 5, 4), 11)
+    x[137] = x[21]
+    ref, ctx = eam_pair(CU_U3, hi, x)
+    ctx.set_launch(256, tpa)
+    out = ctx.compute(3, 5, peratom=True)
+    rho, fp = ctx.eam_rho_fp()
+    rho_ref, fp_ref = ref.eam_rho_fp()
+    assert np.isfinite(rho_ref).all()
+    np.testing.assert_allclose(rho, rho_ref, rtol=1e-11)
+    np.testing.assert_allclose(fp, fp_ref, rtol=0, atol=1e-10 * np.abs(fp_ref).max())
+    rest = np.setdiff1d(np.arange(len(x)), [21, 137])
+    assert force_errors(out["f"][rest], ref.state()[2][rest])[0] <= 1e-11
+    ea = ref.peratom()[0]
+    np.testing.assert_allclose(out["eatom"][rest], ea[rest], rtol=0, atol=1e-10 * np.abs(ea[rest]).max())
+    assert ref.energy_virial()[0] == np.inf and out["eng"] == np.inf
+    ctx.close()
