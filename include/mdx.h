@@ -212,7 +212,9 @@ int mdx_set_profiling(mdx_ctx *ctx, int on);
 int mdx_copy_bandwidth(mdx_ctx *ctx, long nbytes, int iters, double *gbs);
 
 /* Kernel shape of the pair kernels, set by the autotuner (0 = library
-   default, which depends on the atom count): block = threads per workgroup (64..256, multiple of 64), tpa =
+   default, which depends on the atom count): block = threads per workgroup
+   (64..256, multiple of 64, or 512, which the FP64 kernels of one-element eam
+   take while their tables fit LDS and the others run as 256), tpa =
    threads per atom (1, 2, 4, 8, 16 or 32; the `threads_per_atom` keyword of
    the reference's `package gpu`, src/GPU/fix_gpu.cpp:112-150). */
 int mdx_set_launch(mdx_ctx *ctx, int block, int tpa);

@@ -890,8 +890,8 @@ int mdx_get_stats(mdx_ctx *c, mdx_stats *out) {
 int mdx_set_launch(mdx_ctx *c, int block, int tpa) {
   int rc = check_ctx(c);
   if (rc) return rc;
-  if (block != 0 && (block < 64 || block > 256 || block % 64 != 0)) {
-    set_error("block must be a multiple of 64 in [64, 256]");
+  if (block != 0 && block != 512 && (block < 64 || block > 256 || block % 64 != 0)) {
+    set_error("block must be a multiple of 64 in [64, 256], or 512");
     return MDX_ERR_ARG;
   }
   if (tpa != 0 && tpa != 1 && tpa != 2 && tpa != 4 && tpa != 8 && tpa != 16 && tpa != 32) {

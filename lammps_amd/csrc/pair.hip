@@ -932,6 +932,8 @@ Launch pair_launch(const mdx_ctx *c) {
     const bool tables = c->pair_style == MDX_PAIR_EAM && eam_lds_tables(c, l.tpa);
     l.block = tables ? (mixed || c->n <= 10000 ? 256 : 512) : (long)c->n * l.tpa < 1024L * 256 ? 64 : 256;
   }
+  // a shape that was set: only the FP64 eam kernels with LDS tables take 512
+  if (l.block > 256 && (mixed || c->pair_style != MDX_PAIR_EAM || !eam_lds_tables(c, l.tpa))) l.block = 256;
   return l;
 }
 

@@ -710,3 +710,66 @@ def test_coincident_eam_atoms_have_the_density_of_zero_separation(tpa):
     np.testing.assert_allclose(out["eatom"][rest], ea[rest], rtol=0, atol=1e-10 * np.abs(ea[rest]).max())
     assert ref.energy_virial()[0] == np.inf and out["eng"] == np.inf
     ctx.close()
+
+
+@pytest.mark.parametrize("style,cells", [("lj", 5), ("lj", 15), ("lj", 23), ("eam", 6), ("eam", 14), ("eam", 22)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_default_launch_shape_can_be_set_by_value(style, cells, prec):
+    """What get_launch reports can be handed to set_launch and is then in
+    force, and gives the same forces; other blocks above 256 stay refused."""
+    from gpu_helpers import CU_U3
+    from lammps_amd import mdx
+    if style == "lj":
+        lo, hi, x = mdx.lattice("fcc", 0.8442, "lj", (0, 0, 0), (cells,) * 3)
+        ctx = lj_context((0, 0, 0), hi, (1, 1, 1), np.mod(x + 0.01, hi), prec)
+    else:
+        lo, hi, x = copper((cells,) * 3, 2)
+        ctx = mdx.Context(0)
+        ctx.set_box((0, 0, 0), hi, (1, 1, 1))
+        ctx.set_atoms(x, np.ones(len(x), dtype=np.int32), np.array([0.0, 63.55]))
+        mdx.eam_context_tables(ctx, CU_U3)
+        ctx.precision(prec)
+        ctx.neigh_modify(1.0)
+    f = ctx.compute(0, 0)["f"]
+    shape = ctx.get_launch()
+    ctx.set_launch(**shape)
+    assert ctx.get_launch() == shape
+    assert np.array_equal(ctx.compute(0, 0)["f"], f)
+    for block in (320, 384, 448, 576, 1024, 96):
+        with pytest.raises(mdx.MdxError):
+            ctx.set_launch(block, 8)
+    assert ctx.get_launch() == shape
+    # 512 threads are the FP64 eam kernels' with tables in LDS; others run 256
+    ctx.set_launch(512, 8)
+    assert ctx.get_launch() == dict(block=512 if style == "eam" and prec == mdx.FP64 else 256, tpa=8)
+    ctx.set_launch(256, 8)
+    want = ctx.compute(0, 0)["f"]
+    ctx.set_launch(512, 8)
+    assert np.array_equal(ctx.compute(0, 0)["f"], want)
+    tuned = ctx.autotune(2)
+    ctx.set_launch(**tuned)
+    assert ctx.get_launch() == tuned
+    ctx.close()
+
+
+@pytest.mark.parametrize("prec,nr", [("fp64", 799), ("fp64", 800), ("mixed", 1023), ("mixed", 1024)])
+@pytest.mark.parametrize("tpa", [4, 8, 16])
+def test_eam_tables_on_both_sides_of_the_lds_limits(prec, nr, tpa, tmp_path):
+    """One-element tables of the largest size that goes to LDS (800 knots in
+    FP64, 1,024 mixed, the unused knot 0 included) and one knot more: forces,
+    per-atom energies and virials are the oracle's."""
+    from lammps_amd import mdx
+    path = str(tmp_path / "cu.eam")
+    mdx.write_synthetic_funcfl(path, nr=nr, dr=4.99 / (nr - 1))
+    lo, hi, x = copper((6, 5, 5), nr)
+    ref, ctx = eam_pair(path, hi, x)
+    ctx.precision(mdx.FP64 if prec == "fp64" else mdx.MIXED)
+    ea, va = ref.peratom()
+    ftol, etol = (1e-11, 1e-10) if prec == "fp64" else (1e-5, 1e-5)
+    for block in (256, 512):
+        ctx.set_launch(block, tpa)
+        out = ctx.compute(3, 5, peratom=True)
+        assert force_errors(out["f"], ref.state()[2])[0] <= ftol
+        np.testing.assert_allclose(out["eatom"], ea, rtol=0, atol=etol * np.abs(ea).max())
+        np.testing.assert_allclose(out["vatom"], va, rtol=0, atol=etol * np.abs(va).max())
+    ctx.close()
