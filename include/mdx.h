@@ -221,8 +221,9 @@ int mdx_set_launch(mdx_ctx *ctx, int block, int tpa);
 int mdx_get_launch(mdx_ctx *ctx, int *block, int *tpa);
 /* Autotuner (the role of `package gpu ... tpa` chosen by hand in the
    reference, src/GPU/fix_gpu.cpp:112-150): times the force kernel of the
-   current configuration for threads per atom {4, 8, 16} x block {128, 256},
-   `reps` launches each; keeps the fastest and recomputes the forces with it. */
+   current configuration in the default shape and for threads per atom
+   {4, 8, 16} x block {128, 256}, `reps` launches each; keeps the fastest and
+   recomputes the forces with it. */
 int mdx_autotune(mdx_ctx *ctx, int reps);
 /* Timing probe (no counterpart in the reference): the force kernel of a
    non-thermo step of mdx_run (with fix nve fused: force + final integrate +

@@ -91,12 +91,13 @@ int mdx_batch_eam_vjp(mdx_batch *b, const double *gf, double *g_frho, double *g_
    per atom (1..64, power of two), grid (blocks; 0 = one block per
    atom tile).  Kernels loop over their share of atoms, so any grid is valid.
    A kind that was neither set nor tuned takes a shape for the batch's size;
-   the list build always takes its own. */
+   the list build always takes its own, which get_launch reports. */
 int mdx_batch_set_launch(mdx_batch *b, int kind, int block, int tpa, int grid);
 int mdx_batch_get_launch(mdx_batch *b, int kind, int *block, int *tpa, int *grid);
-/* Autotuner: when on, the next call of each kernel kind times a set of
-   (threads per atom, block, grid) candidates on the real inputs, keeps the
-   fastest and finishes with it. */
+/* Autotuner: when on, the next call of each kernel kind but the list build
+   times the default shape (unless it has more than 16 threads per atom) and
+   a set of (threads per atom, block, grid) candidates on the real inputs,
+   keeps the fastest and finishes with it. */
 int mdx_batch_autotune(mdx_batch *b, int on);
 /* accumulated device time (ms) and launch count of a kernel kind */
 int mdx_batch_kernel_time(mdx_batch *b, int kind, double *ms, long *launches);

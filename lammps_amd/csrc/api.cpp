@@ -912,9 +912,6 @@ int mdx_get_launch(mdx_ctx *c, int *block, int *tpa) {
   return MDX_OK;
 }
 
-// Times the pair kernels (no energy/virial) on the current list for each
-// (threads per atom, block) candidate, keeps the fastest, then recomputes
-// the forces with it so f is that of the chosen shape.
 int mdx_time_step_kernel(mdx_ctx *c, int reps, double dt, double ftm2v, double *ms) {
   int rc = check_ctx(c);
   if (rc) return rc;
@@ -974,6 +971,9 @@ int mdx_time_step_kernel(mdx_ctx *c, int reps, double dt, double ftm2v, double *
   return MDX_OK;
 }
 
+// Times the pair kernels (no energy/virial) on the current list for the
+// default shape and each (threads per atom, block) candidate, keeps the
+// fastest, then recomputes the forces with it so f is that of the chosen shape.
 int mdx_autotune(mdx_ctx *c, int reps) {
   int rc = check_ctx(c);
   if (rc) return rc;
@@ -1016,23 +1016,33 @@ int mdx_autotune(mdx_ctx *c, int reps) {
     ig.trig_dev = c->trig_dev;
     igp = &ig;
   }
+  // the default of this size first: another shape has to be faster than it
+  c->launch = mdx::Launch{};
+  std::vector<mdx::Launch> shapes = {pair_launch(c)};
   for (int tpa : {4, 8, 16})
     for (int block : {128, 256}) {
-      c->launch.tpa = tpa;
-      c->launch.block = block;
-      if ((rc = pair_compute(c, 0, igp))) break;  // warm-up
-      e = hipEventRecord(e0, c->stream);
-      for (int r = 0; r < reps && !rc && e == hipSuccess; r++) rc = pair_compute(c, 0, igp);
-      if (!rc && e == hipSuccess) e = hipEventRecord(e1, c->stream);
-      if (!rc && e == hipSuccess) e = hipEventSynchronize(e1);
-      float ms = 0.0f;
-      if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-      if (rc || e != hipSuccess) break;
-      if (ms < best) {
-        best = ms;
-        pick = c->launch;
-      }
+      mdx::Launch l;
+      l.tpa = tpa;
+      l.block = block;
+      shapes.push_back(l);
     }
+  rc = pair_compute(c, 0, igp);  // clocks and caches, before the first shape
+  for (const mdx::Launch &l : shapes) {
+    if (rc) break;
+    c->launch = l;
+    if ((rc = pair_compute(c, 0, igp))) break;  // warm-up
+    e = hipEventRecord(e0, c->stream);
+    for (int r = 0; r < reps && !rc && e == hipSuccess; r++) rc = pair_compute(c, 0, igp);
+    if (!rc && e == hipSuccess) e = hipEventRecord(e1, c->stream);
+    if (!rc && e == hipSuccess) e = hipEventSynchronize(e1);
+    float ms = 0.0f;
+    if (!rc && e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
+    if (rc || e != hipSuccess) break;
+    if (ms < best) {
+      best = ms;
+      pick = l;
+    }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc || e != hipSuccess) {

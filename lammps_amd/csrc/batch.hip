@@ -1319,7 +1319,20 @@ Tune default_tune(const mdx_batch *b, int kind) {
   return t;
 }
 
-Tune tune_of(const mdx_batch *b, int kind) { return b->tune[kind].tpa ? b->tune[kind] : default_tune(b, kind); }
+// the list build's own shape, whatever is set for its kind
+Tune build_tune(int n) {
+  constexpr int per = kBuildBlock / kBuildLanes;
+  Tune t;
+  t.block = kBuildBlock;
+  t.tpa = kBuildLanes;
+  t.grid = std::min(xcd_grid((n + per - 1) / per), kBuildGrid);
+  return t;
+}
+
+Tune tune_of(const mdx_batch *b, int kind) {
+  if (kind == MDX_BK_BUILD) return build_tune(b->n);
+  return b->tune[kind].tpa ? b->tune[kind] : default_tune(b, kind);
+}
 
 // adds the times of the launches since the last call to kms; waits for them
 int resolve_times(mdx_batch *b) {
@@ -1394,9 +1407,13 @@ int persistent_grid(mdx_batch *b, const Tune &t, bool partial_rows = false) {
   return (int)G;
 }
 
-// candidates for the autotuner
-std::vector<Tune> candidates(mdx_batch *b) {
+// candidates for the autotuner, 2 to 16 lanes per atom: the default first
+// where it is one of them (lj above 10,000 atoms, eam always), which the others
+// have to beat
+std::vector<Tune> candidates(const mdx_batch *b, int kind) {
   std::vector<Tune> v;
+  const Tune dflt = default_tune(b, kind);
+  if (dflt.tpa <= 16) v.push_back(dflt);
   for (int tpa : {2, 4, 8, 16})
     for (int block : {128, 256, 512})
       for (int per_cu : {2, 4, 8, 0}) {
@@ -1416,7 +1433,7 @@ int run_kind(mdx_batch *b, int kind, F &&launch) {
   if (b->autotune && !b->tuned[kind]) {
     float best = 1e30f;
     Tune bt = tune_of(b, kind);
-    for (const Tune &t : candidates(b)) {
+    for (const Tune &t : candidates(b, kind)) {
       float ms = 0.0f;
       for (int rep = 0; rep < 2; rep++) {  // second timing counts (warm caches)
         int rc = timed(b, kind, t, launch, &ms);
@@ -1557,9 +1574,8 @@ int build(mdx_batch *b) {
   for (int attempt = 0; attempt < 4; attempt++) {
     if (attempt > 0 && (e = hipMemsetAsync(b->dflags + kFlagInts, 0, sizeof(ListSlot) * kListSlots, b->stream)) != hipSuccess)
       return bfail(e, "build flags");
-    auto launch = [&](const Tune &) {
-      constexpr int per = kBuildBlock / kBuildLanes;
-      const int G = std::min(xcd_grid((n + per - 1) / per), kBuildGrid);
+    auto launch = [&](const Tune &t) {
+      const int G = t.grid;
       auto go = [&](auto kernel) {
         BATCH_LAUNCH(kernel, G, kBuildBlock, 0, n, b->x, b->xq, b->rep, b->geom, b->bin_start, cutneighsq, c_lo, c_hi,
                      reach, b->cap, b->nbr, b->numneigh, reinterpret_cast<ListSlot *>(b->dflags + kFlagInts));
@@ -1567,7 +1583,7 @@ int build(mdx_batch *b) {
       if (b->mirror_ok) go(k_b_build<true>);
       else go(k_b_build<false>);
     };
-    if ((rc = timed(b, MDX_BK_BUILD, Tune{}, launch))) return rc;
+    if ((rc = timed(b, MDX_BK_BUILD, build_tune(n), launch))) return rc;
     b->flag_serial = b->flag_serial == 0x7fffffff ? 1 : b->flag_serial + 1;
     launch_build_flags(b->stream, b->dflags, b->flags_host, b->flag_serial);
     int fl[kFlagInts], got;

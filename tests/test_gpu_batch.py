@@ -414,3 +414,19 @@ def test_coincident_eam_atoms_have_the_density_of_zero_separation(tpa, nknots):
     rest = np.setdiff1d(np.arange(331), [17, 200])
     assert force_errors(f[rest], f_ref[rest])[0] <= 1e-11
     b.close()
+
+
+def test_build_kind_reports_the_shape_it_runs():
+    """The list build takes its own launch shape whatever is set for it."""
+    natoms, lo, hi, per, t, x = ka_batch_inputs(2, 8)
+    b = B.Batch(natoms, lo, hi, per, 2, t)
+    b.set_positions(x)
+    b.lj_init(*ka_tables())
+    shape = b.get_launch(B.BK_BUILD)
+    assert shape["block"] == 256 and shape["tpa"] == 32 and shape["grid"] == 128
+    b.set_launch(B.BK_BUILD, 512, 4, 7)
+    assert b.get_launch(B.BK_BUILD) == shape
+    b.autotune(True)
+    b.lj_forces()
+    assert b.get_launch(B.BK_BUILD) == shape
+    b.close()
