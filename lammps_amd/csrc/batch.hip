@@ -9,7 +9,9 @@
 // holds the neighbour index (bits 0-26) and its periodic image code
 // 9(sx+1) + 3(sy+1) + (sz+1) (bits 27-31).  The ghost coordinate is
 // x_j + s*prd rounded once, as CommBrick::borders forms it
-// (atom_vec_atomic.cpp:290-297).
+// (atom_vec_atomic.cpp:290-297): whether a pair lies inside a cutoff is
+// decided by the FP64 distance to it, in each atom's row by itself.  Away
+// from the cutoff the passes use cheaper separations (kQBand).
 //
 // Every pair kernel is persistent: block b takes a contiguous chunk of
 // atoms (chunks ordered so each XCD gets a contiguous eighth) and loops over
@@ -60,10 +62,11 @@ struct RepGeom {
   int bin_off;
 };
 
-// a pair within kQBand of the cutoff (relative, on rsq) from the fixed-point
-// separation is re-tested on the FP64 positions, so the cutoff decision is
-// the FP64 one
+// A pair within kQBand of the cutoff (relative, on rsq), by the fixed-point or
+// the nearest-image separation, is tested again on the FP64 positions with its
+// image (image_rsq).  kInner: the band's lower end over its upper end.
 constexpr double kQBand = 2e-6;
+constexpr double kInner = 1.0 - 2.0 * kQBand;
 
 __device__ __forceinline__ int4 quantize_rep(const RepGeom &g, const double4 &p) {
   return make_int4((int)(unsigned)(long long)rint((p.x - g.lo[0]) * g.qscale[0]),
@@ -111,6 +114,34 @@ __device__ __forceinline__ void shift_of(int code, double &sx, double &sy, doubl
   sx = (double)(code / 9 - 1);
   sy = (double)((code / 3) % 3 - 1);
   sz = (double)(code % 3 - 1);
+}
+
+// the squared distance from a to the ghost of b under an image code, as the
+// reference forms it
+__device__ __forceinline__ double image_rsq(const double4 &a, const double4 &b, int code, const RepGeom &g) {
+  double sx, sy, sz;
+  shift_of(code, sx, sy, sz);
+  const double ex = a.x - (b.x + sx * g.prd[0]), ey = a.y - (b.y + sy * g.prd[1]), ez = a.z - (b.z + sz * g.prd[2]);
+  return ex * ex + ey * ey + ez * ez;
+}
+// the code under which b sees a's image
+__device__ __forceinline__ int reverse_code(int code) { return 26 - code; }
+
+// A pair's separation rsq lies below chi = cutsq (1 + kQBand): whether it lies
+// inside cutsq in the row of a.
+__device__ __forceinline__ bool row_inside(double rsq, double chi, double cutsq, const double4 &a, const double4 &b,
+                                           int ent, const RepGeom &g) {
+  return rsq < chi * kInner || image_rsq(a, b, (int)((unsigned)ent >> MDX_IDX_BITS), g) < cutsq;
+}
+// The same for a pass that takes a pair once, from one of its two rows: at the
+// cutoff the rounding of the two ghosts can put it into one row's sum only.
+struct PairRows {
+  bool here, there;  // inside in the row of a, in that of b
+};
+__device__ __forceinline__ PairRows pair_rows(const double4 &a, const double4 &b, double cutsq, int ent,
+                                              const RepGeom &g) {
+  const int code = (int)((unsigned)ent >> MDX_IDX_BITS);
+  return {image_rsq(a, b, code, g) < cutsq, image_rsq(b, a, reverse_code(code), g) < cutsq};
 }
 
 __device__ __forceinline__ int local_bin(const RepGeom &g, double x, int d) {
@@ -190,7 +221,9 @@ __global__ void k_b_rank_permute(int n, const int *__restrict__ tmp, const unsig
 // tested in FP32; one within kBuildBand of the cutoff is re-tested on the
 // FP64 positions with its image, so the list is the FP64 test's (the host
 // checks that the mirror is fine enough and that no stencil holds an atom
-// under two images).  The one-loop-per-bin build that this replaces read 250
+// under two images).  A pair on the cutoff that the rounding of its two ghosts
+// puts into one row only is listed in both: the force passes decide each row
+// again, the gradient passes need it in the row they take it from.  The one-loop-per-bin build that this replaces read 250
 // bin starts per atom one after the other and counted rows in two words by
 // atomics: 962 us at 96 x 1,331 atoms, 1.90 ms at 64 x 8,000, 7.32 ms for
 // 512 clusters of 1.33 M atoms.
@@ -319,16 +352,16 @@ __global__ __launch_bounds__(kBuildBlock, 5) void k_b_build(int n, const double4
             keep = keep && rq <= c_hi;
           }
           if (test64) {
-            double sx, sy, sz;
-            shift_of((int)((unsigned)e[u] >> MDX_IDX_BITS), sx, sy, sz);
+            const int code = (int)((unsigned)e[u] >> MDX_IDX_BITS);
             double4 pi = xi, pj = Q ? xi : xj[Q ? 0 : u];
             if constexpr (Q) {
               pi = x[ii];
               pj = gather_x(x, e[u]);
             }
-            const double ex = pi.x - (pj.x + sx * g.prd[0]), ey = pi.y - (pj.y + sy * g.prd[1]),
-                         ez = pi.z - (pj.z + sz * g.prd[2]);
-            keep = ex * ex + ey * ey + ez * ez < cutneighsq;
+            const double rsq = image_rsq(pi, pj, code, g);
+            keep = rsq < cutneighsq;
+            // a pair on the cutoff that the other row holds
+            if (!keep && rsq < cutneighsq * (1.0 + kBuildBand)) keep = image_rsq(pj, pi, reverse_code(code), g) < cutneighsq;
           }
           const unsigned long long m = __ballot(keep) & gmask;
           if (keep) {
@@ -427,6 +460,12 @@ struct RowWalk {
 // (periodic boxes are at least two cutoffs wide, so it is the list's)
 __device__ __forceinline__ double nearest(double d, double prd, double iprd) { return fma(-prd, rint(d * iprd), d); }
 
+// (G_i - G_j) . del of a pair on the cutoff: each row's share if it is inside there
+__device__ __forceinline__ double edge_factor(const PairRows &in, const double4 &gi, const double4 &gj, double dx,
+                                              double dy, double dz) {
+  return (in.here ? gi.x * dx + gi.y * dy + gi.z * dz : 0.0) - (in.there ? gj.x * dx + gj.y * dy + gj.z * dz : 0.0);
+}
+
 // ---------------------------------------------------------------- lj/cut
 
 // MIXED: neighbours are read from the fixed-point mirror (16 B instead of
@@ -441,13 +480,13 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
                                                const int *__restrict__ numneigh, int cap,
                                                const double *__restrict__ tab, ForceOut out) {
   __shared__ double s_tab[T_N * kNT];
-  __shared__ double s_qlo[MIXED ? kNT : 1], s_qhi[MIXED ? kNT : 1];
+  __shared__ double s_qlo[MIXED ? kNT : 1], s_qhi[kNT];
   __shared__ float s_f[MIXED ? 4 * kNT : 1];
   for (int k = threadIdx.x; k < T_N * kNT; k += blockDim.x) s_tab[k] = tab[k];
+  for (int k = threadIdx.x; k < kNT; k += blockDim.x) s_qhi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
   if (MIXED)
     for (int k = threadIdx.x; k < kNT; k += blockDim.x) {
       s_qlo[k] = tab[T_CUTSQ * kNT + k] * (1.0 - kQBand);
-      s_qhi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
       s_f[k] = (float)tab[T_LJ1 * kNT + k];
       s_f[kNT + k] = (float)tab[T_LJ2 * kNT + k];
       s_f[2 * kNT + k] = (float)tab[T_LJ3 * kNT + k];
@@ -490,11 +529,8 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
           const int t = ti * nt1 + qj[u].w;
           bool inside = rsq < s_qlo[t];
           if (!inside && rsq < s_qhi[t]) {
-            double sx, sy, sz;
-            shift_of((unsigned)ent[u] >> MDX_IDX_BITS, sx, sy, sz);
-            const double4 xj = x[ent[u] & MDX_IDX_MASK];
-            const double ex = xi.x - (xj.x + sx * px), ey = xi.y - (xj.y + sy * py), ez = xi.z - (xj.z + sz * pz);
-            inside = ex * ex + ey * ey + ez * ez < s_tab[T_CUTSQ * kNT + t];
+            inside = image_rsq(xi, x[ent[u] & MDX_IDX_MASK], (int)((unsigned)ent[u] >> MDX_IDX_BITS), g) <
+                     s_tab[T_CUTSQ * kNT + t];
           }
           if (inside) {
             const float r2inv = __builtin_amdgcn_rcpf((float)rsq);
@@ -523,7 +559,8 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
                        dz = nearest(xi.z - xj[u].z, pz, g.iprd[2]);
           const double rsq = dx * dx + dy * dy + dz * dz;
           const int t = ti * nt1 + (int)xj[u].w;
-          if (rsq < s_tab[T_CUTSQ * kNT + t]) {
+          const double chi = s_qhi[t];
+          if (rsq < chi && row_inside(rsq, chi, s_tab[T_CUTSQ * kNT + t], xi, xj[u], ent[u], g)) {
             const double r2inv = 1.0 / rsq;
             const double r6inv = r2inv * r2inv * r2inv;
             const double forcelj = r6inv * (s_tab[T_LJ1 * kNT + t] * r6inv - s_tab[T_LJ2 * kNT + t]);
@@ -559,12 +596,12 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
   constexpr bool FEW = NT <= 2;
   constexpr int NP = NT * (NT + 1) / 2;
   constexpr int NA = FEW ? NP : NT;  // sums per lane: type pairs, or the partner's types
-  __shared__ double s_cut[kNT];
+  __shared__ double s_chi[kNT];
   __shared__ double2 s_a[kNT], s_b[kNT];
   __shared__ double s_acc[FEW ? 2 * NP * 16 : 2 * kNT];
   const int cols = nt1 * nt1;
   for (int k = threadIdx.x; k < cols; k += blockDim.x) {
-    s_cut[k] = tab[T_CUTSQ * kNT + k];
+    s_chi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
     s_a[k] = make_double2(tab[T_A1 * kNT + k], tab[T_A2 * kNT + k]);
     s_b[k] = make_double2(tab[T_B1 * kNT + k], tab[T_B2 * kNT + k]);
   }
@@ -608,8 +645,10 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
         const double rsq = dx * dx + dy * dy + dz * dz;
         const int tj = (int)xj[q].w;
         const int t = ti * nt1 + tj;
-        if (rsq < s_cut[t]) {
-          const double a = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
+        const double chi = s_chi[t];
+        if (rsq < chi) {
+          double a = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
+          if (rsq >= chi * kInner) a = edge_factor(pair_rows(xi, xj[q], tab[T_CUTSQ * kNT + t], ent[q], g), gi, gj[q], dx, dy, dz);
           const double r2inv = 1.0 / rsq;
           const double r6inv = r2inv * r2inv * r2inv;
           const double ar8 = a * (r2inv * r6inv);
@@ -707,8 +746,7 @@ __device__ __forceinline__ void r_spline(const EamTab &et, T r, int &m, T &p) {
 }
 
 // Whether the pair (i, entry) lies inside cutsq, and its separation: from the
-// fixed-point mirror with the FP64 re-test within kQBand of the cutoff
-// (MIXED), or from the FP64 positions.
+// fixed-point mirror (MIXED) or the nearest image of the FP64 positions.
 template <bool MIXED>
 __device__ __forceinline__ bool eam_inside(const double4 &xi, const int4 &qi, int i, const double4 *__restrict__ x,
                                            const double4 &xj, const int4 &qj, const RepGeom &g, int ent, double cutsq,
@@ -721,18 +759,14 @@ __device__ __forceinline__ bool eam_inside(const double4 &xi, const int4 &qi, in
     rsq = dx * dx + dy * dy + dz * dz;
     if (rsq < cutsq * (1.0 - kQBand)) return true;
     if (!(rsq < cutsq * (1.0 + kQBand))) return false;
-    double sx, sy, sz;
-    shift_of((int)((unsigned)ent >> MDX_IDX_BITS), sx, sy, sz);
-    const double4 pi = x[i], pj = x[ent & MDX_IDX_MASK];
-    const double ex = pi.x - (pj.x + sx * g.prd[0]), ey = pi.y - (pj.y + sy * g.prd[1]),
-                 ez = pi.z - (pj.z + sz * g.prd[2]);
-    return ex * ex + ey * ey + ez * ez < cutsq;
+    return image_rsq(x[i], x[ent & MDX_IDX_MASK], (int)((unsigned)ent >> MDX_IDX_BITS), g) < cutsq;
   } else {
     dx = nearest(xi.x - xj.x, step[0], ip[0]);
     dy = nearest(xi.y - xj.y, step[1], ip[1]);
     dz = nearest(xi.z - xj.z, step[2], ip[2]);
     rsq = dx * dx + dy * dy + dz * dz;
-    return rsq < cutsq;
+    const double chi = cutsq * (1.0 + kQBand);
+    return rsq < chi && row_inside(rsq, chi, cutsq, xi, xj, ent, g);
   }
 }
 
@@ -953,7 +987,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, true> walk{lane};
-  const double rdr = et.rdr;
+  const double rdr = et.rdr, chi = et.cutsq * (1.0 + kQBand);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -979,13 +1013,15 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
-        if (rsq < et.cutsq) {
+        if (rsq < chi) {
           double r, ri, p;
           int m;
+          double gd = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
+          if (rsq >= chi * kInner) gd = edge_factor(pair_rows(xi, xj[q], et.cutsq, ent[q], g), gi, gj[q], dx, dy, dz);
           sqrt_and_inverse(rsq, r, ri);
           r_spline<double>(et, r, m, p);
           const double4 c = TL ? s_rd[m] : rhor[2 * m];
-          const double b = -((gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz) * ri;
+          const double b = -gd * ri;
           u += b * ((c.x * p + c.y) * p + c.z);
           if ((ent[q] & MDX_IDX_MASK) > i) {
             const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * (gi.w + gj[q].w) * rdr, gzr = gz1 * rdr, pp = p * p;
@@ -1053,6 +1089,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, true> walk{lane};
+  const double chi = et.cutsq * (1.0 + kQBand);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -1077,8 +1114,12 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
-        const double v = xi.w + xj[q].w;
-        if (rsq < et.cutsq && v != 0.0) {
+        double v = xi.w + xj[q].w;
+        if (rsq >= chi * kInner && rsq < chi) {
+          const PairRows in = pair_rows(xi, xj[q], et.cutsq, ent[q], g);
+          v = (in.here ? xi.w : 0.0) + (in.there ? xj[q].w : 0.0);
+        }
+        if (rsq < chi && v != 0.0) {
           double r, ri, p;
           int m;
           sqrt_and_inverse(rsq, r, ri);

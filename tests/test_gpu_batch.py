@@ -430,3 +430,67 @@ def test_build_kind_reports_the_shape_it_runs():
     b.lj_forces()
     assert b.get_launch(B.BK_BUILD) == shape
     b.close()
+
+
+def boundary_pairs(L, cut, want=240):
+    """Two-atom boxes whose atoms lie within a few ulps of `cut` apart through
+    a periodic face: positions [m, 2, 3], only pairs where x_i - (x_j + L),
+    x_j - (x_i - L) and the nearest image of x_i - x_j do not all decide alike."""
+    rng = np.random.default_rng(17)
+    out = []
+    while len(out) < want:
+        d = int(rng.integers(3))
+        x = np.tile(rng.uniform(1.0, 9.0, 3), (2, 1))
+        lowside = rng.uniform(0.0, 1.0)
+        high = L[d] + lowside - cut
+        x[0, d], x[1, d] = high + int(rng.integers(-3, 4)) * np.spacing(high), lowside
+        i, j = (0, 1) if rng.random() < 0.5 else (1, 0)
+        a = x[0, d] - (x[1, d] + L[d])
+        b = x[1, d] - (x[0, d] - L[d])
+        c = (x[0, d] - x[1, d]) - L[d]
+        if len({q * q < cut * cut for q in (a, b, c)}) > 1:
+            out.append(x[[i, j]])
+    return np.array(out)
+
+
+@pytest.mark.parametrize("skin", [0.0, 0.3])
+@pytest.mark.parametrize("tpa", [4, 16])
+def test_pairs_at_the_cutoff_through_a_periodic_face(skin, tpa):
+    """A pair is decided by the FP64 separation from the neighbour's image,
+    x_i - (x_j + shift), in each row by itself: forces, energies and parameter
+    gradients of pairs on the cutoff are the oracle's, in both precisions."""
+    L = np.array([11.3, 12.7, 13.9])
+    one = np.ones((2, 2))
+    rng = np.random.default_rng(1)
+    for style, cut in (("lj", 2.5), ("eam", 4.95)):
+        x = boundary_pairs(L, cut)
+        m = len(x)
+        x = x.reshape(-1, 3)
+        geo = ([2] * m, [[0, 0, 0]] * m, [L] * m, [[1, 1, 1]] * m, 1, np.ones(2 * m, np.int32))
+        ref = FR.Batch(*geo, x)
+        G = rng.normal(size=x.shape)
+        b = B.Batch(*geo)
+        b.set_positions(x)
+        b.skin(skin)
+        for kind in range(1, 7):
+            b.set_launch(kind, 256, tpa, 0)
+        if style == "lj":
+            args = (one, one, one * cut)
+            f_ref, e_ref = ref.lj_forces(*args)
+            g_ref = ref.lj_vjp(*args, G)
+            b.lj_init(*args)
+        else:
+            pot = W.synthetic_knots(64)
+            args = (pot["drho"], pot["dr"], cut, pot["frho"], pot["rhor"], pot["z2r"])
+            ref.eam_set(*args)
+            f_ref, e_ref = ref.eam_forces()[:2]
+            g_ref = ref.eam_vjp(G)
+            b.eam_init(*args)
+        for prec, ftol, etol in ((B.FP64, 1e-11, 1e-12), (B.MIXED, 1e-5, 1e-5)):
+            b.precision(prec)
+            f, e = b.lj_forces() if style == "lj" else b.eam_forces()
+            assert force_errors(f, f_ref)[0] <= ftol
+            assert np.max(np.abs(e - e_ref)) <= etol * np.max(np.abs(e_ref))
+            for gd, gr in zip(b.lj_vjp(G) if style == "lj" else b.eam_vjp(G), g_ref):
+                assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
+        b.close()
