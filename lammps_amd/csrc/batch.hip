@@ -62,11 +62,16 @@ struct RepGeom {
   int bin_off;
 };
 
-// A pair within kQBand of the cutoff (relative, on rsq), by the fixed-point or
-// the nearest-image separation, is tested again on the FP64 positions with its
-// image (image_rsq).  kInner: the band's lower end over its upper end.
+// Pairs at the cutoff are tested again on the FP64 positions with their image
+// (image_rsq).  By the fixed-point separations, those within kQBand of it
+// (relative, on rsq).  By the nearest-image separations of the FP64 passes,
+// those whose rsq has one of the two upper words h and h + 1 around cutsq,
+// h = edge_word(cutsq): at least 2^-21 of it on either side.  So one integer
+// difference says inside (negative), edge (0 or 1) or outside.
 constexpr double kQBand = 2e-6;
-constexpr double kInner = 1.0 - 2.0 * kQBand;
+__device__ __forceinline__ int edge_word(double cutsq) {
+  return __double2hiint(cutsq) - (static_cast<unsigned>(__double2loint(cutsq)) < 0x80000000u ? 1 : 0);
+}
 
 __device__ __forceinline__ int4 quantize_rep(const RepGeom &g, const double4 &p) {
   return make_int4((int)(unsigned)(long long)rint((p.x - g.lo[0]) * g.qscale[0]),
@@ -126,23 +131,6 @@ __device__ __forceinline__ double image_rsq(const double4 &a, const double4 &b, 
 }
 // the code under which b sees a's image
 __device__ __forceinline__ int reverse_code(int code) { return 26 - code; }
-
-// A pair's separation rsq lies below chi = cutsq (1 + kQBand): whether it lies
-// inside cutsq in the row of a.
-__device__ __forceinline__ bool row_inside(double rsq, double chi, double cutsq, const double4 &a, const double4 &b,
-                                           int ent, const RepGeom &g) {
-  return rsq < chi * kInner || image_rsq(a, b, (int)((unsigned)ent >> MDX_IDX_BITS), g) < cutsq;
-}
-// The same for a pass that takes a pair once, from one of its two rows: at the
-// cutoff the rounding of the two ghosts can put it into one row's sum only.
-struct PairRows {
-  bool here, there;  // inside in the row of a, in that of b
-};
-__device__ __forceinline__ PairRows pair_rows(const double4 &a, const double4 &b, double cutsq, int ent,
-                                              const RepGeom &g) {
-  const int code = (int)((unsigned)ent >> MDX_IDX_BITS);
-  return {image_rsq(a, b, code, g) < cutsq, image_rsq(b, a, reverse_code(code), g) < cutsq};
-}
 
 __device__ __forceinline__ int local_bin(const RepGeom &g, double x, int d) {
   int c = (int)floor((x - g.lo[d]) * g.bininv[d]);
@@ -459,11 +447,80 @@ struct RowWalk {
 // separation of a pair within half the box, in FP64: the nearest image
 // (periodic boxes are at least two cutoffs wide, so it is the list's)
 __device__ __forceinline__ double nearest(double d, double prd, double iprd) { return fma(-prd, rint(d * iprd), d); }
+__device__ __forceinline__ double nearest_rsq(const double4 &a, const double4 &b, const double (&prd)[3],
+                                              const double (&iprd)[3], double &dx, double &dy, double &dz) {
+  dx = nearest(a.x - b.x, prd[0], iprd[0]);
+  dy = nearest(a.y - b.y, prd[1], iprd[1]);
+  dz = nearest(a.z - b.z, prd[2], iprd[2]);
+  return dx * dx + dy * dy + dz * dz;
+}
 
-// (G_i - G_j) . del of a pair on the cutoff: each row's share if it is inside there
-__device__ __forceinline__ double edge_factor(const PairRows &in, const double4 &gi, const double4 &gj, double dx,
-                                              double dy, double dz) {
-  return (in.here ? gi.x * dx + gi.y * dy + gi.z * dz : 0.0) - (in.there ? gj.x * dx + gj.y * dy + gj.z * dz : 0.0);
+// A pair that may lie on the cutoff.  There the rounding of the two ghosts can
+// put it into one of its rows only: here() and there() decide for the row of
+// xi and for that of xj.
+struct EdgePair {
+  const int i, ent;
+  const double4 xi, xj;
+  const RepGeom &g;
+  double dx, dy, dz, rsq;
+  __device__ __forceinline__ bool on_edge(int h) const { return (unsigned)(__double2hiint(rsq) - h) < 2u; }
+  __device__ __forceinline__ bool first() const { return (ent & MDX_IDX_MASK) > i; }
+  __device__ __forceinline__ bool here(double cutsq) const { return image_rsq(xi, xj, code(), g) < cutsq; }
+  __device__ __forceinline__ bool there(double cutsq) const { return image_rsq(xj, xi, reverse_code(code()), g) < cutsq; }
+  __device__ __forceinline__ int code() const { return (int)((unsigned)ent >> MDX_IDX_BITS); }
+  // (G_i - G_j) . del, each row's share if the pair is inside there
+  __device__ __forceinline__ double factor(const double4 &gi, const double4 &gj, double cutsq) const {
+    return (here(cutsq) ? gi.x * dx + gi.y * dy + gi.z * dz : 0.0) -
+           (there(cutsq) ? gj.x * dx + gj.y * dy + gj.z * dz : 0.0);
+  }
+};
+
+// The FP64 passes leave a row's pairs on the cutoff's edge for after the loop
+// over it: the loop marks the trip (modulo 32) in a lane's mask, and
+// marked_trips visits every entry of the lane's marked trips.  In the loop the
+// test would hold registers for about one pair in 10^5 (lj gradient, two types:
+// 114 to over 128, which spills; eam pass B 76 to 92); for the same reason the
+// visit loads all it needs anew, from an index the compiler does not see through.
+struct EdgeMarks {
+  unsigned trips = 0, least = ~0u;
+  // where a pair lies: inside the cutoff for certain?  edge pairs are noted
+  __device__ __forceinline__ bool inside(double rsq, int h) {
+    const int u = __double2hiint(rsq) - h;
+    least = min(least, (unsigned)u);
+    return u < 0;
+  }
+  __device__ __forceinline__ void end_trip(int tpa, int k0) {
+    if (least < 2u) {
+      trips |= 1u << (k0 / (4 * tpa) % 32);
+      least = ~0u;
+    }
+  }
+};
+template <int TPA, bool QUAD, typename F>
+__device__ __forceinline__ void marked_trips(const RowWalk<TPA, QUAD> &walk, unsigned mask, int i,
+                                             const double4 *__restrict__ x, const int *__restrict__ rep,
+                                             const RepGeom *__restrict__ geom, const int *__restrict__ nbr,
+                                             const int *__restrict__ numneigh, int cap, F &&pair) {
+  asm volatile("" : "+v"(i));
+  const double4 xi = x[i];
+  const RepGeom &g = geom[rep[i]];
+  const int *row = nbr + (size_t)i * cap;
+  const int jn = numneigh[i];
+#pragma unroll 1
+  while (mask) {
+    const int trip = __ffs(mask) - 1;
+    mask &= mask - 1;
+#pragma unroll 1
+    for (int k0 = walk.first() + trip * 4 * TPA; k0 < jn; k0 += 32 * 4 * TPA)
+#pragma unroll 1
+      for (int u = 0; u < 4; u++) {
+        if (walk.at(k0, u) >= jn) continue;
+        const int ent = row[walk.at(k0, u)];
+        EdgePair e{i, ent, xi, gather_x(x, ent), g};
+        e.rsq = nearest_rsq(e.xi, e.xj, g.prd, g.iprd, e.dx, e.dy, e.dz);
+        pair(e);
+      }
+  }
 }
 
 // ---------------------------------------------------------------- lj/cut
@@ -480,13 +537,16 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
                                                const int *__restrict__ numneigh, int cap,
                                                const double *__restrict__ tab, ForceOut out) {
   __shared__ double s_tab[T_N * kNT];
-  __shared__ double s_qlo[MIXED ? kNT : 1], s_qhi[kNT];
+  __shared__ double s_qlo[MIXED ? kNT : 1], s_qhi[MIXED ? kNT : 1];
+  __shared__ int s_h[MIXED ? 1 : kNT];
   __shared__ float s_f[MIXED ? 4 * kNT : 1];
   for (int k = threadIdx.x; k < T_N * kNT; k += blockDim.x) s_tab[k] = tab[k];
-  for (int k = threadIdx.x; k < kNT; k += blockDim.x) s_qhi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
+  if (!MIXED)
+    for (int k = threadIdx.x; k < kNT; k += blockDim.x) s_h[k] = edge_word(tab[T_CUTSQ * kNT + k]);
   if (MIXED)
     for (int k = threadIdx.x; k < kNT; k += blockDim.x) {
       s_qlo[k] = tab[T_CUTSQ * kNT + k] * (1.0 - kQBand);
+      s_qhi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
       s_f[k] = (float)tab[T_LJ1 * kNT + k];
       s_f[kNT + k] = (float)tab[T_LJ2 * kNT + k];
       s_f[2 * kNT + k] = (float)tab[T_LJ3 * kNT + k];
@@ -544,6 +604,17 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
         }
       }
     } else {
+      auto add = [&](int t, double dx, double dy, double dz, double rsq) {
+        const double r2inv = 1.0 / rsq;
+        const double r6inv = r2inv * r2inv * r2inv;
+        const double forcelj = r6inv * (s_tab[T_LJ1 * kNT + t] * r6inv - s_tab[T_LJ2 * kNT + t]);
+        const double fpair = forcelj * r2inv;
+        fx += dx * fpair;
+        fy += dy * fpair;
+        fz += dz * fpair;
+        e += 0.5 * (r6inv * (s_tab[T_LJ3 * kNT + t] * r6inv - s_tab[T_LJ4 * kNT + t]));
+      };
+      EdgeMarks marks;
       for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
         int ent[4];
         double4 xj[4];
@@ -559,19 +630,15 @@ __global__ __launch_bounds__(1024) void k_b_lj(int n, int nt1, const double4 *__
                        dz = nearest(xi.z - xj[u].z, pz, g.iprd[2]);
           const double rsq = dx * dx + dy * dy + dz * dz;
           const int t = ti * nt1 + (int)xj[u].w;
-          const double chi = s_qhi[t];
-          if (rsq < chi && row_inside(rsq, chi, s_tab[T_CUTSQ * kNT + t], xi, xj[u], ent[u], g)) {
-            const double r2inv = 1.0 / rsq;
-            const double r6inv = r2inv * r2inv * r2inv;
-            const double forcelj = r6inv * (s_tab[T_LJ1 * kNT + t] * r6inv - s_tab[T_LJ2 * kNT + t]);
-            const double fpair = forcelj * r2inv;
-            fx += dx * fpair;
-            fy += dy * fpair;
-            fz += dz * fpair;
-            e += 0.5 * (r6inv * (s_tab[T_LJ3 * kNT + t] * r6inv - s_tab[T_LJ4 * kNT + t]));
-          }
+          if (marks.inside(rsq, s_h[t])) add(t, dx, dy, dz, rsq);
         }
+        marks.end_trip(TPA, k0);
       }
+      if (marks.trips)
+        marked_trips(walk, marks.trips, i, x, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+          const int t = ti * nt1 + (int)p.xj.w;
+          if (p.on_edge(s_h[t]) && p.here(s_tab[T_CUTSQ * kNT + t])) add(t, p.dx, p.dy, p.dz, p.rsq);
+        });
     }
     fx = gsum<TPA>(fx);
     fy = gsum<TPA>(fy);
@@ -596,12 +663,12 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
   constexpr bool FEW = NT <= 2;
   constexpr int NP = NT * (NT + 1) / 2;
   constexpr int NA = FEW ? NP : NT;  // sums per lane: type pairs, or the partner's types
-  __shared__ double s_chi[kNT];
+  __shared__ int s_h[kNT];
   __shared__ double2 s_a[kNT], s_b[kNT];
   __shared__ double s_acc[FEW ? 2 * NP * 16 : 2 * kNT];
   const int cols = nt1 * nt1;
   for (int k = threadIdx.x; k < cols; k += blockDim.x) {
-    s_chi[k] = tab[T_CUTSQ * kNT + k] * (1.0 + kQBand);
+    s_h[k] = edge_word(tab[T_CUTSQ * kNT + k]);
     s_a[k] = make_double2(tab[T_A1 * kNT + k], tab[T_A2 * kNT + k]);
     s_b[k] = make_double2(tab[T_B1 * kNT + k], tab[T_B2 * kNT + k]);
   }
@@ -624,6 +691,22 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
     const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
+    auto add = [&](int tj, double a, double rsq) {  // a: (G_i - G_j) . del
+      const int t = ti * nt1 + tj;
+      const double r2inv = 1.0 / rsq;
+      const double r6inv = r2inv * r2inv * r2inv;
+      const double ar8 = a * (r2inv * r6inv);
+      const double2 ca = s_a[t], cb = s_b[t];
+      const double de = ca.x * r6inv - ca.y, ds = cb.x * r6inv - cb.y;
+      const int slot = FEW ? ti + tj - 2 : tj - 1;  // (1,1), (1,2), (2,2), or the partner's type
+#pragma unroll
+      for (int c = 0; c < NA; c++)
+        if (NA == 1 || slot == c) {
+          ae[c] += ar8 * de;
+          as[c] += ar8 * ds;
+        }
+    };
+    EdgeMarks marks;
     for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4], gj[4];
@@ -644,26 +727,17 @@ __global__ __launch_bounds__(1024) void k_b_lj_vjp(int n, int nt1, const double4
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
         const int tj = (int)xj[q].w;
-        const int t = ti * nt1 + tj;
-        const double chi = s_chi[t];
-        if (rsq < chi) {
-          double a = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
-          if (rsq >= chi * kInner) a = edge_factor(pair_rows(xi, xj[q], tab[T_CUTSQ * kNT + t], ent[q], g), gi, gj[q], dx, dy, dz);
-          const double r2inv = 1.0 / rsq;
-          const double r6inv = r2inv * r2inv * r2inv;
-          const double ar8 = a * (r2inv * r6inv);
-          const double2 ca = s_a[t], cb = s_b[t];
-          const double de = ca.x * r6inv - ca.y, ds = cb.x * r6inv - cb.y;
-          const int slot = FEW ? ti + tj - 2 : tj - 1;  // (1,1), (1,2), (2,2), or the partner's type
-#pragma unroll
-          for (int c = 0; c < NA; c++)
-            if (NA == 1 || slot == c) {
-              ae[c] += ar8 * de;
-              as[c] += ar8 * ds;
-            }
-        }
+        if (marks.inside(rsq, s_h[ti * nt1 + tj]))
+          add(tj, (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz, rsq);
       }
+      marks.end_trip(TPA, k0);
     }
+    if (marks.trips)
+      marked_trips(walk, marks.trips, i, x, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+        const int tj = (int)p.xj.w, t = ti * nt1 + tj;
+        if (p.first() && p.on_edge(s_h[t]))
+          add(tj, p.factor(gin[p.i], gather_x(gin, p.ent), tab[T_CUTSQ * kNT + t]), p.rsq);
+      });
     if constexpr (!FEW) {
 #pragma unroll
       for (int c = 0; c < NA; c++)
@@ -745,29 +819,18 @@ __device__ __forceinline__ void r_spline(const EamTab &et, T r, int &m, T &p) {
   p = pp < (T)1 ? pp : (T)1;
 }
 
-// Whether the pair (i, entry) lies inside cutsq, and its separation: from the
-// fixed-point mirror (MIXED) or the nearest image of the FP64 positions.
-template <bool MIXED>
-__device__ __forceinline__ bool eam_inside(const double4 &xi, const int4 &qi, int i, const double4 *__restrict__ x,
-                                           const double4 &xj, const int4 &qj, const RepGeom &g, int ent, double cutsq,
-                                           const double (&step)[3], const double (&ip)[3], double &dx, double &dy,
-                                           double &dz, double &rsq) {
-  if constexpr (MIXED) {
-    dx = qsep(qi.x, qj.x, step[0]);
-    dy = qsep(qi.y, qj.y, step[1]);
-    dz = qsep(qi.z, qj.z, step[2]);
-    rsq = dx * dx + dy * dy + dz * dz;
-    if (rsq < cutsq * (1.0 - kQBand)) return true;
-    if (!(rsq < cutsq * (1.0 + kQBand))) return false;
-    return image_rsq(x[i], x[ent & MDX_IDX_MASK], (int)((unsigned)ent >> MDX_IDX_BITS), g) < cutsq;
-  } else {
-    dx = nearest(xi.x - xj.x, step[0], ip[0]);
-    dy = nearest(xi.y - xj.y, step[1], ip[1]);
-    dz = nearest(xi.z - xj.z, step[2], ip[2]);
-    rsq = dx * dx + dy * dy + dz * dz;
-    const double chi = cutsq * (1.0 + kQBand);
-    return rsq < chi && row_inside(rsq, chi, cutsq, xi, xj, ent, g);
-  }
+// Whether the pair (i, entry) lies inside cutsq, and its separation, from the
+// fixed-point mirror.
+__device__ __forceinline__ bool eam_inside(const int4 &qi, int i, const double4 *__restrict__ x, const int4 &qj,
+                                           const RepGeom &g, int ent, double cutsq, const double (&step)[3],
+                                           double &dx, double &dy, double &dz, double &rsq) {
+  dx = qsep(qi.x, qj.x, step[0]);
+  dy = qsep(qi.y, qj.y, step[1]);
+  dz = qsep(qi.z, qj.z, step[2]);
+  rsq = dx * dx + dy * dy + dz * dz;
+  if (rsq < cutsq * (1.0 - kQBand)) return true;
+  if (!(rsq < cutsq * (1.0 + kQBand))) return false;
+  return image_rsq(x[i], x[ent & MDX_IDX_MASK], (int)((unsigned)ent >> MDX_IDX_BITS), g) < cutsq;
 }
 
 template <bool MIXED, int TPA, bool TL>
@@ -791,6 +854,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, false> walk{lane};
+  const int h = edge_word(et.cutsq);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -807,34 +871,54 @@ __global__ __launch_bounds__(1024) void k_b_eam_rho(int n, const double4 *__rest
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double acc = 0.0;
-    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
-      int ent[4];
-      double4 xj[MIXED ? 1 : 4];
-      int4 qj[MIXED ? 4 : 1];
-      walk.read(row, k0, jn, i, ent);
+    if constexpr (MIXED) {
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
+        int ent[4];
+        int4 qj[4];
+        walk.read(row, k0, jn, i, ent);
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
-        else xj[u] = gather_x(x, ent[u]);
-      }
+        for (int u = 0; u < 4; u++) qj[u] = gather_q(xq, ent[u]);
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        double dx, dy, dz, rsq;
-        if (walk.at(k0, u) < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
-                                             step, ip, dx, dy, dz, rsq)) {
-          int m;
-          T p;
-          if constexpr (MIXED) {
+        for (int u = 0; u < 4; u++) {
+          double dx, dy, dz, rsq;
+          if (walk.at(k0, u) < jn && eam_inside(qi, i, x, qj[u], g, ent[u], et.cutsq, step, dx, dy, dz, rsq)) {
+            int m;
+            T p;
             (void)eam_index_mixed(rsq, et.rdr, et.nr, m, p);
-          } else {
-            double r, ri;
-            sqrt_and_inverse(rsq, r, ri);
-            r_spline<T>(et, r, m, p);
+            const V c = TL ? s_val[m] : tab[2 * m + 1];
+            acc += (double)(((c.x * p + c.y) * p + c.z) * p + c.w);
           }
-          const V c = TL ? s_val[m] : tab[2 * m + 1];
-          acc += (double)(((c.x * p + c.y) * p + c.z) * p + c.w);
         }
       }
+    } else {
+      auto add = [&](double rsq) {
+        int m;
+        double p, r, ri;
+        sqrt_and_inverse(rsq, r, ri);
+        r_spline<double>(et, r, m, p);
+        const V c = TL ? s_val[m] : tab[2 * m + 1];
+        acc += ((c.x * p + c.y) * p + c.z) * p + c.w;
+      };
+      EdgeMarks marks;
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
+        int ent[4];
+        double4 xj[4];
+        walk.read(row, k0, jn, i, ent);
+#pragma unroll
+        for (int u = 0; u < 4; u++) xj[u] = gather_x(x, ent[u]);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (walk.at(k0, u) >= jn) continue;
+          double dx, dy, dz;
+          const double rsq = nearest_rsq(xi, xj[u], step, ip, dx, dy, dz);
+          if (marks.inside(rsq, h)) add(rsq);
+        }
+        marks.end_trip(TPA, k0);
+      }
+      if (marks.trips)
+        marked_trips(walk, marks.trips, i, x, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+          if (p.on_edge(h) && p.here(et.cutsq)) add(p.rsq);
+        });
     }
     acc = gsum<TPA>(acc);
     if (lane == 0) {
@@ -880,6 +964,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, !MIXED> walk{lane};
+  const int h = edge_word(et.cutsq);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -897,48 +982,87 @@ __global__ __launch_bounds__(1024) void k_b_eam_force(int n, const double4 *__re
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
-    for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
-      int ent[4];
-      double4 xj[MIXED ? 1 : 4];
-      int4 qj[MIXED ? 4 : 1];
-      double fpj[4];
-      walk.read(row, k0, jn, i, ent);
+    if constexpr (MIXED) {
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
+        int ent[4];
+        int4 qj[4];
+        double fpj[4];
+        walk.read(row, k0, jn, i, ent);
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        if constexpr (MIXED) qj[u] = gather_q(xq, ent[u]);
-        else xj[u] = gather_x(x, ent[u]);
-        fpj[u] = gather_d(fp, ent[u]);
-      }
+        for (int u = 0; u < 4; u++) {
+          qj[u] = gather_q(xq, ent[u]);
+          fpj[u] = gather_d(fp, ent[u]);
+        }
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        double dx, dy, dz, rsq;
-        if (walk.at(k0, u) < jn && eam_inside<MIXED>(xi, qi, i, x, xj[MIXED ? 0 : u], qj[MIXED ? u : 0], g, ent[u], et.cutsq,
-                                             step, ip, dx, dy, dz, rsq)) {
-          int m;
-          T p, r, recip;
-          if constexpr (MIXED) {
+        for (int u = 0; u < 4; u++) {
+          double dx, dy, dz, rsq;
+          if (walk.at(k0, u) < jn && eam_inside(qi, i, x, qj[u], g, ent[u], et.cutsq, step, dx, dy, dz, rsq)) {
+            int m;
+            T p, r, recip;
             r = eam_index_mixed(rsq, et.rdr, et.nr, m, p);
             recip = __builtin_amdgcn_rcpf(r);  // hardware reciprocal, 1 ulp
-          } else {
-            sqrt_and_inverse(rsq, r, recip);
-            r_spline<T>(et, r, m, p);
+            const V rd = TL ? s_tab[m] : rtab[2 * m];
+            const V zd = TL ? s_tab[kn + m] : ztab[2 * m];
+            const V zv = TL ? s_tab[2 * kn + m] : ztab[2 * m + 1];
+            const T rhop = (rd.x * p + rd.y) * p + rd.z;
+            const T z2p = (zd.x * p + zd.y) * p + zd.z;
+            const T z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
+            const T phi = z2 * recip;
+            const T phip = z2p * recip - phi * recip;
+            const T psip = (T)fpi * rhop + (T)fpj[u] * rhop + phip;
+            const double fpair = (double)(-psip * recip);
+            fx += dx * fpair;
+            fy += dy * fpair;
+            fz += dz * fpair;
+            e += 0.5 * (double)phi;
           }
-          const V rd = TL ? s_tab[m] : rtab[2 * m];
-          const V zd = TL ? s_tab[kn + m] : ztab[2 * m];
-          const V zv = TL ? s_tab[2 * kn + m] : ztab[2 * m + 1];
-          const T rhop = (rd.x * p + rd.y) * p + rd.z;
-          const T z2p = (zd.x * p + zd.y) * p + zd.z;
-          const T z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
-          const T phi = z2 * recip;
-          const T phip = z2p * recip - phi * recip;
-          const T psip = (T)fpi * rhop + (T)fpj[u] * rhop + phip;
-          const double fpair = (double)(-psip * recip);
-          fx += dx * fpair;
-          fy += dy * fpair;
-          fz += dz * fpair;
-          e += 0.5 * (double)phi;
         }
       }
+    } else {
+      auto add = [&](double fpj, double dx, double dy, double dz, double rsq) {
+        int m;
+        double p, r, recip;
+        sqrt_and_inverse(rsq, r, recip);
+        r_spline<double>(et, r, m, p);
+        const V rd = TL ? s_tab[m] : rtab[2 * m];
+        const V zd = TL ? s_tab[kn + m] : ztab[2 * m];
+        const V zv = TL ? s_tab[2 * kn + m] : ztab[2 * m + 1];
+        const double rhop = (rd.x * p + rd.y) * p + rd.z;
+        const double z2p = (zd.x * p + zd.y) * p + zd.z;
+        const double z2 = ((zv.x * p + zv.y) * p + zv.z) * p + zv.w;
+        const double phi = z2 * recip;
+        const double phip = z2p * recip - phi * recip;
+        const double psip = fpi * rhop + fpj * rhop + phip;
+        const double fpair = -psip * recip;
+        fx += dx * fpair;
+        fy += dy * fpair;
+        fz += dz * fpair;
+        e += 0.5 * phi;
+      };
+      EdgeMarks marks;
+      for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
+        int ent[4];
+        double4 xj[4];
+        double fpj[4];
+        walk.read(row, k0, jn, i, ent);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          xj[u] = gather_x(x, ent[u]);
+          fpj[u] = gather_d(fp, ent[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (walk.at(k0, u) >= jn) continue;
+          double dx, dy, dz;
+          const double rsq = nearest_rsq(xi, xj[u], step, ip, dx, dy, dz);
+          if (marks.inside(rsq, h)) add(fpj[u], dx, dy, dz, rsq);
+        }
+        marks.end_trip(TPA, k0);
+      }
+      if (marks.trips)
+        marked_trips(walk, marks.trips, i, x, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+          if (p.on_edge(h) && p.here(et.cutsq)) add(gather_d(fp, p.ent), p.dx, p.dy, p.dz, p.rsq);
+        });
     }
     fx = gsum<TPA>(fx);
     fy = gsum<TPA>(fy);
@@ -987,7 +1111,8 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, true> walk{lane};
-  const double rdr = et.rdr, chi = et.cutsq * (1.0 + kQBand);
+  const double rdr = et.rdr;
+  const int h = edge_word(et.cutsq);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -998,6 +1123,27 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
     double u = 0.0;
+    auto add = [&](bool once, double gd, double fpsum, double rsq) {  // gd: (G_i - G_j) . del
+      double r, ri, p;
+      int m;
+      sqrt_and_inverse(rsq, r, ri);
+      r_spline<double>(et, r, m, p);
+      const double4 c = TL ? s_rd[m] : rhor[2 * m];
+      const double b = -gd * ri;
+      u += b * ((c.x * p + c.y) * p + c.z);
+      if (once) {
+        const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * fpsum * rdr, gzr = gz1 * rdr, pp = p * p;
+        double *a = mine + m;
+        atomicAdd(a, 3.0 * pp * gzr + gz0 * pp * p);
+        atomicAdd(a + kn, 2.0 * p * gzr + gz0 * pp);
+        atomicAdd(a + 2 * kn, gzr + gz0 * p);
+        atomicAdd(a + 3 * kn, gz0);
+        atomicAdd(a + 4 * kn, 3.0 * pp * grp);
+        atomicAdd(a + 5 * kn, 2.0 * p * grp);
+        atomicAdd(a + 6 * kn, grp);
+      }
+    };
+    EdgeMarks marks;
     for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4], gj[4];
@@ -1013,30 +1159,18 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_a(int n, const double4 *__re
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
-        if (rsq < chi) {
-          double r, ri, p;
-          int m;
-          double gd = (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz;
-          if (rsq >= chi * kInner) gd = edge_factor(pair_rows(xi, xj[q], et.cutsq, ent[q], g), gi, gj[q], dx, dy, dz);
-          sqrt_and_inverse(rsq, r, ri);
-          r_spline<double>(et, r, m, p);
-          const double4 c = TL ? s_rd[m] : rhor[2 * m];
-          const double b = -gd * ri;
-          u += b * ((c.x * p + c.y) * p + c.z);
-          if ((ent[q] & MDX_IDX_MASK) > i) {
-            const double gz1 = b * ri, gz0 = -gz1 * ri, grp = b * (gi.w + gj[q].w) * rdr, gzr = gz1 * rdr, pp = p * p;
-            double *a = mine + m;
-            atomicAdd(a, 3.0 * pp * gzr + gz0 * pp * p);
-            atomicAdd(a + kn, 2.0 * p * gzr + gz0 * pp);
-            atomicAdd(a + 2 * kn, gzr + gz0 * p);
-            atomicAdd(a + 3 * kn, gz0);
-            atomicAdd(a + 4 * kn, 3.0 * pp * grp);
-            atomicAdd(a + 5 * kn, 2.0 * p * grp);
-            atomicAdd(a + 6 * kn, grp);
-          }
-        }
+        if (marks.inside(rsq, h))
+          add((ent[q] & MDX_IDX_MASK) > i, (gi.x - gj[q].x) * dx + (gi.y - gj[q].y) * dy + (gi.z - gj[q].z) * dz,
+              gi.w + gj[q].w, rsq);
       }
+      marks.end_trip(TPA, k0);
     }
+    if (marks.trips)
+      marked_trips(walk, marks.trips, i, x, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+        if (!p.on_edge(h)) return;
+        const double4 ga = gin[p.i], gb = gather_x(gin, p.ent);
+        add(p.first(), p.factor(ga, gb, et.cutsq), ga.w + gb.w, p.rsq);
+      });
     u = gsum<TPA>(u);
     if (lane == 0) {
       // fp = F'(rho_i): dL/dF'(rho_i) = u, dL/drho_i = u F''(rho_i)
@@ -1089,7 +1223,7 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
   const int b0 = chunk_begin(n, apb, &end);
   const int lane = threadIdx.x % TPA;
   const RowWalk<TPA, true> walk{lane};
-  const double chi = et.cutsq * (1.0 + kQBand);
+  const int h = edge_word(et.cutsq);
   for (int base = b0; base < end; base += apb) {
     const int i = base + threadIdx.x / TPA;
     if (i >= end) continue;
@@ -1098,6 +1232,18 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
     const double px = g.prd[0], py = g.prd[1], pz = g.prd[2], ix = g.iprd[0], iy = g.iprd[1], iz = g.iprd[2];
     const int *row = nbr + (size_t)i * cap;
     const int jn = numneigh[i];
+    auto add = [&](double v, double rsq) {  // v: dL/drho of both atoms
+      double r, ri, p;
+      int m;
+      sqrt_and_inverse(rsq, r, ri);
+      r_spline<double>(et, r, m, p);
+      double *a = mine + m;
+      atomicAdd(a, v * p * p * p);
+      atomicAdd(a + kn, v * p * p);
+      atomicAdd(a + 2 * kn, v * p);
+      atomicAdd(a + 3 * kn, v);
+    };
+    EdgeMarks marks;
     for (int k0 = walk.first(); k0 < jn; k0 += 4 * TPA) {
       int ent[4];
       double4 xj[4];
@@ -1114,24 +1260,17 @@ __global__ __launch_bounds__(1024) void k_b_eam_adj_b(int n, const double4 *__re
         const double dx = nearest(xi.x - xj[q].x, px, ix), dy = nearest(xi.y - xj[q].y, py, iy),
                      dz = nearest(xi.z - xj[q].z, pz, iz);
         const double rsq = dx * dx + dy * dy + dz * dz;
-        double v = xi.w + xj[q].w;
-        if (rsq >= chi * kInner && rsq < chi) {
-          const PairRows in = pair_rows(xi, xj[q], et.cutsq, ent[q], g);
-          v = (in.here ? xi.w : 0.0) + (in.there ? xj[q].w : 0.0);
-        }
-        if (rsq < chi && v != 0.0) {
-          double r, ri, p;
-          int m;
-          sqrt_and_inverse(rsq, r, ri);
-          r_spline<double>(et, r, m, p);
-          double *a = mine + m;
-          atomicAdd(a, v * p * p * p);
-          atomicAdd(a + kn, v * p * p);
-          atomicAdd(a + 2 * kn, v * p);
-          atomicAdd(a + 3 * kn, v);
-        }
+        const double v = xi.w + xj[q].w;
+        if (marks.inside(rsq, h) && v != 0.0) add(v, rsq);
       }
+      marks.end_trip(TPA, k0);
     }
+    if (marks.trips)
+      marked_trips(walk, marks.trips, i, xv, rep, geom, nbr, numneigh, cap, [&](const EdgePair &p) {
+        if (!p.first() || !p.on_edge(h)) return;
+        const double v = (p.here(et.cutsq) ? p.xi.w : 0.0) + (p.there(et.cutsq) ? p.xj.w : 0.0);
+        if (v != 0.0) add(v, p.rsq);
+      });
   }
   __syncthreads();
   double *out = partials + (size_t)blockIdx.x * 4 * kn;

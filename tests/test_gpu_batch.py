@@ -494,3 +494,54 @@ def test_pairs_at_the_cutoff_through_a_periodic_face(skin, tpa):
             for gd, gr in zip(b.lj_vjp(G) if style == "lj" else b.eam_vjp(G), g_ref):
                 assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
         b.close()
+
+
+@pytest.mark.parametrize("tpa", [1, 4, 64])
+def test_pairs_at_the_cutoff_in_long_rows(tpa):
+    """The same among other neighbours, in rows of up to 40 trips of one lane:
+    a jittered lattice of about 130 neighbours per atom with such pairs put in."""
+    rng = np.random.default_rng(6)
+    for style, cut, a, sigma in (("lj", 2.5, 0.78, 0.5), ("eam", 4.95, 1.56, None)):
+        L = np.round(np.array([15, 16, 18]) * a, 2)
+        ends = boundary_pairs(L, cut, 60)
+        n = np.floor(L / a).astype(int)
+        grid = np.stack(np.meshgrid(*[np.arange(q) for q in n], indexing="ij"), -1).reshape(-1, 3) * (L / n)
+        grid = np.mod(grid + rng.uniform(-0.1 * a, 0.1 * a, grid.shape), L)
+        taken = []
+        for pair in ends:  # pairs whose atoms keep apart
+            d = (pair[:, None] - np.array(taken).reshape(-1, 3)[None])
+            d -= L * np.round(d / L)
+            if not len(taken) or np.min(np.sum(d * d, -1)) > a * a:
+                taken.extend(pair)
+        taken = np.array(taken)
+        d = grid[:, None] - taken[None]
+        d -= L * np.round(d / L)
+        x = np.concatenate([grid[np.min(np.sum(d * d, -1), 1) > (0.7 * a) ** 2], taken])
+        x = x[rng.permutation(len(x))]
+        assert len(taken) >= 20
+        geo = ([len(x)], [[0, 0, 0]], [L], [[1, 1, 1]], 1, np.ones(len(x), np.int32))
+        ref = FR.Batch(*geo, x)
+        G = rng.normal(size=x.shape)
+        b = B.Batch(*geo)
+        b.set_positions(x)
+        b.skin(0.05 * cut)
+        for kind in range(1, 7):
+            b.set_launch(kind, 256, tpa, 0)
+        if style == "lj":
+            one = np.ones((2, 2))
+            args = (one, one * sigma, one * cut)
+            f_ref, g_ref = ref.lj_forces(*args)[0], ref.lj_vjp(*args, G)
+            b.lj_init(*args)
+            f, g = b.lj_forces()[0], b.lj_vjp(G)
+        else:
+            pot = W.synthetic_knots(64)
+            args = (pot["drho"], pot["dr"], cut, pot["frho"], pot["rhor"], pot["z2r"])
+            ref.eam_set(*args)
+            f_ref, g_ref = ref.eam_forces()[0], ref.eam_vjp(G)
+            b.eam_init(*args)
+            f, g = b.eam_forces()[0], b.eam_vjp(G)
+        assert b.neigh_stats()[1] > (128 if tpa == 1 else 4)
+        assert np.max(np.abs(f - f_ref)) <= 1e-11 * max(1.0, np.sqrt(np.mean(f_ref ** 2)))
+        for gd, gr in zip(g, g_ref):
+            assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
+        b.close()
