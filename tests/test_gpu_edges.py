@@ -773,3 +773,71 @@ def test_eam_tables_on_both_sides_of_the_lds_limits(prec, nr, tpa, tmp_path):
         np.testing.assert_allclose(out["eatom"], ea, rtol=0, atol=etol * np.abs(ea).max())
         np.testing.assert_allclose(out["vatom"], va, rtol=0, atol=etol * np.abs(va).max())
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1024, 1025, 97000])
+def test_moved_positions_are_computed_on_the_old_list(n):
+    """Positions handed over again after a move below half the skin, through
+    mapped memory, one staged piece and several: forces, per-atom energies and
+    virials are the oracle's at the new positions."""
+    from lammps_amd import mdx
+    rng = np.random.default_rng(n)
+    cells = int(np.ceil((n / 4.0) ** (1.0 / 3.0)))
+    lo, hi, x = mdx.lattice("fcc", 0.8442, "lj", (0, 0, 0), (cells,) * 3)
+    x = np.mod(x[rng.permutation(len(x))[:n]] + rng.uniform(-0.05, 0.05, (n, 3)), hi)
+    ctx = lj_context((0, 0, 0), hi, (1, 1, 1), x, mdx.FP64)
+    first = ctx.compute(3, 5, peratom=True)
+    builds = ctx.stats()["total_neighbors"]
+    moved = x + rng.uniform(-0.08, 0.08, x.shape)
+    ctx.set_positions(moved)
+    out = ctx.compute(3, 5, peratom=True)
+    assert ctx.stats()["total_neighbors"] == builds
+    ref = M.Ref(M.LJ)
+    ref.box((0, 0, 0), hi)
+    ref.add_atoms(np.mod(moved, hi), np.ones(n, dtype=np.int32))
+    ref.mass(1, 1.0)
+    ref.pair_lj(2.5)
+    ref.pair_coeff(1, 1, 1.0, 1.0, 2.5)
+    ref.neighbor(0.3)
+    ref.setup()
+    ref.compute(3, 5)
+    ea, va = ref.peratom()
+    f = ref.state()[2]
+    assert force_errors(first["f"], f)[0] > 1e-3  # the move changes the forces
+    assert force_errors(out["f"], f)[0] <= 1e-11
+    np.testing.assert_allclose(out["eatom"], ea, rtol=0, atol=1e-10 * np.abs(ea).max())
+    np.testing.assert_allclose(out["vatom"], va, rtol=0, atol=1e-10 * np.abs(va).max())
+    ctx.close()
+
+
+@pytest.mark.parametrize("style,ntypes", [("lj", 1), ("lj", 2), ("eam", 1)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_mixed_forces_have_the_same_bits_at_four_and_eight_lanes(style, ntypes, fmt):
+    """The default takes four lanes per atom above 40,000 atoms and eight
+    below: a mixed trajectory must not depend on which."""
+    from gpu_helpers import CU_U3
+    from lammps_amd import mdx
+    rng = np.random.default_rng(ntypes)
+    ctx = mdx.Context(0)
+    if style == "lj":
+        lo, hi, x = mdx.lattice("fcc", 0.8442, "lj", (0, 0, 0), (11, 12, 10))
+        x = np.mod(x + rng.uniform(-0.1, 0.1, x.shape), hi)[:-3]
+        ctx.set_box((0, 0, 0), hi, (1, 1, 1))
+        ctx.set_atoms(x, rng.integers(1, ntypes + 1, len(x)).astype(np.int32), np.ones(ntypes + 1))
+        ctx.pair_lj_from_coeffs(ntypes, {(1, 1): (1.0, 1.0, 2.5), (ntypes, ntypes): (0.5, 0.88, 2.2)})
+        ctx.neigh_modify(0.3)
+    else:
+        lo, hi, x = copper((9, 10, 8), 5)
+        ctx.set_box((0, 0, 0), hi, (1, 1, 1))
+        ctx.set_atoms(x[:-3], np.ones(len(x) - 3, dtype=np.int32), np.array([0.0, 63.55]))
+        mdx.eam_context_tables(ctx, CU_U3)
+        ctx.neigh_modify(1.0)
+    ctx.position_format(fmt)
+    ctx.precision(mdx.MIXED)
+    got = []
+    for tpa in (4, 8):
+        ctx.set_launch(256, tpa)
+        got.append([ctx.compute(0, 0)["f"]] + (list(ctx.eam_rho_fp()) if style == "eam" else []))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    ctx.close()
