@@ -11,9 +11,11 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <limits>
 #include <thread>
 #include <vector>
 #include "mdx_internal.h"
+#include "piece_gate.h"
 
 namespace mdx {
 
@@ -399,16 +401,16 @@ int download(mdx_ctx *c, const Seg *segs, int nseg) {
         (void)hipStreamSynchronize(c->stream);
         return hip_fail(e, "download");
       }
-    std::vector<std::atomic<int>> state(last - first);  // 1: in the stage, 2: failed
+    constexpr int kFailed = std::numeric_limits<int>::max();
+    PieceGate gate;
     on_threads(total, [&](int t, int nt) {
       for (size_t k = first; k < last; k++) {
+        const int piece = (int)(k - first);
         if (t == 0) {
-          if (e == hipSuccess) e = hipEventSynchronize(c->stage_ev[k - first]);
-          state[k - first].store(e == hipSuccess ? 1 : 2, std::memory_order_release);
+          e = hipEventSynchronize(c->stage_ev[piece]);
+          gate.raise(e == hipSuccess ? piece + 1 : kFailed);
         }
-        int st;
-        while (!(st = state[k - first].load(std::memory_order_acquire))) std::this_thread::yield();
-        if (st == 2) return;
+        if (gate.wait(piece) == kFailed) return;
         size_t a, b;
         slice(v[k].len, t, nt, a, b);
         if (v[k].add)

@@ -107,3 +107,13 @@ def test_rows_of_bins_stay_in_range_for_atoms_outside_the_box(build_dir):
     _run(["g++", "-std=c++17"] + SAN + ["-I" + os.path.join(ROOT, "lammps_amd", "csrc"),
                                         os.path.join(HERE, "sanitize", "bin_row_checks.cpp"), "-o", exe])
     _run([exe], env=ENV, timeout=60)
+
+
+def test_threads_waiting_for_a_transfer_sleep(build_dir):
+    """The wait of the copy threads (lammps_amd/csrc/piece_gate.h), also under ThreadSanitizer."""
+    src = os.path.join(HERE, "sanitize", "piece_gate_checks.cpp")
+    inc = "-I" + os.path.join(ROOT, "lammps_amd", "csrc")
+    for name, san in (("address", SAN), ("thread", ["-fsanitize=thread", "-g", "-O1"])):
+        exe = os.path.join(build_dir, "piece_gate_" + name)
+        _run(["g++", "-std=c++17"] + san + [inc, src, "-o", exe, "-lpthread"])
+        _run([exe], env=ENV, timeout=120)
