@@ -121,9 +121,10 @@ __device__ __forceinline__ void shift_of(int code, double &sx, double &sy, doubl
   sz = (double)(code % 3 - 1);
 }
 
-// the squared distance from a to the ghost of b under an image code, as the
-// reference forms it
+// the squared distance from a to the ghost of b under an image code, rounded as
+// the reference rounds it (every product and sum)
 __device__ __forceinline__ double image_rsq(const double4 &a, const double4 &b, int code, const RepGeom &g) {
+#pragma clang fp contract(off)
   double sx, sy, sz;
   shift_of(code, sx, sy, sz);
   const double ex = a.x - (b.x + sx * g.prd[0]), ey = a.y - (b.y + sy * g.prd[1]), ez = a.z - (b.z + sz * g.prd[2]);

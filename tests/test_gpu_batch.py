@@ -545,3 +545,37 @@ def test_pairs_at_the_cutoff_in_long_rows(tpa):
         for gd, gr in zip(g, g_ref):
             assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
         b.close()
+
+
+@pytest.mark.parametrize("shell", [(1, 2, 0), (1, 1, 1), (2, 1, 1), (2, 2, 1)])
+@pytest.mark.parametrize("skin", [0.0, 0.2])
+def test_lattice_shell_at_the_cutoff(shell, skin):
+    """A perfect simple-cubic lattice whose spacing is no exact fraction, the
+    cutoff on one of its shells: each of thousands of ties is decided as the
+    oracle's FP64 rounding of every product and sum decides it."""
+    a = 1.1
+    n = 8
+    grid = np.stack(np.meshgrid(*(np.arange(n),) * 3, indexing="ij"), -1).reshape(-1, 3) * a
+    cut = float(np.sqrt(np.sum((np.array(shell) * a) ** 2)))
+    L = n * a
+    geo = ([len(grid)] * 2, [[0, 0, 0]] * 2, [[L, L, L]] * 2, [[1, 1, 1], [0, 0, 0]], 1, np.ones(2 * len(grid), np.int32))
+    x = np.concatenate([grid, grid])
+    one = np.ones((2, 2))
+    args = (one, one, one * cut)
+    ref = FR.Batch(*geo, x)
+    G = np.random.default_rng(3).normal(size=x.shape)
+    f_ref, e_ref = ref.lj_forces(*args)
+    g_ref = ref.lj_vjp(*args, G)
+    b = B.Batch(*geo)
+    b.set_positions(x)
+    b.skin(skin)
+    b.lj_init(*args)
+    for prec, ftol in ((B.FP64, 1e-11), (B.MIXED, 1e-5)):
+        b.precision(prec)
+        f, e = b.lj_forces()
+        scale = 24.0 * (2.0 / a ** 13 - 1.0 / a ** 7)  # a nearest pair's force: the lattice's cancel
+        assert np.max(np.abs(f - f_ref)) <= ftol * scale
+        assert np.max(np.abs(e - e_ref)) <= (1e-12 if prec == B.FP64 else 1e-5) * np.max(np.abs(e_ref))
+        for gd, gr in zip(b.lj_vjp(G), g_ref):
+            assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
+    b.close()
