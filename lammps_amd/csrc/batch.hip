@@ -1753,7 +1753,8 @@ int build(mdx_batch *b) {
   const float c_lo = (float)(cutneighsq * (1.0 - kBuildBand)), c_hi = (float)(cutneighsq * (1.0 + kBuildBand)),
               reach = (float)(cutneighsq * (1.0 + 1e-4));
   for (int attempt = 0; attempt < 4; attempt++) {
-    if (attempt > 0 && (e = hipMemsetAsync(b->dflags + kFlagInts, 0, sizeof(ListSlot) * kListSlots, b->stream)) != hipSuccess)
+    if (attempt > 0 &&
+        (e = hipMemsetAsync(b->dflags + kFlagInts, 0, sizeof(ListSlot) * kListSlots, b->stream)) != hipSuccess)
       return bfail(e, "build flags");
     auto launch = [&](const Tune &t) {
       const int G = t.grid;
@@ -1801,7 +1802,7 @@ ForceOut force_out(mdx_batch *b, double *f) {
 }
 
 // what follows a force pass: replica energies, the copy to a host force array,
-// and the one wait of the call
+// and the wait for both (the list build, when there was one, has waited for its flags)
 int force_results(mdx_batch *b, const ForceOut &out, double *f, double *energy) {
   if (energy)
     hipLaunchKernelGGL(k_b_rep_energy, dim3(b->nrep), dim3(256), 0, b->stream, b->eat, b->off_d, b->rep_host);
@@ -1985,7 +1986,8 @@ int mdx_batch_create(int device, int nrep, const int *natoms, const double *lo, 
   for (int r = 0; r < nrep; r++)
     for (int i = b->off[r]; i < b->off[r + 1]; i++) rep_c[i] = r;
   if ((rc = dalloc(&b->geom, nrep)) || (rc = dalloc(&b->off_d, nrep + 1)) || (rc = dalloc(&b->xin, 3 * (size_t)n)) ||
-      (rc = dalloc(&b->staging, std::max<size_t>(3 * (size_t)n, nrep))) || (rc = dalloc(&b->type_c, n)) || (rc = dalloc(&b->rep_c, n)) ||
+      (rc = dalloc(&b->staging, std::max<size_t>(3 * (size_t)n, nrep))) || (rc = dalloc(&b->type_c, n)) ||
+      (rc = dalloc(&b->rep_c, n)) ||
       (rc = dalloc(&b->xw, n)) || (rc = dalloc(&b->x, n)) || (rc = dalloc(&b->xq, n)) || (rc = dalloc(&b->eat, n)) ||
       (rc = dalloc(&b->g, n)) ||
       (rc = dalloc(&b->rep, n)) || (rc = dalloc(&b->orig, n)) || (rc = dalloc(&b->inv, n)) ||

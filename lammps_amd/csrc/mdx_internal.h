@@ -577,9 +577,9 @@ int compute_noalloc(mdx_ctx *c, int n, const double *x, const int *type, int efl
 // neighbour build (neigh.hip)
 int neigh_setup_grid(mdx_ctx *c);
 int neigh_build(mdx_ctx *c);
-// neigh_build in two halves: the launches (sort, list, an asynchronous copy
-// of the build flags to pinned memory), and the check of those flags, which
-// waits only for that copy.  finish sets *regrow when the list capacity was
+// neigh_build in two halves: the launches (sort, list, and the kernel that
+// writes the build flags to mapped memory, their serial last), and the check of
+// those flags, which waits only for that serial.  finish sets *regrow when the list capacity was
 // too small (the caller rebuilds with neigh_build, which regrows).
 int neigh_build_launch(mdx_ctx *c);
 int neigh_build_finish(mdx_ctx *c, bool *regrow);

@@ -9,9 +9,10 @@
 // grid (binsize = cutneigh/2, src/neighbor.cpp:1580-1620), and stably
 // sorted by bin (counting sort: arrival slots, then ranks by atom index)
 // so that every x-row of bins is one contiguous atom range.  One lane
-// per atom (32 lanes in systems too small to fill the chip that way) then scans the 5x5 rows of its stencil (each row at most 3
-// contiguous segments: wrapped-low, main, wrapped-high; k_build_flat takes
-// them a plane at a time as one candidate stream) and keeps j iff
+// per atom (32 lanes in systems too small to fill the chip that way) then
+// scans the 5x5 rows of its stencil (each row at most 3 contiguous segments:
+// wrapped-low, main, wrapped-high; k_build_flat takes them a plane at a time
+// as one candidate stream) and keeps j iff
 // rsq <= cutneighsq, with the rsq the reference computes for a ghost atom:
 // FP64 without contraction on the periodic image x_j + s*L
 // (atom_vec_atomic.cpp:290-297), decided first on the fixed-point mirror in
@@ -154,8 +155,8 @@ __device__ __forceinline__ void stage_band(const NeighArgs &a, float *lo, float 
   }
 }
 
-// The list pass's counters into the build flags, and the flags into pinned
-// host memory (in place of a copy): one workgroup, one slot per thread.
+// The list pass's counters into the build flags, and the flags into mapped
+// host memory: one workgroup, one slot per thread.
 __global__ __launch_bounds__(kListSlots) void k_build_flags(int *__restrict__ dflags, int *__restrict__ host,
                                                              int serial) {
   __shared__ int s_most[kListSlots / 64];
@@ -1252,8 +1253,8 @@ int alloc_list(mdx_ctx *c, int cap) {
 int launch_list(mdx_ctx *c, bool again);
 
 // The launches of a build: pbc wrap + bins, the stable counting sort, the
-// permutation and the list (capacity maxneigh), then the build flags copied
-// into pinned memory behind them.
+// permutation and the list (capacity maxneigh), then the build flags written
+// to mapped memory behind them.
 int neigh_build_launch(mdx_ctx *c) {
   NeighArgs &a = c->na;
   a.n = c->n;
@@ -1333,8 +1334,8 @@ int neigh_build_launch(mdx_ctx *c) {
   return launch_list(c, false);
 }
 
-// the list pass of a build (the atoms are sorted), with its flags copied
-// into pinned memory behind it; `again`: a repeat after a regrow, whose
+// the list pass of a build (the atoms are sorted), with its flags written to
+// mapped memory behind it; `again`: a repeat after a regrow, whose
 // list flags are cleared first
 int launch_list(mdx_ctx *c, bool again) {
   NeighArgs &a = c->na;

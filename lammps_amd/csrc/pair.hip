@@ -391,92 +391,96 @@ __global__ MDX_PAIR_BOUNDS void k_lj(int n, int npad, int cap, int nt1, double p
     if (AHEAD && 4 * lane < jn) pre = nb4[(size_t)lane * npad];
     for (int kt = TRANS ? 0 : 4 * lane; kt < jn; kt += NS * U * TPA) {
 #pragma unroll
-    for (int h = 0; h < NS; h++) {  // trip h of NS adds into set h
-      const int k0 = kt + h * U * TPA;
-      if (h > 0 && k0 >= jn) break;
-      int jc[U];
-      double4 xj[Q ? 1 : U];
-      int4 qj[Q ? U : 1];
-      if constexpr (TRANS) {
-        int ev[4] = {self, self, self, self};
-        if (k0 + 4 * lane < jn) {  // chunks past the row may lie past the list's capacity
-          const int4 e4 = nb4[(size_t)((k0 >> 2) + lane) * npad];
-          ev[0] = e4.x;
-          ev[1] = e4.y;
-          ev[2] = e4.z;
-          ev[3] = e4.w;
-        }
-        quad_transpose(ev, lane);
-#pragma unroll
-        for (int u = 0; u < U; u++) jc[u] = k0 + 4 * u + lane < jn ? ev[u] : self;
-      } else {
-        const int4 e4 = AHEAD ? pre : nb4[(size_t)(k0 >> 2) * npad];
-        const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-        for (int u = 0; u < U; u++) jc[u] = k0 + u < jn ? ev[u] : self;
-        if (AHEAD && k0 + U * TPA < jn) pre = nb4[(size_t)((k0 + U * TPA) >> 2) * npad];
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (Q) qj[u] = gather_q(xq, jc[u]);
-        else xj[Q ? 0 : u] = gather_x(x, jc[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        // entries carry image bits: test the index, not the sign
-        if ((TRANS ? k0 + 4 * u + lane : k0 + u) >= jn) continue;
-        double delx, dely, delz, rsq;
-        int t;
-        bool inside;
-        if (Q) {
-          delx = qdelta(qi.x, qj[u].x, qs.step[0]);
-          dely = qdelta(qi.y, qj[u].y, qs.step[1]);
-          delz = qdelta(qi.z, qj[u].z, qs.step[2]);
-          rsq = delx * delx + dely * dely + delz * delz;
-          t = ONE ? nt1 + 1 : row + qj[u].w;
-          inside = rsq < (HOIST ? o_clo : s_clo[t]);
-          if (!inside && rsq < (HOIST ? o_chi : s_chi[t])) {
-            double ex, ey, ez;
-            pair_delta(x[i], x[jc[u] & MDX_IDX_MASK], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
-            inside = ex * ex + ey * ey + ez * ez < (HOIST ? o_cut : s_cutsq[t]);
+      for (int h = 0; h < NS; h++) {  // trip h of NS adds into set h
+        const int k0 = kt + h * U * TPA;
+        if (h > 0 && k0 >= jn) break;
+        int jc[U];
+        double4 xj[Q ? 1 : U];
+        int4 qj[Q ? U : 1];
+        if constexpr (TRANS) {
+          int ev[4] = {self, self, self, self};
+          if (k0 + 4 * lane < jn) {  // chunks past the row may lie past the list's capacity
+            const int4 e4 = nb4[(size_t)((k0 >> 2) + lane) * npad];
+            ev[0] = e4.x;
+            ev[1] = e4.y;
+            ev[2] = e4.z;
+            ev[3] = e4.w;
           }
+          quad_transpose(ev, lane);
+#pragma unroll
+          for (int u = 0; u < U; u++) jc[u] = k0 + 4 * u + lane < jn ? ev[u] : self;
         } else {
-          pair_delta(xi, xj[Q ? 0 : u], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz);
-          rsq = delx * delx + dely * dely + delz * delz;
-          t = ONE ? nt1 + 1 : row + static_cast<int>(xj[Q ? 0 : u].w);
-          inside = rsq < (HOIST ? o_cut : s_cutsq[t]);
+          const int4 e4 = AHEAD ? pre : nb4[(size_t)(k0 >> 2) * npad];
+          const int ev[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+          for (int u = 0; u < U; u++) jc[u] = k0 + u < jn ? ev[u] : self;
+          if (AHEAD && k0 + U * TPA < jn) pre = nb4[(size_t)((k0 + U * TPA) >> 2) * npad];
         }
-        if (inside) {
-          double fpair, evdwl = 0.0;
-          if (MIXED) {
-            // hardware reciprocal (1 ulp): well inside the FP32 pair-math budget
-            const float r2inv = __builtin_amdgcn_rcpf((float)rsq);
-            const float r6inv = r2inv * r2inv * r2inv;
-            const float forcelj = r6inv * ((HOIST ? o_f1 : f_lj1[t]) * r6inv - (HOIST ? o_f2 : f_lj2[t]));
-            fpair = (double)(forcelj * r2inv);
-            if (EV) evdwl = HOIST ? (double)(r6inv * (one.f3 * r6inv - one.f4) - one.foff) : (double)(r6inv * (f_lj3[t] * r6inv - f_lj4[t]) - f_off[t]);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (Q) qj[u] = gather_q(xq, jc[u]);
+          else xj[Q ? 0 : u] = gather_x(x, jc[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          // entries carry image bits: test the index, not the sign
+          if ((TRANS ? k0 + 4 * u + lane : k0 + u) >= jn) continue;
+          double delx, dely, delz, rsq;
+          int t;
+          bool inside;
+          if (Q) {
+            delx = qdelta(qi.x, qj[u].x, qs.step[0]);
+            dely = qdelta(qi.y, qj[u].y, qs.step[1]);
+            delz = qdelta(qi.z, qj[u].z, qs.step[2]);
+            rsq = delx * delx + dely * dely + delz * delz;
+            t = ONE ? nt1 + 1 : row + qj[u].w;
+            inside = rsq < (HOIST ? o_clo : s_clo[t]);
+            if (!inside && rsq < (HOIST ? o_chi : s_chi[t])) {
+              double ex, ey, ez;
+              pair_delta(x[i], x[jc[u] & MDX_IDX_MASK], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, ex, ey, ez);
+              inside = ex * ex + ey * ey + ez * ez < (HOIST ? o_cut : s_cutsq[t]);
+            }
           } else {
-            const double r2inv = 1.0 / rsq;
-            const double r6inv = r2inv * r2inv * r2inv;
-            const double forcelj = r6inv * ((HOIST ? o_lj1 : s_lj1[t]) * r6inv - (HOIST ? o_lj2 : s_lj2[t]));
-            fpair = forcelj * r2inv;
-            if (EV) evdwl = HOIST ? r6inv * (one.lj3 * r6inv - one.lj4) - one.off : r6inv * (s_lj3[t] * r6inv - s_lj4[t]) - s_off[t];
+            pair_delta(xi, xj[Q ? 0 : u], (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz);
+            rsq = delx * delx + dely * dely + delz * delz;
+            t = ONE ? nt1 + 1 : row + static_cast<int>(xj[Q ? 0 : u].w);
+            inside = rsq < (HOIST ? o_cut : s_cutsq[t]);
           }
-          fx[h] += delx * fpair;
-          fy[h] += dely * fpair;
-          fz[h] += delz * fpair;
-          if (EV) {
-            e += 0.5 * evdwl;
-            virial_entry(w, ig.pervir, (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz, fpair);
+          if (inside) {
+            double fpair, evdwl = 0.0;
+            if (MIXED) {
+              // hardware reciprocal (1 ulp): well inside the FP32 pair-math budget
+              const float r2inv = __builtin_amdgcn_rcpf((float)rsq);
+              const float r6inv = r2inv * r2inv * r2inv;
+              const float forcelj = r6inv * ((HOIST ? o_f1 : f_lj1[t]) * r6inv - (HOIST ? o_f2 : f_lj2[t]));
+              fpair = (double)(forcelj * r2inv);
+              if (EV)
+                evdwl = HOIST ? (double)(r6inv * (one.f3 * r6inv - one.f4) - one.foff)
+                              : (double)(r6inv * (f_lj3[t] * r6inv - f_lj4[t]) - f_off[t]);
+            } else {
+              const double r2inv = 1.0 / rsq;
+              const double r6inv = r2inv * r2inv * r2inv;
+              const double forcelj = r6inv * ((HOIST ? o_lj1 : s_lj1[t]) * r6inv - (HOIST ? o_lj2 : s_lj2[t]));
+              fpair = forcelj * r2inv;
+              if (EV)
+                evdwl = HOIST ? r6inv * (one.lj3 * r6inv - one.lj4) - one.off
+                              : r6inv * (s_lj3[t] * r6inv - s_lj4[t]) - s_off[t];
+            }
+            fx[h] += delx * fpair;
+            fy[h] += dely * fpair;
+            fz[h] += delz * fpair;
+            if (EV) {
+              e += 0.5 * evdwl;
+              virial_entry(w, ig.pervir, (unsigned)jc[u] >> MDX_IDX_BITS, px, py, pz, delx, dely, delz, fpair);
+            }
           }
         }
       }
-    }
     }
   }
   if (Q && i < n && lane == 0) xi = x[i];
-  finish_atom<TPA, EV, INTEG, kLateV, ACROSS>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
-                              partials);
+  finish_atom<TPA, EV, INTEG, kLateV, ACROSS>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy),
+                                              set_sum<NS>(fz), e, w, ig, vpre, hpre, f, partials);
 }
 
 // ------------------------------------------------------------------ EAM
@@ -734,8 +738,8 @@ __global__ MDX_EAM_BOUNDS(TL && !MIXED) void k_eam_force(int n, int npad, int ca
     if (EV && lane == 0) e += eemb[i];
   }
   if (Q && i < n && lane == 0) xi = x[i];
-  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e, w, ig, vpre, hpre, f,
-                              partials);
+  finish_atom<TPA, EV, INTEG, kLateV>(i, i < n && lane == 0, xi, set_sum<NS>(fx), set_sum<NS>(fy), set_sum<NS>(fz), e,
+                                      w, ig, vpre, hpre, f, partials);
 }
 
 // Resident wavefronts per SIMD of the fused force kernels, held by giving
@@ -823,18 +827,21 @@ void launch_eam_t(mdx_ctx *c, int B, const IntegArgs &ig) {
   ea.clo = ea.cutforcesq * (1.0 - kBand);
   ea.chi = ea.cutforcesq * (1.0 + kBand);
   prof_begin(c, MDX_K_EAM_RHO);
+  const size_t rho_bytes = TL ? kn * (MIXED ? sizeof(float4) : sizeof(double4)) : 0;
   hipLaunchKernelGGL((k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>), dim3(G), dim3(B),
-                     occupancy_lds(static_lds<k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>>(), B, TL ? kn * (MIXED ? sizeof(float4) : sizeof(double4)) : 0, 0), c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs,
-                     c->nbr, c->numneigh, c->rho, c->fp, c->eemb, c->xf, INTEG ? ig.gate : StepGate{});
+                     occupancy_lds(static_lds<k_eam_rho<MIXED, EV, TPA, Q, ONE, TL>>(), B, rho_bytes, 0), c->stream,
+                     c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs, c->nbr,
+                     c->numneigh, c->rho, c->fp, c->eemb, c->xf, INTEG ? ig.gate : StepGate{});
   prof_end(c);
   IntegArgs fi = ig;
   fi.gate.decided = nullptr;  // the density pass has told the host
   prof_begin(c, INTEG ? MDX_K_FUSED : MDX_K_EAM_FORCE);
   const size_t tl_bytes = TL ? kn * (MIXED ? 3 * sizeof(float4) : 5 * sizeof(double2)) : 0;
-  hipLaunchKernelGGL((k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>), dim3(G), dim3(B),
-                     INTEG ? occupancy_lds(static_lds<k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>>(), B, tl_bytes, 0) : tl_bytes, c->stream, c->n, c->npad, c->maxneigh, c->prd[0], c->prd[1],
-                     c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp, c->eemb, c->xf, c->f,
-                     c->partials, fi);
+  const size_t lds =
+      INTEG ? occupancy_lds(static_lds<k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>>(), B, tl_bytes, 0) : tl_bytes;
+  hipLaunchKernelGGL((k_eam_force<MIXED, EV, TPA, INTEG, Q, ONE, TL>), dim3(G), dim3(B), lds, c->stream, c->n, c->npad,
+                     c->maxneigh, c->prd[0], c->prd[1], c->prd[2], ea, c->x, c->xq, c->qs, c->nbr, c->numneigh, c->fp,
+                     c->eemb, c->xf, c->f, c->partials, fi);
   prof_end(c);
   c->last_grid = G;
 }
@@ -915,8 +922,9 @@ int dispatch_prec(mdx_ctx *c, int ev, const IntegArgs &ig) {
 //                   4,000       19.6 / 14.7 / 12.4 / 12.6
 //                  13,500       22.3 / 16.3 / 17.4 / 24.2
 //                 108,000         55 /   58 /   89 /  136
-// Mixed precision takes only 8 and 4, which give the same bits (split_sums):
-// a mixed trajectory amplifies any other difference to its own error.
+// By default mixed precision takes only 8 and 4, which give the same bits
+// (split_sums): a mixed trajectory amplifies any other difference to its own
+// error.  A shape that is set, or found by the autotuner, may be another.
 // Workgroups of one wavefront spread a small launch evenly over the CUs
 // (13,500 lj/cut atoms at 8 lanes: 64 threads 14% faster than 256); with 1024 or more
 // workgroups of 256 there is nothing to gain.  The single-type eam kernels
