@@ -161,6 +161,7 @@ __global__ void k_b_load(int n, const double *__restrict__ xin, const int *__res
     } else if (!(u >= g.lo[d] && u <= hi)) {
       atomicOr(&dflags[4], 1);  // outside a non-periodic box
     }
+    if (u != u) atomicOr(&dflags[7], 1);  // no place: the mirror would give it one
     v[d] = u;
   }
   xw[c] = make_double4(v[0], v[1], v[2], (double)type[c]);
@@ -1388,7 +1389,7 @@ struct mdx_batch {
   size_t scan_bytes = 0;
   int *nbr = nullptr, *numneigh = nullptr;
   int cap = 0;
-  int *dflags = nullptr;       // kFlagWords: [0] max count, [4] outside box, [8..9] u64 total
+  int *dflags = nullptr;       // kFlagWords: [0] max count, [4] outside box, [7] NaN, [8..9] u64 total
   int *flags_host = nullptr;   // mapped copy of the first kFlagInts
   int flag_serial = 0;         // list passes whose flags were asked for (kFlagSerial)
   bool mirror_ok = false;      // the fixed-point mirror can decide the list's candidates
@@ -1752,7 +1753,8 @@ int build(mdx_batch *b) {
   const double cutneighsq = cutneigh * cutneigh;
   const float c_lo = (float)(cutneighsq * (1.0 - kBuildBand)), c_hi = (float)(cutneighsq * (1.0 + kBuildBand)),
               reach = (float)(cutneighsq * (1.0 + 1e-4));
-  for (int attempt = 0; attempt < 4; attempt++) {
+  bool mirror = b->mirror_ok;
+  for (int attempt = 0; attempt < 5; attempt++) {
     if (attempt > 0 &&
         (e = hipMemsetAsync(b->dflags + kFlagInts, 0, sizeof(ListSlot) * kListSlots, b->stream)) != hipSuccess)
       return bfail(e, "build flags");
@@ -1762,7 +1764,7 @@ int build(mdx_batch *b) {
         BATCH_LAUNCH(kernel, G, kBuildBlock, 0, n, b->x, b->xq, b->rep, b->geom, b->bin_start, cutneighsq, c_lo, c_hi,
                      reach, b->cap, b->nbr, b->numneigh, reinterpret_cast<ListSlot *>(b->dflags + kFlagInts));
       };
-      if (b->mirror_ok) go(k_b_build<true>);
+      if (mirror) go(k_b_build<true>);
       else go(k_b_build<false>);
     };
     if ((rc = timed(b, MDX_BK_BUILD, build_tune(n), launch))) return rc;
@@ -1774,6 +1776,10 @@ int build(mdx_batch *b) {
     if (fl[4]) {
       set_error("an atom lies outside its replica's box in a non-periodic dimension");
       return MDX_ERR_ARG;
+    }
+    if (fl[7] && mirror) {  // a coordinate is not a number: FP64 candidates, which reject its pairs
+      mirror = false;
+      continue;
     }
     if (fl[0] <= b->cap) {
       unsigned long long tot;

@@ -579,3 +579,35 @@ def test_lattice_shell_at_the_cutoff(shell, skin):
         for gd, gr in zip(b.lj_vjp(G), g_ref):
             assert np.max(np.abs(gd - gr)) <= 1e-9 * np.max(np.abs(gr))
     b.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, -np.nan])
+@pytest.mark.parametrize("prec", [B.FP64, B.MIXED])
+def test_atom_without_a_place_touches_no_other(prec, bad):
+    """A coordinate that is not a number in a periodic box: the atom has no
+    neighbours, whatever the fixed-point mirror makes of it, and all other
+    atoms have the forces and gradients of the batch without it."""
+    natoms, lo, hi, per, t, x = ka_batch_inputs(2, 9)
+    n = natoms[0]
+    lost = int(np.argmin(np.sum(x[:n] ** 2, 1)))  # beside the box's corner, among neighbours
+    keep = np.delete(np.arange(2 * n), lost)
+    G = np.random.default_rng(2).normal(size=x.shape)
+    tab = ka_tables()
+    want = B.Batch([n - 1, n], lo, hi, per, 2, t[keep])
+    want.set_positions(x[keep])
+    got = B.Batch(natoms, lo, hi, per, 2, t)
+    broken = x.copy()
+    broken[lost, 1] = np.copysign(np.nan, 1.0 if not np.signbit(bad) else -1.0)
+    got.set_positions(broken)
+    out = []
+    for b, g in ((want, G[keep]), (got, G)):
+        b.precision(prec)
+        b.lj_init(*tab)
+        out.append((b.neigh_stats()[0], b.lj_forces(), b.lj_vjp(g)))
+        b.close()
+    assert out[0][0] == out[1][0]
+    assert not out[1][1][0][lost].any()
+    assert force_errors(out[1][1][0][keep], out[0][1][0])[0] <= 1e-12
+    assert np.max(np.abs(out[0][1][1] - out[1][1][1])) <= 1e-12 * np.max(np.abs(out[0][1][1]))
+    for a, c in zip(out[0][2], out[1][2]):
+        assert rel(c, a) <= 1e-12
