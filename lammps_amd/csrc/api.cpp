@@ -741,8 +741,7 @@ int mdx_run(mdx_ctx *c, int nsteps, double dt, double ftm2v, int thermo_every, m
     set_error("mdx_run: nsteps >= 0 and dt > 0 required");
     return MDX_ERR_ARG;
   }
-  // set up anew too after a step whose build failed: it left no list
-  if ((!c->run_setup_done || !c->built) && (rc = mdx_setup(c, cb, user))) return rc;
+  if (!c->run_setup_done && (rc = mdx_setup(c, cb, user))) return rc;
   const double dtv = dt, dtf = 0.5 * dt * ftm2v;
   const long last = c->ntimestep + nsteps;
   // Fused path: the force kernel of step n also runs fix nve's final

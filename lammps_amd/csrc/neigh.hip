@@ -1255,7 +1255,7 @@ int launch_list(mdx_ctx *c, bool again);
 // The launches of a build: pbc wrap + bins, the stable counting sort, the
 // permutation and the list (capacity maxneigh), then the build flags written
 // to mapped memory behind them.
-int neigh_build_launch(mdx_ctx *c) {
+static int launch_all(mdx_ctx *c) {
   NeighArgs &a = c->na;
   a.n = c->n;
   a.npad = c->npad;
@@ -1356,7 +1356,7 @@ int launch_list(mdx_ctx *c, bool again) {
 // Waits for the flags of the last list pass and checks them: errors as the
 // reference reports them, else *regrow when the largest row exceeded the
 // capacity (the capacity is grown here, the caller lists again).
-int neigh_build_finish(mdx_ctx *c, bool *regrow) {
+static int check_build(mdx_ctx *c, bool *regrow) {
   *regrow = false;
   if (c->n == 0) return MDX_OK;
   int serial;
@@ -1396,6 +1396,18 @@ int neigh_build_finish(mdx_ctx *c, bool *regrow) {
   return MDX_OK;
 }
 
+// A build that failed leaves no list: the next mdx_run sets up anew.
+int neigh_build_launch(mdx_ctx *c) {
+  const int rc = launch_all(c);
+  if (rc) c->run_setup_done = false;
+  return rc;
+}
+int neigh_build_finish(mdx_ctx *c, bool *regrow) {
+  const int rc = check_build(c, regrow);
+  if (rc) c->run_setup_done = false;
+  return rc;
+}
+
 // list build; regrow the per-atom capacity and list again on overflow
 int neigh_build(mdx_ctx *c) {
   int rc = neigh_build_launch(c);
@@ -1407,8 +1419,9 @@ int neigh_build(mdx_ctx *c) {
   }
   if (!rc && !c->built) {
     set_error("neighbour list capacity could not be grown to fit");
-    return MDX_ERR_OVERFLOW;
+    rc = MDX_ERR_OVERFLOW;
   }
+  if (rc) c->run_setup_done = false;
   return rc;
 }
 
