@@ -35,7 +35,8 @@ def fake(tmp_path_factory):
 
 @pytest.mark.parametrize("what", ["batch_lj", "batch_eam", "context_lj", "context_eam", "context_run"])
 def test_each_allocation_failing_once(fake, what):
-    env = dict(os.environ, LD_PRELOAD=fake, FAKE_HIP=fake, MDX_HIP_RUNTIME="rocm", PYTHONPATH=ROOT)
+    preload = " ".join(q for q in (fake, os.environ.get("LD_PRELOAD")) if q)
+    env = dict(os.environ, LD_PRELOAD=preload, FAKE_HIP=fake, MDX_HIP_RUNTIME="rocm", PYTHONPATH=ROOT)
     r = subprocess.run([sys.executable, os.path.abspath(__file__), what], capture_output=True, text=True, env=env,
                        timeout=300)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
